@@ -149,10 +149,10 @@ struct dh_ctx_s {
   size_t h_tables_n = 0;
   dh::Status* d_status_host = nullptr;  // device address of h_status
   DevBuf<uint32_t> export_buf;  // RGBA staging of dh_canvas_read_rgba
-  DevBuf<dh_gui_vertex> gui_vtx;  // GUI overlay draw list
-  DevBuf<uint4> gui_tri, gui_clip;
-  DevBuf<uint4> gui_rec;          // dh::kGuiRecBytes per triangle
-  DevBuf<uint32_t> gui_err;
+  DevBuf<uint4> gui_list, gui_rec;  // GUI overlay: draw list (dh::GuiLayout), dh::kGuiRecBytes per triangle
+  uint4* h_gui = nullptr;           // coherent pinned staging: an error word's 16 bytes, then the draw list
+  uint4* d_gui_host = nullptr;      // its device address
+  size_t h_gui_n = 0;               // uint4s
   uint64_t scratch_cap = 0;     // 0 = none; else frame scratch may not grow past it (DH_E_BUDGET)
   uint64_t scratch_need = 0;    // bytes the last frame refused by the cap asked for
   uint32_t cap_tri = 0, cap_pairs = 0;
@@ -177,6 +177,14 @@ struct dh_ctx_s {
 };
 
 namespace {
+
+void release_gui(dh_ctx c) {
+  c->gui_list.release();
+  c->gui_rec.release();
+  if (c->h_gui) hipHostFree(c->h_gui);
+  c->h_gui = c->d_gui_host = nullptr;
+  c->h_gui_n = 0;
+}
 
 int fail(dh_ctx c, int code, const std::string& msg) {
   if (c) c->err = msg;
@@ -395,7 +403,7 @@ extern "C" int dh_ctx_destroy(dh_ctx c) {
   c->tile_cnt.release(); c->tile_start.release();
   c->status.release(); c->tables.release(); c->draws = nullptr; c->views = nullptr; c->export_buf.release();
   c->tdraws.release(); c->grp.release(); c->tperm.release(); c->sort_n.release();
-  c->gui_vtx.release(); c->gui_tri.release(); c->gui_clip.release(); c->gui_rec.release(); c->gui_err.release();
+  release_gui(c);
   if (c->h_status) hipHostFree(c->h_status);
   if (c->h_tables) hipHostFree(c->h_tables);
   for (int i = 0; i < 5; i++)
@@ -1230,22 +1238,34 @@ extern "C" int dh_draw_gui(dh_ctx c, dh_handle canvas, const dh_gui_vertex* vtx,
   }
   if (tris.empty()) return DH_OK;
   HIPCHK(c, hipSetDevice(c->device));
-  HIPCHK(c, c->gui_vtx.ensure(n_vtx));
-  HIPCHK(c, c->gui_tri.ensure(tris.size()));
-  HIPCHK(c, c->gui_clip.ensure(clips.size()));
-  HIPCHK(c, c->gui_rec.ensure(tris.size() * (dh::kGuiRecBytes / sizeof(uint4))));
-  HIPCHK(c, c->gui_err.ensure(1));
-  HIPCHK(c, hipMemcpyAsync(c->gui_vtx.p, vtx, n_vtx * sizeof(dh_gui_vertex), hipMemcpyHostToDevice, c->stream));
-  HIPCHK(c, hipMemcpyAsync(c->gui_tri.p, tris.data(), tris.size() * sizeof(uint4), hipMemcpyHostToDevice, c->stream));
-  HIPCHK(c, hipMemcpyAsync(c->gui_clip.p, clips.data(), clips.size() * sizeof(uint4), hipMemcpyHostToDevice,
-                           c->stream));
-  HIPCHK(c, hipMemsetAsync(c->gui_err.p, 0, 4, c->stream));
-  HIPCHK(c, dh::enqueue_gui(c->gui_vtx.p, c->gui_tri.p, (uint32_t)tris.size(), c->gui_clip.p, c->gui_rec.p, cv.W,
-                            cv.H, ft.d, ft.w, ft.h, ft.comp, cv.bgra, cv.depth, c->gui_err.p, c->stream));
-  uint32_t err = 0;
-  HIPCHK(c, hipMemcpyAsync(&err, c->gui_err.p, 4, hipMemcpyDeviceToHost, c->stream));
+  // one buffer, written once into pinned memory and copied by the first kernel
+  dh::GuiLayout lay;
+  lay.clip = 0;
+  lay.tri = clips.size() * sizeof(uint4);
+  lay.vtx = lay.tri + tris.size() * sizeof(uint4);
+  lay.bytes = (lay.vtx + n_vtx * sizeof(dh_gui_vertex) + 15) & ~(size_t)15;
+  const size_t n16 = lay.bytes / sizeof(uint4);
+  HIPCHK(c, c->gui_list.ensure(n16));
+  HIPCHK(c, c->gui_rec.ensure((tris.size() * dh::kGuiRecBytes + 15) / sizeof(uint4)));
+  if (c->h_gui_n < n16 + 1) {
+    if (c->h_gui) hipHostFree(c->h_gui);
+    c->h_gui = c->d_gui_host = nullptr;
+    c->h_gui_n = 0;
+    HIPCHK(c, hipHostMalloc(reinterpret_cast<void**>(&c->h_gui), (n16 + 1) * sizeof(uint4), hipHostMallocCoherent));
+    HIPCHK(c, hipHostGetDevicePointer(reinterpret_cast<void**>(&c->d_gui_host), c->h_gui, 0));
+    c->h_gui_n = n16 + 1;
+  }
+  volatile uint32_t* const err = reinterpret_cast<volatile uint32_t*>(c->h_gui);
+  uint8_t* const list = reinterpret_cast<uint8_t*>(c->h_gui + 1);
+  *err = 0;
+  memcpy(list + lay.clip, clips.data(), clips.size() * sizeof(uint4));
+  memcpy(list + lay.tri, tris.data(), tris.size() * sizeof(uint4));
+  memcpy(list + lay.vtx, vtx, n_vtx * sizeof(dh_gui_vertex));
+  HIPCHK(c, dh::enqueue_gui(c->d_gui_host + 1, c->gui_list.p, lay, (uint32_t)tris.size(), c->gui_rec.p, cv.W, cv.H,
+                            ft.d, ft.w, ft.h, ft.comp, cv.bgra, cv.depth, reinterpret_cast<uint32_t*>(c->d_gui_host),
+                            c->stream));
   HIPCHK(c, hipStreamSynchronize(c->stream));
-  if (err) return fail(c, DH_E_TEXCOORD, "font sample outside the texture (get_rgba_slice would panic)");
+  if (*err) return fail(c, DH_E_TEXCOORD, "font sample outside the texture (get_rgba_slice would panic)");
   return DH_OK;
 }
 
@@ -1318,7 +1338,7 @@ void ctx_release_scratch(dh_ctx c) {
   c->tile_cnt.release(); c->tile_start.release();
   c->status.release(); c->tables.release(); c->draws = nullptr; c->views = nullptr; c->export_buf.release();
   c->tdraws.release(); c->grp.release(); c->tperm.release(); c->sort_n.release();
-  c->gui_vtx.release(); c->gui_tri.release(); c->gui_clip.release(); c->gui_rec.release(); c->gui_err.release();
+  release_gui(c);
   c->cap_tri = c->cap_pairs = 0;
 }
 }  // namespace dh

@@ -18,10 +18,18 @@ void ctx_set_scratch_cap(dh_ctx c, uint64_t cap);
 uint64_t ctx_scratch_need(dh_ctx c);
 int mesh_triangles(dh_ctx c, dh_handle mesh, uint32_t* n_tri);
 void ctx_release_scratch(dh_ctx c);
-hipError_t enqueue_gui(const dh_gui_vertex* vtx, const uint4* tris, uint32_t n_tri, const uint4* clips, void* recs,
-                       int W, int H, const uint8_t* font, int32_t fw, int32_t fh, int32_t fcomp, uint32_t* bgra,
-                       const float* depth, uint32_t* error, hipStream_t s);
-constexpr size_t kGuiRecBytes = 144;  // sizeof(GuiRec)
+// A GUI draw list in one buffer: byte offsets (multiples of 16) of its clip
+// rectangles, triangles and vertices, and its size (a multiple of 16).
+struct GuiLayout {
+  size_t clip, tri, vtx, bytes;
+};
+// src: the list in pinned host memory (its device address), copied to dst by
+// the first kernel; recs: kGuiRecBytes per triangle of scratch; *error (device
+// address of a pinned word) is set to 1 where a font sample leaves the image.
+hipError_t enqueue_gui(const uint4* src, uint4* dst, const GuiLayout& g, uint32_t n_tri, void* recs, int W, int H,
+                       const uint8_t* font, int32_t fw, int32_t fh, int32_t fcomp, uint32_t* bgra, const float* depth,
+                       uint32_t* error, hipStream_t s);
+constexpr size_t kGuiRecBytes = 152;  // a 144-byte record and an 8-byte scan rectangle
 hipError_t enqueue_bgra_to_rgba(const uint32_t* src, uint32_t* dst, uint32_t n, hipStream_t s);
 // The fixed RGBA staging array of dh_canvas_read_rgba_noalloc: at most
 // kRgbaScratchPixels pixels (one 3840x2160 frame, 31.6 MiB per device).
