@@ -107,7 +107,7 @@ struct dh_ctx_s {
   // a second stream (default priority) for independent kernels of a frame,
   // forked from and joined back to `stream` with these events
   hipStream_t side = nullptr;
-  hipEvent_t xev[4] = {nullptr, nullptr, nullptr, nullptr};
+  hipEvent_t xev[2] = {nullptr, nullptr};
   std::string err;
   std::shared_ptr<ResPool> res;
   // raster configuration
@@ -123,7 +123,7 @@ struct dh_ctx_s {
   DevBuf<dh::SetupRec> setup;
   DevBuf<dh::ShadeRec> shade;
   DevBuf<uint32_t> bincnt, binoff, big;
-  DevBuf<uint32_t> keys0, keys1, vals0, vals1;
+  DevBuf<uint32_t> keys, vals0, vals1;  // keys: 2 cap_pairs
   DevBuf<uint32_t> hist, partials;
   DevBuf<uint2> ranges;
   DevBuf<uint32_t> tile_cnt, tile_start;
@@ -247,10 +247,10 @@ size_t tables_bytes(uint64_t n_draws, uint64_t n_views) {
 uint64_t scratch_bytes_after(dh_ctx c, uint64_t n_in, uint64_t cap_tri, uint64_t cap_pairs, uint64_t n_tiles,
                              uint64_t n_pixels, uint64_t n_draws, uint64_t n_views) {
   auto mx = [](uint64_t have, uint64_t want) { return std::max<uint64_t>(have, std::max<uint64_t>(want, 1)); };
-  uint64_t b = mx(c->cnt.n, n_in) + 4 * mx(c->blk.n, 3 * ((n_in + 255) / 256 + 1)) + 4 * mx(c->surv.n, 2 * n_in);
+  uint64_t b = mx(c->cnt.n, n_in) + 4 * mx(c->blk.n, 3 * dh::geom_blk_stride((n_in + 255) / 256)) + 4 * mx(c->surv.n, 2 * n_in);
   b += (sizeof(dh::SetupRec) * mx(c->setup.n, cap_tri)) + sizeof(dh::ShadeRec) * mx(c->shade.n, cap_tri);
   b += 4 * (mx(c->bincnt.n, cap_tri) + mx(c->binoff.n, cap_tri) + mx(c->big.n, 3 * cap_tri + 4));
-  b += 4 * (mx(c->keys0.n, cap_pairs) + mx(c->keys1.n, cap_pairs) + mx(c->vals0.n, cap_pairs) + mx(c->vals1.n, cap_pairs));
+  b += 4 * (mx(c->keys.n, 2 * cap_pairs) + mx(c->vals0.n, cap_pairs) + mx(c->vals1.n, cap_pairs));
   b += 4 * (mx(c->hist.n, dh::kRadixHistEntries) + mx(c->partials.n, 1024)) + 8 * mx(c->ranges.n, n_tiles);
   b += 4 * (mx(c->tile_cnt.n, 2 * n_tiles) + mx(c->tile_start.n, n_tiles) + mx(c->vis.n, n_pixels));
   b += sizeof(dh::Status) * mx(c->status.n, 2) + mx(c->tables.n, tables_bytes(n_draws, n_views));
@@ -261,15 +261,14 @@ uint64_t scratch_bytes_after(dh_ctx c, uint64_t n_in, uint64_t cap_tri, uint64_t
 int ensure_scratch(dh_ctx c, uint32_t n_in, uint32_t cap_tri, uint32_t cap_pairs, uint32_t n_tiles,
                    uint32_t n_pixels, uint32_t n_draws, uint32_t n_views) {
   HIPCHK(c, c->cnt.ensure(n_in));
-  HIPCHK(c, c->blk.ensure(3ull * ((n_in + 255) / 256 + 1)));  // output, unclipped and clipped emitter counts
+  HIPCHK(c, c->blk.ensure(3ull * dh::geom_blk_stride((n_in + 255) / 256)));  // output, unclipped and clipped emitter counts
   HIPCHK(c, c->surv.ensure(2ull * n_in));
   HIPCHK(c, c->setup.ensure(cap_tri));
   HIPCHK(c, c->shade.ensure(cap_tri));
   HIPCHK(c, c->bincnt.ensure(cap_tri));
   HIPCHK(c, c->binoff.ensure(cap_tri));
   HIPCHK(c, c->big.ensure(3ull * cap_tri + 4));  // flag bytes, then 8-byte bin boxes (16-byte aligned)
-  HIPCHK(c, c->keys0.ensure(cap_pairs));
-  HIPCHK(c, c->keys1.ensure(cap_pairs));
+  HIPCHK(c, c->keys.ensure(2ull * cap_pairs));
   HIPCHK(c, c->vals0.ensure(cap_pairs));
   HIPCHK(c, c->vals1.ensure(cap_pairs));
   HIPCHK(c, c->hist.ensure(dh::kRadixHistEntries));
@@ -297,8 +296,8 @@ int ensure_scratch(dh_ctx c, uint32_t n_in, uint32_t cap_tri, uint32_t cap_pairs
     c->views = reinterpret_cast<dh::DevView*>(c->tables.p + c->tables_view_off);
   }
   c->cap_tri = (uint32_t)std::min<size_t>(c->setup.n, 0xFFFFFFF0u);
-  c->cap_pairs = (uint32_t)std::min<size_t>(c->keys0.n, 0xFFFFFFF0u);
-  // binning keeps the wide-triangle list (up to cap_tri entries) in keys[1]
+  c->cap_pairs = (uint32_t)std::min<size_t>(c->vals0.n, 0xFFFFFFF0u);
+  // binning keeps the wide-triangle list (up to cap_tri entries) in keys[1] or vals[1]
   if (c->cap_pairs < c->cap_tri) return fail(c, DH_E_CAPACITY, "bin buffers smaller than the triangle records");
   return DH_OK;
 }
@@ -337,7 +336,7 @@ int ctx_new(int32_t device, std::shared_ptr<ResPool> pool, dh_ctx* out) {
   hipError_t e = hipSetDevice(device);
   if (e == hipSuccess) e = hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking);
   if (e == hipSuccess) e = hipStreamCreateWithFlags(&c->side, hipStreamNonBlocking);
-  for (int i = 0; i < 4 && e == hipSuccess; i++) e = hipEventCreateWithFlags(&c->xev[i], hipEventDisableTiming);
+  for (int i = 0; i < 2 && e == hipSuccess; i++) e = hipEventCreateWithFlags(&c->xev[i], hipEventDisableTiming);
   // the frame's last kernel writes the status words here (coherent: no copy, no cache flush)
   if (e == hipSuccess)
     e = hipHostMalloc(reinterpret_cast<void**>(&c->h_status), 2 * sizeof(dh::Status), hipHostMallocCoherent);
@@ -398,7 +397,7 @@ extern "C" int dh_ctx_destroy(dh_ctx c) {
   if (c->graph) hipGraphDestroy(c->graph);
   c->cnt.release(); c->blk.release(); c->surv.release(); c->setup.release(); c->shade.release();
   c->bincnt.release(); c->binoff.release(); c->big.release();
-  c->keys0.release(); c->keys1.release(); c->vals0.release(); c->vals1.release();
+  c->keys.release(); c->vals0.release(); c->vals1.release();
   c->hist.release(); c->partials.release(); c->ranges.release(); c->vis.release();
   c->tile_cnt.release(); c->tile_start.release();
   c->status.release(); c->tables.release(); c->draws = nullptr; c->views = nullptr; c->export_buf.release();
@@ -408,7 +407,7 @@ extern "C" int dh_ctx_destroy(dh_ctx c) {
   if (c->h_tables) hipHostFree(c->h_tables);
   for (int i = 0; i < 5; i++)
     if (c->ev[i]) hipEventDestroy(c->ev[i]);
-  for (int i = 0; i < 4; i++)
+  for (int i = 0; i < 2; i++)
     if (c->xev[i]) hipEventDestroy(c->xev[i]);
   if (c->side) hipStreamDestroy(c->side);
   if (c->stream) hipStreamDestroy(c->stream);
@@ -827,8 +826,8 @@ dh::PipeArgs make_args(dh_ctx c, const dh::DevMaterial* mats, uint32_t n_in, uin
   a.tile_cnt = c->tile_cnt.p;
   a.tile_cur = c->tile_cnt.p + n_tiles;
   a.tile_start = c->tile_start.p;
-  a.keys[0] = c->keys0.p;
-  a.keys[1] = c->keys1.p;
+  a.keys[0] = c->keys.p;
+  a.keys[1] = c->keys.p + c->cap_pairs;
   a.vals[0] = c->vals0.p;
   a.vals[1] = c->vals1.p;
   a.cap_pairs = c->cap_pairs;
@@ -839,7 +838,7 @@ dh::PipeArgs make_args(dh_ctx c, const dh::DevMaterial* mats, uint32_t n_in, uin
   a.status = c->status.p;
   for (int i = 0; i < 5; i++) a.ev[i] = events ? c->ev[i] : nullptr;
   a.side = c->side;
-  for (int i = 0; i < 4; i++) a.xev[i] = c->xev[i];
+  for (int i = 0; i < 2; i++) a.xev[i] = c->xev[i];
   return a;
 }
 
@@ -912,7 +911,7 @@ int render_views(dh_ctx c, const dh_view* views, uint32_t n_views, bool use_grap
     // everything a captured launch sequence bakes in
     std::vector<uint64_t> gkey = key;
     const void* ptrs[] = {c->cnt.p, c->blk.p, c->surv.p, c->setup.p, c->shade.p, c->bincnt.p, c->binoff.p, c->big.p,
-                          c->keys0.p, c->keys1.p, c->vals0.p, c->vals1.p, c->hist.p, c->partials.p, c->ranges.p,
+                          c->keys.p, c->vals0.p, c->vals1.p, c->hist.p, c->partials.p, c->ranges.p,
                           c->tile_cnt.p, c->tile_start.p, c->vis.p, c->status.p, c->draws, c->views,
                           c->d_tables_host};
     for (const void* p : ptrs) gkey.push_back((uint64_t)(uintptr_t)p);
@@ -1292,7 +1291,7 @@ namespace dh {
 uint64_t ctx_scratch_bytes(dh_ctx c) {
   uint64_t b = 0;
   b += c->cnt.n + 4 * (c->blk.n + c->surv.n) + sizeof(SetupRec) * c->setup.n + sizeof(ShadeRec) * c->shade.n;
-  b += 4 * (c->bincnt.n + c->binoff.n + c->big.n + c->keys0.n + c->keys1.n + c->vals0.n + c->vals1.n);
+  b += 4 * (c->bincnt.n + c->binoff.n + c->big.n + c->keys.n + c->vals0.n + c->vals1.n);
   b += 4 * (c->hist.n + c->partials.n + c->tile_cnt.n + c->tile_start.n + c->vis.n) + 8 * c->ranges.n;
   b += sizeof(Status) * c->status.n + c->tables.n;
   return b;
@@ -1333,7 +1332,7 @@ void ctx_release_scratch(dh_ctx c) {
   drop_graph(c);
   c->cnt.release(); c->blk.release(); c->surv.release(); c->setup.release(); c->shade.release();
   c->bincnt.release(); c->binoff.release(); c->big.release();
-  c->keys0.release(); c->keys1.release(); c->vals0.release(); c->vals1.release();
+  c->keys.release(); c->vals0.release(); c->vals1.release();
   c->hist.release(); c->partials.release(); c->ranges.release(); c->vis.release();
   c->tile_cnt.release(); c->tile_start.release();
   c->status.release(); c->tables.release(); c->draws = nullptr; c->views = nullptr; c->export_buf.release();

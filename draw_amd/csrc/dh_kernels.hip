@@ -12,18 +12,14 @@
 //                    (1047-1063), raster setup (canvas.rs:585-666) -> SetupRec +
 //                    ShadeRec at its output id; with ordered bins also the
 //                    conservative tile count, and the near-first depth key
-//   4 k_wide_list, k_bin_count_wide  triangles spanning many tiles: listed,
-//                    then counted a wave each (k_bin_count counts per tile for
-//                    unordered bins)
-//   5 near first     stable 8-bit radix pass of the triangles by depth key,
-//                    their counts gathered in that order
-//   6 scan           -> bin entry offsets
-//   7 k_bin_emit(_wide)  (tile, triangle) pairs in that order
-//   8 radix sort     stable LSD sort of the pairs by tile -> per-tile lists,
-//                    near first (or in submission order)
-//   9 tile ranges    [start, end) of every tile's list: written by the sort's
-//                    scatter from its scanned histogram when the tile key
-//                    takes one pass, else by k_tile_ranges from the sorted keys
+//   4 k_pair_hist    near first (the default bins): (tile, triangle) pairs of
+//                    each chunk of triangles counted by the tile's low digit
+//   5 k_row_scan     -> each chunk's place in each digit's segment
+//   6 k_pair_scatter the pairs into their segments
+//   7 k_pair_sort    one workgroup per segment: its tiles' lists, near first,
+//                    and the tile ranges.  (Submission order: k_wide_list,
+//                    k_bin_count_wide, scan, k_bin_emit(_wide), a stable radix
+//                    sort of the pairs by tile, k_tile_ranges.)
 //  10 k_raster       one workgroup per screen tile: coverage and the strict
 //                    depth test (canvas.rs:668-682, 923) into an LDS visibility
 //                    buffer of (depth key << 32 | triangle id); the result does
@@ -707,55 +703,16 @@ __device__ inline uint32_t wave_tiles(const Spans& g, int TS, int lane, int* s_l
 
 // Ordered bins keep, per clipped triangle, a bin box: x the tile key of the
 // corner (cx0, cy0) of its tile box, y its tiles as bits 4 * (ty - cy0) +
-// (tx - cx0) (low 16 bits, within the at most 4 x 4 box) and the view's tiles
-// per row (high 16 bits), so that the pair emit finds every tile key from
-// these 8 bytes alone; x = kWideBox for a wide triangle, whose tiles a wave
-// counts and emits later.  They live in the flag buffer after the flag bytes
-// (12 bytes per clipped triangle in all).
+// (tx - cx0) (low 16 bits, within the at most 4 x 4 box; none for a dropped
+// triangle) and the view's tiles per row (high 16 bits), so that the pair
+// kernels find every tile key from these 8 bytes alone; x = kWideBox for a
+// wide triangle, whose tiles a wave counts and emits later.  They live in the
+// byte buffer after one byte per triangle (12 bytes per clipped triangle in all).
 constexpr uint32_t kWideBox = 0xFFFFFFFFu;
 __device__ __host__ inline uint2* bin_boxes(void* big, uint32_t cap_tri) {
   return reinterpret_cast<uint2*>(reinterpret_cast<uint8_t*>(big) + ((cap_tri + 15u) & ~15u));
 }
 
-// Ordered bins, one clipped triangle of view vw: its flag byte (0 binned here,
-// 1 wide, 2 dropped: no tiles, and its records were not stored), its bin box
-// and, when it is not wide, its tile count.
-__device__ inline void bin_count_one(const SetupRec& r, int TS, uint32_t i, const DevView& vw,
-                                     uint32_t* __restrict__ bincnt, uint8_t* __restrict__ wflag,
-                                     uint2* __restrict__ boxes) {
-  uint32_t c = 0, mask = 0, key0 = 0;
-  bool is_wide = false;
-  if (!(r.flags & kDrop)) {
-    Spans g;
-    spans_init(r, TS, g);
-    is_wide = bin_is_wide(g);
-    key0 = vw.tile_base + (uint32_t)g.cy0 * vw.ntx + (uint32_t)g.cx0;
-    if (!is_wide)
-      c = thread_tiles(g, TS, [&](uint32_t, int ty, int tx) { mask |= 1u << (4 * (ty - g.cy0) + (tx - g.cx0)); });
-  }
-  wflag[i] = is_wide ? 1u : ((r.flags & kDrop) ? 2u : 0u);
-  boxes[i] = make_uint2(is_wide ? kWideBox : key0, mask | (vw.ntx << 16));
-  if (!is_wide) bincnt[i] = c;
-}
-
-// The pairs of a triangle that is not wide from its bin box, its e-th tile at
-// position o + e (tiles in the order of the count pass).
-__device__ inline void emit_box_pairs(uint2 box, uint32_t i, uint32_t o, uint32_t cap_pairs,
-                                      uint32_t* __restrict__ keys, uint32_t* __restrict__ vals) {
-  const uint32_t ntx = box.y >> 16;
-  uint32_t mask = box.y & 0xFFFFu;
-  while (mask) {
-    const uint32_t b = (uint32_t)__builtin_ctz(mask);
-    mask &= mask - 1u;
-    if (o < cap_pairs) {
-      keys[o] = box.x + (b >> 2) * ntx + (b & 3u);
-      vals[o] = i;
-    }
-    o++;
-  }
-}
-
-// ================================================================== geometry
 // Near-first binning order: an 8-bit key of the nearest vertex depth, 16
 // steps per octave above depth_base (the float bits of half the near-plane
 // distance), so 16 octaves of depth; monotonic for positive depths, others
@@ -768,6 +725,90 @@ __device__ inline uint32_t depth_order_key(const SetupRec& r, uint32_t depth_bas
   return min((b - depth_base) >> 19, (1u << kDepthKeyBits) - 1u);
 }
 
+// How an emit prepares the binning: nothing (unordered bins), submission
+// order (flag byte, bin box, tile count per triangle) or near first (depth
+// key byte, bin box, and the list of wide triangles).
+constexpr int kBinNone = 0, kBinSubmit = 1, kBinNear = 2;
+
+// One clipped triangle of view vw: its byte (submission order: 0 binned here,
+// 1 wide, 2 dropped; near first: its depth key), its bin box and, for
+// submission order, its tile count when it is not wide.  (A dropped triangle
+// has no tiles, and its records are not stored.)  Returns whether it is wide.
+template <int BIN>
+__device__ inline bool bin_count_one(const SetupRec& r, int TS, uint32_t i, const DevView& vw,
+                                     uint32_t* __restrict__ bincnt, uint8_t* __restrict__ wflag,
+                                     uint2* __restrict__ boxes) {
+  uint32_t c = 0, mask = 0, key0 = 0;
+  bool is_wide = false;
+  if (!(r.flags & kDrop)) {
+    Spans g;
+    spans_init(r, TS, g);
+    is_wide = bin_is_wide(g);
+    key0 = vw.tile_base + (uint32_t)g.cy0 * vw.ntx + (uint32_t)g.cx0;
+    if (!is_wide)
+      c = thread_tiles(g, TS, [&](uint32_t, int ty, int tx) { mask |= 1u << (4 * (ty - g.cy0) + (tx - g.cx0)); });
+  }
+  boxes[i] = make_uint2(is_wide ? kWideBox : key0, mask | (vw.ntx << 16));
+  if constexpr (BIN == kBinNear) {
+    wflag[i] = (uint8_t)depth_order_key(r, vw.depth_base);
+  } else {
+    wflag[i] = is_wide ? 1u : ((r.flags & kDrop) ? 2u : 0u);
+    if (!is_wide) bincnt[i] = c;
+  }
+  return is_wide;
+}
+
+// The wide triangles an emit block meets, gathered in LDS and appended to the
+// frame's list with one atomic per block (an atomic per wave on that one word
+// would serialize a large frame's emits); more than the buffer holds go to
+// the list one by one.  The list's order does not matter.
+constexpr uint32_t kWideBuf = 512;
+struct WideBuf {
+  uint32_t n, base;
+  uint32_t id[kWideBuf];
+};
+__device__ inline void wide_push(WideBuf& b, uint32_t i, Status* status, uint32_t* __restrict__ list) {
+  const uint32_t p = atomicAdd(&b.n, 1u);
+  if (p < kWideBuf) b.id[p] = i;
+  else list[atomicAdd(&status->n_wide, 1u)] = i;
+}
+// Every thread of the block calls it, after its last wide_push.
+__device__ inline void wide_flush(WideBuf& b, Status* status, uint32_t* __restrict__ list) {
+  __syncthreads();
+  const uint32_t n = min(b.n, kWideBuf);
+  if (n == 0u) return;
+  if (threadIdx.x == 0) b.base = atomicAdd(&status->n_wide, n);
+  __syncthreads();
+  for (uint32_t k = threadIdx.x; k < n; k += blockDim.x) list[b.base + k] = b.id[k];
+}
+
+// Calls f(tile key) for every tile of a bin box (none for a wide triangle,
+// whose mask is empty).
+template <class F>
+__device__ inline void box_tiles(uint2 box, F f) {
+  const uint32_t ntx = box.y >> 16;
+  uint32_t mask = box.y & 0xFFFFu;
+  while (mask) {
+    const uint32_t b = (uint32_t)__builtin_ctz(mask);
+    mask &= mask - 1u;
+    f(box.x + (b >> 2) * ntx + (b & 3u));
+  }
+}
+
+// The pairs of a triangle that is not wide from its bin box, its e-th tile at
+// position o + e (tiles in the order of the count pass).
+__device__ inline void emit_box_pairs(uint2 box, uint32_t i, uint32_t o, uint32_t cap_pairs,
+                                      uint32_t* __restrict__ keys, uint32_t* __restrict__ vals) {
+  box_tiles(box, [&](uint32_t key) {
+    if (o < cap_pairs) {
+      keys[o] = key;
+      vals[o] = i;
+    }
+    o++;
+  });
+}
+
+// ================================================================== geometry
 // Small single-view frames: at most kSmallBinTris input triangles and
 // kSmallBinTiles tiles take single-workgroup kernels for the geometry lists
 // (k_geom_small) and the binning (k_bin_small), and one launch for both emits.
@@ -935,13 +976,13 @@ __global__ __launch_bounds__(256) void k_geom_compact(uint32_t n_in, const uint8
 // One thread per emitting input triangle of one list (dense: culled
 // triangles take no lane).  The unclipped list (CLIP false) skips the
 // clipper, whose attribute registers would otherwise size the whole kernel.
-template <bool BIN>
+template <int BIN>
 __device__ __forceinline__ void geom_emit_clipped(uint32_t j, const DevDraw* __restrict__ draws, uint32_t n_draws,
                                                   const DevView* __restrict__ views, const uint2* __restrict__ surv,
                                                   const DevMaterial* __restrict__ mats, SetupRec* __restrict__ setup,
                                                   ShadeRec* __restrict__ shade, uint32_t cap_tri, Status* __restrict__ status,
                                                   int TS, uint32_t* __restrict__ bincnt, uint8_t* __restrict__ wflag,
-                                                  uint32_t* __restrict__ dkey, uint32_t span) {
+                                                  uint32_t* __restrict__ wide_list, WideBuf* wide, uint32_t span) {
   const uint2 sv = surv[status->n_simple + j];
   const uint32_t t = sv.x, base = sv.y;
   // the lanes of the wave still in the loop
@@ -981,14 +1022,16 @@ __device__ __forceinline__ void geom_emit_clipped(uint32_t j, const DevDraw* __r
     uint4 ro[6], so[9];
     make_setup<false>(fr, A, B, C, material, mats[material], view, group, ro, so, rec);
     // with ordered bins nothing reads a dropped triangle's records
-    if (!BIN || !(rec.flags & kDrop)) {
+    if (BIN == kBinNone || !(rec.flags & kDrop)) {
 #pragma unroll
       for (int q = 0; q < 6; q++) reinterpret_cast<uint4*>(setup + idx)[q] = ro[q];
 #pragma unroll
       for (int q = 0; q < 9; q++) reinterpret_cast<uint4*>(shade + idx)[q] = so[q];
     }
-    if (BIN) bin_count_one(rec, TS, idx, views[view], bincnt, wflag, bin_boxes(wflag, cap_tri));
-    if (dkey) dkey[idx] = depth_order_key(rec, views[view].depth_base);
+    if constexpr (BIN != kBinNone) {
+      const bool is_wide = bin_count_one<BIN>(rec, TS, idx, views[view], bincnt, wflag, bin_boxes(wflag, cap_tri));
+      if (BIN == kBinNear && is_wide) wide_push(*wide, idx, status, wide_list);
+    }
   };
   cull_and_clip(fr, v[0], v[1], v[2], !(dr.flags & kDrawNoCull), out);
 }
@@ -996,13 +1039,14 @@ __device__ __forceinline__ void geom_emit_clipped(uint32_t j, const DevDraw* __r
 // One unclipped list entry per lane (every lane of the wave calls it; lanes
 // past the list end with active false): one record each at the entry's output
 // id, stored through the wave's LDS area stage[64 * 9].
-template <bool BIN>
+template <int BIN>
 __device__ __forceinline__ void geom_emit_simple(uint32_t j, bool active, uint4* stage, const DevDraw* __restrict__ draws,
                                                  uint32_t n_draws, const DevView* __restrict__ views,
                                                  const uint2* __restrict__ surv, const DevMaterial* __restrict__ mats,
                                                  SetupRec* __restrict__ setup, ShadeRec* __restrict__ shade, uint32_t cap_tri,
                                                  Status* __restrict__ status, int TS, uint32_t* __restrict__ bincnt,
-                                                 uint8_t* __restrict__ wflag, uint32_t* __restrict__ dkey, uint32_t span) {
+                                                 uint8_t* __restrict__ wflag, uint32_t* __restrict__ wide_list,
+                                                 WideBuf* wide, uint32_t span) {
   uint4 ro[6], so[9];
   uint32_t idx = 0;
   bool ok = false, skip = false;
@@ -1044,9 +1088,11 @@ __device__ __forceinline__ void geom_emit_simple(uint32_t j, bool active, uint4*
       make_setup<true>(fr, v[0], v[1], v[2], dr.material, mats[dr.material], dr.view, dr.group, ro, so, rec);
       ok = true;
       // with ordered bins nothing reads a dropped triangle's records
-      skip = BIN && (rec.flags & kDrop);
-      if (BIN) bin_count_one(rec, TS, idx, views[dr.view], bincnt, wflag, bin_boxes(wflag, cap_tri));
-      if (dkey) dkey[idx] = depth_order_key(rec, views[dr.view].depth_base);
+      skip = BIN != kBinNone && (rec.flags & kDrop);
+      if constexpr (BIN != kBinNone) {
+        const bool is_wide = bin_count_one<BIN>(rec, TS, idx, views[dr.view], bincnt, wflag, bin_boxes(wflag, cap_tri));
+        if (BIN == kBinNear && is_wide) wide_push(*wide, idx, status, wide_list);
+      }
     }
   }
   wave_store<6>(stage, ro, ok, idx, reinterpret_cast<uint4*>(setup), skip);
@@ -1056,27 +1102,35 @@ __device__ __forceinline__ void geom_emit_simple(uint32_t j, bool active, uint4*
 // A grid-stride loop over one list (its length is on the device), so that the
 // grid can be capped well below one thread per input triangle.  The unclipped
 // list goes a wave at a time (its records leave through LDS).
-template <bool BIN, bool CLIP>
+template <int BIN, bool CLIP>
 __global__ __launch_bounds__(256) void k_geom_emit(const DevDraw* __restrict__ draws, uint32_t n_draws,
                                                    const DevView* __restrict__ views,
                                                    const uint2* __restrict__ surv,
                                                    const DevMaterial* __restrict__ mats, SetupRec* __restrict__ setup,
                                                    ShadeRec* __restrict__ shade, uint32_t cap_tri,
                                                    Status* __restrict__ status, int TS, uint32_t* __restrict__ bincnt,
-                                                   uint8_t* __restrict__ wflag, uint32_t* __restrict__ dkey, uint32_t span) {
+                                                   uint8_t* __restrict__ wflag, uint32_t* __restrict__ wide_list,
+                                                   uint32_t span) {
+  __shared__ uint32_t s_wide[BIN == kBinNear ? sizeof(WideBuf) / 4 : 1];
+  WideBuf* const wide = reinterpret_cast<WideBuf*>(s_wide);
+  if constexpr (BIN == kBinNear) {
+    if (threadIdx.x == 0) wide->n = 0u;
+    __syncthreads();
+  }
   if constexpr (CLIP) {
     const uint32_t n = status->n_clip;
     for (uint32_t j = blockIdx.x * 256u + threadIdx.x; j < n; j += gridDim.x * 256u)
       geom_emit_clipped<BIN>(j, draws, n_draws, views, surv, mats, setup, shade, cap_tri, status, TS, bincnt, wflag,
-                             dkey, span);
+                             wide_list, wide, span);
   } else {
     __shared__ uint4 s_stage[4][64 * 9];
     const uint32_t n = status->n_simple;
     const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
     for (uint32_t j0 = blockIdx.x * 256u + wave * 64u; j0 < n; j0 += gridDim.x * 256u)
       geom_emit_simple<BIN>(j0 + lane, j0 + lane < n, s_stage[wave], draws, n_draws, views, surv, mats, setup, shade,
-                            cap_tri, status, TS, bincnt, wflag, dkey, span);
+                            cap_tri, status, TS, bincnt, wflag, wide_list, wide, span);
   }
+  if constexpr (BIN == kBinNear) wide_flush(*wide, status, wide_list);
 }
 
 // Both emitter lists of a small frame in one launch on the stream (for a few
@@ -1087,7 +1141,7 @@ __global__ __launch_bounds__(256) void k_geom_emit(const DevDraw* __restrict__ d
 // No occupancy floor: the grid (at most 128 blocks) fills a fraction of the
 // chip, so registers go to the clipped path (167-172 VGPRs, no spills)
 // rather than to waves that would have nothing to run.
-template <bool BIN>
+template <int BIN>
 __global__ __launch_bounds__(256) void k_geom_emit_both(const DevDraw* __restrict__ draws, uint32_t n_draws,
                                                         const DevView* __restrict__ views,
                                                         const uint2* __restrict__ surv,
@@ -1095,7 +1149,13 @@ __global__ __launch_bounds__(256) void k_geom_emit_both(const DevDraw* __restric
                                                         SetupRec* __restrict__ setup, ShadeRec* __restrict__ shade,
                                                         uint32_t cap_tri, Status* __restrict__ status, int TS,
                                                         uint32_t* __restrict__ bincnt, uint8_t* __restrict__ wflag,
-                                                        uint32_t* __restrict__ dkey, uint32_t g_clip) {
+                                                        uint32_t* __restrict__ wide_list, uint32_t g_clip) {
+  __shared__ uint32_t s_wide[BIN == kBinNear ? sizeof(WideBuf) / 4 : 1];
+  WideBuf* const wide = reinterpret_cast<WideBuf*>(s_wide);
+  if constexpr (BIN == kBinNear) {
+    if (threadIdx.x == 0) wide->n = 0u;
+    __syncthreads();
+  }
   __shared__ uint4 s_stage[4][64 * 9];
   const uint64_t G = gridDim.x, b = blockIdx.x;
   const uint32_t c0 = (uint32_t)(b * g_clip / G), c1 = (uint32_t)((b + 1) * g_clip / G);
@@ -1103,36 +1163,47 @@ __global__ __launch_bounds__(256) void k_geom_emit_both(const DevDraw* __restric
     const uint32_t n = status->n_clip;
     for (uint32_t j = c0 * 256u + threadIdx.x; j < n; j += g_clip * 256u)
       geom_emit_clipped<BIN>(j, draws, n_draws, views, surv, mats, setup, shade, cap_tri, status, TS, bincnt, wflag,
-                             dkey, kSparseSpan);
+                             wide_list, wide, kSparseSpan);
   } else {
     const uint32_t ub = (uint32_t)b - c0, g_simple = (uint32_t)G - g_clip;
     const uint32_t n = status->n_simple;
     const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
     for (uint32_t j0 = ub * 256u + wave * 64u; j0 < n; j0 += g_simple * 256u)
       geom_emit_simple<BIN>(j0 + lane, j0 + lane < n, s_stage[wave], draws, n_draws, views, surv, mats, setup, shade,
-                            cap_tri, status, TS, bincnt, wflag, dkey, kSparseSpan);
+                            cap_tri, status, TS, bincnt, wflag, wide_list, wide, kSparseSpan);
   }
+  if constexpr (BIN == kBinNear) wide_flush(*wide, status, wide_list);
 }
 
-// First clipped-triangle id of each view: the exclusive prefix of the clip
-// counts at the view's first input triangle (blk_off holds the scanned block
-// sums).  Shading subtracts it, so a view's winner ids do not depend on the
-// other views of a batch.
-__global__ void k_view_id_base(DevView* __restrict__ views, uint32_t n_views, uint32_t n_in,
-                               const uint8_t* __restrict__ cnt, const uint32_t* __restrict__ blk_off,
-                               const Status* __restrict__ status) {
-  const uint32_t v = blockIdx.x * blockDim.x + threadIdx.x;
-  if (v >= n_views) return;
-  const uint32_t t0 = views[v].tri_begin;
-  uint32_t base;
-  if (t0 >= n_in) {
-    base = status->n_out;
-  } else {
-    const uint32_t b = t0 >> 8;
-    base = blk_off[b];
-    for (uint32_t t = b << 8; t < t0; t++) base += cnt[t] & kCntMask;
+// Clipped triangles before input triangle t0: its block's scanned count and
+// the counts before it in the block, a wave's lanes taking four each (every
+// lane calls it; one thread alone needs up to 255 dependent loads, 20 us of a
+// 32-view batch).
+__device__ inline uint32_t wave_id_before(uint32_t t0, uint32_t n_in, const uint8_t* __restrict__ cnt,
+                                          const uint32_t* __restrict__ blk_off, const Status* __restrict__ status) {
+  if (t0 >= n_in) return status->n_out;
+  const uint32_t lane = threadIdx.x & 63u, b = t0 >> 8;
+  uint32_t s = 0;
+#pragma unroll
+  for (uint32_t k = 0; k < 4u; k++) {
+    const uint32_t t = (b << 8) + 64u * k + lane;
+    if (t < t0) s += cnt[t] & kCntMask;
   }
-  views[v].id_base = base;
+#pragma unroll
+  for (int o = 32; o; o >>= 1) s += __shfl_xor(s, o, 64);
+  return blk_off[b] + s;
+}
+
+// First clipped-triangle id of each view (a wave per view).  Shading subtracts
+// it, so a view's winner ids do not depend on the other views of a batch.
+__global__ __launch_bounds__(256) void k_view_id_base(DevView* __restrict__ views, uint32_t n_views, uint32_t n_in,
+                                                      const uint8_t* __restrict__ cnt,
+                                                      const uint32_t* __restrict__ blk_off,
+                                                      const Status* __restrict__ status) {
+  const uint32_t v = (blockIdx.x * 256u + threadIdx.x) >> 6;
+  if (v >= n_views) return;  // the whole wave
+  const uint32_t id = wave_id_before(views[v].tri_begin, n_in, cnt, blk_off, status);
+  if ((threadIdx.x & 63u) == 0u) views[v].id_base = id;
 }
 
 // ====================================================================== scan
@@ -1211,8 +1282,11 @@ __global__ __launch_bounds__(256) void k_scan_apply(const uint32_t* in, uint32_t
   }
 }
 
-// Scans of at most 4 * 1024 elements whose count the host knows: one block.
-// Up to three independent scans of n <= 4096 values, one block each.
+// Up to three independent exclusive scans of n values each (n known to the
+// host), one block of 1024 threads each, 8192 values at a time with a carry:
+// the per-block counts of the geometry pass, for which one launch of a few
+// rounds is shorter than two launches per scan (20,000 blocks: a 5M-triangle
+// frame, 27 us in six launches, 20 in one).
 struct ScanSeg {
   const uint32_t* in;
   uint32_t* out;
@@ -1224,7 +1298,8 @@ struct ScanSegs {
   ScanSeg s[3];
 };
 
-__global__ __launch_bounds__(1024) void k_scan_small(ScanSegs segs, uint32_t n) {
+__global__ __launch_bounds__(1024) void k_scan_segs(ScanSegs segs, uint32_t n) {
+  constexpr int kPer = 8;
   const ScanSeg& g = segs.s[blockIdx.x];
   const uint32_t* in = g.in;  // may be out (in-place scans)
   uint32_t* out = g.out;
@@ -1233,33 +1308,48 @@ __global__ __launch_bounds__(1024) void k_scan_small(ScanSegs segs, uint32_t n) 
   const uint32_t cap_check = g.cap_check, overflow_bit = g.overflow_bit;
   __shared__ uint32_t s_w[16];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const uint32_t i0 = threadIdx.x * 4u;
-  uint32_t v[4];
+  uint32_t carry = 0;
+  uint32_t v[kPer];
+  auto load = [&](uint32_t t0) {
+    const uint32_t i0 = t0 + threadIdx.x * (uint32_t)kPer;
 #pragma unroll
-  for (int k = 0; k < 4; k++) v[k] = (i0 + k < n) ? in[i0 + k] : 0u;
-  const uint32_t s4 = v[0] + v[1] + v[2] + v[3];
-  uint32_t x = s4;
+    for (int k = 0; k < kPer; k++) v[k] = (i0 + k < n) ? in[i0 + k] : 0u;
+  };
+  load(0u);
+  for (uint32_t t0 = 0; t0 < n; t0 += 1024u * kPer) {
+    const uint32_t i0 = t0 + threadIdx.x * (uint32_t)kPer;
+    uint32_t c[kPer], sum = 0;
 #pragma unroll
-  for (int o = 1; o < 64; o <<= 1) {
-    const uint32_t y = __shfl_up(x, o, 64);
-    if (lane >= o) x += y;
-  }
-  if (lane == 63) s_w[wave] = x;
-  __syncthreads();
-  uint32_t before = 0, all = 0;
-  for (int w = 0; w < 16; w++) {
-    if (w < wave) before += s_w[w];
-    all += s_w[w];
-  }
-  uint32_t ex = before + x - s4;
+    for (int k = 0; k < kPer; k++) {
+      c[k] = v[k];
+      sum += c[k];
+    }
+    if (t0 + 1024u * kPer < n) load(t0 + 1024u * kPer);  // the next round's, behind this round's barriers
+    uint32_t x = sum;
 #pragma unroll
-  for (int k = 0; k < 4; k++) {
-    if (i0 + k < n) out[i0 + k] = ex;
-    ex += v[k];
+    for (int o = 1; o < 64; o <<= 1) {
+      const uint32_t y = __shfl_up(x, o, 64);
+      if (lane >= o) x += y;
+    }
+    if (lane == 63) s_w[wave] = x;
+    __syncthreads();
+    uint32_t before = carry, all = 0;
+    for (int w = 0; w < 16; w++) {
+      if (w < wave) before += s_w[w];
+      all += s_w[w];
+    }
+    uint32_t ex = before + x - sum;
+#pragma unroll
+    for (int k = 0; k < kPer; k++) {
+      if (i0 + k < n) out[i0 + k] = ex;
+      ex += c[k];
+    }
+    carry += all;
+    __syncthreads();
   }
   if (threadIdx.x == 0) {
-    if (total_out) *total_out = all;
-    if (overflow_word && all > cap_check) atomicOr(overflow_word, overflow_bit);
+    if (total_out) *total_out = carry;
+    if (overflow_word && carry > cap_check) atomicOr(overflow_word, overflow_bit);
   }
 }
 
@@ -1270,7 +1360,7 @@ static void scan_u32(const uint32_t* in, uint32_t* out, const uint32_t* n_ptr, u
   if (!n_ptr && n_const <= 4096u && !idx) {
     ScanSegs g{};
     g.s[0] = ScanSeg{in, out, total_out, overflow_word, cap_check, overflow_bit};
-    hipLaunchKernelGGL(k_scan_small, dim3(1), dim3(1024), 0, s, g, n_const);
+    hipLaunchKernelGGL(k_scan_segs, dim3(1), dim3(1024), 0, s, g, n_const);
     return;
   }
   hipLaunchKernelGGL(k_scan_reduce, dim3(kScanG), dim3(256), 0, s, in, n_ptr, n_const, cap, partials, idx);
@@ -1423,68 +1513,6 @@ __global__ __launch_bounds__(256) void k_bin_emit(const SetupRec* __restrict__ s
   }
 }
 
-// Near-first pairs with the scan of their counts fused in: block b takes
-// chunk b of the depth order (the chunks of k_scan_reduce, whose sums are in
-// partials), scans the counts bincnt[order[j]] from the sums before it, and
-// emits each triangle's pairs at its offset from its bin box (a wide
-// triangle's offset goes to binoff for k_bin_emit_wide).  The ids, counts and
-// boxes of up to four rounds of 256 are loaded before the first round's scan,
-// so that a block waits on two dependent loads per four rounds.  Block 0
-// publishes the pair total and the overflow flag.
-__global__ __launch_bounds__(256) void k_bin_emit_near(Status* status, uint32_t cap_tri,
-                                                       const uint8_t* __restrict__ wflag,
-                                                       uint32_t* __restrict__ binoff, const uint32_t* __restrict__ order,
-                                                       const uint32_t* __restrict__ bincnt,
-                                                       const uint32_t* __restrict__ partials, uint32_t cap_pairs,
-                                                       uint32_t* __restrict__ keys, uint32_t* __restrict__ vals) {
-  __shared__ uint32_t s_tmp[4];
-  constexpr int kRounds = 4;
-  const uint32_t n = min(status->n_out, cap_tri);
-  const uint32_t C = scan_chunk(n);
-  const uint32_t b0 = blockIdx.x * C, b1 = min(b0 + C, n);
-  const uint2* boxes = bin_boxes(const_cast<uint8_t*>(wflag), cap_tri);
-  const uint32_t upto = blockIdx.x == 0 ? (uint32_t)kScanG : blockIdx.x;
-  uint32_t p = 0;
-  for (uint32_t k = threadIdx.x; k < upto; k += 256) p += partials[k];
-  uint32_t sum;
-  block_exclusive_scan256(p, s_tmp, &sum);
-  uint32_t running = 0;
-  if (blockIdx.x == 0) {
-    if (threadIdx.x == 0) {
-      status->n_pairs = sum;
-      if (sum > cap_pairs) atomicOr(&status->overflow, 2u);
-    }
-  } else {
-    running = sum;
-  }
-  for (uint32_t tg = b0; tg < b1; tg += 256u * kRounds) {
-    uint32_t id[kRounds], c[kRounds];
-    uint2 box[kRounds];
-#pragma unroll
-    for (int k = 0; k < kRounds; k++) {
-      const uint32_t j = tg + 256u * k + threadIdx.x;
-      id[k] = j < b1 ? order[j] : 0u;
-    }
-#pragma unroll
-    for (int k = 0; k < kRounds; k++) {
-      const bool act = tg + 256u * k + threadIdx.x < b1;
-      c[k] = act ? bincnt[id[k]] : 0u;
-      box[k] = act ? boxes[id[k]] : make_uint2(0u, 0u);
-    }
-#pragma unroll
-    for (int k = 0; k < kRounds; k++) {
-      uint32_t tot;
-      const uint32_t o = block_exclusive_scan256(c[k], s_tmp, &tot) + running;
-      running += tot;
-      if (tg + 256u * k + threadIdx.x >= b1) continue;
-      if (box[k].x == kWideBox)
-        binoff[id[k]] = o;
-      else
-        emit_box_pairs(box[k], id[k], o, cap_pairs, keys, vals);
-    }
-  }
-}
-
 template <bool ORDERED>
 __global__ __launch_bounds__(256) void k_bin_emit_wide(const SetupRec* __restrict__ setup,
                                                        const DevView* __restrict__ views, const Status* status,
@@ -1517,8 +1545,8 @@ __global__ __launch_bounds__(256) void k_bin_emit_wide(const SetupRec* __restric
 // Binning of a small single-view frame in one workgroup of 1024 threads,
 // in place of the general path's dozen launches (which a frame of a few
 // thousand triangles spends mostly starting and draining): per-tile counts
-// with LDS atomics from each triangle's bin box (a wave per wide triangle,
-// as k_bin_count_wide), their scan into the tile ranges, then each
+// with LDS atomics from each triangle's bin box (a wave per wide triangle of
+// the emits' list), their scan into the tile ranges, then each
 // triangle's id written into its tiles' lists at LDS-atomic cursors.  The
 // lists are unordered, which changes no result: a tile's visibility is the
 // minimum of its fragments' keys whatever the order (the transparent pass,
@@ -1528,7 +1556,7 @@ __global__ __launch_bounds__(256) void k_bin_emit_wide(const SetupRec* __restric
 __global__ __launch_bounds__(1024) void k_bin_small(const SetupRec* __restrict__ setup,
                                                     const DevView* __restrict__ views, Status* __restrict__ status,
                                                     uint32_t cap_tri, int TS, const uint8_t* __restrict__ wflag,
-                                                    uint32_t* __restrict__ wide_list, uint32_t n_tiles,
+                                                    const uint32_t* __restrict__ wide_list, uint32_t n_tiles,
                                                     uint32_t cap_pairs, uint32_t* __restrict__ vals,
                                                     uint2* __restrict__ ranges) {
   __shared__ uint32_t s_cnt[kSmallBinTiles];
@@ -1536,10 +1564,8 @@ __global__ __launch_bounds__(1024) void k_bin_small(const SetupRec* __restrict__
   __shared__ int s_lo[16][64];
   __shared__ uint32_t s_off[16][64];
   __shared__ uint32_t s_w[16];
-  __shared__ uint32_t s_nwide;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   for (uint32_t k = (uint32_t)tid; k < n_tiles; k += 1024u) s_cnt[k] = 0u;
-  if (tid == 0) s_nwide = 0u;
   __syncthreads();
   const uint32_t n = min(status->n_out, cap_tri);
   const uint2* boxes = bin_boxes(const_cast<uint8_t*>(wflag), cap_tri);
@@ -1547,15 +1573,7 @@ __global__ __launch_bounds__(1024) void k_bin_small(const SetupRec* __restrict__
   // one pass over the triangles' tiles: f(tile key) for each
   auto each_tile = [&](auto f) {
     for (uint32_t i = (uint32_t)tid; i < n; i += 1024u) {
-      if (wflag[i] != 0u) continue;  // wide (below) or dropped
-      const uint2 box = boxes[i];
-      const uint32_t ntx = box.y >> 16;
-      uint32_t mask = box.y & 0xFFFFu;
-      while (mask) {
-        const uint32_t b = (uint32_t)__builtin_ctz(mask);
-        mask &= mask - 1u;
-        f(i, box.x + (b >> 2) * ntx + (b & 3u));
-      }
+      box_tiles(boxes[i], [&](uint32_t key) { f(i, key); });
     }
   };
   auto each_wide_tile = [&](uint32_t nw, auto f) {
@@ -1570,12 +1588,9 @@ __global__ __launch_bounds__(1024) void k_bin_small(const SetupRec* __restrict__
       });
     }
   };
-  // counts, and the list of wide triangles
-  for (uint32_t i = (uint32_t)tid; i < n; i += 1024u)
-    if (wflag[i] == 1u) wide_list[atomicAdd(&s_nwide, 1u)] = i;
+  // counts
   each_tile([&](uint32_t, uint32_t key) { atomicAdd(&s_cnt[key], 1u); });
-  __syncthreads();
-  const uint32_t nw = s_nwide;
+  const uint32_t nw = status->n_wide;
   each_wide_tile(nw, [&](uint32_t, uint32_t key) { atomicAdd(&s_cnt[key], 1u); });
   __syncthreads();
   // exclusive scan of the counts, 1024 tiles at a time with a carry
@@ -1736,77 +1751,286 @@ __global__ __launch_bounds__(256) void k_radix_scatter(const uint32_t* __restric
   }
 }
 
-// One-pass sort by keys below DIG (256 or 2048) whose order within a key is
-// free: the near-first depth order and tile lists, whose entries only need to
-// stay roughly in depth order (a tile's visibility does not depend on the
-// order of its list).  Each block owns one contiguous chunk of the input
-// (chunks contiguous per XCD, as above), so the histogram has DIG x 256
-// entries instead of DIG per wave, and its items take their output slots
-// with LDS atomic increments of their key's cursor: a key's entries come
-// chunk by chunk in input order, in any order within a chunk.
-constexpr int kRadixBG = 256;   // blocks (chunks) of the unordered one-pass sort
-constexpr int kRadixBT = 1024;  // threads per chunk: 16 waves, one block per CU
-static_assert(2048u * kRadixBG <= kRadixHistEntries, "histogram size");
+// ======================================================== near-first tile lists
+// The default bins: every tile's list, roughly near first, in four launches
+// and without an intermediate array of pairs in triangle order.  Nothing here
+// has to be stable: a tile's visibility does not depend on its list's order.
+//  k_pair_hist     the triangles (bin boxes) are cut into kPairChunks
+//                  contiguous chunks, the wide list into as many; a block per
+//                  chunk counts its (tile, triangle) pairs by digit, the
+//                  tile key's low bits;
+//  k_row_scan      a block per digit scans the chunks' counts;
+//  k_pair_scatter  the blocks of k_pair_hist write their pairs at LDS cursors
+//                  into the digit's segment, as (rest of the key << 8 | depth
+//                  key, triangle);
+//  k_pair_sort     a block per segment sorts it by (tile, depth level) with
+//                  LDS counters and writes the ids and the tiles' ranges.
+// Neighbouring tiles lie in different segments, so a crowded part of the
+// screen is spread over all of them; the depth order costs no pass of its own.
+// (Before: a depth sort of the triangles, a gathered scan, a pair emit and one
+// or two more sort passes with their scans, 13 to 18 launches of 3 to 15 us
+// each.  1M-triangle 1080p frame: 387 -> 358 us; 150k triangles at 1237x709: 208
+// -> 166 us; 500k triangles at 3840x2160: 300 -> 249 us.)
+constexpr int kPairChunks = 256;         // blocks of 1024 threads: one per CU, twice (triangles, wide triangles)
+constexpr int kPairT = 1024;
+constexpr int kPairU = 4;                // boxes in flight per thread
+constexpr int kPairCols = 2 * kPairChunks;  // histogram columns: wide chunks first, then the others
+constexpr uint32_t kPairCounters = 8192;    // k_pair_sort's LDS counters: tiles of a segment x depth levels
+// 256 segments, or 2048 where they would leave a segment fewer than 16 depth
+// levels; beyond kPairMaxTiles a segment has more tiles than counters.
+constexpr uint32_t kPairFewTiles = 256u * (kPairCounters / 16u);
+constexpr uint32_t kPairMaxTiles = 2048u * kPairCounters;
+static_assert(2048u * (kPairCols + 1u) <= kRadixHistEntries, "histogram and digit totals");
 
-__device__ inline uint32_t radix_chunk_blk(uint32_t n) { return (((n + kRadixBG - 1u) / kRadixBG) + 255u) & ~255u; }
-
-template <int DIG>
-__global__ __launch_bounds__(kRadixBT) void k_radix_hist_blk(const uint32_t* __restrict__ keys, const uint32_t* n_ptr,
-                                                             uint32_t cap, uint32_t* __restrict__ hist) {
-  __shared__ uint32_t h[DIG];
-  const int tid = threadIdx.x;
-  const uint32_t n = min(*n_ptr, cap);
-  const uint32_t C = radix_chunk_blk(n);
-  const uint32_t cb = xcd_remap(blockIdx.x, gridDim.x);
+// Visits the pairs of one chunk: f(tile key, triangle, depth key).  The wide
+// chunks' waves take the listed triangles in turn.
+template <class F>
+__device__ inline void pair_chunk(const uint8_t* __restrict__ dkey, const uint32_t* __restrict__ wide_list,
+                                  const SetupRec* __restrict__ setup, const DevView* __restrict__ views,
+                                  const Status* __restrict__ status, uint32_t cap_tri, int TS, int (*s_lo)[64],
+                                  uint32_t (*s_off)[64], F f) {
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  if (blockIdx.x < (uint32_t)kPairChunks) {
+    const uint32_t n = min(status->n_wide, cap_tri);
+    const uint32_t w0 = blockIdx.x + (uint32_t)kPairChunks * (uint32_t)wave;
+    for (uint32_t w = w0; w < n; w += (uint32_t)(kPairChunks * (kPairT / 64))) {
+      const uint32_t i = (uint32_t)__builtin_amdgcn_readfirstlane((int)wide_list[w]);
+      const SetupRec r = setup[i];
+      const DevView& vw = views[r.view];
+      const uint32_t dk = dkey[i];
+      Spans g;
+      spans_init(r, TS, g);
+      spans_init_rows(r, g);
+      wave_tiles(g, TS, lane, s_lo[wave], s_off[wave], [&](uint32_t, int ty, int tx) {
+        f(vw.tile_base + (uint32_t)ty * vw.ntx + (uint32_t)tx, i, dk);
+      });
+    }
+    return;
+  }
+  const uint32_t n = min(status->n_out, cap_tri);
+  // consecutive chunks on one XCD: their runs in a segment are neighbours
+  const uint32_t cb = xcd_remap(blockIdx.x - (uint32_t)kPairChunks, (uint32_t)kPairChunks);
+  const uint32_t C = (n + (uint32_t)kPairChunks - 1u) / (uint32_t)kPairChunks;
   const uint32_t b0 = min(cb * C, n), b1 = min(b0 + C, n);
-  for (int d = tid; d < DIG; d += kRadixBT) h[d] = 0u;
-  __syncthreads();
-  for (uint32_t tb = b0; tb < b1; tb += (uint32_t)kRadixBT * kRadixU) {
-    uint32_t k[kRadixU];
+  const uint2* boxes = bin_boxes(const_cast<uint8_t*>(dkey), cap_tri);
+  for (uint32_t tb = b0; tb < b1; tb += (uint32_t)(kPairT * kPairU)) {
+    uint2 box[kPairU];
+    uint32_t dk[kPairU];
 #pragma unroll
-    for (int u = 0; u < kRadixU; u++) {
-      const uint32_t i = tb + (uint32_t)kRadixBT * (uint32_t)u + (uint32_t)tid;
-      k[u] = i < b1 ? keys[i] : 0u;
+    for (int u = 0; u < kPairU; u++) {
+      const uint32_t i = tb + (uint32_t)(kPairT * u + tid);
+      box[u] = i < b1 ? boxes[i] : make_uint2(0u, 0u);
+      dk[u] = i < b1 ? dkey[i] : 0u;
     }
 #pragma unroll
-    for (int u = 0; u < kRadixU; u++)
-      if (tb + (uint32_t)kRadixBT * (uint32_t)u + (uint32_t)tid < b1) atomicAdd(&h[k[u] & (DIG - 1u)], 1u);
+    for (int u = 0; u < kPairU; u++)
+      box_tiles(box[u], [&](uint32_t key) { f(key, tb + (uint32_t)(kPairT * u + tid), dk[u]); });
   }
-  __syncthreads();
-  for (int d = tid; d < DIG; d += kRadixBT) hist[(uint32_t)d * kRadixBG + cb] = h[d];
 }
 
-// vout[slot] = vin[i] (vin null: i itself) for the chunk's items, slots from
-// the scanned histogram (hist_off); ranges (may be null): [start, end) of each
-// of the first n_ranges keys in the output.
+__device__ inline uint32_t pair_col() {
+  return blockIdx.x < (uint32_t)kPairChunks
+             ? blockIdx.x
+             : (uint32_t)kPairChunks + xcd_remap(blockIdx.x - (uint32_t)kPairChunks, (uint32_t)kPairChunks);
+}
+
 template <int DIG>
-__global__ __launch_bounds__(kRadixBT) void k_radix_scatter_blk(const uint32_t* __restrict__ kin,
-                                                                const uint32_t* __restrict__ vin,
-                                                                uint32_t* __restrict__ vout, const uint32_t* n_ptr,
-                                                                uint32_t cap, const uint32_t* __restrict__ hist_off,
-                                                                uint2* __restrict__ ranges, uint32_t n_ranges) {
-  __shared__ uint32_t run[DIG];
-  const int tid = threadIdx.x;
-  const uint32_t n = min(*n_ptr, cap);
-  const uint32_t C = radix_chunk_blk(n);
-  const uint32_t cb = xcd_remap(blockIdx.x, gridDim.x);
-  const uint32_t b0 = min(cb * C, n), b1 = min(b0 + C, n);
-  if (ranges)
-    for (uint32_t d = blockIdx.x * (uint32_t)kRadixBT + (uint32_t)tid; d < n_ranges; d += gridDim.x * (uint32_t)kRadixBT)
-      ranges[d] = make_uint2(hist_off[d * kRadixBG], d + 1u < (uint32_t)DIG ? hist_off[(d + 1u) * kRadixBG] : n);
-  for (int d = tid; d < DIG; d += kRadixBT) run[d] = hist_off[(uint32_t)d * kRadixBG + cb];
+__global__ __launch_bounds__(kPairT) void k_pair_hist(const uint8_t* __restrict__ dkey,
+                                                      const uint32_t* __restrict__ wide_list,
+                                                      const SetupRec* __restrict__ setup,
+                                                      const DevView* __restrict__ views,
+                                                      const Status* __restrict__ status, uint32_t cap_tri, int TS,
+                                                      uint32_t* __restrict__ hist) {
+  __shared__ uint32_t h[DIG];
+  __shared__ int s_lo[kPairT / 64][64];
+  __shared__ uint32_t s_off[kPairT / 64][64];
+  for (int d = threadIdx.x; d < DIG; d += kPairT) h[d] = 0u;
   __syncthreads();
-  for (uint32_t tb = b0; tb < b1; tb += (uint32_t)kRadixBT * kRadixU) {
-    uint32_t k[kRadixU], v[kRadixU];
+  pair_chunk(dkey, wide_list, setup, views, status, cap_tri, TS, s_lo, s_off,
+             [&](uint32_t key, uint32_t, uint32_t) { atomicAdd(&h[key & (DIG - 1u)], 1u); });
+  __syncthreads();
+  const uint32_t col = pair_col();
+  for (int d = threadIdx.x; d < DIG; d += kPairT) hist[(uint32_t)d * kPairCols + col] = h[d];
+}
+
+// Row d of the histogram to its exclusive scan, its total to totals[d].
+__global__ __launch_bounds__(kPairCols) void k_row_scan(uint32_t* __restrict__ hist, uint32_t* __restrict__ totals) {
+  __shared__ uint32_t s_w[kPairCols / 64];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  uint32_t* const row = hist + (uint64_t)blockIdx.x * kPairCols;
+  const uint32_t v = row[threadIdx.x];
+  uint32_t x = v;
 #pragma unroll
-    for (int u = 0; u < kRadixU; u++) {
-      const uint32_t i = tb + (uint32_t)kRadixBT * (uint32_t)u + (uint32_t)tid;
-      k[u] = i < b1 ? kin[i] : 0u;
-      v[u] = i < b1 ? (vin ? vin[i] : i) : 0u;
+  for (int o = 1; o < 64; o <<= 1) {
+    const uint32_t y = __shfl_up(x, o, 64);
+    if (lane >= o) x += y;
+  }
+  if (lane == 63) s_w[wave] = x;
+  __syncthreads();
+  uint32_t before = 0, all = 0;
+#pragma unroll
+  for (int w = 0; w < kPairCols / 64; w++) {
+    if (w < wave) before += s_w[w];
+    all += s_w[w];
+  }
+  row[threadIdx.x] = before + x - v;
+  if (threadIdx.x == 0) totals[blockIdx.x] = all;
+}
+
+// Exclusive scan of s[0, N) in LDS by a block of T threads (all call it, the
+// values stored before a barrier); returns the total.
+template <int T>
+__device__ inline uint32_t lds_exclusive_scan(uint32_t* s, uint32_t n, uint32_t* s_w /*[T/64]*/) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  uint32_t carry = 0;
+  for (uint32_t k0 = 0; k0 < n; k0 += 4u * T) {
+    const uint32_t k = k0 + 4u * threadIdx.x;
+    uint32_t v[4];
+#pragma unroll
+    for (int j = 0; j < 4; j++) v[j] = k + j < n ? s[k + j] : 0u;
+    const uint32_t s4 = v[0] + v[1] + v[2] + v[3];
+    uint32_t x = s4;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const uint32_t y = __shfl_up(x, o, 64);
+      if (lane >= o) x += y;
     }
+    if (lane == 63) s_w[wave] = x;
+    __syncthreads();
+    uint32_t before = carry, all = 0;
 #pragma unroll
-    for (int u = 0; u < kRadixU; u++)
-      if (tb + (uint32_t)kRadixBT * (uint32_t)u + (uint32_t)tid < b1) vout[atomicAdd(&run[k[u] & (DIG - 1u)], 1u)] = v[u];
+    for (int w = 0; w < T / 64; w++) {
+      if (w < wave) before += s_w[w];
+      all += s_w[w];
+    }
+    uint32_t ex = before + x - s4;
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+      if (k + j < n) s[k + j] = ex;
+      ex += v[j];
+    }
+    carry += all;
+    __syncthreads();
+  }
+  return carry;
+}
+
+template <int DIG>
+__global__ __launch_bounds__(kPairT) void k_pair_scatter(const uint8_t* __restrict__ dkey,
+                                                         const uint32_t* __restrict__ wide_list,
+                                                         const SetupRec* __restrict__ setup,
+                                                         const DevView* __restrict__ views, Status* __restrict__ status,
+                                                         uint32_t cap_tri, int TS, const uint32_t* __restrict__ hist,
+                                                         const uint32_t* __restrict__ totals, uint32_t cap_pairs,
+                                                         uint2* __restrict__ pairs) {
+  constexpr int kShift = DIG == 256 ? 8 : 11;
+  __shared__ uint32_t cur[DIG];
+  __shared__ int s_lo[kPairT / 64][64];
+  __shared__ uint32_t s_off[kPairT / 64][64];
+  __shared__ uint32_t s_w[kPairT / 64];
+  const uint32_t col = pair_col();
+  for (int d = threadIdx.x; d < DIG; d += kPairT) cur[d] = totals[d];
+  __syncthreads();
+  const uint32_t all = lds_exclusive_scan<kPairT>(cur, DIG, s_w);
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    status->n_pairs = all;
+    if (all > cap_pairs) atomicOr(&status->overflow, 2u);
+  }
+  for (int d = threadIdx.x; d < DIG; d += kPairT) cur[d] += hist[(uint32_t)d * kPairCols + col];
+  __syncthreads();
+  pair_chunk(dkey, wide_list, setup, views, status, cap_tri, TS, s_lo, s_off,
+             [&](uint32_t key, uint32_t i, uint32_t dk) {
+               const uint32_t pos = atomicAdd(&cur[key & (DIG - 1u)], 1u);
+               if (pos < cap_pairs) pairs[pos] = make_uint2((key >> kShift) << 8 | dk, i);
+             });
+}
+
+// Segment d holds the pairs of the tiles d, d + DIG, d + 2 DIG, ...: nh of
+// them.  Counters per (tile, depth level): the depth keys between the
+// segment's smallest and largest, 2^s to a level, with s as small as the
+// counters allow.  Pairs past cap_pairs (flagged by the scatter) are left out.
+constexpr int kSortT = 512, kSortU = 8;
+template <int DIG>
+__global__ __launch_bounds__(kSortT) void k_pair_sort(const uint2* __restrict__ pairs,
+                                                      const uint32_t* __restrict__ totals, uint32_t cap_pairs,
+                                                      uint32_t n_tiles, uint32_t* __restrict__ vals,
+                                                      uint2* __restrict__ ranges) {
+  __shared__ uint32_t cnt[kPairCounters];
+  __shared__ uint32_t s_w[kSortT / 64];
+  __shared__ uint32_t s_mn, s_mx, s_base;
+  const uint32_t d = blockIdx.x, tid = threadIdx.x;
+  const uint32_t nh = d < n_tiles ? (n_tiles - d + DIG - 1u) / DIG : 0u;
+  if (nh == 0u) return;  // the whole block
+  // the segment's start: the sum of the totals before it
+  if (tid == 0) {
+    s_mn = 255u;
+    s_mx = 0u;
+    s_base = 0u;
+  }
+  __syncthreads();
+  uint32_t p = 0;
+  for (uint32_t k = tid; k < d; k += kSortT) p += totals[k];
+#pragma unroll
+  for (int o = 32; o; o >>= 1) p += __shfl_xor(p, o, 64);
+  if ((tid & 63u) == 0u && p) atomicAdd(&s_base, p);
+  __syncthreads();
+  const uint32_t base = min(s_base, cap_pairs);
+  const uint32_t n = min(totals[d], cap_pairs - base);
+  uint2 it[kSortU];
+  auto load = [&](uint32_t t0) {
+#pragma unroll
+    for (int u = 0; u < kSortU; u++) {
+      const uint32_t i = t0 + (uint32_t)(kSortT * u) + tid;
+      it[u] = i < n ? pairs[base + i] : make_uint2(0u, 0u);
+    }
+  };
+  // up to kSortT * kSortU pairs stay in registers, more are read three times
+  constexpr uint32_t kRound = kSortT * kSortU;
+  const bool once = n <= kRound;
+  uint32_t mn = 255u, mx = 0u;
+  for (uint32_t t0 = 0; t0 < n; t0 += kRound) {
+    load(t0);
+#pragma unroll
+    for (int u = 0; u < kSortU; u++)
+      if (t0 + (uint32_t)(kSortT * u) + tid < n) {
+        mn = min(mn, it[u].x & 255u);
+        mx = max(mx, it[u].x & 255u);
+      }
+  }
+#pragma unroll
+  for (int o = 32; o; o >>= 1) {
+    mn = min(mn, (uint32_t)__shfl_xor(mn, o, 64));
+    mx = max(mx, (uint32_t)__shfl_xor(mx, o, 64));
+  }
+  if ((tid & 63u) == 0u) {
+    atomicMin(&s_mn, mn);
+    atomicMax(&s_mx, mx);
+  }
+  __syncthreads();
+  mn = s_mn;
+  mx = max(s_mx, mn);
+  uint32_t s = 0;
+  while ((((mx - mn) >> s) + 1u) * nh > kPairCounters) s++;  // ends: s = 8 leaves one level, nh <= kPairCounters
+  const uint32_t L = ((mx - mn) >> s) + 1u;
+  for (uint32_t k = tid; k < nh * L; k += kSortT) cnt[k] = 0u;
+  __syncthreads();
+  auto slot = [&](uint32_t x) { return (x >> 8) * L + (((x & 255u) - mn) >> s); };
+  for (uint32_t t0 = 0; t0 < n; t0 += kRound) {
+    if (!once) load(t0);
+#pragma unroll
+    for (int u = 0; u < kSortU; u++)
+      if (t0 + (uint32_t)(kSortT * u) + tid < n) atomicAdd(&cnt[slot(it[u].x)], 1u);
+  }
+  __syncthreads();
+  lds_exclusive_scan<kSortT>(cnt, nh * L, s_w);
+  for (uint32_t h = tid; h < nh; h += kSortT)
+    ranges[h * DIG + d] = make_uint2(base + cnt[h * L], base + (h + 1u < nh ? cnt[(h + 1u) * L] : n));
+  __syncthreads();
+  for (uint32_t t0 = 0; t0 < n; t0 += kRound) {
+    if (!once) load(t0);
+#pragma unroll
+    for (int u = 0; u < kSortU; u++)
+      if (t0 + (uint32_t)(kSortT * u) + tid < n) vals[base + atomicAdd(&cnt[slot(it[u].x)], 1u)] = it[u].y;
   }
 }
 
@@ -1834,23 +2058,15 @@ __global__ __launch_bounds__(256) void k_tile_ranges(const uint32_t* __restrict_
 }
 
 // ======================================================== transparent pass
-// First opaque clipped-triangle id of each object group (the same prefix as
-// k_view_id_base, at the group's first opaque input triangle).
-__global__ void k_group_base(const uint32_t* __restrict__ grp_first, uint32_t n_groups, uint32_t n_in,
-                             const uint8_t* __restrict__ cnt, const uint32_t* __restrict__ blk_off,
-                             const Status* __restrict__ status, uint32_t* __restrict__ grp_base) {
-  const uint32_t g = blockIdx.x * blockDim.x + threadIdx.x;
-  if (g >= n_groups) return;
-  const uint32_t t0 = grp_first[g];
-  uint32_t base;
-  if (t0 >= n_in) {
-    base = status->n_out;
-  } else {
-    const uint32_t b = t0 >> 8;
-    base = blk_off[b];
-    for (uint32_t t = b << 8; t < t0; t++) base += cnt[t] & kCntMask;
-  }
-  grp_base[g] = base;
+// First opaque clipped-triangle id of each object group (a wave per group).
+__global__ __launch_bounds__(256) void k_group_base(const uint32_t* __restrict__ grp_first, uint32_t n_groups,
+                                                    uint32_t n_in, const uint8_t* __restrict__ cnt,
+                                                    const uint32_t* __restrict__ blk_off,
+                                                    const Status* __restrict__ status, uint32_t* __restrict__ grp_base) {
+  const uint32_t g = (blockIdx.x * 256u + threadIdx.x) >> 6;
+  if (g >= n_groups) return;  // the whole wave
+  const uint32_t id = wave_id_before(grp_first[g], n_in, cnt, blk_off, status);
+  if ((threadIdx.x & 63u) == 0u) grp_base[g] = id;
 }
 
 // Sort keys of a transparent mesh's triangles (scene/mod.rs:1100-1115): the
@@ -1905,23 +2121,7 @@ void enqueue_mesh_streams(const uint32_t* tri, uint32_t n_tri, const float* pos,
 // n_ranges in the sorted order; not written otherwise.
 int enqueue_radix_sort(uint32_t* const keys[2], uint32_t* const vals[2], const uint32_t* n_ptr, uint32_t cap,
                        int key_bits, uint32_t* hist, uint32_t* partials, hipStream_t s, bool keys_out,
-                       uint2* ranges, uint32_t n_ranges, bool stable) {
-  if (!stable && !keys_out && key_bits <= 11) {
-    if (key_bits <= 8) {
-      const uint32_t nh = 256u * kRadixBG;
-      hipLaunchKernelGGL(k_radix_hist_blk<256>, dim3(kRadixBG), dim3(kRadixBT), 0, s, keys[0], n_ptr, cap, hist);
-      scan_u32(hist, hist, nullptr, nh, nh, partials, nullptr, 0, nullptr, 0, s);
-      hipLaunchKernelGGL(k_radix_scatter_blk<256>, dim3(kRadixBG), dim3(kRadixBT), 0, s, keys[0], vals[0], vals[1],
-                         n_ptr, cap, hist, ranges, ranges ? n_ranges : 0u);
-    } else {
-      const uint32_t nh = 2048u * kRadixBG;
-      hipLaunchKernelGGL(k_radix_hist_blk<2048>, dim3(kRadixBG), dim3(kRadixBT), 0, s, keys[0], n_ptr, cap, hist);
-      scan_u32(hist, hist, nullptr, nh, nh, partials, nullptr, 0, nullptr, 0, s);
-      hipLaunchKernelGGL(k_radix_scatter_blk<2048>, dim3(kRadixBG), dim3(kRadixBT), 0, s, keys[0], vals[0], vals[1],
-                         n_ptr, cap, hist, ranges, ranges ? n_ranges : 0u);
-    }
-    return 1;
-  }
+                       uint2* ranges, uint32_t n_ranges) {
   int cur = 0;
   // one 8-bit pass for keys of up to 8 bits, one 11-bit pass up to 11 bits
   const bool one_pass = key_bits > 8 && key_bits <= 11;
@@ -1976,17 +2176,22 @@ static void join(hipStream_t s, const PipeArgs& a, int i) {
 // Status reset, geometry, view bases and binning of one pipeline pass;
 // returns the arguments the per-tile stages read (tile lists in b.vals[0]).
 PipeArgs enqueue_front(const PipeArgs& a, hipStream_t s) {
-  // near-first lists keep the depth sort in keys[1] / vals[1] (behind the
-  // wide-triangle list), which needs cap_pairs >= 3 cap_tri
-  const bool depth_sorted = a.ordered_bins && a.depth_order && (uint64_t)a.cap_pairs >= 3ull * a.cap_tri;
+  // near-first lists (k_pair_*); a frame of more tiles than their counters
+  // take is binned in submission order
+  const bool near = a.ordered_bins && a.depth_order && a.n_tiles <= kPairMaxTiles;
   // a small single-view frame is binned by one workgroup (k_bin_small)
-  const bool small_bins = depth_sorted && a.n_views == 1 && a.n_tiles <= kSmallBinTiles &&
+  const bool small_bins = near && a.n_views == 1 && a.n_tiles <= kSmallBinTiles &&
                           a.n_tri_in <= kSmallBinTris;
   if (a.ev[0]) (void)hipEventRecord(a.ev[0], s);
   hipLaunchKernelGGL(k_frame_begin, dim3(a.tables_src ? std::min<uint32_t>(cdiv(a.tables_words, 1024), 64u) : 1u),
                      dim3(256), 0, s, reinterpret_cast<uint32_t*>(a.status), (uint32_t)(sizeof(Status) / 4),
                      a.tables_src, a.tables_dst, a.tables_src ? a.tables_words : 0u);
   const uint32_t n_blk = cdiv(a.n_tri_in, 256);
+  uint8_t* const wflag = reinterpret_cast<uint8_t*>(a.big);
+  // the wide-triangle list: near first in vals[1], which the pair kernels
+  // leave alone; else in keys[1] until the radix sort needs it (both hold
+  // cap_pairs >= cap_tri entries)
+  uint32_t* const wide_list = near ? a.vals[1] : a.keys[1];
   // a small single-view frame: one workgroup builds the emitter lists, and
   // both emits share one launch on this stream
   const bool small_geom = a.n_views == 1 && a.n_tri_in <= kSmallBinTris;
@@ -1994,40 +2199,31 @@ PipeArgs enqueue_front(const PipeArgs& a, hipStream_t s) {
   if (n_blk && small_geom) {
     hipLaunchKernelGGL(k_geom_small, dim3(1), dim3(1024), 0, s, a.draws, a.n_draws, a.views, a.n_tri_in, a.cnt, a.blk,
                        a.status, a.cap_tri, a.surv);
-    uint8_t* wf = reinterpret_cast<uint8_t*>(a.big);
-    uint32_t* dk = depth_sorted && !small_bins ? a.keys[1] + a.cap_tri : nullptr;
     const uint32_t g_simple = n_blk, g_clip = n_blk;
-    if (a.ordered_bins)
-      hipLaunchKernelGGL(k_geom_emit_both<true>, dim3(g_clip + g_simple), dim3(256), 0, s, a.draws, a.n_draws,
-                         a.views, a.surv, a.mats, a.setup, a.shade, a.cap_tri, a.status, a.TS, a.bincnt, wf, dk,
-                         g_clip);
+    if (near)
+      hipLaunchKernelGGL(k_geom_emit_both<kBinNear>, dim3(g_clip + g_simple), dim3(256), 0, s, a.draws, a.n_draws,
+                         a.views, a.surv, a.mats, a.setup, a.shade, a.cap_tri, a.status, a.TS, nullptr, wflag,
+                         wide_list, g_clip);
+    else if (a.ordered_bins)
+      hipLaunchKernelGGL(k_geom_emit_both<kBinSubmit>, dim3(g_clip + g_simple), dim3(256), 0, s, a.draws, a.n_draws,
+                         a.views, a.surv, a.mats, a.setup, a.shade, a.cap_tri, a.status, a.TS, a.bincnt, wflag,
+                         nullptr, g_clip);
     else
-      hipLaunchKernelGGL(k_geom_emit_both<false>, dim3(g_clip + g_simple), dim3(256), 0, s, a.draws, a.n_draws,
+      hipLaunchKernelGGL(k_geom_emit_both<kBinNone>, dim3(g_clip + g_simple), dim3(256), 0, s, a.draws, a.n_draws,
                          a.views, a.surv, a.mats, a.setup, a.shade, a.cap_tri, a.status, a.TS, nullptr, nullptr,
                          nullptr, g_clip);
   } else if (n_blk) {
-    uint32_t* blk_simple = a.blk + n_blk + 1;
-    uint32_t* blk_clip = a.blk + 2 * (n_blk + 1);
+    uint32_t* blk_simple = a.blk + geom_blk_stride(n_blk);
+    uint32_t* blk_clip = a.blk + 2 * geom_blk_stride(n_blk);
     hipLaunchKernelGGL(k_geom_count, dim3(n_blk), dim3(256), 0, s, a.draws, a.n_draws, a.views, a.n_tri_in, a.cnt,
                        a.blk, blk_simple, blk_clip);
-    if (n_blk <= 4096u) {
-      ScanSegs g{};
-      g.s[0] = ScanSeg{a.blk, a.blk, &a.status->n_out, &a.status->overflow, a.cap_tri, 1u};
-      g.s[1] = ScanSeg{blk_simple, blk_simple, &a.status->n_simple, nullptr, 0u, 0u};
-      g.s[2] = ScanSeg{blk_clip, blk_clip, &a.status->n_clip, nullptr, 0u, 0u};
-      hipLaunchKernelGGL(k_scan_small, dim3(3), dim3(1024), 0, s, g, n_blk);
-    } else {
-      scan_u32(a.blk, a.blk, nullptr, n_blk, n_blk, a.partials, &a.status->n_out, a.cap_tri, &a.status->overflow,
-               1u, s);
-      scan_u32(blk_simple, blk_simple, nullptr, n_blk, n_blk, a.partials, &a.status->n_simple, 0u, nullptr, 0u, s);
-      scan_u32(blk_clip, blk_clip, nullptr, n_blk, n_blk, a.partials, &a.status->n_clip, 0u, nullptr, 0u, s);
-    }
+    ScanSegs g{};
+    g.s[0] = ScanSeg{a.blk, a.blk, &a.status->n_out, &a.status->overflow, a.cap_tri, 1u};
+    g.s[1] = ScanSeg{blk_simple, blk_simple, &a.status->n_simple, nullptr, 0u, 0u};
+    g.s[2] = ScanSeg{blk_clip, blk_clip, &a.status->n_clip, nullptr, 0u, 0u};
+    hipLaunchKernelGGL(k_scan_segs, dim3(3), dim3(1024), 0, s, g, n_blk);
     hipLaunchKernelGGL(k_geom_compact, dim3(n_blk), dim3(256), 0, s, a.n_tri_in, a.cnt, a.blk, blk_simple, blk_clip,
                        a.status, a.surv);
-    // ordered bins: the per-triangle tile counts and wide flags come with the
-    // records, and for near-first lists each record's depth key
-    uint8_t* wf = reinterpret_cast<uint8_t*>(a.big);
-    uint32_t* dk = depth_sorted && !small_bins ? a.keys[1] + a.cap_tri : nullptr;
     // the unclipped and clipped emits write disjoint outputs: the clipped
     // one runs beside the other on the side stream.  Capped grids (the lists'
     // lengths are on the device): 2048 and 1024 blocks, a grid-stride loop
@@ -2037,77 +2233,77 @@ PipeArgs enqueue_front(const PipeArgs& a, hipStream_t s) {
     const hipStream_t s2 = fork(s, a, 0);
     // (the clipped emit, the longer one per thread, starts first on the main
     // stream; the unclipped one waits for the fork on the side stream)
-    if (a.ordered_bins) {
-      hipLaunchKernelGGL((k_geom_emit<true, true>), dim3(g_clip), dim3(256), 0, s, a.draws, a.n_draws, a.views,
-                         a.surv, a.mats, a.setup, a.shade, a.cap_tri, a.status, a.TS, a.bincnt, wf, dk, span);
-      hipLaunchKernelGGL((k_geom_emit<true, false>), dim3(g_simple), dim3(256), 0, s2, a.draws, a.n_draws, a.views,
-                         a.surv, a.mats, a.setup, a.shade, a.cap_tri, a.status, a.TS, a.bincnt, wf, dk, span);
+    if (near) {
+      hipLaunchKernelGGL((k_geom_emit<kBinNear, true>), dim3(g_clip), dim3(256), 0, s, a.draws, a.n_draws, a.views,
+                         a.surv, a.mats, a.setup, a.shade, a.cap_tri, a.status, a.TS, nullptr, wflag, wide_list, span);
+      hipLaunchKernelGGL((k_geom_emit<kBinNear, false>), dim3(g_simple), dim3(256), 0, s2, a.draws, a.n_draws, a.views,
+                         a.surv, a.mats, a.setup, a.shade, a.cap_tri, a.status, a.TS, nullptr, wflag, wide_list, span);
+    } else if (a.ordered_bins) {
+      hipLaunchKernelGGL((k_geom_emit<kBinSubmit, true>), dim3(g_clip), dim3(256), 0, s, a.draws, a.n_draws, a.views,
+                         a.surv, a.mats, a.setup, a.shade, a.cap_tri, a.status, a.TS, a.bincnt, wflag, nullptr, span);
+      hipLaunchKernelGGL((k_geom_emit<kBinSubmit, false>), dim3(g_simple), dim3(256), 0, s2, a.draws, a.n_draws, a.views,
+                         a.surv, a.mats, a.setup, a.shade, a.cap_tri, a.status, a.TS, a.bincnt, wflag, nullptr, span);
     } else {
-      hipLaunchKernelGGL((k_geom_emit<false, true>), dim3(g_clip), dim3(256), 0, s, a.draws, a.n_draws, a.views,
+      hipLaunchKernelGGL((k_geom_emit<kBinNone, true>), dim3(g_clip), dim3(256), 0, s, a.draws, a.n_draws, a.views,
                          a.surv, a.mats, a.setup, a.shade, a.cap_tri, a.status, a.TS, nullptr, nullptr, nullptr, span);
-      hipLaunchKernelGGL((k_geom_emit<false, false>), dim3(g_simple), dim3(256), 0, s2, a.draws, a.n_draws, a.views,
+      hipLaunchKernelGGL((k_geom_emit<kBinNone, false>), dim3(g_simple), dim3(256), 0, s2, a.draws, a.n_draws, a.views,
                          a.surv, a.mats, a.setup, a.shade, a.cap_tri, a.status, a.TS, nullptr, nullptr, nullptr, span);
     }
     join(s, a, 1);
   }
   if (a.n_views > 1)
-    hipLaunchKernelGGL(k_view_id_base, dim3(cdiv(a.n_views, 256)), dim3(256), 0, s, const_cast<DevView*>(a.views),
+    hipLaunchKernelGGL(k_view_id_base, dim3(cdiv(a.n_views, 4)), dim3(256), 0, s, const_cast<DevView*>(a.views),
                        a.n_views, a.n_tri_in, a.cnt, a.blk, a.status);
   if (a.ev[1]) (void)hipEventRecord(a.ev[1], s);
   // 4-8 binning
   const uint32_t gb = std::min<uint32_t>(cdiv(a.cap_tri, 256), 4096u);
-  uint8_t* wflag = reinterpret_cast<uint8_t*>(a.big);
-  // the wide-triangle list lives in keys[1] until the radix sort needs it
-  // (cap_pairs >= cap_tri); a wave per listed triangle, up to 16384 waves
-  uint32_t* wide_list = a.keys[1];
   const uint32_t gl = std::min<uint32_t>(cdiv(a.cap_tri, 4096), 1024u);
   const uint32_t gw = std::min<uint32_t>(cdiv(a.cap_tri, 64), 4096u);
   PipeArgs b = a;
   if (small_bins) {
     hipLaunchKernelGGL(k_bin_small, dim3(1), dim3(1024), 0, s, a.setup, a.views, a.status, a.cap_tri, a.TS, wflag,
                        wide_list, a.n_tiles, a.cap_pairs, a.vals[0], a.ranges);
-  } else if (a.ordered_bins) {
-    // the wide-triangle list and counts (keys[1][0, cap_tri), bincnt) beside
-    // the depth sort (keys[1] + cap_tri .., vals[1], hist, partials)
-    const hipStream_t s2 = depth_sorted ? fork(s, a, 2) : s;
-    hipLaunchKernelGGL(k_wide_list, dim3(gl), dim3(256), 0, s2, wflag, a.status, a.cap_tri, wide_list,
-                       reinterpret_cast<uint32_t*>(a.ranges), 2u * a.n_tiles);
-    hipLaunchKernelGGL(k_bin_count_wide<true>, dim3(gw), dim3(256), 0, s2, a.setup, a.views, a.status, a.TS,
-                       wide_list, a.bincnt, a.tile_cnt);
-    if (depth_sorted) {
-      // near first: the clipped triangles in depth-key order (one 8-bit
-      // pass over keys[1] + cap_tri, the values the triangle ids themselves,
-      // in chunk order within a key; results in vals[1] + cap_tri, the
-      // sorted keys not written), then the bin offsets in that order
-      uint32_t* const dkeys[2] = {a.keys[1] + a.cap_tri, a.keys[1] + 2ull * a.cap_tri};
-      uint32_t* const dvals[2] = {nullptr, a.vals[1] + a.cap_tri};
-      const int dc = enqueue_radix_sort(dkeys, dvals, &a.status->n_out, a.cap_tri, kDepthKeyBits, a.hist,
-                                        a.partials, s, false, nullptr, 0u, false);
-      join(s, a, 3);
-      uint32_t* order = dvals[dc];
-      // the scan of the counts in that order: its chunk sums here, the rest
-      // inside the pair emit
-      hipLaunchKernelGGL(k_scan_reduce, dim3(kScanG), dim3(256), 0, s, a.bincnt, &a.status->n_out, 0u, a.cap_tri,
-                         a.partials, order);
-      hipLaunchKernelGGL(k_bin_emit_near, dim3(kScanG), dim3(256), 0, s, a.status, a.cap_tri, wflag, a.binoff,
-                         order, a.bincnt, a.partials, a.cap_pairs, a.keys[0], a.vals[0]);
+  } else if (near) {
+    uint2* const pairs = reinterpret_cast<uint2*>(a.keys[0]);  // keys[0] and keys[1] are one buffer
+    const bool few = a.n_tiles <= kPairFewTiles;
+    const uint32_t dig = few ? 256u : 2048u;
+    uint32_t* const totals = a.hist + (size_t)dig * kPairCols;
+    const dim3 gp(kPairCols), bp(kPairT);
+    if (few)
+      hipLaunchKernelGGL(k_pair_hist<256>, gp, bp, 0, s, wflag, wide_list, a.setup, a.views, a.status, a.cap_tri, a.TS,
+                         a.hist);
+    else
+      hipLaunchKernelGGL(k_pair_hist<2048>, gp, bp, 0, s, wflag, wide_list, a.setup, a.views, a.status, a.cap_tri,
+                         a.TS, a.hist);
+    hipLaunchKernelGGL(k_row_scan, dim3(dig), dim3(kPairCols), 0, s, a.hist, totals);
+    if (few) {
+      hipLaunchKernelGGL(k_pair_scatter<256>, gp, bp, 0, s, wflag, wide_list, a.setup, a.views, a.status, a.cap_tri,
+                         a.TS, a.hist, totals, a.cap_pairs, pairs);
+      hipLaunchKernelGGL(k_pair_sort<256>, dim3(dig), dim3(kSortT), 0, s, pairs, totals, a.cap_pairs, a.n_tiles,
+                         a.vals[0], a.ranges);
     } else {
-      scan_u32(a.bincnt, a.binoff, &a.status->n_out, 0, a.cap_tri, a.partials, &a.status->n_pairs, a.cap_pairs,
-               &a.status->overflow, 2u, s);
-      hipLaunchKernelGGL(k_bin_emit<true>, dim3(gb), dim3(256), 0, s, a.setup, a.views, a.status, a.cap_tri, a.TS,
-                         wflag, a.binoff, a.tile_start, a.tile_cur, a.cap_pairs, a.keys[0], a.vals[0]);
+      hipLaunchKernelGGL(k_pair_scatter<2048>, gp, bp, 0, s, wflag, wide_list, a.setup, a.views, a.status, a.cap_tri,
+                         a.TS, a.hist, totals, a.cap_pairs, pairs);
+      hipLaunchKernelGGL(k_pair_sort<2048>, dim3(dig), dim3(kSortT), 0, s, pairs, totals, a.cap_pairs, a.n_tiles,
+                         a.vals[0], a.ranges);
     }
+  } else if (a.ordered_bins) {
+    hipLaunchKernelGGL(k_wide_list, dim3(gl), dim3(256), 0, s, wflag, a.status, a.cap_tri, wide_list,
+                       reinterpret_cast<uint32_t*>(a.ranges), 2u * a.n_tiles);
+    hipLaunchKernelGGL(k_bin_count_wide<true>, dim3(gw), dim3(256), 0, s, a.setup, a.views, a.status, a.TS,
+                       wide_list, a.bincnt, a.tile_cnt);
+    scan_u32(a.bincnt, a.binoff, &a.status->n_out, 0, a.cap_tri, a.partials, &a.status->n_pairs, a.cap_pairs,
+             &a.status->overflow, 2u, s);
+    hipLaunchKernelGGL(k_bin_emit<true>, dim3(gb), dim3(256), 0, s, a.setup, a.views, a.status, a.cap_tri, a.TS,
+                       wflag, a.binoff, a.tile_start, a.tile_cur, a.cap_pairs, a.keys[0], a.vals[0]);
     hipLaunchKernelGGL(k_bin_emit_wide<true>, dim3(gw), dim3(256), 0, s, a.setup, a.views, a.status, wide_list,
                        a.TS, a.binoff, a.tile_start, a.tile_cur, a.cap_pairs, a.keys[0], a.vals[0]);
     // radix sort by tile key (one pass when the key has at most 11 bits, else
     // stable 8-bit passes), then the tile ranges: from the one pass's scanned
-    // histogram, else from the sorted keys.  Near-first lists take the one
-    // pass with free order within a chunk of the depth order;
-    // submission-ordered lists stay stable.
+    // histogram, else from the sorted keys
     const bool one_pass = a.key_bits <= 11;
     const int cur = enqueue_radix_sort(a.keys, a.vals, &a.status->n_pairs, a.cap_pairs, a.key_bits, a.hist,
-                                       a.partials, s, !one_pass, one_pass ? a.ranges : nullptr, a.n_tiles,
-                                       !depth_sorted);
+                                       a.partials, s, !one_pass, one_pass ? a.ranges : nullptr, a.n_tiles);
     b.vals[0] = a.vals[cur];
     if (!one_pass)
       hipLaunchKernelGGL(k_tile_ranges, dim3(std::min<uint32_t>(cdiv(a.cap_pairs, 256), 4096u)), dim3(256), 0, s,
@@ -2139,7 +2335,7 @@ PipeArgs enqueue_front(const PipeArgs& a, hipStream_t s) {
 // reference's sort_by on the mesh's triangle vector does.
 void enqueue_transparent_prep(const PipeArgs& opaque, const TransArgs& t, hipStream_t s) {
   if (t.n_groups)
-    hipLaunchKernelGGL(k_group_base, dim3(cdiv(t.n_groups, 256)), dim3(256), 0, s, t.grp_first, t.n_groups,
+    hipLaunchKernelGGL(k_group_base, dim3(cdiv(t.n_groups, 4)), dim3(256), 0, s, t.grp_first, t.n_groups,
                        opaque.n_tri_in, opaque.cnt, opaque.blk, opaque.status, t.grp_base);
   for (uint32_t m = 0; m < t.n_meshes; m++) {
     const TransMesh& tm = t.meshes[m];

@@ -6,6 +6,8 @@
 namespace dh {
 
 constexpr uint32_t kRadixHistEntries = 2048u * 1024u;  // (up to 11-bit) digits x radix-sort waves
+// words between the three segments of per-block geometry counts
+__host__ __device__ constexpr uint64_t geom_blk_stride(uint64_t n_blk) { return n_blk + 1u; }
 
 struct PipeArgs {
   // inputs
@@ -23,8 +25,8 @@ struct PipeArgs {
   int raster_kind;     // 0: waves own 8x8 quadrants; 1: triangle-parallel rectangle sweeps
   // scratch
   uint8_t* cnt;        // [n_tri_in] clipped-triangle count per input triangle
-  uint32_t* blk;       // [3 * (ceil(n_tri_in/256) + 1)] per-block counts -> offsets: clipped triangles,
-                       // then (each ceil(n_tri_in/256) + 1 further) unclipped and clipped emitters
+  uint32_t* blk;       // [3 * geom_blk_stride(ceil(n_tri_in/256))] per-block counts -> offsets: clipped
+                       // triangles, then (each a stride further) unclipped and clipped emitters
   uint2* surv;         // [n_tri_in] (input triangle, first output id) of the emitting triangles: the
                        // unclipped ones in order, then the clipped ones in order
   SetupRec* setup;     // [cap_tri]
@@ -32,18 +34,19 @@ struct PipeArgs {
   uint32_t cap_tri;
   uint32_t* bincnt;    // [cap_tri]
   uint32_t* binoff;    // [cap_tri]
-  uint32_t* big;       // [3 cap_tri + 4] words: a byte per triangle (1 = wide, binned by a wave; 2 =
-                       // dropped), then 16-byte aligned an 8-byte bin box per triangle (ordered bins)
+  uint32_t* big;       // [3 cap_tri + 4] words: a byte per triangle (near-first bins: its depth key; else
+                       // 1 = wide, binned by a wave; 2 = dropped), then 16-byte aligned an 8-byte bin box
+                       // per triangle (ordered bins)
   bool ordered_bins;   // stable radix sort (per-tile lists in submission order)
   bool shade_in_raster;  // kind 0 rasters shade their own tiles (no visibility buffer, no k_shade)
-  bool depth_order;    // ordered bins: per-tile lists near first (triangles sorted by depth key before binning)
+  bool depth_order;    // ordered bins: per-tile lists near first (k_pair_*)
   uint32_t* tile_cnt;  // [2 * n_tiles] per-tile counts, then per-tile cursors
   uint32_t* tile_cur;  // = tile_cnt + n_tiles
   uint32_t* tile_start;  // [n_tiles] exclusive scan of tile_cnt
-  uint32_t* keys[2];   // [cap_pairs] each
+  uint32_t* keys[2];   // [cap_pairs] each, adjacent: one array of 8-byte pairs for the near-first lists
   uint32_t* vals[2];
   uint32_t cap_pairs;
-  uint32_t* hist;      // [256 * kRadixG]
+  uint32_t* hist;      // [kRadixHistEntries]
   uint32_t* partials;  // [1024]
   uint2* ranges;       // [n_tiles]
   uint32_t* vis;       // [n_pixels] winner id per pixel
@@ -56,9 +59,9 @@ struct PipeArgs {
   hipEvent_t ev[5];    // optional stage events (all null when not profiling)
   // independent kernels fork onto `side` (null: everything on the main
   // stream) and join back with xev[] (fork 0 / join 1: the two geometry
-  // emits; fork 2 / join 3: the wide-triangle counts beside the depth sort)
+  // emits)
   hipStream_t side;
-  hipEvent_t xev[4];
+  hipEvent_t xev[2];
 };
 
 // One transparent mesh (device pointers): its triangles, sorted in place.
@@ -93,7 +96,7 @@ void enqueue_mesh_streams(const uint32_t* tri, uint32_t n_tri, const float* pos,
                           float* soa, hipStream_t s);
 int enqueue_radix_sort(uint32_t* const keys[2], uint32_t* const vals[2], const uint32_t* n_ptr, uint32_t cap,
                        int key_bits, uint32_t* hist, uint32_t* partials, hipStream_t s, bool keys_out,
-                       uint2* ranges, uint32_t n_ranges, bool stable = true);
+                       uint2* ranges, uint32_t n_ranges);
 void enqueue_transparent_prep(const PipeArgs& opaque, const TransArgs& t, hipStream_t s);
 void enqueue_blend(const PipeArgs& b, const TransArgs& t, hipStream_t s);
 bool raster_config_supported(int TS, int waves, int kind);
