@@ -116,7 +116,7 @@ struct alignas(16) SetupRec {
   float ea[4];            // edge bc (alpha): A, B, C, D
   float eb[4];            // edge ca (beta)
   float eg[4];            // edge ab (gamma)
-  float f[4];             // f_alpha, f_beta, f_gama, (unused)
+  float f[4];             // f_alpha, f_beta, f_gama; kUvSafe: RN(1 / f_alpha), else 0
   float d[4];             // a_depth, b_depth, c_depth, (unused)
   uint32_t rx, ry;        // x0 | x1 << 16, y0 | y1 << 16 (inclusive scan rectangle)
   uint32_t flags, view;
@@ -170,8 +170,25 @@ __host__ __device__ inline uint64_t f2usize(float v) {
   if (v >= 18446744073709551616.0f) return ~0ull;
   return (uint64_t)v;
 }
+// e / f, correctly rounded, from y = RN(1 / f): Markstein's sequence (IBM J.
+// Res. Dev. 34, 1990).  With y correctly rounded, e y is within 1.5 ulp of the
+// quotient, the first residual step brings it within one ulp, and a second one
+// from there gives the correctly rounded quotient.  For integers e, f below
+// 2^24 in magnitude no step under- or overflows.  5 instructions; the general
+// division takes some 10, one of them at quarter rate.
+__host__ __device__ inline float div_known(float e, float f, float y) {
+  float q = e * y;
+  q = fmaf(fmaf(-q, f, e), y, q);
+  return fmaf(fmaf(-q, f, e), y, q);
+}
+
 // Rust `f32 as u8`.
 __host__ __device__ inline uint32_t f2u8(float v) {
+#ifdef __HIP_DEVICE_COMPILE__
+  uint32_t u;  // truncates, saturates and takes NaN to 0, as the cast does
+  asm("v_cvt_u32_f32 %0, %1" : "=v"(u) : "v"(v));
+  return u < 255u ? u : 255u;
+#endif
   if (!(v > 0.0f)) return 0;
   if (v >= 255.0f) return 255;
   return (uint32_t)v;

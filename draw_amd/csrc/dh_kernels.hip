@@ -471,7 +471,10 @@ __device__ inline void make_setup(const FrameParamsPod& fr, const FV& A, const F
     rec.eb[k] = eb[k];
     rec.eg[k] = eg[k];
   }
-  rec.f[0] = fa; rec.f[1] = fb; rec.f[2] = fg; rec.f[3] = 0.0f;
+  rec.f[0] = fa; rec.f[1] = fb; rec.f[2] = fg;
+  // with `exact` the three normalizers are one value (twice the signed area),
+  // an integer below 2^24: its reciprocal stands for three divisions a pixel
+  rec.f[3] = (flags & kUvSafe) ? 1.0f / fa : 0.0f;
   rec.d[0] = A.d; rec.d[1] = B.d; rec.d[2] = C.d; rec.d[3] = zlb;
   rec.rx = x0 | (x1 << 16);
   rec.ry = y0 | (y1 << 16);
@@ -2366,10 +2369,12 @@ void enqueue_status_out(const Status* dev, Status* host_dev_ptr, uint32_t n, hip
 // One shard of a sort-last frame: geometry, binning, raster, then the packed
 // u64 visibility (no shading: dh_shade_shard shades after the merge).
 void enqueue_visibility(const PipeArgs& a, uint32_t shard, uint64_t* out, hipStream_t s) {
-  const PipeArgs b = enqueue_front(a, s);
+  PipeArgs b = enqueue_front(a, s);
+  b.pack_out = out;
+  b.pack_tag = shard << kShardShift;
   enqueue_raster(b, s);
   if (a.ev[3]) (void)hipEventRecord(a.ev[3], s);
-  enqueue_vis_pack(a, shard, out, s);
+  if (a.raster_kind != 0) enqueue_vis_pack(a, shard, out, s);
   if (a.ev[4]) (void)hipEventRecord(a.ev[4], s);
 }
 

@@ -50,6 +50,8 @@ struct PipeArgs {
   uint32_t* partials;  // [1024]
   uint2* ranges;       // [n_tiles]
   uint32_t* vis;       // [n_pixels] winner id per pixel
+  uint64_t* pack_out;  // [n_pixels] packed visibility of a shard frame (kind-0 rasters that do not shade)
+  uint32_t pack_tag;   // shard << kShardShift
   Status* status;
   // the frame's draw/view tables, copied by the frame's first kernel from
   // coherent pinned host memory (tables_src: its device address; null: none)

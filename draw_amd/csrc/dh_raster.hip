@@ -18,9 +18,16 @@ struct FragOut {
 // Barycentrics and depth at a pixel, canvas.rs:673-682.
 __device__ inline FragOut bary(const SetupRec& r, float x, float y) {
   FragOut o;
-  o.al = edge_eval(r.ea, x, y) / r.f[0];
-  o.be = edge_eval(r.eb, x, y) / r.f[1];
-  o.ga = edge_eval(r.eg, x, y) / r.f[2];
+  const float ea = edge_eval(r.ea, x, y), eb = edge_eval(r.eb, x, y), eg = edge_eval(r.eg, x, y);
+  if (r.f[3] != 0.0f) {  // exact integers and one normalizer (make_setup)
+    o.al = div_known(ea, r.f[0], r.f[3]);
+    o.be = div_known(eb, r.f[0], r.f[3]);
+    o.ga = div_known(eg, r.f[0], r.f[3]);
+  } else {
+    o.al = ea / r.f[0];
+    o.be = eb / r.f[1];
+    o.ga = eg / r.f[2];
+  }
   o.d = (o.al * r.d[0] + o.be * r.d[1]) + o.ga * r.d[2];
   return o;
 }
@@ -63,133 +70,191 @@ __device__ inline uint32_t wave_max_u32(uint32_t v) {
 }
 
 // ===================================================================== shade
-__device__ inline void fetch_rgb(const uint8_t* img, int32_t comp, uint64_t off, uint32_t c[3]) {
-  if (comp == 4) {
-    const uint32_t w = *reinterpret_cast<const uint32_t*>(img + off);
-    c[0] = w & 255u; c[1] = (w >> 8) & 255u; c[2] = (w >> 16) & 255u;
-  } else {
-    c[0] = img[off]; c[1] = img[off + 1]; c[2] = img[off + 2];
-  }
+// k / 255 for every byte k (Pixel::normalized_as_vec3, canvas.rs:81-87), in an
+// LDS table that the shading reads, the block's nt threads filling it together.
+// The caller places a barrier between the fill and the first shade_pixel.
+__device__ inline void fill_unit_table(float* unit, int tid, int nt) {
+  constexpr float kInv = 1.0f / 255.0f;
+  for (int k = tid; k < 256; k += nt) unit[k] = div_known((float)k, 255.0f, kInv);
 }
 
-// k / 255 for every byte k (Pixel::normalized_as_vec3, canvas.rs:81-87),
-// divided once per workgroup into an LDS table that the shading reads, the
-// block's nt threads filling it together.  The caller places a barrier
-// between the fill and the first shade_pixel.
-__device__ inline void fill_unit_table(float* unit, int tid, int nt) {
-  for (int k = tid; k < 256; k += nt) unit[k] = (float)k / 255.0f;
+// TextureMap::get_rgb_slice's byte offset (rgb_offset) in 32-bit arithmetic:
+// true where the floored coordinates lie in the map, which most do; ok as
+// rgb_offset returns it.  small: the map has fewer than 2^32 bytes.
+__device__ __forceinline__ bool rgb_offset_in_map(int32_t w, int32_t h, int32_t comp, float u, float v, bool small,
+                                         uint32_t* off) {
+  const float mu = (float)w - 1.0f, mv = (float)h - 1.0f;
+  // f32 as usize: NaN and negatives are 0
+  const float fu = fmaxf(floorf(u * mu), 0.0f), fv = fmaxf(floorf(v * mv), 0.0f);
+  *off = (((uint32_t)h - 1u - (uint32_t)fv) * (uint32_t)w + (uint32_t)fu) * (uint32_t)comp;
+  return small && fu <= mu && fv <= mv;
+}
+__device__ inline bool small_map(int32_t w, int32_t h, int32_t comp) {
+  return (uint64_t)w * (uint64_t)h * (uint64_t)comp < 0xFFFFFFFFull;
+}
+
+__device__ inline uint32_t fetch_rgb(const uint8_t* img, int32_t comp, uint64_t off) {
+  if (comp == 4) return *reinterpret_cast<const uint32_t*>(img + off);
+  return (uint32_t)img[off] | ((uint32_t)img[off + 1] << 8) | ((uint32_t)img[off + 2] << 16);
 }
 
 // Shading of a covered pixel, canvas.rs:685-741; returns B | G<<8 | R<<16 | A<<24.
 // unit: the k / 255 table (fill_unit_table).
-__device__ inline uint32_t shade_pixel(const ShadeRec& s, const DevMaterial& m, const FragOut& o, Status* status,
+__device__ __forceinline__ uint32_t shade_pixel(const ShadeRec& s, const DevMaterial& m, const FragOut& o, Status* status,
                                        const float* unit) {
   const float u = (s.uv[0] * o.al + s.uv[2] * o.be) + s.uv[4] * o.ga;
   const float v = (s.uv[1] * o.al + s.uv[3] * o.be) + s.uv[5] * o.ga;
-  uint64_t okd, oka;
-  const bool ok1 = rgb_offset(m.kd_w, m.kd_h, m.kd_comp, u, v, &okd);
-  const bool ok2 = rgb_offset(m.ka_w, m.ka_h, m.ka_comp, u, v, &oka);
-  if (!(ok1 && ok2)) {
-    atomicOr(&status->error, 1u);
-    okd = 0;
-    oka = 0;
+  uint32_t skd, ska;
+  const bool in1 = rgb_offset_in_map(m.kd_w, m.kd_h, m.kd_comp, u, v, small_map(m.kd_w, m.kd_h, m.kd_comp), &skd);
+  const bool in2 = rgb_offset_in_map(m.ka_w, m.ka_h, m.ka_comp, u, v, small_map(m.ka_w, m.ka_h, m.ka_comp), &ska);
+  uint64_t okd = skd, oka = ska;
+  if (!(in1 && in2)) {
+    const bool ok1 = rgb_offset(m.kd_w, m.kd_h, m.kd_comp, u, v, &okd);
+    const bool ok2 = rgb_offset(m.ka_w, m.ka_h, m.ka_comp, u, v, &oka);
+    if (!(ok1 && ok2)) {
+      atomicOr(&status->error, 1u);
+      okd = 0;
+      oka = 0;
+    }
   }
-  uint32_t dk[3], ak[3];
-  fetch_rgb(m.kd_img, m.kd_comp, okd, dk);
-  fetch_rgb(m.ka_img, m.ka_comp, oka, ak);
-  const V3 diffuse = v3(unit[dk[0]], unit[dk[1]], unit[dk[2]]);
-  const V3 ambient = v3(unit[ak[0]], unit[ak[1]], unit[ak[2]]);
+  const uint32_t dk = fetch_rgb(m.kd_img, m.kd_comp, okd), ak = fetch_rgb(m.ka_img, m.ka_comp, oka);
   const V3 pn = add(add(muls(v3(s.n[0], s.n[1], s.n[2]), o.al), muls(v3(s.n[3], s.n[4], s.n[5]), o.be)),
                     muls(v3(s.n[6], s.n[7], s.n[8]), o.ga));
   const V3 pl = add(add(muls(v3(s.l[0], s.l[1], s.l[2]), o.al), muls(v3(s.l[3], s.l[4], s.l[5]), o.be)),
                     muls(v3(s.l[6], s.l[7], s.l[8]), o.ga));
-  const V3 ph = add(add(muls(v3(s.h[0], s.h[1], s.h[2]), o.al), muls(v3(s.h[3], s.h[4], s.h[5]), o.be)),
-                    muls(v3(s.h[6], s.h[7], s.h[8]), o.ga));
-  const V3 c_l = v3(m.ks[0], m.ks[1], m.ks[2]);
-  const V3 c_r = v3(diffuse.x * m.kd[0], diffuse.y * m.kd[1], diffuse.z * m.kd[2]);
-  const V3 c_a = v3(ambient.x * m.ka[0], ambient.y * m.ka[1], ambient.z * m.ka[2]);
   const float dln = dot(pl, pn);
   const float mx = (dln > 0.0f) ? dln : 0.0f;  // 0.0_f32.max(x); the sign of a zero is irrelevant below
   const float sfac = 1.0f - mx;
+  const V3 ph = add(add(muls(v3(s.h[0], s.h[1], s.h[2]), o.al), muls(v3(s.h[3], s.h[4], s.h[5]), o.be)),
+                    muls(v3(s.h[6], s.h[7], s.h[8]), o.ga));
+  const float h2 = powi_f(dot(ph, pn), m.power);
+  const V3 diffuse = v3(unit[dk & 255u], unit[(dk >> 8) & 255u], unit[(dk >> 16) & 255u]);
+  const V3 ambient = v3(unit[ak & 255u], unit[(ak >> 8) & 255u], unit[(ak >> 16) & 255u]);
+  const V3 c_l = v3(m.ks[0], m.ks[1], m.ks[2]);
+  const V3 c_r = v3(diffuse.x * m.kd[0], diffuse.y * m.kd[1], diffuse.z * m.kd[2]);
+  const V3 c_a = v3(ambient.x * m.ka[0], ambient.y * m.ka[1], ambient.z * m.ka[2]);
   const V3 inner = add(c_a, muls(c_l, sfac));
   const V3 t1 = v3(c_r.x * inner.x, c_r.y * inner.y, c_r.z * inner.z);
-  const float h2 = powi_f(dot(ph, pn), m.power);
   const V3 col = add(t1, muls(c_l, h2));
   const V3 sc = muls(col, 255.0f);
   return f2u8(sc.z) | (f2u8(sc.y) << 8) | (f2u8(sc.x) << 16) | (255u << 24);
 }
 
-// Shading of up to 64 pixels by one wave; every lane calls it.  A lane's
-// pixel (x, y) of view vw has winner id, or kNone (the clear colour); lanes
-// with active false have no pixel.  Runs of equal winners along the wave load
-// their records once into run[slot] (up to R runs; more take per-lane loads):
-// the texture address units cost per requested byte per lane, and a run of
-// pixels shares one triangle's 224 record bytes.  A material shared by the
-// whole wave is read with scalar loads.
+// The clear colour, and a pixel's three outputs.
+__device__ inline uint32_t clear_word(const DevView& vw) {
+  const uint8_t* c = vw.fr.clear_bgra;
+  return (uint32_t)c[0] | ((uint32_t)c[1] << 8) | ((uint32_t)c[2] << 16) | ((uint32_t)c[3] << 24);
+}
+__device__ inline void write_pixel(const DevView& vw, uint32_t W, uint32_t H, uint32_t x, uint32_t y, uint32_t bgra,
+                                   float depth, uint32_t winner) {
+  const uint32_t p = y * W + x;
+  vw.out_bgra[(H - 1u - y) * W + x] = bgra;  // draw_pixel_coord row flip, canvas.rs:955
+  vw.out_depth[p] = depth;
+  if (vw.out_winner) vw.out_winner[p] = winner;
+}
+
+// Shading of up to 64 pixels by one wave; every lane calls it.  A lane's pixel
+// (x, y) of view vw has winner id, or kNone (the clear colour); lanes with
+// active false have no pixel.  A run of equal winners along the wave's 64
+// pixels shares one triangle's records: the words of up to R runs (14 of 16
+// bytes each) are loaded once, spread over the lanes, into the wave's LDS area
+// run, and the others read them there (the texture address units cost per
+// requested byte per lane); more runs take per-lane loads (taking them R at a
+// time instead cost the soup a quarter of its raster time).  A material shared
+// by all lanes at work is read with scalar loads.
+constexpr int shade_run_words(int R) { return 14 * R + (R + 3) / 4; }  // uint4s: the records, then the runs' ids
 template <int R>
-__device__ inline void shade_wave(uint32_t id, bool active, uint32_t x, uint32_t y, const DevView& vw,
+__device__ __forceinline__ void shade_wave(uint32_t id, bool active, uint32_t x, uint32_t y, const DevView& vw,
                                   const SetupRec* __restrict__ setup, const ShadeRec* __restrict__ shade,
-                                  const DevMaterial* __restrict__ mats, Status* __restrict__ status,
-                                  uint4 (*run)[14], const float* unit) {
+                                  const DevMaterial* __restrict__ mats, Status* __restrict__ status, uint4* run,
+                                  const float* unit) {
+  constexpr int kIt = (14 * R + 63) / 64;
+  static_assert(kIt <= 4, "run words");
   const uint32_t lane = threadIdx.x & 63u;
+  uint32_t* const run_id = reinterpret_cast<uint32_t*>(run + 14 * R);
   const bool covered = active && id != kNone;
   const uint32_t key = covered ? id : kSkip;
   // runs: a covered lane starts one unless the lane before holds the same id
   const uint32_t prev = (uint32_t)__shfl_up((int)key, 1, 64);
   const bool start = covered && (lane == 0u || prev != key);
   const uint64_t sm = __ballot(start);
-  SetupRec r;
-  ShadeRec sh;
-  if (__popcll(sm) <= R) {
-    const uint32_t slot = (uint32_t)__popcll(sm & (~0ull >> (63u - lane))) - 1u;  // the last start at or before
-    uint4* const rs_run = run[covered ? slot : 0u];
-    if (start) {
-      const uint4* rs = reinterpret_cast<const uint4*>(setup + id);
-      const uint4* ss = reinterpret_cast<const uint4*>(shade + id);
-#pragma unroll
-      for (int q = 0; q < 5; q++) rs_run[q] = rs[q];
-#pragma unroll
-      for (int q = 0; q < 9; q++) rs_run[5 + q] = ss[q];
-    }
-    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-    if (covered) {
-      uint4* rd = reinterpret_cast<uint4*>(&r);
-      uint4* sd = reinterpret_cast<uint4*>(&sh);
-#pragma unroll
-      for (int q = 0; q < 5; q++) rd[q] = rs_run[q];
-#pragma unroll
-      for (int q = 0; q < 9; q++) sd[q] = rs_run[5 + q];
-    }
-    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-  } else if (covered) {
-    const uint4* rs = reinterpret_cast<const uint4*>(setup + id);
-    uint4* rd = reinterpret_cast<uint4*>(&r);
-#pragma unroll
-    for (int q = 0; q < 5; q++) rd[q] = rs[q];
-    sh = shade[id];
-  }
-  if (!active) return;
+  const uint32_t n_run = (uint32_t)__popcll(sm);
+  const uint32_t slot = (uint32_t)__popcll(sm & (~0ull >> (63u - lane))) - 1u;  // the last start at or before
   const uint32_t W = (uint32_t)vw.fr.W, H = (uint32_t)vw.fr.H;
-  uint32_t bgra;
-  float depth;
-  if (!covered) {
-    const uint8_t* c = vw.fr.clear_bgra;
-    bgra = (uint32_t)c[0] | ((uint32_t)c[1] << 8) | ((uint32_t)c[2] << 16) | ((uint32_t)c[3] << 24);
-    depth = vw.fr.clear_depth;
-  } else {
+  auto shade_from = [&](const SetupRec& r, const ShadeRec& sh) {  // the covered lanes
     const FragOut o = bary(r, (float)x, (float)y);
-    // one material for the wave's covered pixels: scalar loads
+    // one material for the lanes at work: scalar loads
     const uint32_t m0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)sh.material);
+    uint32_t bgra;
     if (__ballot(sh.material != m0) == 0ull)
       bgra = shade_pixel(sh, mats[m0], o, status, unit);
     else
       bgra = shade_pixel(sh, mats[sh.material], o, status, unit);
-    depth = o.d;
+    write_pixel(vw, W, H, x, y, bgra, o.d, id - vw.id_base);
+  };
+  SetupRec r0;
+  ShadeRec sh0;
+  uint4* rd = reinterpret_cast<uint4*>(&r0);
+  uint4* sd = reinterpret_cast<uint4*>(&sh0);
+  if (n_run <= (uint32_t)R) {
+    if (start) run_id[slot] = id;
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    uint4 w0{}, w1{}, w2{}, w3{};  // named values, not an array, which would live in scratch memory
+    auto each_word = [&](auto f) {  // f(this lane's word index, its register)
+      f(lane, w0);
+      if constexpr (kIt > 1) f(64u + lane, w1);
+      if constexpr (kIt > 2) f(128u + lane, w2);
+      if constexpr (kIt > 3) f(192u + lane, w3);
+    };
+    each_word([&](uint32_t k, uint4& w) {
+      if (k >= 14u * n_run) return;
+      const uint32_t s = k / 14u, q = k - 14u * s;
+      const uint32_t rid = run_id[s];
+      w = *(q < 5u ? reinterpret_cast<const uint4*>(setup + rid) + q
+                   : reinterpret_cast<const uint4*>(shade + rid) + (q - 5u));
+    });
+    each_word([&](uint32_t k, const uint4& w) {
+      if (k < 14u * n_run) run[k] = w;
+    });
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    if (covered) {
+#pragma unroll
+      for (int q = 0; q < 5; q++) rd[q] = run[14u * slot + q];
+#pragma unroll
+      for (int q = 0; q < 9; q++) sd[q] = run[14u * slot + 5 + q];
+    }
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+  } else if (covered) {
+    const uint4* rs = reinterpret_cast<const uint4*>(setup + id);
+#pragma unroll
+    for (int q = 0; q < 5; q++) rd[q] = rs[q];
+    sh0 = shade[id];
   }
-  const uint32_t p = y * W + x;
-  vw.out_bgra[(H - 1u - y) * W + x] = bgra;  // draw_pixel_coord row flip, canvas.rs:955
-  vw.out_depth[p] = depth;
-  if (vw.out_winner) vw.out_winner[p] = covered ? id - vw.id_base : kNone;
+  if (covered) shade_from(r0, sh0);
+  if (active && !covered) write_pixel(vw, W, H, x, y, clear_word(vw), vw.fr.clear_depth, kNone);
+}
+
+// The 16-byte word wd of a record whose P lanes hold its words: lane part sp
+// has words sp, sp + P, ... in q0, q1, ... (DPP moves within the P lanes).
+template <int CTRL>
+__device__ inline uint4 dpp_u4(uint4 v) {
+  auto mv = [](uint32_t x) { return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, CTRL, 0xF, 0xF, false); };
+  return make_uint4(mv(v.x), mv(v.y), mv(v.z), mv(v.w));
+}
+template <int P, int WD>
+__device__ inline uint4 part_word(int sp, const uint4& q0, const uint4& q1, const uint4& q2, const uint4& q3,
+                                  const uint4& q4, const uint4& q5) {
+  constexpr int J = WD / P, SRC = WD % P;
+  const uint4& q = J == 0 ? q0 : J == 1 ? q1 : J == 2 ? q2 : J == 3 ? q3 : J == 4 ? q4 : q5;
+  if constexpr (P == 1) return q;
+  if constexpr (P == 2) return dpp_u4<SRC == 0 ? 0xA0 : 0xF5>(q);  // quad_perm [0,0,2,2] or [1,1,3,3]
+  if constexpr (P == 4) return dpp_u4<SRC * 0x55>(q);              // quad_perm: one lane's
+  if constexpr (P == 8) {  // that of its quad, then the other quad's by row_half_mirror
+    const uint4 b = dpp_u4<(SRC & 3) * 0x55>(q);
+    const uint4 o = dpp_u4<0x141>(b);
+    const bool mine = (sp >> 2) == (SRC >> 2);
+    return make_uint4(mine ? b.x : o.x, mine ? b.y : o.y, mine ? b.z : o.z, mine ? b.w : o.w);
+  }
 }
 
 // Per-tile visibility.  The tile's bin list is near first (or in submission
@@ -201,54 +266,71 @@ __device__ inline void shade_wave(uint32_t id, bool active, uint32_t x, uint32_t
 //  1. records are staged in LDS in chunks of CH, each with the mask of the
 //     tile's quadrants it can cover (its scan rectangle and, for an exact
 //     record, exact per-quadrant edge tests), computed once for all waves;
-//  2. lanes pre-filter 64 records at once: the wave's bits of that mask and
+//  2. a wave that has staged many small records rasterizes those at once, a
+//     record to P lanes (convert);
+//  3. lanes pre-filter 64 records at once: the wave's bits of that mask and
 //     its largest recorded depth (hierarchical Z);
-//  3. the wave visits the hits in order; lanes test coverage of their own
+//  4. the wave visits the hits in order; lanes test coverage of their own
 //     pixel without division (covered_fast) and against their pixel's recorded
 //     depth, and append covered fragments to a per-wave LDS queue;
-//  4. the queue is drained densely: divisions, depth, key, atomicMin.
+//  5. the queue is drained densely: divisions, depth, key, atomicMin.
 // Early-Z only drops a fragment whose depth lower bound is strictly above a
 // depth already recorded at its pixel, so it cannot be the minimum nor tie it.
 // SHADE: the workgroup shades its tile's pixels itself once the tile's
 // visibility is final (the tiles that finish first shade while others still
-// rasterize), else it writes the winners to vis_out for k_shade.
+// rasterize), else it writes the tile's packed visibility to pack_out (see
+// k_vis_pack).
+//
+// What bounds it is how many waves a CU holds to cover the chains of dependent
+// loads (tile range, ids, records, then the winners' records and texels), so
+// the staged record is kept small: an exact record (two-FMA edge values, below)
+// needs only the 64 bytes the visits and the divisions read, and any other one
+// is read from global memory where it is visited.  Five waves per SIMD are
+// asked of the compiler (96 VGPRs; four were the rule at 112, six spill): with
+// the batch of 32 views on <32, 4>, three, four and five waves took 700, 555
+// and 486 us.  All together, with the divisions by div_known (raster us, before
+// -> after): 32-view batch <32, 4> 770 -> 474; 12 mixed requests <16, 1> 432 ->
+// 397; 500k-triangle mesh at 4K 164 -> 146; 5M micro-triangles 155 -> 86; the
+// 1M-triangle 1080p soup, whose lists are long and visits many, 152 -> 151.
 template <int TS, int QPW, bool SHADE>
-__global__ __launch_bounds__(64 * (TS / 8) * (TS / 8) / QPW) void k_raster(
+__global__ __launch_bounds__(64 * (TS / 8) * (TS / 8) / QPW) __attribute__((amdgpu_waves_per_eu(5))) void k_raster(
     const DevView* __restrict__ views, uint32_t n_views, const uint2* __restrict__ ranges,
     const uint32_t* __restrict__ vals, const SetupRec* __restrict__ setup, const ShadeRec* __restrict__ shade,
-    const DevMaterial* __restrict__ mats, uint32_t* __restrict__ vis_out, Status* __restrict__ status) {
+    const DevMaterial* __restrict__ mats, unsigned long long* __restrict__ pack_out, uint32_t tag,
+    Status* __restrict__ status) {
   constexpr int QS = TS / 8, NQ = QS * QS, NW = NQ / QPW, NT = 64 * NW;
   constexpr int CH = 128;    // records staged per round
   // fragment queue per wave: drained once it holds more than kQFlush entries,
   // checked before each triangle, which appends at most 64 per quadrant
   constexpr int kQFlush = 224, QCAP = kQFlush + 64 * QPW;
-  // the staged chunk: records, edge constants, depth-bound keys, ids,
-  // quadrant masks (one LDS area, which the shading epilogue reuses for its
-  // record runs).  A workgroup's LDS must fit in one of the CU's two 80 KB
-  // halves, so <32, 2> (8 waves, 80 VGPRs) keeps below 40 KB to fit two per
-  // half and run three per CU.
-  constexpr int kChunkU4 = CH * (sizeof(SetupRec) + 48 + 4 + 4 + 4) / 16;
-  __shared__ uint4 s_chunk[kChunkU4];
-  SetupRec* const s_rec = reinterpret_cast<SetupRec*>(s_chunk);
-  // per edge of an exact record: s*A, s*B and E, the edge's exact value
-  // s*e - t at the tile origin (s = sign(f); t = 0 on a tie edge, else 1)
-  float4 (*const s_pre)[3] = reinterpret_cast<float4 (*)[3]>(s_chunk + CH * sizeof(SetupRec) / 16);
-  uint32_t* const s_zk = reinterpret_cast<uint32_t*>(s_chunk + CH * (sizeof(SetupRec) + 48) / 16);  // depth-bound key
-  uint32_t* const s_id = s_zk + CH;
+  // One LDS area: the staged chunk (64 bytes a record, depth-bound keys, ids,
+  // quadrant masks), then the waves' queues; the shading epilogue reuses it
+  // all for its record runs.  A workgroup's LDS must fit in one of the CU's
+  // two 80 KB halves: 26.6 KB for <32, 4> (six workgroups per CU), 17.4 KB
+  // for <16, 1> (eight).
+  constexpr int kChunkU4 = CH * 4 + 3 * CH / 4, kBufU4 = kChunkU4 + NW * QCAP / 4;
+  __shared__ uint4 s_buf[kBufU4];
+  // per record: per edge s*A, s*B and E = s*e - t, the edge's exact value at
+  // the tile origin less t (s = sign(f); t = 0 on a tie edge, else 1), with t
+  // as the sign of the fourth word: |f|, RN(1 / |f|), 1; then its vertex
+  // depths and id
+  float4 (*const s_e)[4] = reinterpret_cast<float4 (*)[4]>(s_buf);
+  uint32_t* const s_zk = reinterpret_cast<uint32_t*>(s_buf + CH * 4);  // depth-bound key
+  uint32_t* const s_id = s_zk + CH;  // for the visits of records that are not exact
   // the tile's quadrants a record can cover (bit Q: quadrant row Q / QS,
   // column Q % QS), | kQExact for an exact record
   uint32_t* const s_qm = s_id + CH;
   __shared__ unsigned long long s_vis[TS * TS];
-  __shared__ uint32_t s_q[NW][QCAP];
   __shared__ uint32_t s_nfrag;  // the tile's fragment count (one global atomic per tile)
   __shared__ uint32_t s_wmax[NW];  // each wave's largest recorded depth key, as of its last flush
   __shared__ float s_unit[SHADE ? 256 : 1];
   // How an exact hit's edge constants reach the wave.  kLdsHit: broadcast
-  // reads of the staged s_pre.  Otherwise the pre-filtering lane reads them
+  // reads of the staged record.  Otherwise the pre-filtering lane reads them
   // and the wave takes them with readlanes: with one quadrant per wave a hit
   // has too little work to cover the LDS latency.
   constexpr bool kLdsHit = QPW >= 2;
   constexpr uint32_t kQExact = 1u << 16;
+  constexpr int kSmallPx = 8;  // largest side of a small record's rectangle within the tile
 
   const uint32_t tile = xcd_remap(blockIdx.x, gridDim.x);
   const DevView& vw = views[wave_find_view_tile(views, n_views, tile)];
@@ -260,6 +342,15 @@ __global__ __launch_bounds__(64 * (TS / 8) * (TS / 8) / QPW) void k_raster(
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform: keeps the wave's geometry scalar
   const uint2 rg = ranges[tile];
+  if (SHADE && rg.x >= rg.y) {  // nothing to rasterize: the clear values (the whole block)
+    const uint32_t clear = clear_word(vw);
+    for (int p = tid; p < TS * TS; p += NT) {
+      const uint32_t px = (uint32_t)(tx0 + p % TS), py = (uint32_t)(ty0 + p / TS);
+      if ((int)px < W && (int)py < H) write_pixel(vw, (uint32_t)W, (uint32_t)H, px, py, clear, clear_depth, kNone);
+    }
+    return;
+  }
+  uint32_t* const s_q = reinterpret_cast<uint32_t*>(s_buf + kChunkU4) + wave * QCAP;
 
   // Pixels off the screen start at key 0, below every fragment's (depth
   // keys of recorded fragments and staged depth bounds are >= 1), so the
@@ -271,7 +362,6 @@ __global__ __launch_bounds__(64 * (TS / 8) * (TS / 8) / QPW) void k_raster(
   if constexpr (SHADE) fill_unit_table(s_unit, tid, NT);  // read after the barrier before the shading
 
   const int lx = lane & 7, ly = lane >> 3;
-  const uint64_t lanemask_lt = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
   // The wave's quadrants: QPW consecutive ones in row-major order (part of a
   // quadrant row, or whole rows), bits wq0 .. wq0 + QPW - 1 of a record's
   // quadrant mask.
@@ -283,10 +373,10 @@ __global__ __launch_bounds__(64 * (TS / 8) * (TS / 8) / QPW) void k_raster(
   for (int qq = 0; qq < QPW; qq++) {
     const int Q = wq0 + qq;
     lp[qq] = ((Q / QS) * 8 + ly) * TS + (Q % QS) * 8 + lx;
-    const int px = tx0 + (Q % QS) * 8 + lx, py = ty0 + (Q / QS) * 8 + ly;
-    dxf[qq] = (float)(px - tx0);
-    dyf[qq] = (float)(py - ty0);
-    zk[qq] = (px < W && py < H) ? 0xFFFFFFFFu : 0u;
+    const int dx = (Q % QS) * 8 + lx, dy = (Q / QS) * 8 + ly;
+    dxf[qq] = (float)dx;
+    dyf[qq] = (float)dy;
+    zk[qq] = (tx0 + dx < W && ty0 + dy < H) ? 0xFFFFFFFFu : 0u;
   }
   uint32_t wmax = 0xFFFFFFFFu;  // largest recorded depth key over the wave's pixels
   // ...and over each of its quadrants (hierarchical Z per quadrant, with 4
@@ -299,21 +389,27 @@ __global__ __launch_bounds__(64 * (TS / 8) * (TS / 8) / QPW) void k_raster(
   uint32_t qn = 0;
   uint32_t nfrag = 0;
 
-  auto submit = [&](const SetupRec& r, uint32_t id, int px, int py) {
-    const FragOut o = bary(r, (float)px, (float)py);
-    if (!(r.flags & kUvSafe) && !uv_ok(shade, mats, id, o)) atomicOr(&status->error, 1u);
-    if (o.d < clear_depth) {
-      const unsigned long long key = ((unsigned long long)depth_key(o.d) << 32) | id;
-      atomicMin(&s_vis[(py - ty0) * TS + (px - tx0)], key);
-    }
-  };
+  // Queued fragments, all of exact records: (s*e) / |f| is e / f (the sign of a
+  // zero aside, which no depth key sees), one |f| for the three edges.
   auto flush = [&]() {
     __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");  // queue writes by other lanes of this wave
     for (uint32_t j = (uint32_t)lane; j < qn; j += 64) {
-      const uint32_t q = s_q[wave][j];
+      const uint32_t q = s_q[j];
       const uint32_t k = q >> 16, l = q & 0xFFFFu;
       if (s_zk[k] > (uint32_t)(s_vis[l] >> 32)) continue;  // early-Z recheck
-      submit(s_rec[k], s_id[k], tx0 + (int)(l % TS), ty0 + (int)(l / TS));
+      const float fx = (float)(l % TS), fy = (float)(l / TS);
+      const float f = fabsf(s_e[k][0].w), y = fabsf(s_e[k][1].w);
+      float v[3];
+#pragma unroll
+      for (int e = 0; e < 3; e++) {
+        const float4 c = s_e[k][e];
+        const float t = (float)(__float_as_uint(c.w) >> 31);
+        v[e] = div_known(fmaf(c.x, fx, fmaf(c.y, fy, c.z)) + t, f, y);
+      }
+      const float4 dd = s_e[k][3];
+      const float d = (v[0] * dd.x + v[1] * dd.y) + v[2] * dd.z;
+      if (d < clear_depth)
+        atomicMin(&s_vis[l], ((unsigned long long)depth_key(d) << 32) | __float_as_uint(dd.w));
     }
     nfrag += qn;
     qn = 0;
@@ -335,8 +431,7 @@ __global__ __launch_bounds__(64 * (TS / 8) * (TS / 8) / QPW) void k_raster(
 
   // Staging: P consecutive lanes of one wave per record of a chunk (P = NT /
   // CH, at least 1).  Lane part sp loads the record's 16-byte words sp,
-  // sp + P, ... and stores them into LDS; the P lanes read back the words
-  // they need (stores of their own wave: no barrier) and each tests the
+  // sp + P, ...; the P lanes exchange them (part_word) and each tests the
   // quadrant rows sp, sp + P, ... of the tile; an OR over the P lanes joins
   // the rows.  With NT >= CH the loads run ahead of the raster: while a chunk
   // is rasterized, the next chunk's words (their ids loaded a chunk earlier)
@@ -365,28 +460,15 @@ __global__ __launch_bounds__(64 * (TS / 8) * (TS / 8) / QPW) void k_raster(
     return v;
   };
   uint32_t tile_wmax = 0xFFFFFFFFu;  // the tile's largest recorded depth key (s_wmax), for stage
-  // Record i of a chunk into LDS, from this lane's words.
-  auto stage = [&](int i, uint32_t id, uint4 q0, uint4 q1, uint4 q2, uint4 q3, uint4 q4, uint4 q5) {
-    uint4* dst = reinterpret_cast<uint4*>(s_rec + i);
-    if (sp < 6) dst[sp] = q0;
-    if constexpr (NPC > 1) if (sp + P < 6) dst[sp + P] = q1;
-    if constexpr (NPC > 2) if (sp + 2 * P < 6) dst[sp + 2 * P] = q2;
-    if constexpr (NPC > 3) if (sp + 3 * P < 6) dst[sp + 3 * P] = q3;
-    if constexpr (NPC > 4) if (sp + 4 * P < 6) dst[sp + 4 * P] = q4;
-    if constexpr (NPC > 5) if (sp + 5 * P < 6) dst[sp + 5 * P] = q5;
-    uint4 w0, w1, w2, w3, w5;
-    uint32_t zb;  // the depth lower bound's bits
-    if constexpr (P == 1) {
-      w5 = q5;
-      zb = q4.w;
-    } else {
-      __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");  // the other parts' stores
-      w5 = dst[5];
-      zb = __float_as_uint(s_rec[i].d[3]);
-    }
+  // Record i of a chunk into LDS, from this lane's words.  Returns, for a
+  // small record that some quadrant may see, its rectangle within the tile as
+  // x | y << 8 | w << 16 | h << 24, else 0.
+  auto stage = [&](int i, uint32_t id, const uint4& q0, const uint4& q1, const uint4& q2, const uint4& q3,
+                   const uint4& q4, const uint4& q5) -> uint32_t {
+    const uint4 w4 = part_word<P, 4>(sp, q0, q1, q2, q3, q4, q5);
     // depth bound key, at least 1: only off-screen pixels hold key 0 (a
     // fragment key of 0 is a NaN depth, which never passes the depth test)
-    const uint32_t zkey = max(depth_key(__uint_as_float(zb)), 1u);
+    const uint32_t zkey = max(depth_key(__uint_as_float(w4.w)), 1u);
     if (sp == 0) {
       s_id[i] = id;
       s_zk[i] = zkey;
@@ -396,19 +478,17 @@ __global__ __launch_bounds__(64 * (TS / 8) * (TS / 8) / QPW) void k_raster(
     // quadrants, and no edge work.
     if (zkey > tile_wmax) {
       if (sp == 0) s_qm[i] = 0u;
-      return;
+      return 0u;
     }
-    if constexpr (P == 1) {
-      w0 = q0; w1 = q1; w2 = q2; w3 = q3;
-    } else {
-      w0 = dst[0]; w1 = dst[1]; w2 = dst[2]; w3 = dst[3];
-    }
+    const uint4 w5 = part_word<P, 5>(sp, q0, q1, q2, q3, q4, q5);
     // The tile's quadrants the scan rectangle meets: quadrant column c meets
     // [x0, x1] iff floor((x0 - tx0) / 8) <= c <= floor((x1 - tx0) / 8), rows
     // likewise.
     const uint32_t flags = w5.z;
-    const int c0 = max(((int)(w5.x & 0xFFFFu) - tx0) >> 3, 0), c1 = min(((int)(w5.x >> 16) - tx0) >> 3, QS - 1);
-    const int r0 = max(((int)(w5.y & 0xFFFFu) - ty0) >> 3, 0), r1 = min(((int)(w5.y >> 16) - ty0) >> 3, QS - 1);
+    const int rx0 = (int)(w5.x & 0xFFFFu) - tx0, rx1 = (int)(w5.x >> 16) - tx0;
+    const int ry0 = (int)(w5.y & 0xFFFFu) - ty0, ry1 = (int)(w5.y >> 16) - ty0;
+    const int c0 = max(rx0 >> 3, 0), c1 = min(rx1 >> 3, QS - 1);
+    const int r0 = max(ry0 >> 3, 0), r1 = min(ry1 >> 3, QS - 1);
     uint32_t qmask = 0;
     if (c0 <= c1 && r0 <= r1) {
       const uint32_t cols = (2u << c1) - (1u << c0);
@@ -416,7 +496,7 @@ __global__ __launch_bounds__(64 * (TS / 8) * (TS / 8) / QPW) void k_raster(
       for (int rr = 0; rr < QS; rr++)
         if (rr >= r0 && rr <= r1) qmask |= cols << (rr * QS);
     }
-    // Exact records.  With S = |A| x1 + |B| y1 + |C| + |D| over the tile's
+    // Exact records (whose texture reads cannot fail either).  With S = |A| x1 + |B| y1 + |C| + |D| over the tile's
     // largest pixel coordinates (x1, y1) below 2^24 - 216 on every edge (the
     // float S is within 3 units of the exact one), every product and partial
     // sum of the edge function at the tile's pixels is an integer of
@@ -426,54 +506,107 @@ __global__ __launch_bounds__(64 * (TS / 8) * (TS / 8) / QPW) void k_raster(
     // bounding box need no separate test: a covered pixel is inside the
     // snapped triangle, hence inside its bounding box unless it is off the
     // screen.
-    bool exact = (flags & kFast) != 0u;
-    float sA[3], sB[3], E[3];
-    const uint4 edge[3] = {w0, w1, w2};
+    // ...less the quadrants an edge rules out: an edge's largest value over
+    // quadrant (qx, qy) is at its pixel (8 qx + (sA > 0 ? 7 : 0), 8 qy +
+    // (sB > 0 ? 7 : 0)) of the tile, computed exactly (a pixel of the tile);
+    // below zero there, no pixel of the quadrant is covered.  qv: the
+    // smallest of the three edges' values, for this lane's quadrant rows.
+    bool exact = (flags & (kFast | kUvSafe)) == (kFast | kUvSafe);
+    constexpr int RQ = QS >= P ? QS / P : 1;
+    float qv[RQ][QS];
+#pragma unroll
+    for (int j = 0; j < RQ; j++)
+#pragma unroll
+      for (int qx = 0; qx < QS; qx++) qv[j][qx] = INFINITY;
+    const uint4 w3 = part_word<P, 3>(sp, q0, q1, q2, q3, q4, q5);
     const uint32_t fb[3] = {w3.x, w3.y, w3.z};
     const float tx0f = (float)tx0, ty0f = (float)ty0, tx1f = (float)(tx0 + TS - 1), ty1f = (float)(ty0 + TS - 1);
 #pragma unroll
     for (int e = 0; e < 3; e++) {
+      const uint4 q = e == 0   ? part_word<P, 0>(sp, q0, q1, q2, q3, q4, q5)
+                      : e == 1 ? part_word<P, 1>(sp, q0, q1, q2, q3, q4, q5)
+                               : part_word<P, 2>(sp, q0, q1, q2, q3, q4, q5);
       const float sg = __uint_as_float(fb[e]) > 0.0f ? 1.0f : -1.0f;
-      const float A = __uint_as_float(edge[e].x), B = __uint_as_float(edge[e].y);
-      const float C = __uint_as_float(edge[e].z), D = __uint_as_float(edge[e].w);
-      sA[e] = sg * A;
-      sB[e] = sg * B;
-      const float S = (fabsf(sA[e]) * tx1f + fabsf(sB[e]) * ty1f) + (fabsf(C) + fabsf(D));
+      const float A = __uint_as_float(q.x), B = __uint_as_float(q.y);
+      const float C = __uint_as_float(q.z), D = __uint_as_float(q.w);
+      const float sA = sg * A, sB = sg * B;
+      const float S = (fabsf(sA) * tx1f + fabsf(sB) * ty1f) + (fabsf(C) + fabsf(D));
       if (!(S < 16777000.0f)) exact = false;
-      E[e] = ((sA[e] * tx0f + sB[e] * ty0f) + sg * (C - D)) - ((flags & (kTieA << e)) ? 0.0f : 1.0f);
-      if (e % P == sp) s_pre[i][e] = make_float4(sA[e], sB[e], E[e], 0.0f);
-    }
-    if (exact) {  // the same on the record's P lanes
-      // ...less the quadrants an edge rules out: an edge's largest value over
-      // quadrant (qx, qy) is at its pixel (8 qx + (sA > 0 ? 7 : 0), 8 qy +
-      // (sB > 0 ? 7 : 0)) of the tile, computed exactly (a pixel of the
-      // tile) as cv[qx] + sB * 8 qy; below zero there, no pixel of the
-      // quadrant is covered.
-      float cv[3][QS];
+      const bool tie = (flags & (kTieA << e)) != 0u;
+      const float E = ((sA * tx0f + sB * ty0f) + sg * (C - D)) - (tie ? 0.0f : 1.0f);
+      const uint32_t fm = e == 0 ? w3.x : e == 1 ? w3.w : 0x3F800000u;
+      const uint32_t fw = (fm & 0x7FFFFFFFu) | (tie ? 0u : 0x80000000u);
+      if (e % P == sp) s_e[i][e] = make_float4(sA, sB, E, __uint_as_float(fw));
+      const float top = fmaf(sA, sA > 0.0f ? 7.0f : 0.0f, fmaf(sB, sB > 0.0f ? 7.0f : 0.0f, E));
 #pragma unroll
-      for (int e = 0; e < 3; e++) {
-        cv[e][0] = fmaf(sA[e], sA[e] > 0.0f ? 7.0f : 0.0f, fmaf(sB[e], sB[e] > 0.0f ? 7.0f : 0.0f, E[e]));
+      for (int j = 0; j < RQ; j++) {
+        const float rv = fmaf(sB, (float)(8 * (sp + j * P)), top);
 #pragma unroll
-        for (int k = 1; k < QS; k++) cv[e][k] = fmaf(sA[e], (float)(8 * k), cv[e][0]);
+        for (int qx = 0; qx < QS; qx++) qv[j][qx] = fminf(qv[j][qx], fmaf(sA, (float)(8 * qx), rv));
       }
+    }
+    if (3 % P == sp)
+      s_e[i][3] = make_float4(__uint_as_float(w4.x), __uint_as_float(w4.y), __uint_as_float(w4.z), __uint_as_float(id));
+    uint32_t small = 0u;
+    if (exact) {  // the same on the record's P lanes
       uint32_t keep = 0;
 #pragma unroll
-      for (int j = 0; j < (QS >= P ? QS / P : 1); j++) {
+      for (int j = 0; j < RQ; j++) {
         const int qy = sp + j * P;
         if (QS >= P || qy < QS) {
-          float rv[3];
 #pragma unroll
-          for (int e = 0; e < 3; e++) rv[e] = sB[e] * (float)(8 * qy);
-#pragma unroll
-          for (int qx = 0; qx < QS; qx++) {
-            const float v = fminf(fminf(cv[0][qx] + rv[0], cv[1][qx] + rv[1]), cv[2][qx] + rv[2]);
-            keep |= (v >= 0.0f ? 1u : 0u) << (qy * QS + qx);
-          }
+          for (int qx = 0; qx < QS; qx++) keep |= (qv[j][qx] >= 0.0f ? 1u : 0u) << (qy * QS + qx);
         }
       }
-      qmask = (qmask & or_parts(keep)) | kQExact;
+      qmask &= or_parts(keep);
+      const int x0 = max(rx0, 0), x1 = min(rx1, TS - 1), y0 = max(ry0, 0), y1 = min(ry1, TS - 1);
+      if (qmask != 0u && x1 - x0 < kSmallPx && y1 - y0 < kSmallPx)
+        small = (uint32_t)x0 | (uint32_t)y0 << 8 | (uint32_t)(x1 - x0 + 1) << 16 | (uint32_t)(y1 - y0 + 1) << 24;
+      qmask |= kQExact;
     }
     if (sp == 0) s_qm[i] = qmask;
+    return small;
+  };
+  // The small records that the wave has just staged (record i of this lane,
+  // its rectangle sm as stage returned it, 0 if none), all at once: each of a
+  // record's P lanes walks its rows of the rectangle, and the covered pixels
+  // join the wave's fragment queue.  One record at a time, a visit costs some
+  // 100 instructions for the 64 pixels of a quadrant of which a small triangle
+  // covers a few; here a step costs about 20 for one pixel of every small
+  // record, so it pays when the wave has more than two records per step
+  // (32-view batch: raster 775 -> 580 us; 5M micro-triangles 154 -> 87 us; with
+  // fewer records per step meshes of larger triangles lost up to a half).
+  // Every lane of the wave calls it.
+  auto convert = [&](int i, uint32_t sm) {
+    const int w = (int)((sm >> 16) & 0xFFu), h = (int)(sm >> 24);
+    const uint32_t cnt = (uint32_t)__popcll(__ballot(h > 0 && sp == 0));
+    if (cnt < 4u) return;
+    const uint32_t mw = wave_max_u32((uint32_t)w), mh = wave_max_u32((uint32_t)h);
+    if (cnt < 2u * ((mh + (uint32_t)P - 1u) / (uint32_t)P) * mw) return;
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");  // the record's P lanes' stores
+    if (h > 0 && sp == 0) s_qm[i] = 0u;  // settled here
+    const float4 e0 = s_e[i][0], e1 = s_e[i][1], e2 = s_e[i][2];
+    const int x = (int)(sm & 0xFFu), y = (int)((sm >> 8) & 0xFFu);
+    for (int r = sp;; r += P) {
+      const bool row = r < h;
+      if (__ballot(row) == 0ull) break;
+      const float fx = (float)x, fy = (float)(y + r);
+      float w0 = fmaf(e0.x, fx, fmaf(e0.y, fy, e0.z));
+      float w1 = fmaf(e1.x, fx, fmaf(e1.y, fy, e1.z));
+      float w2 = fmaf(e2.x, fx, fmaf(e2.y, fy, e2.z));
+      for (int c = 0;; c++) {
+        const bool on = row && c < w;
+        if (__ballot(on) == 0ull) break;
+        const bool cov = on && fminf(fminf(w0, w1), w2) >= 0.0f;
+        const uint64_t m = __ballot(cov);
+        if (cov) s_q[lanes_below(m, qn)] = ((uint32_t)i << 16) | (uint32_t)((y + r) * TS + x + c);
+        qn += (uint32_t)__popcll(m);
+        if (qn > (uint32_t)(QCAP - 64)) flush();
+        w0 += e0.x;
+        w1 += e1.x;
+        w2 += e2.x;
+      }
+    }
   };
   uint32_t pf_id = 0, pf_id2 = 0;  // ids of the next chunk and of the one after it
   uint4 p0{}, p1{}, p2{}, p3{}, p4{}, p5{};  // this lane's words of the next chunk's record
@@ -492,13 +625,20 @@ __global__ __launch_bounds__(64 * (TS / 8) * (TS / 8) / QPW) void k_raster(
 #pragma unroll
     for (int w = 0; w < NW; w++) tile_wmax = max(tile_wmax, s_wmax[w]);
     if constexpr (kPrefetch) {
-      if (sr < n) stage(sr, pf_id, p0, p1, p2, p3, p4, p5);
+      uint32_t sm = 0u;
+      if (sr < n) sm = stage(sr, pf_id, p0, p1, p2, p3, p4, p5);
+      convert(min(sr, CH - 1), sm);
     } else {
-      for (int i = tid; i < n; i += NT) {
-        const uint32_t id = vals[base + i];
-        uint4 w0, w1, w2, w3, w4, w5;
-        load_words(id, w0, w1, w2, w3, w4, w5);
-        stage(i, id, w0, w1, w2, w3, w4, w5);
+      for (int i0 = 0; i0 < n; i0 += NT) {
+        const int i = i0 + tid;
+        uint32_t sm = 0u;
+        if (i < n) {
+          const uint32_t id = vals[base + i];
+          uint4 w0, w1, w2, w3, w4, w5;
+          load_words(id, w0, w1, w2, w3, w4, w5);
+          sm = stage(i, id, w0, w1, w2, w3, w4, w5);
+        }
+        convert(min(i, CH - 1), sm);
       }
     }
     __syncthreads();
@@ -530,7 +670,7 @@ __global__ __launch_bounds__(64 * (TS / 8) * (TS / 8) / QPW) void k_raster(
           if (hit && wexact) {
 #pragma unroll
             for (int e = 0; e < 3; e++) {
-              const float4 q = s_pre[g0 + lane][e];
+              const float4 q = s_e[g0 + lane][e];
               pA[e] = q.x;
               pB[e] = q.y;
               pE[e] = q.z;
@@ -542,6 +682,7 @@ __global__ __launch_bounds__(64 * (TS / 8) * (TS / 8) / QPW) void k_raster(
       // minimum does not depend on the order of the visits).
       uint64_t hf = __ballot(hit && wexact);
       uint64_t hs = __ballot(hit) & ~hf;
+      const bool slow = hs != 0ull;
       while (hf) {
         const int kl = (int)__builtin_ctzll(hf);
         const int k = g0 + kl;
@@ -555,7 +696,7 @@ __global__ __launch_bounds__(64 * (TS / 8) * (TS / 8) / QPW) void k_raster(
         if constexpr (kLdsHit) {
 #pragma unroll
           for (int e = 0; e < 3; e++) {
-            const float4 q = s_pre[k][e];
+            const float4 q = s_e[k][e];
             A[e] = q.x;
             B[e] = q.y;
             E[e] = q.z;
@@ -584,7 +725,7 @@ __global__ __launch_bounds__(64 * (TS / 8) * (TS / 8) / QPW) void k_raster(
           const bool inside = fminf(fminf(w0, w1), w2) >= 0.0f, nearer = zkey <= zk[qq];
           const bool cov = inside & nearer;
           const uint64_t m = __ballot(inside) & __ballot(nearer);
-          uint32_t* const qb = &s_q[wave][qn];
+          uint32_t* const qb = &s_q[qn];
           if (cov) qb[lanes_below(m, 0u)] = ((uint32_t)k << 16) | (uint32_t)lp[qq];
           qn += (uint32_t)__popcll(m);
         }
@@ -593,8 +734,8 @@ __global__ __launch_bounds__(64 * (TS / 8) * (TS / 8) / QPW) void k_raster(
         const int kl = (int)__builtin_ctzll(hs);
         const int k = g0 + kl;
         hs &= hs - 1;
-        if (qn > kQFlush) flush();
-        const SetupRec& r = s_rec[k];
+        const uint32_t id = (uint32_t)__builtin_amdgcn_readfirstlane((int)s_id[k]);
+        const SetupRec& r = setup[id];
         const uint32_t hx = r.rx, hy = r.ry;
         const int rx0 = (int)(hx & 0xFFFFu), rx1 = (int)(hx >> 16);
         const int ry0 = (int)(hy & 0xFFFFu), ry1 = (int)(hy >> 16);
@@ -608,37 +749,28 @@ __global__ __launch_bounds__(64 * (TS / 8) * (TS / 8) / QPW) void k_raster(
           const int px = qx0 + lx, py = qy0 + ly;
           const bool in = px >= rx0 && px <= rx1 && py >= ry0 && py <= ry1;
           const float xf = (float)px, yf = (float)py;
-          if (flags & kFast) {
-            bool cov = false;
-            if (in && !(zkey > zk[qq])) {
-              const float e0 = edge_eval(r.ea, xf, yf);
-              const float e1 = edge_eval(r.eb, xf, yf);
-              const float e2 = edge_eval(r.eg, xf, yf);
-              cov = covered_fast(e0, r.f[0], flags & kTieA) && covered_fast(e1, r.f[1], flags & kTieB) &&
-                    covered_fast(e2, r.f[2], flags & kTieG);
-            }
-            const uint64_t m = __ballot(cov);
-            if (m) {
-              if (cov) {
-                const uint32_t pos = qn + (uint32_t)__popcll(m & lanemask_lt);
-                s_q[wave][pos] = ((uint32_t)k << 16) | (uint32_t)lp[qq];
-              }
-              qn += (uint32_t)__popcll(m);
-            }
-          } else {
+          bool cov = false;
+          FragOut o{};
+          if ((flags & kFast) && in && !(zkey > zk[qq])) {
+            cov = covered_fast(edge_eval(r.ea, xf, yf), r.f[0], flags & kTieA) &&
+                  covered_fast(edge_eval(r.eb, xf, yf), r.f[1], flags & kTieB) &&
+                  covered_fast(edge_eval(r.eg, xf, yf), r.f[2], flags & kTieG);
+            if (cov) o = bary(r, xf, yf);
+          } else if (!(flags & kFast) && in) {
             // Any other triangle: the reference's predicate on the divided values.
-            bool cov = false;
-            if (in) {
-              const FragOut o = bary(r, xf, yf);
-              cov = o.al >= 0.0f && o.be >= 0.0f && o.ga >= 0.0f && (o.al > 0.0f || (flags & kTieA)) &&
-                    (o.be > 0.0f || (flags & kTieB)) && (o.ga > 0.0f || (flags & kTieG));
-            }
-            if (cov) submit(r, s_id[k], px, py);
-            nfrag += (uint32_t)__popcll(__ballot(cov));
+            o = bary(r, xf, yf);
+            cov = o.al >= 0.0f && o.be >= 0.0f && o.ga >= 0.0f && (o.al > 0.0f || (flags & kTieA)) &&
+                  (o.be > 0.0f || (flags & kTieB)) && (o.ga > 0.0f || (flags & kTieG));
           }
+          if (cov) {
+            if (!(flags & kUvSafe) && !uv_ok(shade, mats, id, o)) atomicOr(&status->error, 1u);
+            if (o.d < clear_depth)
+              atomicMin(&s_vis[lp[qq]], ((unsigned long long)depth_key(o.d) << 32) | id);
+          }
+          nfrag += (uint32_t)__popcll(__ballot(cov));
         }
       }
-      if (qn) flush();
+      if (qn || slow) flush();  // (slow visits record their fragments themselves)
     }
   }
   // A wave with fragments ran the chunk loop, whose barriers order this
@@ -649,23 +781,24 @@ __global__ __launch_bounds__(64 * (TS / 8) * (TS / 8) / QPW) void k_raster(
   if (tid == 0 && s_nfrag) atomicAdd(&status->frags[tile % kFragWords], s_nfrag);
   if constexpr (SHADE) {
     // each wave shades 64 consecutive pixels of the tile at a time, its
-    // record runs in its share of the chunk area
-    constexpr int R = (int)(kChunkU4 / (NW * 14)) < 16 ? (int)(kChunkU4 / (NW * 14)) : 16;
-    uint4 (*const run)[14] = reinterpret_cast<uint4 (*)[14]>(s_chunk) + wave * R;
+    // record runs in its share of the LDS area
+    constexpr int kU4 = kBufU4 / NW;
+    constexpr int R = kU4 >= shade_run_words(16) ? 16 : (4 * kU4 - 3) / 57;
+    static_assert(R >= 1 && shade_run_words(R) <= kU4, "run area");
     for (int p0 = wave * 64; p0 < TS * TS; p0 += NT) {
       const int p = p0 + lane;
       const int px = tx0 + p % TS, py = ty0 + p / TS;
       const bool on = px < W && py < H;
       const unsigned long long v = s_vis[p];
       shade_wave<R>((v == ~0ull) ? kNone : (uint32_t)v, on, (uint32_t)px, (uint32_t)py, vw, setup, shade, mats,
-                    status, run, s_unit);
+                    status, s_buf + wave * kU4, s_unit);
     }
   } else {
     for (int p = tid; p < TS * TS; p += NT) {
       const int px = tx0 + p % TS, py = ty0 + p / TS;
       if (px < W && py < H) {
         const unsigned long long v = s_vis[p];
-        vis_out[vw.px_base + (uint32_t)py * (uint32_t)W + (uint32_t)px] = (v == ~0ull) ? kNone : (uint32_t)v;
+        pack_out[(uint32_t)py * (uint32_t)W + (uint32_t)px] = v == ~0ull ? v : v | tag;
       }
     }
   }
@@ -847,7 +980,7 @@ __global__ __launch_bounds__(256) void k_shade(const DevView* __restrict__ views
                                                const uint32_t* __restrict__ vis, const SetupRec* __restrict__ setup,
                                                const ShadeRec* __restrict__ shade,
                                                const DevMaterial* __restrict__ mats, Status* __restrict__ status) {
-  __shared__ uint4 s_run[4][kShadeRuns][14];  // setup bytes 0-79, then the 144 shade bytes
+  __shared__ uint4 s_run[4][shade_run_words(kShadeRuns)];
   __shared__ float s_unit[256];
   fill_unit_table(s_unit, (int)threadIdx.x, 256);
   __syncthreads();
@@ -992,10 +1125,11 @@ static void launch_raster(const PipeArgs& a, hipStream_t s) {
   constexpr int NT = 64 * (TS / 8) * (TS / 8) / QPW;
   if (a.shade_in_raster)
     hipLaunchKernelGGL((k_raster<TS, QPW, true>), dim3(a.n_tiles), dim3(NT), 0, s, a.views, a.n_views, a.ranges,
-                       a.vals[0], a.setup, a.shade, a.mats, a.vis, a.status);
+                       a.vals[0], a.setup, a.shade, a.mats, nullptr, 0u, a.status);
   else
     hipLaunchKernelGGL((k_raster<TS, QPW, false>), dim3(a.n_tiles), dim3(NT), 0, s, a.views, a.n_views, a.ranges,
-                       a.vals[0], a.setup, a.shade, a.mats, a.vis, a.status);
+                       a.vals[0], a.setup, a.shade, a.mats, reinterpret_cast<unsigned long long*>(a.pack_out),
+                       a.pack_tag, a.status);
 }
 
 template <int TS, int NW>
@@ -1060,7 +1194,8 @@ void enqueue_blend(const PipeArgs& b, const TransArgs& t, hipStream_t s) {
 // raster's atomicMin kept (bary and depth_key at the winner's pixel), with
 // ids ordered by (shard, submission) -- so the u64 minimum over the shards
 // of a frame split by submission range is the single-GPU winner, ties
-// included.  No winner: ~0.
+// included.  No winner: ~0.  (The kind-0 raster writes the same from its own
+// visibility buffer.)
 __global__ __launch_bounds__(256) void k_vis_pack(const DevView* __restrict__ views, uint32_t n_pixels,
                                                   const uint32_t* __restrict__ vis, const SetupRec* __restrict__ setup,
                                                   uint32_t tag, unsigned long long* __restrict__ out) {
