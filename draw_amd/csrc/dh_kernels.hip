@@ -545,7 +545,12 @@ struct Spans {
   int cx0, cx1, cy0, cy1;
   bool exact;
   float fa[3], fb[3], fk[3], fm[3];  // per-tile corner test (tile_may_cover)
-  double a[3], b[3], k[3], m[3];     // per-row spans of wide triangles (spans_row)
+};
+// Per-row spans of a wide triangle (spans_row).
+struct SpanRows {
+  int cx0, cx1;
+  bool exact;
+  double a[3], b[3], k[3], m[3];
 };
 
 // Bounds and the per-tile test's constants.  The test evaluates
@@ -580,8 +585,11 @@ __device__ inline void spans_init(const SetupRec& r, int TS, Spans& g) {
   }
 }
 
-// The per-row constants of a wide triangle (after spans_init), in double.
-__device__ inline void spans_init_rows(const SetupRec& r, Spans& g) {
+// The per-row constants of a wide triangle with tile box c, in double.
+__device__ inline void spans_init_rows(const SetupRec& r, const Spans& c, SpanRows& g) {
+  g.cx0 = c.cx0;
+  g.cx1 = c.cx1;
+  g.exact = c.exact;
   if (!g.exact) return;
   const uint32_t x1 = r.rx >> 16, y1 = r.ry >> 16;
   const float* es[3] = {r.ea, r.eb, r.eg};
@@ -599,7 +607,7 @@ __device__ inline void spans_init_rows(const SetupRec& r, Spans& g) {
 }
 
 // Columns [lo, hi] of tile row ty that may hold covered pixels (lo > hi: none).
-__device__ inline void spans_row(const Spans& g, int TS, int ty, int* lo, int* hi) {
+__device__ inline void spans_row(const SpanRows& g, int TS, int ty, int* lo, int* hi) {
   int l = g.cx0, h = g.cx1;
   if (g.exact) {
     const double ya = (double)(ty * TS), yb = (double)(ty * TS + TS - 1);
@@ -668,16 +676,41 @@ __device__ inline uint32_t thread_tiles(const Spans& g, int TS, F f) {
   return e;
 }
 
-// Wave version: lanes take tile rows, a wave scan places each row's span and
-// the entries are spread over the lanes.  s_lo/s_off: 64-entry LDS scratch of
-// this wave.  Returns the tile count (wave-uniform).
+// Wave version, for a wide triangle.  A box of at most kBoxTiles tiles: lanes
+// take its tiles and test each as the narrow triangles' are.  A larger one:
+// lanes take tile rows, a wave scan places each row's span (in double) and the
+// entries are spread over the lanes.  f(e, ty, tx) with e numbering the tiles;
+// returns the tile count (wave-uniform).  The rows cost some 250 instructions a
+// triangle, most of them double divisions, 64 tests about 30 (1M-triangle 1080p
+// soup: k_pair_hist 18.9 -> 13.4 us).
+constexpr int kBoxTiles = 256;
+struct WaveRows {  // a wave's LDS scratch
+  int lo[64];
+  uint32_t off[64];
+};
 template <class F>
-__device__ inline uint32_t wave_tiles(const Spans& g, int TS, int lane, int* s_lo, uint32_t* s_off, F f) {
+__device__ inline uint32_t wave_tiles(const SetupRec& r, const Spans& g, int TS, int lane, WaveRows& s, F f) {
   uint32_t o = 0;
+  const int nx = g.cx1 - g.cx0 + 1, n = nx * (g.cy1 - g.cy0 + 1);
+  if (n <= kBoxTiles) {
+    const float inv = 1.0f / (float)nx;
+    for (int t0 = 0; t0 < n; t0 += 64) {
+      const int t = t0 + lane;
+      const int dy = (int)(((float)t + 0.5f) * inv);  // t / nx: exact for t < 512
+      const int ty = g.cy0 + dy, tx = g.cx0 + (t - dy * nx);
+      const bool on = t < n && tile_may_cover(g, TS, tx, ty);
+      const uint64_t m = __ballot(on);
+      if (on) f(o + (uint32_t)__popcll(m & lanemask_lt_u64(lane)), ty, tx);
+      o += (uint32_t)__popcll(m);
+    }
+    return o;
+  }
+  SpanRows sr;
+  spans_init_rows(r, g, sr);
   for (int row0 = g.cy0; row0 <= g.cy1; row0 += 64) {
     const int ty = row0 + lane;
     int lo = 0, hi = -1;
-    if (ty <= g.cy1) spans_row(g, TS, ty, &lo, &hi);
+    if (ty <= g.cy1) spans_row(sr, TS, ty, &lo, &hi);
     const uint32_t c = hi >= lo ? (uint32_t)(hi - lo + 1) : 0u;
     uint32_t x = c;
 #pragma unroll
@@ -686,8 +719,8 @@ __device__ inline uint32_t wave_tiles(const Spans& g, int TS, int lane, int* s_l
       if (lane >= d) x += y;
     }
     const uint32_t total = (uint32_t)__shfl((int)x, 63, 64);
-    s_lo[lane] = lo;
-    s_off[lane] = x - c;
+    s.lo[lane] = lo;
+    s.off[lane] = x - c;
     __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
     for (uint32_t e = (uint32_t)lane; e < total; e += 64) {
       // the row of entry e: the last row whose offset is <= e (rows without
@@ -695,13 +728,84 @@ __device__ inline uint32_t wave_tiles(const Spans& g, int TS, int lane, int* s_l
       int k = 0;
 #pragma unroll
       for (int step = 32; step >= 1; step >>= 1)
-        if (s_off[k + step] <= e) k += step;
-      f(o + e, row0 + k, s_lo[k] + (int)(e - s_off[k]));
+        if (s.off[k + step] <= e) k += step;
+      f(o + e, row0 + k, s.lo[k] + (int)(e - s.off[k]));
     }
     o += total;
     __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
   }
   return o;
+}
+
+// The wide triangles list[w], list[w + step], ... (below n) of one wave:
+// f(tile key, triangle) for each of their tiles, lanes over a triangle's
+// tiles.  Each lane first fetches and prepares one of the wave's next 64
+// triangles, so that the chain of dependent loads (id, record, view) is paid
+// once for all of them and the visits take their constants from registers; a
+// wave per triangle paid some 2 us of latency for each (k_bin_small of a
+// 2312-triangle frame of 3600 tiles: 105 -> 38 us).  For the one workgroup of
+// k_bin_small only: the pair kernels have 4096 waves and few triangles for
+// each, and its 90 VGPRs would keep their wide and other blocks from sharing a
+// CU (k_pair_scatter of a frame with few wide triangles 6 -> 15 us).
+template <class F>
+__device__ inline void wave_wide_tiles(const uint32_t* __restrict__ list, uint32_t w, uint32_t step, uint32_t n,
+                                       const SetupRec* __restrict__ setup, const DevView* __restrict__ views,
+                                       int TS, WaveRows& rows, F f) {
+  const int lane = threadIdx.x & 63;
+  for (uint64_t w0 = w; w0 < n; w0 += 64ull * step) {
+    const uint64_t at = w0 + (uint64_t)step * (uint32_t)lane;
+    const bool on = at < n;
+    uint32_t id = 0, key0 = 0, ntx = 0;
+    Spans g;
+    g.cx0 = g.cy0 = g.cx1 = g.cy1 = 0;
+    g.exact = false;
+#pragma unroll
+    for (int e = 0; e < 3; e++) g.fa[e] = g.fb[e] = g.fk[e] = g.fm[e] = 0.0f;
+    if (on) {
+      id = list[at];
+      const SetupRec r = setup[id];
+      spans_init(r, TS, g);
+      const DevView& vw = views[r.view];
+      ntx = vw.ntx;
+      key0 = vw.tile_base + (uint32_t)g.cy0 * ntx + (uint32_t)g.cx0;
+    }
+    // without edge tests every margin is infinite
+#pragma unroll
+    for (int e = 0; e < 3; e++) g.fm[e] = g.exact ? g.fm[e] : INFINITY;
+    const int nx = g.cx1 - g.cx0 + 1, ny = g.cy1 - g.cy0 + 1;
+    auto bi = [](int v, int b) { return __builtin_amdgcn_readlane(v, b); };
+    auto bf = [](float v, int b) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), b)); };
+    for (uint64_t m = __ballot(on); m; m &= m - 1) {
+      const int b = (int)__builtin_ctzll(m);
+      const uint32_t i = (uint32_t)bi((int)id, b), k0 = (uint32_t)bi((int)key0, b), row = (uint32_t)bi((int)ntx, b);
+      const int unx = bi(nx, b), nt = unx * bi(ny, b);
+      if (nt > kBoxTiles) {
+        const SetupRec r = setup[i];
+        Spans u;
+        spans_init(r, TS, u);
+        wave_tiles(r, u, TS, lane, rows, [&](uint32_t, int ty, int tx) {
+          f(k0 + (uint32_t)(ty - u.cy0) * row + (uint32_t)(tx - u.cx0), i);
+        });
+        continue;
+      }
+      Spans u;
+      u.exact = true;
+#pragma unroll
+      for (int e = 0; e < 3; e++) {
+        u.fa[e] = bf(g.fa[e], b);
+        u.fb[e] = bf(g.fb[e], b);
+        u.fk[e] = bf(g.fk[e], b);
+        u.fm[e] = bf(g.fm[e], b);
+      }
+      const int cx0 = bi(g.cx0, b), cy0 = bi(g.cy0, b);
+      const float inv = 1.0f / (float)unx;
+      for (int t0 = 0; t0 < nt; t0 += 64) {
+        const int t = t0 + lane;
+        const int dy = (int)(((float)t + 0.5f) * inv), dx = t - dy * unx;  // exact: t < 512
+        if (t < nt && tile_may_cover(u, TS, cx0 + dx, cy0 + dy)) f(k0 + (uint32_t)dy * row + (uint32_t)dx, i);
+      }
+    }
+  }
 }
 
 // Ordered bins keep, per clipped triangle, a bin box: x the tile key of the
@@ -1449,16 +1553,14 @@ __global__ __launch_bounds__(256) void k_bin_count_wide(const SetupRec* __restri
                                                         const DevView* __restrict__ views, const Status* status,
                                                         int TS, const uint32_t* __restrict__ wide_list,
                                                         uint32_t* __restrict__ bincnt, uint32_t* __restrict__ tile_cnt) {
-  __shared__ int s_lo[4][64];
-  __shared__ uint32_t s_off[4][64];
+  __shared__ WaveRows s_rows[4];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   for_each_wide(wide_list, status, [&](uint32_t i) {
     const SetupRec r = setup[i];
     const DevView& vw = views[r.view];
     Spans g;
     spans_init(r, TS, g);
-    spans_init_rows(r, g);
-    const uint32_t c = wave_tiles(g, TS, lane, s_lo[wave], s_off[wave], [&](uint32_t, int ty, int tx) {
+    const uint32_t c = wave_tiles(r, g, TS, lane, s_rows[wave], [&](uint32_t, int ty, int tx) {
       if (!ORDERED) atomicAdd(&tile_cnt[vw.tile_base + (uint32_t)ty * vw.ntx + (uint32_t)tx], 1u);
     });
     if (ORDERED && lane == 0) bincnt[i] = c;
@@ -1524,17 +1626,15 @@ __global__ __launch_bounds__(256) void k_bin_emit_wide(const SetupRec* __restric
                                                        const uint32_t* __restrict__ tile_start,
                                                        uint32_t* __restrict__ tile_cur, uint32_t cap_pairs,
                                                        uint32_t* __restrict__ keys, uint32_t* __restrict__ vals) {
-  __shared__ int s_lo[4][64];
-  __shared__ uint32_t s_off[4][64];
+  __shared__ WaveRows s_rows[4];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   for_each_wide(wide_list, status, [&](uint32_t i) {
     const SetupRec r = setup[i];
     const DevView& vw = views[r.view];
     Spans g;
     spans_init(r, TS, g);
-    spans_init_rows(r, g);
     const uint32_t o = ORDERED ? binoff[i] : 0u;
-    wave_tiles(g, TS, lane, s_lo[wave], s_off[wave], [&](uint32_t e, int ty, int tx) {
+    wave_tiles(r, g, TS, lane, s_rows[wave], [&](uint32_t e, int ty, int tx) {
       const uint32_t key = vw.tile_base + (uint32_t)ty * vw.ntx + (uint32_t)tx;
       const uint32_t pos = ORDERED ? o + e : tile_start[key] + atomicAdd(&tile_cur[key], 1u);
       if (pos < cap_pairs) {
@@ -1564,9 +1664,8 @@ __global__ __launch_bounds__(1024) void k_bin_small(const SetupRec* __restrict__
                                                     uint2* __restrict__ ranges) {
   __shared__ uint32_t s_cnt[kSmallBinTiles];
   __shared__ uint32_t s_cur[kSmallBinTiles];
-  __shared__ int s_lo[16][64];
-  __shared__ uint32_t s_off[16][64];
   __shared__ uint32_t s_w[16];
+  __shared__ WaveRows s_rows[16];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   for (uint32_t k = (uint32_t)tid; k < n_tiles; k += 1024u) s_cnt[k] = 0u;
   __syncthreads();
@@ -1580,16 +1679,8 @@ __global__ __launch_bounds__(1024) void k_bin_small(const SetupRec* __restrict__
     }
   };
   auto each_wide_tile = [&](uint32_t nw, auto f) {
-    for (uint32_t w = (uint32_t)wave; w < nw; w += 16u) {
-      const uint32_t i = (uint32_t)__builtin_amdgcn_readfirstlane((int)wide_list[w]);
-      const SetupRec r = setup[i];
-      Spans g;
-      spans_init(r, TS, g);
-      spans_init_rows(r, g);
-      wave_tiles(g, TS, lane, s_lo[wave], s_off[wave], [&](uint32_t, int ty, int tx) {
-        f(i, vw.tile_base + (uint32_t)ty * vw.ntx + (uint32_t)tx);
-      });
-    }
+    wave_wide_tiles(wide_list, (uint32_t)wave, 16u, nw, setup, views, TS, s_rows[wave],
+                    [&](uint32_t key, uint32_t i) { f(i, key); });
   };
   // counts
   each_tile([&](uint32_t, uint32_t key) { atomicAdd(&s_cnt[key], 1u); });
@@ -1785,26 +1876,23 @@ constexpr uint32_t kPairFewTiles = 256u * (kPairCounters / 16u);
 constexpr uint32_t kPairMaxTiles = 2048u * kPairCounters;
 static_assert(2048u * (kPairCols + 1u) <= kRadixHistEntries, "histogram and digit totals");
 
-// Visits the pairs of one chunk: f(tile key, triangle, depth key).  The wide
-// chunks' waves take the listed triangles in turn.
+// Visits the pairs of one chunk: f(tile key, triangle, depth key).
 template <class F>
 __device__ inline void pair_chunk(const uint8_t* __restrict__ dkey, const uint32_t* __restrict__ wide_list,
                                   const SetupRec* __restrict__ setup, const DevView* __restrict__ views,
-                                  const Status* __restrict__ status, uint32_t cap_tri, int TS, int (*s_lo)[64],
-                                  uint32_t (*s_off)[64], F f) {
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+                                  const Status* __restrict__ status, uint32_t cap_tri, int TS, WaveRows* s_rows, F f) {
+  const int tid = threadIdx.x;
   if (blockIdx.x < (uint32_t)kPairChunks) {
+    const int lane = tid & 63, wave = tid >> 6;
     const uint32_t n = min(status->n_wide, cap_tri);
-    const uint32_t w0 = blockIdx.x + (uint32_t)kPairChunks * (uint32_t)wave;
-    for (uint32_t w = w0; w < n; w += (uint32_t)(kPairChunks * (kPairT / 64))) {
+    for (uint32_t w = blockIdx.x + (uint32_t)(kPairChunks * wave); w < n; w += (uint32_t)(kPairChunks * (kPairT / 64))) {
       const uint32_t i = (uint32_t)__builtin_amdgcn_readfirstlane((int)wide_list[w]);
       const SetupRec r = setup[i];
       const DevView& vw = views[r.view];
       const uint32_t dk = dkey[i];
       Spans g;
       spans_init(r, TS, g);
-      spans_init_rows(r, g);
-      wave_tiles(g, TS, lane, s_lo[wave], s_off[wave], [&](uint32_t, int ty, int tx) {
+      wave_tiles(r, g, TS, lane, s_rows[wave], [&](uint32_t, int ty, int tx) {
         f(vw.tile_base + (uint32_t)ty * vw.ntx + (uint32_t)tx, i, dk);
       });
     }
@@ -1845,11 +1933,10 @@ __global__ __launch_bounds__(kPairT) void k_pair_hist(const uint8_t* __restrict_
                                                       const Status* __restrict__ status, uint32_t cap_tri, int TS,
                                                       uint32_t* __restrict__ hist) {
   __shared__ uint32_t h[DIG];
-  __shared__ int s_lo[kPairT / 64][64];
-  __shared__ uint32_t s_off[kPairT / 64][64];
+  __shared__ WaveRows s_rows[kPairT / 64];
   for (int d = threadIdx.x; d < DIG; d += kPairT) h[d] = 0u;
   __syncthreads();
-  pair_chunk(dkey, wide_list, setup, views, status, cap_tri, TS, s_lo, s_off,
+  pair_chunk(dkey, wide_list, setup, views, status, cap_tri, TS, s_rows,
              [&](uint32_t key, uint32_t, uint32_t) { atomicAdd(&h[key & (DIG - 1u)], 1u); });
   __syncthreads();
   const uint32_t col = pair_col();
@@ -1918,8 +2005,11 @@ __device__ inline uint32_t lds_exclusive_scan(uint32_t* s, uint32_t n, uint32_t*
   return carry;
 }
 
+// Held to 64 VGPRs (a dozen spilled words, in the rows of large triangles), so
+// that a wide block and another share a CU: 20 -> 18 us on the 1M-triangle
+// soup; k_pair_hist, without the scatter's waits, lost more to the spills.
 template <int DIG>
-__global__ __launch_bounds__(kPairT) void k_pair_scatter(const uint8_t* __restrict__ dkey,
+__global__ __launch_bounds__(kPairT) __attribute__((amdgpu_waves_per_eu(8))) void k_pair_scatter(const uint8_t* __restrict__ dkey,
                                                          const uint32_t* __restrict__ wide_list,
                                                          const SetupRec* __restrict__ setup,
                                                          const DevView* __restrict__ views, Status* __restrict__ status,
@@ -1928,8 +2018,7 @@ __global__ __launch_bounds__(kPairT) void k_pair_scatter(const uint8_t* __restri
                                                          uint2* __restrict__ pairs) {
   constexpr int kShift = DIG == 256 ? 8 : 11;
   __shared__ uint32_t cur[DIG];
-  __shared__ int s_lo[kPairT / 64][64];
-  __shared__ uint32_t s_off[kPairT / 64][64];
+  __shared__ WaveRows s_rows[kPairT / 64];
   __shared__ uint32_t s_w[kPairT / 64];
   const uint32_t col = pair_col();
   for (int d = threadIdx.x; d < DIG; d += kPairT) cur[d] = totals[d];
@@ -1941,7 +2030,7 @@ __global__ __launch_bounds__(kPairT) void k_pair_scatter(const uint8_t* __restri
   }
   for (int d = threadIdx.x; d < DIG; d += kPairT) cur[d] += hist[(uint32_t)d * kPairCols + col];
   __syncthreads();
-  pair_chunk(dkey, wide_list, setup, views, status, cap_tri, TS, s_lo, s_off,
+  pair_chunk(dkey, wide_list, setup, views, status, cap_tri, TS, s_rows,
              [&](uint32_t key, uint32_t i, uint32_t dk) {
                const uint32_t pos = atomicAdd(&cur[key & (DIG - 1u)], 1u);
                if (pos < cap_pairs) pairs[pos] = make_uint2((key >> kShift) << 8 | dk, i);
