@@ -335,6 +335,38 @@ __device__ inline int cull_and_clip(const FrameParamsPod& fr, const V& a, const 
   return cnt;
 }
 
+// clip_plane's count alone.
+__device__ inline int clip_count(const float* pl, V3 a, V3 b, V3 c) {
+  const float fa = plane_f(pl, a), fb = plane_f(pl, b), fc = plane_f(pl, c);
+  if (fa > 0.0f && fb > 0.0f && fc > 0.0f) return 1;
+  if (fa <= 0.0f && fb <= 0.0f && fc <= 0.0f) return 0;
+  const bool r1 = fa * fc >= 0.0f;
+  const bool r2 = !r1 && (fb * fc >= 0.0f);
+  return (r1 ? fb : (r2 ? fa : fc)) <= 0.0f ? 2 : 1;
+}
+
+// One output of clip_plane (the second: of a triangle with two), in place.
+__device__ inline void clip_select(const float* pl, FV& a, FV& b, FV& c, bool second) {
+  FV o0, o1, o2, p0, p1, p2;
+  (void)clip_plane(pl, a, b, c, o0, o1, o2, p0, p1, p2);
+  a = selv(second, p0, o0);
+  b = selv(second, p1, o1);
+  c = selv(second, p2, o2);
+}
+
+// Output k of cull_and_clip, in place, of a triangle that has more than k.
+// The first near output's far count says which of the two near outputs it
+// comes from; the attributes then go through the two cuts once.
+__device__ inline void clip_output(const FrameParamsPod& fr, FV& a, FV& b, FV& c, uint32_t k) {
+  const PV pa{a.p}, pb{b.p}, pc{c.p};
+  PV n0, n1, n2, m0, m1, m2;
+  (void)clip_plane(fr.planes[0], pa, pb, pc, n0, n1, n2, m0, m1, m2);
+  const uint32_t nf = (uint32_t)clip_count(fr.planes[1], n0.p, n1.p, n2.p);
+  const bool from_second = k >= nf;
+  clip_select(fr.planes[0], a, b, c, from_second);
+  clip_select(fr.planes[1], a, b, c, (from_second ? k - nf : k) == 1u);
+}
+
 // ====================================================================== setup
 // Rectangle::from_coords + Rectangle::clip along one axis (canvas.rs:315-350,
 // 646-658).
@@ -350,9 +382,6 @@ __device__ inline void rect_axis(uint64_t a0, uint64_t a1, uint64_t smax, uint32
 // snapping (canvas.rs:585-587, 896-904), edge constants, normalizers,
 // tie-break products (660-666) and the scan rectangle (640-658).  Writes the
 // SetupRec and ShadeRec of one clipped triangle with 16-byte stores.
-// TINY_DROP: drop a FAST triangle of at most 3x3 pixels that covers none of
-// them (the unclipped emits; the clipper's registers leave no room for it).
-template <bool TINY_DROP>
 __device__ inline void make_setup(const FrameParamsPod& fr, const FV& A, const FV& B, const FV& C, uint32_t material,
                                   const DevMaterial& mat, uint32_t view, uint32_t group, uint4 (&ro)[6],
                                   uint4 (&so)[9], SetupRec& rec) {
@@ -408,7 +437,7 @@ __device__ inline void make_setup(const FrameParamsPod& fr, const FV& A, const F
   // (0) A FAST triangle whose scan rectangle is at most 3x3 pixels and holds
   // no covered pixel: the raster's own test (covered_fast at each pixel of
   // the rectangle) settled here, where the triangle is still in registers.
-  if (TINY_DROP && (flags & kFast) && x1 - x0 <= 2u && y1 - y0 <= 2u) {
+  if ((flags & kFast) && x1 - x0 <= 2u && y1 - y0 <= 2u) {
     bool any = false;
 #pragma unroll
     for (uint32_t k = 0; k < 9u; k++) {
@@ -918,7 +947,7 @@ __device__ inline void emit_box_pairs(uint2 box, uint32_t i, uint32_t o, uint32_
 // ================================================================== geometry
 // Small single-view frames: at most kSmallBinTris input triangles and
 // kSmallBinTiles tiles take single-workgroup kernels for the geometry lists
-// (k_geom_small) and the binning (k_bin_small), and one launch for both emits.
+// (k_geom_small) and the binning (k_bin_small).
 constexpr uint32_t kSmallBinTiles = 4096;  // LDS counters and cursors: 32 KB
 constexpr uint32_t kSmallBinTris = 16384;  // LDS count bytes: 16 KB
 
@@ -1080,89 +1109,24 @@ __global__ __launch_bounds__(256) void k_geom_compact(uint32_t n_in, const uint8
 
 
 
-// One thread per emitting input triangle of one list (dense: culled
-// triangles take no lane).  The unclipped list (CLIP false) skips the
-// clipper, whose attribute registers would otherwise size the whole kernel.
+// One output of an emitting input triangle per lane (every lane of the wave
+// calls it; lanes without an output with active false): list entry sv, output
+// k of the clipper for CLIP, else the triangle itself.  Its records leave
+// through the wave's LDS area stage[64 * 9].
 template <int BIN>
-__device__ __forceinline__ void geom_emit_clipped(uint32_t j, const DevDraw* __restrict__ draws, uint32_t n_draws,
-                                                  const DevView* __restrict__ views, const uint2* __restrict__ surv,
-                                                  const DevMaterial* __restrict__ mats, SetupRec* __restrict__ setup,
-                                                  ShadeRec* __restrict__ shade, uint32_t cap_tri, Status* __restrict__ status,
-                                                  int TS, uint32_t* __restrict__ bincnt, uint8_t* __restrict__ wflag,
-                                                  uint32_t* __restrict__ wide_list, WideBuf* wide, uint32_t span) {
-  const uint2 sv = surv[status->n_simple + j];
-  const uint32_t t = sv.x, base = sv.y;
-  // the lanes of the wave still in the loop
-  const bool sparse = wave_sparse(true, t, span);
-  const DevDraw& dr = draws[wave_find_draw(draws, n_draws, t, true)];
-  const FrameParamsPod& fr = views[dr.view].fr;
-  const uint32_t lt = t - dr.tri_begin;
-  const V3 cam = v3(fr.cam[0], fr.cam[1], fr.cam[2]);
-  const V3 L = v3(fr.light[0], fr.light[1], fr.light[2]);
-  FV v[3];
-  V3 P[3], N[3];
-  float U[3], W[3];
-  tri_vertices(dr, lt, sparse, P, N, U, W);
-#pragma unroll
-  for (int k = 0; k < 3; k++) {
-    const V3 p = P[k];
-    v[k].p = p;
-    // per-vertex visual info, scene/mod.rs:920-925
-    const V3 eye_dir = sub(p, cam);
-    const V3 light = normalized(sub(p, L));
-    const V3 eye = normalized(eye_dir);
-    v[k].d = norm(eye_dir);
-    v[k].l = light;
-    v[k].h = normalized(add(light, eye));
-    v[k].n = N[k];
-    v[k].u = U[k];
-    v[k].v = W[k];
-  }
-  const uint32_t material = dr.material, view = dr.view, group = dr.group;
-  auto out = [&](int k, const FV& A, const FV& B, const FV& C) {
-    const uint32_t idx = base + (uint32_t)k;
-    if (idx >= cap_tri) {
-      atomicOr(&status->overflow, 1u);
-      return;
-    }
-    SetupRec rec;
-    uint4 ro[6], so[9];
-    make_setup<false>(fr, A, B, C, material, mats[material], view, group, ro, so, rec);
-    // with ordered bins nothing reads a dropped triangle's records
-    if (BIN == kBinNone || !(rec.flags & kDrop)) {
-#pragma unroll
-      for (int q = 0; q < 6; q++) reinterpret_cast<uint4*>(setup + idx)[q] = ro[q];
-#pragma unroll
-      for (int q = 0; q < 9; q++) reinterpret_cast<uint4*>(shade + idx)[q] = so[q];
-    }
-    if constexpr (BIN != kBinNone) {
-      const bool is_wide = bin_count_one<BIN>(rec, TS, idx, views[view], bincnt, wflag, bin_boxes(wflag, cap_tri));
-      if (BIN == kBinNear && is_wide) wide_push(*wide, idx, status, wide_list);
-    }
-  };
-  cull_and_clip(fr, v[0], v[1], v[2], !(dr.flags & kDrawNoCull), out);
-}
-
-// One unclipped list entry per lane (every lane of the wave calls it; lanes
-// past the list end with active false): one record each at the entry's output
-// id, stored through the wave's LDS area stage[64 * 9].
-template <int BIN>
-__device__ __forceinline__ void geom_emit_simple(uint32_t j, bool active, uint4* stage, const DevDraw* __restrict__ draws,
-                                                 uint32_t n_draws, const DevView* __restrict__ views,
-                                                 const uint2* __restrict__ surv, const DevMaterial* __restrict__ mats,
-                                                 SetupRec* __restrict__ setup, ShadeRec* __restrict__ shade, uint32_t cap_tri,
-                                                 Status* __restrict__ status, int TS, uint32_t* __restrict__ bincnt,
-                                                 uint8_t* __restrict__ wflag, uint32_t* __restrict__ wide_list,
-                                                 WideBuf* wide, uint32_t span) {
+__device__ __forceinline__ void geom_emit_one(uint2 sv, bool active, bool clip, uint32_t k, uint4* stage,
+                                              const DevDraw* __restrict__ draws, uint32_t n_draws,
+                                              const DevView* __restrict__ views, const DevMaterial* __restrict__ mats,
+                                              SetupRec* __restrict__ setup, ShadeRec* __restrict__ shade,
+                                              uint32_t cap_tri, Status* __restrict__ status, int TS,
+                                              uint32_t* __restrict__ bincnt, uint8_t* __restrict__ wflag,
+                                              uint32_t* __restrict__ wide_list, WideBuf* wide, uint32_t span) {
   uint4 ro[6], so[9];
-  uint32_t idx = 0;
+  const uint32_t t = sv.x, idx = sv.y + k;
   bool ok = false, skip = false;
-  const uint2 sv = active ? surv[j] : make_uint2(0u, 0u);
-  const bool sparse = wave_sparse(active, sv.x, span);
-  const uint32_t d = wave_find_draw(draws, n_draws, sv.x, active);
+  const bool sparse = wave_sparse(active, t, span);
+  const uint32_t d = wave_find_draw(draws, n_draws, t, active);
   if (active) {
-    const uint32_t t = sv.x;
-    idx = sv.y;
     const DevDraw& dr = draws[d];
     const FrameParamsPod& fr = views[dr.view].fr;
     const uint32_t lt = t - dr.tri_begin;
@@ -1173,26 +1137,27 @@ __device__ __forceinline__ void geom_emit_simple(uint32_t j, bool active, uint4*
     float U[3], W[3];
     tri_vertices(dr, lt, sparse, P, N, U, W);
 #pragma unroll
-    for (int k = 0; k < 3; k++) {
-      const V3 p = P[k];
-      v[k].p = p;
+    for (int q = 0; q < 3; q++) {
+      const V3 p = P[q];
+      v[q].p = p;
       // per-vertex visual info, scene/mod.rs:920-925
       const V3 eye_dir = sub(p, cam);
       const V3 light = normalized(sub(p, L));
       const V3 eye = normalized(eye_dir);
-      v[k].d = norm(eye_dir);
-      v[k].l = light;
-      v[k].h = normalized(add(light, eye));
-      v[k].n = N[k];
-      v[k].u = U[k];
-      v[k].v = W[k];
+      v[q].d = norm(eye_dir);
+      v[q].l = light;
+      v[q].h = normalized(add(light, eye));
+      v[q].n = N[q];
+      v[q].u = U[q];
+      v[q].v = W[q];
     }
+    // passed the back-face and lateral tests in k_geom_count
+    if (clip) clip_output(fr, v[0], v[1], v[2], k);
     if (idx >= cap_tri) {
       atomicOr(&status->overflow, 1u);
     } else {
-      // passed the back-face and lateral tests in k_geom_count
       SetupRec rec;
-      make_setup<true>(fr, v[0], v[1], v[2], dr.material, mats[dr.material], dr.view, dr.group, ro, so, rec);
+      make_setup(fr, v[0], v[1], v[2], dr.material, mats[dr.material], dr.view, dr.group, ro, so, rec);
       ok = true;
       // with ordered bins nothing reads a dropped triangle's records
       skip = BIN != kBinNone && (rec.flags & kDrop);
@@ -1206,78 +1171,49 @@ __device__ __forceinline__ void geom_emit_simple(uint32_t j, bool active, uint4*
   wave_store<9>(stage, so, ok, idx, reinterpret_cast<uint4*>(shade), skip);
 }
 
-// A grid-stride loop over one list (its length is on the device), so that the
-// grid can be capped well below one thread per input triangle.  The unclipped
-// list goes a wave at a time (its records leave through LDS).
-template <int BIN, bool CLIP>
-__global__ __launch_bounds__(256) void k_geom_emit(const DevDraw* __restrict__ draws, uint32_t n_draws,
-                                                   const DevView* __restrict__ views,
-                                                   const uint2* __restrict__ surv,
-                                                   const DevMaterial* __restrict__ mats, SetupRec* __restrict__ setup,
-                                                   ShadeRec* __restrict__ shade, uint32_t cap_tri,
-                                                   Status* __restrict__ status, int TS, uint32_t* __restrict__ bincnt,
-                                                   uint8_t* __restrict__ wflag, uint32_t* __restrict__ wide_list,
-                                                   uint32_t span) {
-  __shared__ uint32_t s_wide[BIN == kBinNear ? sizeof(WideBuf) / 4 : 1];
-  WideBuf* const wide = reinterpret_cast<WideBuf*>(s_wide);
-  if constexpr (BIN == kBinNear) {
-    if (threadIdx.x == 0) wide->n = 0u;
-    __syncthreads();
-  }
-  if constexpr (CLIP) {
-    const uint32_t n = status->n_clip;
-    for (uint32_t j = blockIdx.x * 256u + threadIdx.x; j < n; j += gridDim.x * 256u)
-      geom_emit_clipped<BIN>(j, draws, n_draws, views, surv, mats, setup, shade, cap_tri, status, TS, bincnt, wflag,
-                             wide_list, wide, span);
-  } else {
-    __shared__ uint4 s_stage[4][64 * 9];
-    const uint32_t n = status->n_simple;
-    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
-    for (uint32_t j0 = blockIdx.x * 256u + wave * 64u; j0 < n; j0 += gridDim.x * 256u)
-      geom_emit_simple<BIN>(j0 + lane, j0 + lane < n, s_stage[wave], draws, n_draws, views, surv, mats, setup, shade,
-                            cap_tri, status, TS, bincnt, wflag, wide_list, wide, span);
-  }
-  if constexpr (BIN == kBinNear) wide_flush(*wide, status, wide_list);
-}
-
-// Both emitter lists of a small frame in one launch on the stream (for a few
-// thousand triangles the fork to a second stream and the join back cost more
-// than the emits): of its g_clip + g_simple blocks, g_clip run the clipped
-// list and the others the unclipped one, interleaved in proportion (block b
-// is a clipped block when floor((b + 1) g_clip / G) > floor(b g_clip / G)).
-// No occupancy floor: the grid (at most 128 blocks) fills a fraction of the
-// chip, so registers go to the clipped path (167-172 VGPRs, no spills)
-// rather than to waves that would have nothing to run.
+// Both emitter lists (dense: culled triangles take no lane) in one launch, a
+// wave per unit of 64 lanes, the clipped list's units first: two lanes a
+// clipped triangle, for its even and its odd outputs (it has at most four, and
+// seldom more than two), one an unclipped one.  The lists' lengths are on the
+// device, so the grid is capped and the waves stride over the units.
+//
+// A clipped triangle is a long chain of dependent work.  With a lane each, up
+// to four inlined copies of the setup (28 KB of code) and 168 VGPRs, its list
+// took 25 us even when short, on a second stream beside the other list's
+// launch: the fork and the join cost some 15 us more.  One copy of the setup
+// serves both lists here (17 KB, 122 VGPRs), at the four waves per SIMD that
+// the LDS of the record stores allows.  Frames, before -> after: 62k triangles
+// at 800x600 with a GUI 194 -> 179 us, 150k at 1237x709 168 -> 152, the
+// 1M-triangle 1080p soup 357 -> 339, two 125k-triangle shards 403 -> 391.
 template <int BIN>
-__global__ __launch_bounds__(256) void k_geom_emit_both(const DevDraw* __restrict__ draws, uint32_t n_draws,
-                                                        const DevView* __restrict__ views,
-                                                        const uint2* __restrict__ surv,
-                                                        const DevMaterial* __restrict__ mats,
-                                                        SetupRec* __restrict__ setup, ShadeRec* __restrict__ shade,
-                                                        uint32_t cap_tri, Status* __restrict__ status, int TS,
-                                                        uint32_t* __restrict__ bincnt, uint8_t* __restrict__ wflag,
-                                                        uint32_t* __restrict__ wide_list, uint32_t g_clip) {
+__global__ __launch_bounds__(256, 4) void k_geom_emit(const DevDraw* __restrict__ draws, uint32_t n_draws,
+                                                      const DevView* __restrict__ views,
+                                                      const uint2* __restrict__ surv, const uint8_t* __restrict__ cnt,
+                                                      const DevMaterial* __restrict__ mats,
+                                                      SetupRec* __restrict__ setup, ShadeRec* __restrict__ shade,
+                                                      uint32_t cap_tri, Status* __restrict__ status, int TS,
+                                                      uint32_t* __restrict__ bincnt, uint8_t* __restrict__ wflag,
+                                                      uint32_t* __restrict__ wide_list, uint32_t span) {
   __shared__ uint32_t s_wide[BIN == kBinNear ? sizeof(WideBuf) / 4 : 1];
+  __shared__ uint4 s_stage[4][64 * 9];
   WideBuf* const wide = reinterpret_cast<WideBuf*>(s_wide);
   if constexpr (BIN == kBinNear) {
     if (threadIdx.x == 0) wide->n = 0u;
     __syncthreads();
   }
-  __shared__ uint4 s_stage[4][64 * 9];
-  const uint64_t G = gridDim.x, b = blockIdx.x;
-  const uint32_t c0 = (uint32_t)(b * g_clip / G), c1 = (uint32_t)((b + 1) * g_clip / G);
-  if (c1 > c0) {
-    const uint32_t n = status->n_clip;
-    for (uint32_t j = c0 * 256u + threadIdx.x; j < n; j += g_clip * 256u)
-      geom_emit_clipped<BIN>(j, draws, n_draws, views, surv, mats, setup, shade, cap_tri, status, TS, bincnt, wflag,
-                             wide_list, wide, kSparseSpan);
-  } else {
-    const uint32_t ub = (uint32_t)b - c0, g_simple = (uint32_t)G - g_clip;
-    const uint32_t n = status->n_simple;
-    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
-    for (uint32_t j0 = ub * 256u + wave * 64u; j0 < n; j0 += g_simple * 256u)
-      geom_emit_simple<BIN>(j0 + lane, j0 + lane < n, s_stage[wave], draws, n_draws, views, surv, mats, setup, shade,
-                            cap_tri, status, TS, bincnt, wflag, wide_list, wide, kSparseSpan);
+  const uint32_t lane = threadIdx.x & 63u;
+  const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const uint32_t n_simple = status->n_simple, n_clip = status->n_clip;
+  const uint32_t uc = (n_clip + 31u) / 32u, us = (n_simple + 63u) / 64u;
+  for (uint32_t u = blockIdx.x * 4u + wave; u < uc + us; u += gridDim.x * 4u) {
+    const bool clip = u < uc;
+    const uint32_t j = clip ? u * 32u + (lane >> 1) : (u - uc) * 64u + lane;
+    const bool in = j < (clip ? n_clip : n_simple);
+    const uint2 sv = in ? surv[clip ? n_simple + j : j] : make_uint2(0u, 0u);
+    const uint32_t c = in ? (clip ? (uint32_t)cnt[sv.x] & kCntMask : 1u) : 0u;
+    for (uint32_t k = clip ? lane & 1u : 0u; __ballot(k < c) != 0ull; k += 2u)
+      geom_emit_one<BIN>(sv, k < c, clip, k, s_stage[wave], draws, n_draws, views, mats, setup, shade, cap_tri, status,
+                         TS, bincnt, wflag, wide_list, wide, span);
   }
   if constexpr (BIN == kBinNear) wide_flush(*wide, status, wide_list);
 }
@@ -2249,22 +2185,6 @@ int enqueue_radix_sort(uint32_t* const keys[2], uint32_t* const vals[2], const u
   return cur;
 }
 
-// Fork: work launched on the returned stream runs beside the main stream's
-// (the side stream waits for everything enqueued on `s` so far).  Without a
-// side stream it is `s` itself.
-static hipStream_t fork(hipStream_t s, const PipeArgs& a, int i) {
-  if (!a.side) return s;
-  (void)hipEventRecord(a.xev[i], s);
-  (void)hipStreamWaitEvent(a.side, a.xev[i], 0);
-  return a.side;
-}
-// Join: the main stream waits for everything enqueued on the side stream.
-static void join(hipStream_t s, const PipeArgs& a, int i) {
-  if (!a.side) return;
-  (void)hipEventRecord(a.xev[i], a.side);
-  (void)hipStreamWaitEvent(s, a.xev[i], 0);
-}
-
 // Status reset, geometry, view bases and binning of one pipeline pass;
 // returns the arguments the per-tile stages read (tile lists in b.vals[0]).
 PipeArgs enqueue_front(const PipeArgs& a, hipStream_t s) {
@@ -2284,26 +2204,12 @@ PipeArgs enqueue_front(const PipeArgs& a, hipStream_t s) {
   // leave alone; else in keys[1] until the radix sort needs it (both hold
   // cap_pairs >= cap_tri entries)
   uint32_t* const wide_list = near ? a.vals[1] : a.keys[1];
-  // a small single-view frame: one workgroup builds the emitter lists, and
-  // both emits share one launch on this stream
+  // a small single-view frame: one workgroup builds the emitter lists
   const bool small_geom = a.n_views == 1 && a.n_tri_in <= kSmallBinTris;
   // 1-3 geometry with ordered compaction
   if (n_blk && small_geom) {
     hipLaunchKernelGGL(k_geom_small, dim3(1), dim3(1024), 0, s, a.draws, a.n_draws, a.views, a.n_tri_in, a.cnt, a.blk,
                        a.status, a.cap_tri, a.surv);
-    const uint32_t g_simple = n_blk, g_clip = n_blk;
-    if (near)
-      hipLaunchKernelGGL(k_geom_emit_both<kBinNear>, dim3(g_clip + g_simple), dim3(256), 0, s, a.draws, a.n_draws,
-                         a.views, a.surv, a.mats, a.setup, a.shade, a.cap_tri, a.status, a.TS, nullptr, wflag,
-                         wide_list, g_clip);
-    else if (a.ordered_bins)
-      hipLaunchKernelGGL(k_geom_emit_both<kBinSubmit>, dim3(g_clip + g_simple), dim3(256), 0, s, a.draws, a.n_draws,
-                         a.views, a.surv, a.mats, a.setup, a.shade, a.cap_tri, a.status, a.TS, a.bincnt, wflag,
-                         nullptr, g_clip);
-    else
-      hipLaunchKernelGGL(k_geom_emit_both<kBinNone>, dim3(g_clip + g_simple), dim3(256), 0, s, a.draws, a.n_draws,
-                         a.views, a.surv, a.mats, a.setup, a.shade, a.cap_tri, a.status, a.TS, nullptr, nullptr,
-                         nullptr, g_clip);
   } else if (n_blk) {
     uint32_t* blk_simple = a.blk + geom_blk_stride(n_blk);
     uint32_t* blk_clip = a.blk + 2 * geom_blk_stride(n_blk);
@@ -2316,32 +2222,20 @@ PipeArgs enqueue_front(const PipeArgs& a, hipStream_t s) {
     hipLaunchKernelGGL(k_scan_segs, dim3(3), dim3(1024), 0, s, g, n_blk);
     hipLaunchKernelGGL(k_geom_compact, dim3(n_blk), dim3(256), 0, s, a.n_tri_in, a.cnt, a.blk, blk_simple, blk_clip,
                        a.status, a.surv);
-    // the unclipped and clipped emits write disjoint outputs: the clipped
-    // one runs beside the other on the side stream.  Capped grids (the lists'
-    // lengths are on the device): 2048 and 1024 blocks, a grid-stride loop
-    // beyond that.
-    const uint32_t g_simple = std::min<uint32_t>(n_blk, 2048u), g_clip = std::min<uint32_t>(n_blk, 1024u);
+  }
+  if (n_blk) {
+    // at most twice the blocks that fit, to even out the units (their number is on the device)
+    const dim3 ge(std::min<uint32_t>(2u * n_blk, 2048u));
     const uint32_t span = (uint64_t)a.n_tri_in >= (uint64_t)a.n_pixels ? kSparseSpanDense : kSparseSpan;
-    const hipStream_t s2 = fork(s, a, 0);
-    // (the clipped emit, the longer one per thread, starts first on the main
-    // stream; the unclipped one waits for the fork on the side stream)
-    if (near) {
-      hipLaunchKernelGGL((k_geom_emit<kBinNear, true>), dim3(g_clip), dim3(256), 0, s, a.draws, a.n_draws, a.views,
-                         a.surv, a.mats, a.setup, a.shade, a.cap_tri, a.status, a.TS, nullptr, wflag, wide_list, span);
-      hipLaunchKernelGGL((k_geom_emit<kBinNear, false>), dim3(g_simple), dim3(256), 0, s2, a.draws, a.n_draws, a.views,
-                         a.surv, a.mats, a.setup, a.shade, a.cap_tri, a.status, a.TS, nullptr, wflag, wide_list, span);
-    } else if (a.ordered_bins) {
-      hipLaunchKernelGGL((k_geom_emit<kBinSubmit, true>), dim3(g_clip), dim3(256), 0, s, a.draws, a.n_draws, a.views,
-                         a.surv, a.mats, a.setup, a.shade, a.cap_tri, a.status, a.TS, a.bincnt, wflag, nullptr, span);
-      hipLaunchKernelGGL((k_geom_emit<kBinSubmit, false>), dim3(g_simple), dim3(256), 0, s2, a.draws, a.n_draws, a.views,
-                         a.surv, a.mats, a.setup, a.shade, a.cap_tri, a.status, a.TS, a.bincnt, wflag, nullptr, span);
-    } else {
-      hipLaunchKernelGGL((k_geom_emit<kBinNone, true>), dim3(g_clip), dim3(256), 0, s, a.draws, a.n_draws, a.views,
-                         a.surv, a.mats, a.setup, a.shade, a.cap_tri, a.status, a.TS, nullptr, nullptr, nullptr, span);
-      hipLaunchKernelGGL((k_geom_emit<kBinNone, false>), dim3(g_simple), dim3(256), 0, s2, a.draws, a.n_draws, a.views,
-                         a.surv, a.mats, a.setup, a.shade, a.cap_tri, a.status, a.TS, nullptr, nullptr, nullptr, span);
-    }
-    join(s, a, 1);
+    if (near)
+      hipLaunchKernelGGL(k_geom_emit<kBinNear>, ge, dim3(256), 0, s, a.draws, a.n_draws, a.views, a.surv, a.cnt, a.mats,
+                         a.setup, a.shade, a.cap_tri, a.status, a.TS, nullptr, wflag, wide_list, span);
+    else if (a.ordered_bins)
+      hipLaunchKernelGGL(k_geom_emit<kBinSubmit>, ge, dim3(256), 0, s, a.draws, a.n_draws, a.views, a.surv, a.cnt,
+                         a.mats, a.setup, a.shade, a.cap_tri, a.status, a.TS, a.bincnt, wflag, nullptr, span);
+    else
+      hipLaunchKernelGGL(k_geom_emit<kBinNone>, ge, dim3(256), 0, s, a.draws, a.n_draws, a.views, a.surv, a.cnt,
+                         a.mats, a.setup, a.shade, a.cap_tri, a.status, a.TS, nullptr, nullptr, nullptr, span);
   }
   if (a.n_views > 1)
     hipLaunchKernelGGL(k_view_id_base, dim3(cdiv(a.n_views, 4)), dim3(256), 0, s, const_cast<DevView*>(a.views),

@@ -59,11 +59,6 @@ struct PipeArgs {
   uint32_t* tables_dst;
   uint32_t tables_words;
   hipEvent_t ev[5];    // optional stage events (all null when not profiling)
-  // independent kernels fork onto `side` (null: everything on the main
-  // stream) and join back with xev[] (fork 0 / join 1: the two geometry
-  // emits)
-  hipStream_t side;
-  hipEvent_t xev[2];
 };
 
 // One transparent mesh (device pointers): its triangles, sorted in place.
