@@ -161,9 +161,8 @@ struct dh_ctx_s {
   std::vector<dh::TransMesh> h_tmeshes;
   std::vector<uint32_t> h_grp_first;  // first opaque input triangle of each object group
   uint64_t n_tin = 0, max_tmesh = 0;
-  DevBuf<dh::DevDraw> tdraws;
-  DevBuf<uint32_t> grp;       // [2 * groups]: first input triangle, then first clipped id
-  DevBuf<uint32_t> tperm;     // [9 * max_tmesh]
+  DevBuf<uint32_t> grp;       // [groups]: first clipped id
+  DevBuf<uint32_t> tperm;     // the triangles being sorted (TransArgs::perm_tmp)
   DevBuf<uint32_t> sort_n;    // [1]
   dh_stats stats = {};
   // captured batch launch (DH_BATCH_GRAPH)
@@ -238,6 +237,11 @@ size_t draw_bytes(uint64_t n_draws) { return (std::max<uint64_t>(n_draws, 1) * s
 size_t tables_bytes(uint64_t n_draws, uint64_t n_views) {
   return draw_bytes(n_draws) + std::max<uint64_t>(n_views, 1) * sizeof(dh::DevView);
 }
+// ...then, for a frame with transparent meshes, their draws and the groups' first triangles.
+size_t tdraws_off(uint64_t n_draws, uint64_t n_views) { return (tables_bytes(n_draws, n_views) + 255) & ~(size_t)255; }
+size_t groups_off(uint64_t n_draws, uint64_t n_views, uint64_t n_tdraws) {
+  return tdraws_off(n_draws, n_views) + draw_bytes(n_tdraws);
+}
 
 // Bytes every scratch buffer would hold after ensure_scratch with these sizes.
 uint64_t scratch_bytes_after(dh_ctx c, uint64_t n_in, uint64_t cap_tri, uint64_t cap_pairs, uint64_t n_tiles,
@@ -255,7 +259,7 @@ uint64_t scratch_bytes_after(dh_ctx c, uint64_t n_in, uint64_t cap_tri, uint64_t
 
 // Grow every scratch buffer to the given capacities.
 int ensure_scratch(dh_ctx c, uint32_t n_in, uint32_t cap_tri, uint32_t cap_pairs, uint32_t n_tiles,
-                   uint32_t n_pixels, uint32_t n_draws, uint32_t n_views) {
+                   uint32_t n_pixels, uint32_t n_draws, uint32_t n_views, uint32_t n_tdraws, uint32_t n_groups) {
   HIPCHK(c, c->cnt.ensure(n_in));
   HIPCHK(c, c->blk.ensure(3ull * dh::geom_blk_stride((n_in + 255) / 256)));  // output, unclipped and clipped emitter counts
   HIPCHK(c, c->surv.ensure(2ull * n_in));
@@ -275,7 +279,8 @@ int ensure_scratch(dh_ctx c, uint32_t n_in, uint32_t cap_tri, uint32_t cap_pairs
   HIPCHK(c, c->vis.ensure(n_pixels));
   HIPCHK(c, c->status.ensure(2));  // opaque pass, transparent pass
   {
-    const size_t need = tables_bytes(n_draws, n_views);
+    const size_t need = n_tdraws ? groups_off(n_draws, n_views, n_tdraws) + 4ull * n_groups
+                                 : tables_bytes(n_draws, n_views);
     if (c->tables.n < need || !c->tables.p) {
       HIPCHK(c, c->tables.ensure(need));
     }
@@ -395,7 +400,7 @@ extern "C" int dh_ctx_destroy(dh_ctx c) {
   c->hist.release(); c->partials.release(); c->ranges.release(); c->vis.release();
   c->tile_cnt.release(); c->tile_start.release();
   c->status.release(); c->tables.release(); c->draws = nullptr; c->views = nullptr; c->export_buf.release();
-  c->tdraws.release(); c->grp.release(); c->tperm.release(); c->sort_n.release();
+  c->grp.release(); c->tperm.release(); c->sort_n.release();
   release_gui(c);
   if (c->h_status) hipHostFree(c->h_status);
   if (c->h_tables) hipHostFree(c->h_tables);
@@ -878,24 +883,28 @@ int render_views(dh_ctx c, const dh_view* views, uint32_t n_views, bool use_grap
         return fail(c, DH_E_BUDGET, "frame scratch would exceed the context's cap");
       }
     }
+    const uint32_t n_groups = (uint32_t)c->h_grp_first.size();
     rc = ensure_scratch(c, (uint32_t)n_max, (uint32_t)want_tri, (uint32_t)want_pairs, n_tiles, n_pixels,
-                        (uint32_t)c->h_draws.size(), (uint32_t)c->h_views.size());
+                        (uint32_t)c->h_draws.size(), (uint32_t)c->h_views.size(), (uint32_t)c->h_tdraws.size(),
+                        n_groups);
     if (rc) return rc;
-    // both tables into the pinned staging (the previous frame has completed);
+    // the tables into the pinned staging (the previous frame has completed);
     // the frame's first kernel copies them to the device
     memcpy(c->h_tables, c->h_draws.data(), c->h_draws.size() * sizeof(dh::DevDraw));
     memcpy(c->h_tables + c->tables_view_off, c->h_views.data(), c->h_views.size() * sizeof(dh::DevView));
     c->tables_used = c->tables_view_off + c->h_views.size() * sizeof(dh::DevView);
-    const uint32_t n_groups = (uint32_t)c->h_grp_first.size();
+    const size_t td_off = tdraws_off(c->h_draws.size(), c->h_views.size());
+    const size_t grp_off = groups_off(c->h_draws.size(), c->h_views.size(), c->h_tdraws.size());
+    // the sorted triangles' copies: all meshes at once, up to 64 MB more than the largest needs
+    const uint64_t perm_chunks = std::max<uint64_t>(c->max_tmesh / 1024 + 1,
+                                                    std::min<uint64_t>(c->n_tin / 1024 + c->h_tmeshes.size(), 1820));
     if (transparent) {
-      HIPCHK(c, c->tdraws.ensure(c->h_tdraws.size()));
-      HIPCHK(c, c->grp.ensure(2ull * n_groups));
-      HIPCHK(c, c->tperm.ensure(9ull * c->max_tmesh));
+      HIPCHK(c, c->grp.ensure(n_groups));
+      HIPCHK(c, c->tperm.ensure(9ull * 1024 * perm_chunks));
       HIPCHK(c, c->sort_n.ensure(1));
-      HIPCHK(c, hipMemcpyAsync(c->tdraws.p, c->h_tdraws.data(), c->h_tdraws.size() * sizeof(dh::DevDraw),
-                               hipMemcpyHostToDevice, c->stream));
-      HIPCHK(c, hipMemcpyAsync(c->grp.p, c->h_grp_first.data(), n_groups * sizeof(uint32_t), hipMemcpyHostToDevice,
-                               c->stream));
+      memcpy(c->h_tables + td_off, c->h_tdraws.data(), c->h_tdraws.size() * sizeof(dh::DevDraw));
+      memcpy(c->h_tables + grp_off, c->h_grp_first.data(), n_groups * sizeof(uint32_t));
+      c->tables_used = grp_off + n_groups * sizeof(uint32_t);
     }
     // everything a captured launch sequence bakes in
     std::vector<uint64_t> gkey = key;
@@ -931,16 +940,18 @@ int render_views(dh_ctx c, const dh_view* views, uint32_t n_views, bool use_grap
         for (int k = 0; k < 3; k++) ta.cam[k] = c->h_views[0].fr.cam[k];
         ta.sort_n = c->sort_n.p;
         ta.perm_tmp = c->tperm.p;
-        ta.grp_first = c->grp.p;
-        ta.grp_base = c->grp.p + n_groups;
+        ta.perm_chunks = (uint32_t)perm_chunks;
+        ta.grp_first = reinterpret_cast<const uint32_t*>(c->tables.p + grp_off);
+        ta.grp_base = c->grp.p;
         ta.n_groups = n_groups;
         ta.pass = make_args(c, mats, (uint32_t)c->n_tin, n_tiles, n_pixels, false);
-        ta.pass.draws = c->tdraws.p;
+        ta.pass.draws = reinterpret_cast<const dh::DevDraw*>(c->tables.p + td_off);
         ta.pass.tables_src = nullptr;  // copied by the opaque pass
         ta.pass.n_draws = (uint32_t)c->h_tdraws.size();
         ta.pass.status = c->status.p + 1;
         ta.pass.ordered_bins = true;  // blending needs every tile list in submission order
         ta.pass.depth_order = false;
+        ta.pass.blend_lists = true;
         dh::enqueue_transparent_prep(oa, ta, c->stream);
         const dh::PipeArgs tb = dh::enqueue_front(ta.pass, c->stream);
         dh::enqueue_blend(tb, ta, c->stream);
@@ -1325,7 +1336,7 @@ void ctx_release_scratch(dh_ctx c) {
   c->hist.release(); c->partials.release(); c->ranges.release(); c->vis.release();
   c->tile_cnt.release(); c->tile_start.release();
   c->status.release(); c->tables.release(); c->draws = nullptr; c->views = nullptr; c->export_buf.release();
-  c->tdraws.release(); c->grp.release(); c->tperm.release(); c->sort_n.release();
+  c->grp.release(); c->tperm.release(); c->sort_n.release();
   release_gui(c);
   c->cap_tri = c->cap_pairs = 0;
 }

@@ -1812,6 +1812,19 @@ constexpr uint32_t kPairFewTiles = 256u * (kPairCounters / 16u);
 constexpr uint32_t kPairMaxTiles = 2048u * kPairCounters;
 static_assert(2048u * (kPairCols + 1u) <= kRadixHistEntries, "histogram and digit totals");
 
+// SUBMIT lists hold each tile's triangles in submission order, which the
+// transparent pass blends in: the depth key gives way to the high bits of the
+// id, and k_pair_sort places the few ids that share them by counting.  For at
+// most kPairSubmitTris input triangles: a tile's ids that share a key number
+// at most 1/256 of the frame's triangles (with 256 levels), so counting stays
+// far below the tile's blending.  (A transparent pass of 19,600 triangles on
+// 3600 tiles took 13 launches from its emits to the blend by a stable sort of
+// tile keys.)
+constexpr uint32_t kPairSubmitTris = 65536;
+__device__ inline uint32_t submit_shift(uint32_t n) {  // (n - 1) >> shift <= 255
+  return n > 256u ? 24u - (uint32_t)__builtin_clz(n - 1u) : 0u;
+}
+
 // Visits the pairs of one chunk: f(tile key, triangle, depth key).
 template <class F>
 __device__ inline void pair_chunk(const uint8_t* __restrict__ dkey, const uint32_t* __restrict__ wide_list,
@@ -1944,7 +1957,7 @@ __device__ inline uint32_t lds_exclusive_scan(uint32_t* s, uint32_t n, uint32_t*
 // Held to 64 VGPRs (a dozen spilled words, in the rows of large triangles), so
 // that a wide block and another share a CU: 20 -> 18 us on the 1M-triangle
 // soup; k_pair_hist, without the scatter's waits, lost more to the spills.
-template <int DIG>
+template <int DIG, bool SUBMIT>
 __global__ __launch_bounds__(kPairT) __attribute__((amdgpu_waves_per_eu(8))) void k_pair_scatter(const uint8_t* __restrict__ dkey,
                                                          const uint32_t* __restrict__ wide_list,
                                                          const SetupRec* __restrict__ setup,
@@ -1966,8 +1979,10 @@ __global__ __launch_bounds__(kPairT) __attribute__((amdgpu_waves_per_eu(8))) voi
   }
   for (int d = threadIdx.x; d < DIG; d += kPairT) cur[d] += hist[(uint32_t)d * kPairCols + col];
   __syncthreads();
+  const uint32_t sh = submit_shift(min(status->n_out, cap_tri));
   pair_chunk(dkey, wide_list, setup, views, status, cap_tri, TS, s_rows,
              [&](uint32_t key, uint32_t i, uint32_t dk) {
+               if (SUBMIT) dk = i >> sh;
                const uint32_t pos = atomicAdd(&cur[key & (DIG - 1u)], 1u);
                if (pos < cap_pairs) pairs[pos] = make_uint2((key >> kShift) << 8 | dk, i);
              });
@@ -1977,12 +1992,14 @@ __global__ __launch_bounds__(kPairT) __attribute__((amdgpu_waves_per_eu(8))) voi
 // them.  Counters per (tile, depth level): the depth keys between the
 // segment's smallest and largest, 2^s to a level, with s as small as the
 // counters allow.  Pairs past cap_pairs (flagged by the scatter) are left out.
+// SUBMIT: vals is a scratch array, and each id goes to out at its rank among
+// the ids of its counter.
 constexpr int kSortT = 512, kSortU = 8;
-template <int DIG>
+template <int DIG, bool SUBMIT>
 __global__ __launch_bounds__(kSortT) void k_pair_sort(const uint2* __restrict__ pairs,
                                                       const uint32_t* __restrict__ totals, uint32_t cap_pairs,
-                                                      uint32_t n_tiles, uint32_t* __restrict__ vals,
-                                                      uint2* __restrict__ ranges) {
+                                                      uint32_t n_tiles, uint32_t* vals, uint2* __restrict__ ranges,
+                                                      uint32_t* __restrict__ out) {
   __shared__ uint32_t cnt[kPairCounters];
   __shared__ uint32_t s_w[kSortT / 64];
   __shared__ uint32_t s_mn, s_mx, s_base;
@@ -2060,10 +2077,24 @@ __global__ __launch_bounds__(kSortT) void k_pair_sort(const uint2* __restrict__ 
     for (int u = 0; u < kSortU; u++)
       if (t0 + (uint32_t)(kSortT * u) + tid < n) vals[base + atomicAdd(&cnt[slot(it[u].x)], 1u)] = it[u].y;
   }
+  if constexpr (SUBMIT) {
+    __syncthreads();  // a counter now holds its ids' end, which is the next one's start
+    for (uint32_t t0 = 0; t0 < n; t0 += kRound) {
+      if (!once) load(t0);
+#pragma unroll
+      for (int u = 0; u < kSortU; u++) {
+        if (t0 + (uint32_t)(kSortT * u) + tid >= n) continue;
+        const uint32_t k = slot(it[u].x), lo = k ? cnt[k - 1u] : 0u, hi = cnt[k];
+        uint32_t r = lo;
+        for (uint32_t j = lo; j < hi; j++) r += vals[base + j] < it[u].y ? 1u : 0u;
+        out[base + r] = it[u].y;
+      }
+    }
+  }
 }
 
-// A pass's first kernel: its Status words cleared and (opaque pass) the
-// draw/view tables copied in from pinned host memory.
+// A frame's first kernel: the Status words of its passes cleared and the
+// draw, view and group tables copied in from pinned host memory.
 __global__ __launch_bounds__(256) void k_frame_begin(uint32_t* __restrict__ status, uint32_t status_words,
                                                      const uint32_t* __restrict__ src, uint32_t* __restrict__ dst,
                                                      uint32_t n_words) {
@@ -2097,24 +2128,107 @@ __global__ __launch_bounds__(256) void k_group_base(const uint32_t* __restrict__
   if ((threadIdx.x & 63u) == 0u) grp_base[g] = id;
 }
 
-// Sort keys of a transparent mesh's triangles (scene/mod.rs:1100-1115): the
+// Sort key of a transparent mesh's triangle (scene/mod.rs:1100-1115): the
 // distance from the camera to the centroid (a + b + c) / 3, ordered by
 // f32::total_cmp reversed.  key = ~(order-preserving bits of the distance),
 // so an ascending stable sort gives the descending total order with ties in
 // the current triangle order.
+__device__ inline uint32_t tsort_key(const uint32_t* __restrict__ t9, const float* __restrict__ pos, V3 cam) {
+  const V3 a = ld3(pos, t9[0]), b = ld3(pos, t9[1]), c = ld3(pos, t9[2]);
+  const V3 ctr = divs(add(add(a, b), c), 3.0f);
+  const float d = norm(sub(ctr, cam));  // Vec3::dist, linalg.rs:177-180
+  const uint32_t u = __float_as_uint(d);
+  const uint32_t k = (u & 0x80000000u) ? ~u : (u | 0x80000000u);  // total order as unsigned
+  return ~k;
+}
+
 __global__ __launch_bounds__(256) void k_tsort_keys(const uint32_t* __restrict__ tri, uint32_t n,
                                                     const float* __restrict__ pos, float cx, float cy, float cz,
                                                     uint32_t* __restrict__ keys, uint32_t* __restrict__ vals) {
   const uint32_t i = blockIdx.x * 256u + threadIdx.x;
   if (i >= n) return;
-  const uint32_t* t9 = tri + 9ull * i;
-  const V3 a = ld3(pos, t9[0]), b = ld3(pos, t9[1]), c = ld3(pos, t9[2]);
-  const V3 ctr = divs(add(add(a, b), c), 3.0f);
-  const float d = norm(sub(ctr, v3(cx, cy, cz)));  // Vec3::dist, linalg.rs:177-180
-  const uint32_t u = __float_as_uint(d);
-  const uint32_t k = (u & 0x80000000u) ? ~u : (u | 0x80000000u);  // total order as unsigned
-  keys[i] = ~k;
+  keys[i] = tsort_key(tri + 9ull * i, pos, v3(cx, cy, cz));
   vals[i] = i;
+}
+
+// The sort of transparent meshes of at most kTsortMax triangles, up to
+// kTsortMeshes of them at once, in two launches:
+//  k_tsort_chunks  a block per kTsortChunk triangles sorts their (key, index)
+//                  words, all different, in registers and LDS, and copies the
+//                  triangles out of the mesh;
+//  k_tsort_merge   sixteen lanes per triangle add up its ranks in the mesh's
+//                  chunks by binary searches and write it to its place.
+// A radix sort took 18 launches a mesh, each about as long as starting it; it
+// stays for larger meshes, whose searches (a sixteenth of n / 1024 chunks a
+// lane) would outgrow it.
+constexpr uint32_t kTsortChunk = 1024, kTsortMax = 32768, kTsortMeshes = 16;
+struct TsortBatch {
+  TransMesh m[kTsortMeshes];
+  uint32_t first[kTsortMeshes + 1];  // each mesh's first chunk
+  uint32_t n;
+  float cam[3];
+};
+__device__ inline uint32_t tsort_mesh(const TsortBatch& b, uint32_t chunk) {
+  uint32_t m = 0;
+  while (m + 1u < b.n && b.first[m + 1u] <= chunk) m++;
+  return m;
+}
+
+__global__ __launch_bounds__(kTsortChunk) void k_tsort_chunks(TsortBatch b, unsigned long long* __restrict__ words,
+                                                              uint32_t* __restrict__ tmp) {
+  __shared__ unsigned long long s_x[2][kTsortChunk];
+  const uint32_t tid = threadIdx.x, m = tsort_mesh(b, blockIdx.x);
+  const TransMesh tm = b.m[m];
+  const uint32_t i0 = (blockIdx.x - b.first[m]) * kTsortChunk, n = min(kTsortChunk, tm.n_tri - i0);
+  const uint32_t* src = tm.tri + 9ull * i0;
+  uint32_t* dst = tmp + 9ull * kTsortChunk * blockIdx.x;
+  for (uint32_t w = tid; w < 9u * n; w += kTsortChunk) dst[w] = src[w];
+  unsigned long long v = ~0ull;  // after every real word
+  if (tid < n)
+    v = (unsigned long long)tsort_key(src + 9u * tid, tm.pos, v3(b.cam[0], b.cam[1], b.cam[2])) << 32 | (i0 + tid);
+  int buf = 0;
+  for (uint32_t k = 2; k <= kTsortChunk; k <<= 1) {  // bitonic
+    for (uint32_t j = k >> 1; j; j >>= 1) {
+      unsigned long long o;
+      if (j < 64u) {
+        o = __shfl_xor(v, (int)j, 64);
+      } else {
+        s_x[buf][tid] = v;
+        __syncthreads();
+        o = s_x[buf][tid ^ j];
+        buf ^= 1;  // the next exchange writes while slower waves still read this one
+      }
+      const bool low = ((tid & j) == 0u) == ((tid & k) == 0u);
+      v = (o < v) == low ? o : v;
+    }
+  }
+  words[(uint64_t)kTsortChunk * blockIdx.x + tid] = v;
+}
+
+__global__ __launch_bounds__(256) void k_tsort_merge(TsortBatch b, const unsigned long long* __restrict__ words,
+                                                     const uint32_t* __restrict__ tmp) {
+  const uint32_t e = (blockIdx.x * 256u + threadIdx.x) >> 4, l = threadIdx.x & 15u;
+  const uint32_t chunk = e / kTsortChunk, m = tsort_mesh(b, chunk);
+  const unsigned long long v = words[e];
+  uint32_t rank = 0;
+  if (v != ~0ull) {
+    for (uint32_t c = b.first[m] + l; c < b.first[m + 1u]; c += 16u) {
+      if (c == chunk) {
+        rank += e % kTsortChunk;
+        continue;
+      }
+      const unsigned long long* w = words + (uint64_t)kTsortChunk * c;
+      uint32_t p = 0;  // words of the chunk below v
+#pragma unroll
+      for (uint32_t s = kTsortChunk / 2u; s; s >>= 1)
+        if (w[p + s - 1u] < v) p += s;
+      rank += p + (w[p] < v ? 1u : 0u);
+    }
+  }
+#pragma unroll
+  for (int o = 8; o; o >>= 1) rank += __shfl_xor(rank, o, 16);
+  if (v != ~0ull && l < 9u)
+    b.m[m].tri[9ull * rank + l] = tmp[9ull * ((uint64_t)kTsortChunk * b.first[m] + (uint32_t)v) + l];
 }
 
 // out[i] = tri[order[i]] (9 indices per triangle).
@@ -2190,14 +2304,16 @@ int enqueue_radix_sort(uint32_t* const keys[2], uint32_t* const vals[2], const u
 PipeArgs enqueue_front(const PipeArgs& a, hipStream_t s) {
   // near-first lists (k_pair_*); a frame of more tiles than their counters
   // take is binned in submission order
-  const bool near = a.ordered_bins && a.depth_order && a.n_tiles <= kPairMaxTiles;
+  const bool submit = a.ordered_bins && a.blend_lists && a.n_tri_in <= kPairSubmitTris && a.n_tiles <= kPairMaxTiles;
+  const bool near = (a.ordered_bins && a.depth_order && a.n_tiles <= kPairMaxTiles) || submit;
   // a small single-view frame is binned by one workgroup (k_bin_small)
-  const bool small_bins = near && a.n_views == 1 && a.n_tiles <= kSmallBinTiles &&
+  const bool small_bins = near && !submit && a.n_views == 1 && a.n_tiles <= kSmallBinTiles &&
                           a.n_tri_in <= kSmallBinTris;
   if (a.ev[0]) (void)hipEventRecord(a.ev[0], s);
-  hipLaunchKernelGGL(k_frame_begin, dim3(a.tables_src ? std::min<uint32_t>(cdiv(a.tables_words, 1024), 64u) : 1u),
-                     dim3(256), 0, s, reinterpret_cast<uint32_t*>(a.status), (uint32_t)(sizeof(Status) / 4),
-                     a.tables_src, a.tables_dst, a.tables_src ? a.tables_words : 0u);
+  if (a.tables_src)  // (the transparent pass's were the opaque pass's work)
+    hipLaunchKernelGGL(k_frame_begin, dim3(std::min<uint32_t>(cdiv(a.tables_words, 1024), 64u)), dim3(256), 0, s,
+                       reinterpret_cast<uint32_t*>(a.status), (uint32_t)(2 * sizeof(Status) / 4), a.tables_src,
+                       a.tables_dst, a.tables_words);
   const uint32_t n_blk = cdiv(a.n_tri_in, 256);
   uint8_t* const wflag = reinterpret_cast<uint8_t*>(a.big);
   // the wide-triangle list: near first in vals[1], which the pair kernels
@@ -2262,16 +2378,19 @@ PipeArgs enqueue_front(const PipeArgs& a, hipStream_t s) {
       hipLaunchKernelGGL(k_pair_hist<2048>, gp, bp, 0, s, wflag, wide_list, a.setup, a.views, a.status, a.cap_tri,
                          a.TS, a.hist);
     hipLaunchKernelGGL(k_row_scan, dim3(dig), dim3(kPairCols), 0, s, a.hist, totals);
-    if (few) {
-      hipLaunchKernelGGL(k_pair_scatter<256>, gp, bp, 0, s, wflag, wide_list, a.setup, a.views, a.status, a.cap_tri,
-                         a.TS, a.hist, totals, a.cap_pairs, pairs);
-      hipLaunchKernelGGL(k_pair_sort<256>, dim3(dig), dim3(kSortT), 0, s, pairs, totals, a.cap_pairs, a.n_tiles,
-                         a.vals[0], a.ranges);
+    auto lists = [&](auto scatter, auto sort) {
+      hipLaunchKernelGGL(scatter, gp, bp, 0, s, wflag, wide_list, a.setup, a.views, a.status, a.cap_tri, a.TS, a.hist,
+                         totals, a.cap_pairs, pairs);
+      hipLaunchKernelGGL(sort, dim3(dig), dim3(kSortT), 0, s, pairs, totals, a.cap_pairs, a.n_tiles, a.vals[0],
+                         a.ranges, a.vals[1]);  // (the wide list there has been read)
+    };
+    if (submit) {
+      if (few) lists(k_pair_scatter<256, true>, k_pair_sort<256, true>);
+      else lists(k_pair_scatter<2048, true>, k_pair_sort<2048, true>);
+      b.vals[0] = a.vals[1];
     } else {
-      hipLaunchKernelGGL(k_pair_scatter<2048>, gp, bp, 0, s, wflag, wide_list, a.setup, a.views, a.status, a.cap_tri,
-                         a.TS, a.hist, totals, a.cap_pairs, pairs);
-      hipLaunchKernelGGL(k_pair_sort<2048>, dim3(dig), dim3(kSortT), 0, s, pairs, totals, a.cap_pairs, a.n_tiles,
-                         a.vals[0], a.ranges);
+      if (few) lists(k_pair_scatter<256, false>, k_pair_sort<256, false>);
+      else lists(k_pair_scatter<2048, false>, k_pair_sort<2048, false>);
     }
   } else if (a.ordered_bins) {
     hipLaunchKernelGGL(k_wide_list, dim3(gl), dim3(256), 0, s, wflag, a.status, a.cap_tri, wide_list,
@@ -2323,9 +2442,34 @@ void enqueue_transparent_prep(const PipeArgs& opaque, const TransArgs& t, hipStr
   if (t.n_groups)
     hipLaunchKernelGGL(k_group_base, dim3(cdiv(t.n_groups, 4)), dim3(256), 0, s, t.grp_first, t.n_groups,
                        opaque.n_tri_in, opaque.cnt, opaque.blk, opaque.status, t.grp_base);
+  // a batch's triangles fit perm_tmp, their words the pair buffer (a mesh alone always does)
+  const uint32_t max_chunks = std::min(t.perm_chunks, opaque.cap_pairs / kTsortChunk);
+  TsortBatch b{};
+  for (int k = 0; k < 3; k++) b.cam[k] = t.cam[k];
+  auto sort_batch = [&]() {
+    const uint32_t chunks = b.first[b.n];
+    if (chunks) {
+      unsigned long long* const words = reinterpret_cast<unsigned long long*>(opaque.keys[0]);
+      hipLaunchKernelGGL(k_tsort_chunks, dim3(chunks), dim3(kTsortChunk), 0, s, b, words, t.perm_tmp);
+      hipLaunchKernelGGL(k_tsort_merge, dim3(chunks * (kTsortChunk / 16u)), dim3(256), 0, s, b, words, t.perm_tmp);
+    }
+    b.n = 0;
+  };
   for (uint32_t m = 0; m < t.n_meshes; m++) {
     const TransMesh& tm = t.meshes[m];
     if (tm.n_tri < 2) continue;
+    if (tm.n_tri <= kTsortMax) {
+      const uint32_t chunks = cdiv(tm.n_tri, kTsortChunk);
+      bool seen = false;  // drawn twice: sorted once
+      for (uint32_t k = 0; k < b.n; k++) seen |= b.m[k].tri == tm.tri;
+      if (seen) continue;
+      if (b.n == kTsortMeshes || (b.n && b.first[b.n] + chunks > max_chunks)) sort_batch();
+      b.m[b.n] = tm;
+      b.first[b.n + 1u] = b.first[b.n] + chunks;
+      b.n++;
+      continue;
+    }
+    sort_batch();
     hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(64), 0, s, t.sort_n, tm.n_tri, 1u);
     hipLaunchKernelGGL(k_tsort_keys, dim3(cdiv(tm.n_tri, 256)), dim3(256), 0, s, tm.tri, tm.n_tri, tm.pos,
                        t.cam[0], t.cam[1], t.cam[2], opaque.keys[0], opaque.vals[0]);
@@ -2335,6 +2479,7 @@ void enqueue_transparent_prep(const PipeArgs& opaque, const TransArgs& t, hipStr
                        tm.n_tri, t.perm_tmp);
     (void)hipMemcpyAsync(tm.tri, t.perm_tmp, 36ull * tm.n_tri, hipMemcpyDeviceToDevice, s);
   }
+  sort_batch();
 }
 
 // The frame's status words into coherent pinned host memory (one wave, in

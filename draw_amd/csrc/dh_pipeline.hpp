@@ -40,6 +40,7 @@ struct PipeArgs {
   bool ordered_bins;   // stable radix sort (per-tile lists in submission order)
   bool shade_in_raster;  // kind 0 rasters shade their own tiles (no visibility buffer, no k_shade)
   bool depth_order;    // ordered bins: per-tile lists near first (k_pair_*)
+  bool blend_lists;    // ordered bins of a transparent pass: lists in submission order by k_pair_* where they fit
   uint32_t* tile_cnt;  // [2 * n_tiles] per-tile counts, then per-tile cursors
   uint32_t* tile_cur;  // = tile_cnt + n_tiles
   uint32_t* tile_start;  // [n_tiles] exclusive scan of tile_cnt
@@ -54,7 +55,8 @@ struct PipeArgs {
   uint32_t pack_tag;   // shard << kShardShift
   Status* status;
   // the frame's draw/view tables, copied by the frame's first kernel from
-  // coherent pinned host memory (tables_src: its device address; null: none)
+  // coherent pinned host memory (tables_src: its device address; null: the
+  // frame's earlier pass did that, and cleared this pass's status)
   const uint32_t* tables_src;
   uint32_t* tables_dst;
   uint32_t tables_words;
@@ -74,7 +76,8 @@ struct TransArgs {
   uint32_t n_meshes;
   float cam[3];
   uint32_t* sort_n;            // [1] device scratch: item count of a sort
-  uint32_t* perm_tmp;          // [9 * max transparent mesh triangles]
+  uint32_t* perm_tmp;          // [9 * 1024 * perm_chunks]: the triangles being sorted
+  uint32_t perm_chunks;        // at least those of the largest mesh
   const uint32_t* grp_first;   // [n_groups] first opaque input triangle of each object group
   uint32_t* grp_base;          // [n_groups] -> first opaque clipped-triangle id of each group
   uint32_t n_groups;

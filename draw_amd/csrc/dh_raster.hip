@@ -1021,6 +1021,12 @@ __device__ inline uint32_t blend_px(uint32_t bg, uint32_t c, float a) {
 // is not before the winner's (transparent meshes are drawn after their own
 // object's opaque meshes, scene/mod.rs:1088) and its depth is < D.  Lanes own
 // pixels and apply the tile's transparent triangles in submission order.
+// Each wave owns 8x8 quadrants of the tile: its lanes test 64 staged records'
+// scan rectangles against the quadrant at once, the wave visits those that meet
+// it for their coverage alone, and each lane then shades the records of its own
+// pixel, all lanes together.  Shading is a chain of some 2 us from the records
+// to the texel: a visit of every record of the tile's list used to cost it,
+// now only as many rounds as a pixel has layers do.
 template <int TS>
 __global__ __launch_bounds__(256) void k_blend(const DevView* __restrict__ views, const uint2* __restrict__ ranges,
                                                const uint32_t* __restrict__ vals, const SetupRec* __restrict__ setup,
@@ -1028,32 +1034,35 @@ __global__ __launch_bounds__(256) void k_blend(const DevView* __restrict__ views
                                                const DevMaterial* __restrict__ mats,
                                                const uint32_t* __restrict__ grp_base, uint32_t n_groups,
                                                Status* __restrict__ status) {
-  constexpr int PPT = (TS * TS + 255) / 256;
+  constexpr int QS = TS / 8, NQ = QS * QS, QPW = (NQ + 3) / 4;  // quadrants per wave: wave, wave + 4, ...
   constexpr int CH = 64;
-  __shared__ SetupRec s_rec[CH];
-  __shared__ uint32_t s_id[CH];
+  __shared__ uint4 s_rec[CH][15];  // the setup record's 6 words, the shading record's 9
   __shared__ float s_unit[256];
   const uint32_t tile = xcd_remap(blockIdx.x, gridDim.x);
+  const uint2 rg = ranges[tile];
+  if (rg.x >= rg.y) return;  // nothing to blend (the whole block)
   const DevView& vw = views[0];
   const int W = vw.fr.W, H = vw.fr.H;
   const int tx0 = (int)(tile % vw.ntx) * TS, ty0 = (int)(tile / vw.ntx) * TS;
-  const int tid = threadIdx.x;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   fill_unit_table(s_unit, tid, 256);  // read after the chunk loop's first barrier
-  uint32_t col[PPT];
-  float D[PPT];
-  int gw[PPT];
-  bool ok[PPT];
+  uint32_t col[QPW];
+  float D[QPW];
+  int gw[QPW];
+  bool ok[QPW], drawn[QPW];
 #pragma unroll
-  for (int q = 0; q < PPT; q++) {
-    const int p = tid + 256 * q;
-    const int px = tx0 + p % TS, py = ty0 + p / TS;
-    ok[q] = p < TS * TS && px < W && py < H;
-    col[q] = 0;
-    D[q] = 0.0f;
-    gw[q] = -1;
-    if (ok[q]) {
-      col[q] = vw.out_bgra[(uint32_t)(H - 1 - py) * (uint32_t)W + (uint32_t)px];
-      D[q] = vw.out_depth[(uint32_t)py * (uint32_t)W + (uint32_t)px];
+  for (int j = 0; j < QPW; j++) {
+    const int Q = wave + 4 * j;
+    const int px = tx0 + (Q % QS) * 8 + (lane & 7), py = ty0 + (Q / QS) * 8 + (lane >> 3);
+    ok[j] = Q < NQ && px < W && py < H;
+    drawn[j] = false;
+    col[j] = 0;
+    D[j] = 0.0f;
+    gw[j] = -1;
+    if (ok[j]) {
+      col[j] = vw.out_bgra[(uint32_t)(H - 1 - py) * (uint32_t)W + (uint32_t)px];
+      D[j] = vw.out_depth[(uint32_t)py * (uint32_t)W + (uint32_t)px];
       const uint32_t w = vw.out_winner[(uint32_t)py * (uint32_t)W + (uint32_t)px];
       if (w != kNone) {  // last group whose first id is <= w
         uint32_t lo = 0, hi = n_groups;
@@ -1062,58 +1071,78 @@ __global__ __launch_bounds__(256) void k_blend(const DevView* __restrict__ views
           if (grp_base[mid] <= w) lo = mid;
           else hi = mid;
         }
-        gw[q] = (int)lo;
+        gw[j] = (int)lo;
       }
     }
   }
-  const uint2 rg = ranges[tile];
   for (uint32_t base = rg.x; base < rg.y; base += CH) {
     const int n = (int)min((uint32_t)CH, rg.y - base);
     __syncthreads();
-    for (int i = tid; i < n * 6; i += 256) {
-      const int k = i / 6, w = i % 6;
+    for (int i = tid; i < n * 15; i += 256) {
+      const int k = i / 15, w = i - 15 * k;
       const uint32_t id = vals[base + k];
-      if (w == 0) s_id[k] = id;
-      reinterpret_cast<uint4*>(s_rec + k)[w] = reinterpret_cast<const uint4*>(setup + id)[w];
+      s_rec[k][w] = w < 6 ? reinterpret_cast<const uint4*>(setup + id)[w]
+                          : reinterpret_cast<const uint4*>(shade + id)[w - 6];
     }
     __syncthreads();
-    for (int k = 0; k < n; k++) {
-      const SetupRec& r = s_rec[k];
-      if (r.flags & kDrop) continue;
-      const int rx0 = (int)(r.rx & 0xFFFFu), rx1 = (int)(r.rx >> 16);
-      const int ry0 = (int)(r.ry & 0xFFFFu), ry1 = (int)(r.ry >> 16);
+    // the lane's record: its scan rectangle, empty when there is none to visit
+    int rx0 = 1, rx1 = 0, ry0 = 1, ry1 = 0;
+    if (lane < n) {
+      const uint4 h = s_rec[lane][5];
+      if (!(h.z & kDrop)) {
+        rx0 = (int)(h.x & 0xFFFFu);
+        rx1 = (int)(h.x >> 16);
+        ry0 = (int)(h.y & 0xFFFFu);
+        ry1 = (int)(h.y >> 16);
+      }
+    }
 #pragma unroll
-      for (int q = 0; q < PPT; q++) {
-        const int p = tid + 256 * q;
-        const int px = tx0 + p % TS, py = ty0 + p / TS;
-        if (!ok[q] || px < rx0 || px > rx1 || py < ry0 || py > ry1) continue;
-        const float xf = (float)px, yf = (float)py;
+    for (int j = 0; j < QPW; j++) {
+      const int Q = wave + 4 * j;
+      if (Q >= NQ) break;
+      const int qx = tx0 + (Q % QS) * 8, qy = ty0 + (Q / QS) * 8;
+      const int px = qx + (lane & 7), py = qy + (lane >> 3);
+      const float xf = (float)px, yf = (float)py;
+      uint64_t hits = __ballot(rx0 <= rx1 && ry0 <= ry1 && rx0 <= qx + 7 && rx1 >= qx && ry0 <= qy + 7 && ry1 >= qy);
+      // the records that cover the lane's pixel, then their shading in order
+      uint64_t mine = 0;
+      for (; hits; hits &= hits - 1) {
+        const int k = (int)__builtin_ctzll(hits);
+        const SetupRec& r = *reinterpret_cast<const SetupRec*>(s_rec[k]);
+        const int x0 = __builtin_amdgcn_readlane(rx0, k), x1 = __builtin_amdgcn_readlane(rx1, k);
+        const int y0 = __builtin_amdgcn_readlane(ry0, k), y1 = __builtin_amdgcn_readlane(ry1, k);
+        if (!ok[j] || px < x0 || px > x1 || py < y0 || py > y1) continue;
         bool cov;
-        FragOut o;
         if (r.flags & kFast) {
           cov = covered_fast(edge_eval(r.ea, xf, yf), r.f[0], r.flags & kTieA) &&
                 covered_fast(edge_eval(r.eb, xf, yf), r.f[1], r.flags & kTieB) &&
                 covered_fast(edge_eval(r.eg, xf, yf), r.f[2], r.flags & kTieG);
-          if (cov) o = bary(r, xf, yf);
         } else {
-          o = bary(r, xf, yf);
+          const FragOut o = bary(r, xf, yf);
           cov = o.al >= 0.0f && o.be >= 0.0f && o.ga >= 0.0f && (o.al > 0.0f || (r.flags & kTieA)) &&
                 (o.be > 0.0f || (r.flags & kTieB)) && (o.ga > 0.0f || (r.flags & kTieG));
         }
-        if (!cov) continue;
+        if (cov) mine |= 1ull << k;
+      }
+      for (; mine; mine &= mine - 1) {
+        const int k = (int)__builtin_ctzll(mine);
+        const FragOut o = bary(*reinterpret_cast<const SetupRec*>(s_rec[k]), xf, yf);
         // both maps are sampled before the depth test (canvas.rs:689-695)
-        const ShadeRec& sr = shade[s_id[k]];
+        const ShadeRec& sr = *reinterpret_cast<const ShadeRec*>(s_rec[k] + 6);
         const DevMaterial& m = mats[sr.material];
         const uint32_t c = shade_pixel(sr, m, o, status, s_unit);
-        if (o.d < D[q] && (int)sr.group >= gw[q]) col[q] = blend_px(col[q], c, m.alpha);
+        if (o.d < D[j] && (int)sr.group >= gw[j]) {
+          col[j] = blend_px(col[j], c, m.alpha);
+          drawn[j] = true;
+        }
       }
     }
   }
 #pragma unroll
-  for (int q = 0; q < PPT; q++) {
-    const int p = tid + 256 * q;
-    const int px = tx0 + p % TS, py = ty0 + p / TS;
-    if (ok[q]) vw.out_bgra[(uint32_t)(H - 1 - py) * (uint32_t)W + (uint32_t)px] = col[q];
+  for (int j = 0; j < QPW; j++) {
+    const int Q = wave + 4 * j;
+    const int px = tx0 + (Q % QS) * 8 + (lane & 7), py = ty0 + (Q / QS) * 8 + (lane >> 3);
+    if (drawn[j]) vw.out_bgra[(uint32_t)(H - 1 - py) * (uint32_t)W + (uint32_t)px] = col[j];
   }
 }
 
