@@ -566,8 +566,7 @@ __device__ inline void wave_store(uint4* stage, const uint4 (&v)[N], bool ok, ui
 // |e - (Ax+By+C-D)| <= 4.01 u S, S = |A|x + |B|y + |C| + |D|; a pixel can only
 // be covered when sign(f) * e >= 0 on all three edges.  Each edge's
 // exact-arithmetic function, widened by that bound (plus 1), therefore gives
-// a superset of the tiles holding covered pixels: per tile for triangles of a
-// few tiles (tile_may_cover), per tile row for wide ones (spans_row).  Other
+// a superset of the tiles holding covered pixels (tile_may_cover).  Other
 // triangles, and those within one tile, are binned to every tile of their
 // scan rectangle.
 struct Spans {
@@ -575,13 +574,6 @@ struct Spans {
   bool exact;
   float fa[3], fb[3], fk[3], fm[3];  // per-tile corner test (tile_may_cover)
 };
-// Per-row spans of a wide triangle (spans_row).
-struct SpanRows {
-  int cx0, cx1;
-  bool exact;
-  double a[3], b[3], k[3], m[3];
-};
-
 // Bounds and the per-tile test's constants.  The test evaluates
 // G_f = fl(fl(fl(a xc) + fl(b yc)) + fl(s (C - D))) at the tile corner
 // (xc, yc) maximising the edge's exact function G = a x + b y + s (C - D).
@@ -614,59 +606,6 @@ __device__ inline void spans_init(const SetupRec& r, int TS, Spans& g) {
   }
 }
 
-// The per-row constants of a wide triangle with tile box c, in double.
-__device__ inline void spans_init_rows(const SetupRec& r, const Spans& c, SpanRows& g) {
-  g.cx0 = c.cx0;
-  g.cx1 = c.cx1;
-  g.exact = c.exact;
-  if (!g.exact) return;
-  const uint32_t x1 = r.rx >> 16, y1 = r.ry >> 16;
-  const float* es[3] = {r.ea, r.eb, r.eg};
-#pragma unroll
-  for (int i = 0; i < 3; i++) {
-    const double A = es[i][0], B = es[i][1], C = es[i][2], D = es[i][3];
-    const double s = r.f[i] > 0.0f ? 1.0 : -1.0;
-    const double S = fabs(A) * (double)x1 + fabs(B) * (double)y1 + fabs(C) + fabs(D);
-    g.a[i] = s * A;
-    g.b[i] = s * B;
-    g.k[i] = s * (C - D);
-    g.m[i] = 4.02 * 5.9604644775390625e-08 * S + 1.0 + 1e-9 * S;
-    if (!isfinite(S)) g.exact = false;
-  }
-}
-
-// Columns [lo, hi] of tile row ty that may hold covered pixels (lo > hi: none).
-__device__ inline void spans_row(const SpanRows& g, int TS, int ty, int* lo, int* hi) {
-  int l = g.cx0, h = g.cx1;
-  if (g.exact) {
-    const double ya = (double)(ty * TS), yb = (double)(ty * TS + TS - 1);
-#pragma unroll
-    for (int i = 0; i < 3; i++) {
-      const double K = g.k[i] + fmax(g.b[i] * ya, g.b[i] * yb);
-      const double a = g.a[i];
-      if (a > 0.0) {
-        // need a*(c*TS + TS-1) + K >= -m
-        double xl = (-g.m[i] - K) / a - 1.0;
-        double c = (xl - (double)(TS - 1)) / (double)TS;
-        c = fmin(fmax(c, -1.0), 1.0e6);
-        const int ci = (int)ceil(c);
-        l = max(l, ci);
-      } else if (a < 0.0) {
-        // need a*(c*TS) + K >= -m
-        double xr = (K + g.m[i]) / (-a) + 1.0;
-        double c = xr / (double)TS;
-        c = fmin(fmax(c, -2.0), 1.0e6);
-        const int ci = (int)floor(c);
-        h = min(h, ci);
-      } else if (K < -g.m[i]) {
-        h = l - 1;
-      }
-    }
-  }
-  *lo = l;
-  *hi = h;
-}
-
 // Work split: a triangle whose tile range is more than kWideSpan tiles tall
 // or wide is binned by a whole wave (lanes over rows, then over entries); the
 // rest by one thread each (at most kWideSpan^2 entries).  The split only
@@ -679,18 +618,22 @@ __device__ inline bool bin_is_wide(const Spans& g) {
 
 __device__ inline uint64_t lanemask_lt_u64(int lane) { return lane == 0 ? 0ull : (~0ull >> (64 - lane)); }
 
-// Tile (tx, ty) may hold a covered pixel: every edge's function, widened by
-// fm (see spans_init), reaches 0 at the tile corner maximising it.
-__device__ inline bool tile_may_cover(const Spans& g, int TS, int tx, int ty) {
+// The tiles (tx0..tx1, ty0..ty1) of the box may hold a covered pixel: every
+// edge's function, widened by fm (see spans_init), reaches 0 at their corner
+// maximising it.
+__device__ inline bool tiles_may_cover(const Spans& g, int TS, int tx0, int tx1, int ty0, int ty1) {
   if (!g.exact) return true;
-  const float xa = (float)(tx * TS), xb = (float)(tx * TS + TS - 1);
-  const float ya = (float)(ty * TS), yb = (float)(ty * TS + TS - 1);
+  const float xa = (float)(tx0 * TS), xb = (float)(tx1 * TS + TS - 1);
+  const float ya = (float)(ty0 * TS), yb = (float)(ty1 * TS + TS - 1);
 #pragma unroll
   for (int i = 0; i < 3; i++) {
     const float v = (g.fa[i] * (g.fa[i] > 0.0f ? xb : xa) + g.fb[i] * (g.fb[i] > 0.0f ? yb : ya)) + g.fk[i];
     if (v < -g.fm[i]) return false;
   }
   return true;
+}
+__device__ inline bool tile_may_cover(const Spans& g, int TS, int tx, int ty) {
+  return tiles_may_cover(g, TS, tx, tx, ty, ty);
 }
 
 // Calls f(e, ty, tx) for every tile of a triangle that is not wide (at most
@@ -705,135 +648,142 @@ __device__ inline uint32_t thread_tiles(const Spans& g, int TS, F f) {
   return e;
 }
 
-// Wave version, for a wide triangle.  A box of at most kBoxTiles tiles: lanes
-// take its tiles and test each as the narrow triangles' are.  A larger one:
-// lanes take tile rows, a wave scan places each row's span (in double) and the
-// entries are spread over the lanes.  f(e, ty, tx) with e numbering the tiles;
-// returns the tile count (wave-uniform).  The rows cost some 250 instructions a
-// triangle, most of them double divisions, 64 tests about 30 (1M-triangle 1080p
-// soup: k_pair_hist 18.9 -> 13.4 us).
+// Wave version, for a wide triangle (uniform arguments).  A box of at most
+// kBoxTiles tiles: lanes take its tiles and test each as the narrow triangles'
+// are.  A larger one: lanes take its blocks of 8x8 tiles, and the tiles of a
+// block that may hold a covered pixel are tested at once.  f(e, tx, ty) with e
+// numbering the tiles; returns the tile count.  part, parts: a share of the box
+// (the waves of a block take one each), numbered within the share.
 constexpr int kBoxTiles = 256;
-struct WaveRows {  // a wave's LDS scratch
-  int lo[64];
-  uint32_t off[64];
-};
 template <class F>
-__device__ inline uint32_t wave_tiles(const SetupRec& r, const Spans& g, int TS, int lane, WaveRows& s, F f) {
+__device__ inline uint32_t wave_tiles(const Spans& g, int TS, int part, int parts, F f) {
+  const int lane = threadIdx.x & 63;
   uint32_t o = 0;
   const int nx = g.cx1 - g.cx0 + 1, n = nx * (g.cy1 - g.cy0 + 1);
-  if (n <= kBoxTiles) {
-    const float inv = 1.0f / (float)nx;
-    for (int t0 = 0; t0 < n; t0 += 64) {
-      const int t = t0 + lane;
-      const int dy = (int)(((float)t + 0.5f) * inv);  // t / nx: exact for t < 512
-      const int ty = g.cy0 + dy, tx = g.cx0 + (t - dy * nx);
-      const bool on = t < n && tile_may_cover(g, TS, tx, ty);
-      const uint64_t m = __ballot(on);
-      if (on) f(o + (uint32_t)__popcll(m & lanemask_lt_u64(lane)), ty, tx);
-      o += (uint32_t)__popcll(m);
+  auto tile = [&](bool on, int tx, int ty) {
+    on = on && tile_may_cover(g, TS, tx, ty);
+    const uint64_t m = __ballot(on);
+    if (on) f(o + (uint32_t)__popcll(m & lanemask_lt_u64(lane)), tx, ty);
+    o += (uint32_t)__popcll(m);
+  };
+  const bool large = n > kBoxTiles;
+  const int bx = large ? (nx + 7) >> 3 : nx, nb = large ? bx * ((g.cy1 - g.cy0 + 8) >> 3) : n;
+  const float inv = 1.0f / (float)bx;
+  for (int t0 = 64 * part; t0 < nb; t0 += 64 * parts) {
+    const int t = t0 + lane;
+    // t / bx: the quotient is off by at most one (t < 2^20), and exact for t < 512
+    int dy = (int)(((float)t + 0.5f) * inv);
+    if (large) {
+      dy -= dy * bx > t ? 1 : 0;
+      dy += (dy + 1) * bx <= t ? 1 : 0;
+      const int x0 = g.cx0 + 8 * (t - dy * bx), y0 = g.cy0 + 8 * dy;
+      const bool may = t < nb && tiles_may_cover(g, TS, x0, min(x0 + 7, g.cx1), y0, min(y0 + 7, g.cy1));
+      for (uint64_t m = __ballot(may); m; m &= m - 1) {
+        const int b = (int)__builtin_ctzll(m);
+        const int tx = __builtin_amdgcn_readlane(x0, b) + (lane & 7), ty = __builtin_amdgcn_readlane(y0, b) + (lane >> 3);
+        tile(tx <= g.cx1 && ty <= g.cy1, tx, ty);
+      }
+    } else {
+      tile(t < nb, g.cx0 + (t - dy * bx), g.cy0 + dy);
     }
-    return o;
-  }
-  SpanRows sr;
-  spans_init_rows(r, g, sr);
-  for (int row0 = g.cy0; row0 <= g.cy1; row0 += 64) {
-    const int ty = row0 + lane;
-    int lo = 0, hi = -1;
-    if (ty <= g.cy1) spans_row(sr, TS, ty, &lo, &hi);
-    const uint32_t c = hi >= lo ? (uint32_t)(hi - lo + 1) : 0u;
-    uint32_t x = c;
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-      const uint32_t y = (uint32_t)__shfl_up((int)x, d, 64);
-      if (lane >= d) x += y;
-    }
-    const uint32_t total = (uint32_t)__shfl((int)x, 63, 64);
-    s.lo[lane] = lo;
-    s.off[lane] = x - c;
-    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-    for (uint32_t e = (uint32_t)lane; e < total; e += 64) {
-      // the row of entry e: the last row whose offset is <= e (rows without
-      // entries share their successor's offset, so the last one has entries)
-      int k = 0;
-#pragma unroll
-      for (int step = 32; step >= 1; step >>= 1)
-        if (s.off[k + step] <= e) k += step;
-      f(o + e, row0 + k, s.lo[k] + (int)(e - s.off[k]));
-    }
-    o += total;
-    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
   }
   return o;
 }
 
-// The wide triangles list[w], list[w + step], ... (below n) of one wave:
-// f(tile key, triangle) for each of their tiles, lanes over a triangle's
+// The constants of a wide triangle's visit.
+struct WideTri {
+  Spans g;  // (without edge tests: exact, and every margin infinite)
+  uint32_t key0, ntx, id, dk;
+};
+__device__ inline WideTri wide_tri(uint32_t id, const SetupRec* __restrict__ setup, const DevView* __restrict__ views,
+                                   const uint8_t* __restrict__ dkey, int TS) {
+  WideTri w;
+  const SetupRec r = setup[id];
+  w.id = id;
+  w.dk = dkey ? dkey[id] : 0u;
+  spans_init(r, TS, w.g);
+  const DevView& vw = views[r.view];
+  w.ntx = vw.ntx;
+  w.key0 = vw.tile_base + (uint32_t)w.g.cy0 * vw.ntx + (uint32_t)w.g.cx0;
+#pragma unroll
+  for (int e = 0; e < 3; e++) {
+    if (!w.g.exact) w.g.fa[e] = w.g.fb[e] = w.g.fk[e] = 0.0f;
+    w.g.fm[e] = w.g.exact ? w.g.fm[e] : INFINITY;
+  }
+  w.g.exact = true;
+  return w;
+}
+
+// Triangles of larger boxes that the waves of a block share out.
+constexpr uint32_t kLargeBuf = 64;
+struct LargeBuf {
+  uint32_t n;
+  WideTri t[kLargeBuf];
+};
+
+// The wide triangles list[w], list[w + step], ... (below n) of one of a block's
+// NW waves: f(tile key, triangle, its byte of dkey if given) for each of their
 // tiles.  Each lane first fetches and prepares one of the wave's next 64
 // triangles, so that the chain of dependent loads (id, record, view) is paid
 // once for all of them and the visits take their constants from registers; a
 // wave per triangle paid some 2 us of latency for each (k_bin_small of a
-// 2312-triangle frame of 3600 tiles: 105 -> 38 us).  For the one workgroup of
-// k_bin_small only: the pair kernels have 4096 waves and few triangles for
-// each, and its 90 VGPRs would keep their wide and other blocks from sharing a
-// CU (k_pair_scatter of a frame with few wide triangles 6 -> 15 us).
-template <class F>
+// 2312-triangle frame of 3600 tiles: 105 -> 38 us).  Triangles of larger boxes
+// wait in the block's LDS until every wave is done with the others, and then
+// every wave takes a share of each: the entries of a screen-sized one alone
+// kept its wave for 20 us.  Every wave of the block calls it; large.n is 0
+// before, after a barrier.
+template <int NW, class F>
 __device__ inline void wave_wide_tiles(const uint32_t* __restrict__ list, uint32_t w, uint32_t step, uint32_t n,
                                        const SetupRec* __restrict__ setup, const DevView* __restrict__ views,
-                                       int TS, WaveRows& rows, F f) {
-  const int lane = threadIdx.x & 63;
-  for (uint64_t w0 = w; w0 < n; w0 += 64ull * step) {
-    const uint64_t at = w0 + (uint64_t)step * (uint32_t)lane;
-    const bool on = at < n;
-    uint32_t id = 0, key0 = 0, ntx = 0;
-    Spans g;
-    g.cx0 = g.cy0 = g.cx1 = g.cy1 = 0;
-    g.exact = false;
-#pragma unroll
-    for (int e = 0; e < 3; e++) g.fa[e] = g.fb[e] = g.fk[e] = g.fm[e] = 0.0f;
-    if (on) {
-      id = list[at];
-      const SetupRec r = setup[id];
-      spans_init(r, TS, g);
-      const DevView& vw = views[r.view];
-      ntx = vw.ntx;
-      key0 = vw.tile_base + (uint32_t)g.cy0 * ntx + (uint32_t)g.cx0;
+                                       const uint8_t* __restrict__ dkey, int TS, LargeBuf& large, F f) {
+  if (n == 0u) return;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  bool shared = false;  // visiting the block's large triangles
+  for (uint64_t w0 = w;; w0 += 64ull * step) {
+    WideTri q{};
+    bool on;
+    if (w0 < n) {
+      const uint64_t at = w0 + (uint64_t)step * (uint32_t)lane;
+      on = at < n;
+      if (on) {
+        q = wide_tri(list[at], setup, views, dkey, TS);
+        if ((q.g.cx1 - q.g.cx0 + 1) * (q.g.cy1 - q.g.cy0 + 1) > kBoxTiles) {
+          const uint32_t p = atomicAdd(&large.n, 1u);
+          if (p < kLargeBuf) {
+            large.t[p] = q;
+            on = false;
+          }
+        }
+      }
+    } else {
+      __syncthreads();
+      shared = true;
+      on = (uint32_t)lane < min(large.n, kLargeBuf);
+      if (on) q = large.t[lane];
     }
-    // without edge tests every margin is infinite
-#pragma unroll
-    for (int e = 0; e < 3; e++) g.fm[e] = g.exact ? g.fm[e] : INFINITY;
-    const int nx = g.cx1 - g.cx0 + 1, ny = g.cy1 - g.cy0 + 1;
-    auto bi = [](int v, int b) { return __builtin_amdgcn_readlane(v, b); };
+    auto bi = [](auto v, int b) { return (decltype(v))__builtin_amdgcn_readlane((int)v, b); };
     auto bf = [](float v, int b) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), b)); };
     for (uint64_t m = __ballot(on); m; m &= m - 1) {
       const int b = (int)__builtin_ctzll(m);
-      const uint32_t i = (uint32_t)bi((int)id, b), k0 = (uint32_t)bi((int)key0, b), row = (uint32_t)bi((int)ntx, b);
-      const int unx = bi(nx, b), nt = unx * bi(ny, b);
-      if (nt > kBoxTiles) {
-        const SetupRec r = setup[i];
-        Spans u;
-        spans_init(r, TS, u);
-        wave_tiles(r, u, TS, lane, rows, [&](uint32_t, int ty, int tx) {
-          f(k0 + (uint32_t)(ty - u.cy0) * row + (uint32_t)(tx - u.cx0), i);
-        });
-        continue;
-      }
       Spans u;
       u.exact = true;
+      u.cx0 = bi(q.g.cx0, b);
+      u.cx1 = bi(q.g.cx1, b);
+      u.cy0 = bi(q.g.cy0, b);
+      u.cy1 = bi(q.g.cy1, b);
 #pragma unroll
       for (int e = 0; e < 3; e++) {
-        u.fa[e] = bf(g.fa[e], b);
-        u.fb[e] = bf(g.fb[e], b);
-        u.fk[e] = bf(g.fk[e], b);
-        u.fm[e] = bf(g.fm[e], b);
+        u.fa[e] = bf(q.g.fa[e], b);
+        u.fb[e] = bf(q.g.fb[e], b);
+        u.fk[e] = bf(q.g.fk[e], b);
+        u.fm[e] = bf(q.g.fm[e], b);
       }
-      const int cx0 = bi(g.cx0, b), cy0 = bi(g.cy0, b);
-      const float inv = 1.0f / (float)unx;
-      for (int t0 = 0; t0 < nt; t0 += 64) {
-        const int t = t0 + lane;
-        const int dy = (int)(((float)t + 0.5f) * inv), dx = t - dy * unx;  // exact: t < 512
-        if (t < nt && tile_may_cover(u, TS, cx0 + dx, cy0 + dy)) f(k0 + (uint32_t)dy * row + (uint32_t)dx, i);
-      }
+      const uint32_t id = bi(q.id, b), dk = bi(q.dk, b), ntx = bi(q.ntx, b), key0 = bi(q.key0, b);
+      wave_tiles(u, TS, shared ? wave : 0, shared ? NW : 1, [&](uint32_t, int tx, int ty) {
+        f(key0 + (uint32_t)(ty - u.cy0) * ntx + (uint32_t)(tx - u.cx0), id, dk);
+      });
     }
+    if (shared) return;
   }
 }
 
@@ -945,11 +895,15 @@ __device__ inline void emit_box_pairs(uint2 box, uint32_t i, uint32_t o, uint32_
 }
 
 // ================================================================== geometry
-// Small single-view frames: at most kSmallBinTris input triangles and
-// kSmallBinTiles tiles take single-workgroup kernels for the geometry lists
-// (k_geom_small) and the binning (k_bin_small).
-constexpr uint32_t kSmallBinTiles = 4096;  // LDS counters and cursors: 32 KB
-constexpr uint32_t kSmallBinTris = 16384;  // LDS count bytes: 16 KB
+// Small single-view frames: at most kSmallBinTris input triangles take one
+// workgroup for the geometry lists (k_geom_small), and with at most
+// kSmallBinTiles tiles one for the binning (k_bin_small): a launch each in
+// place of three and four.  One CU's issue rate sets the limits (frame times,
+// one workgroup -> general kernels): a torus of 2304 triangles on 300 tiles 60
+// -> 67 us, on 1900 74 -> 80, on 2304 90 -> 86, on 3600 117 -> 88; soups of
+// 300 triangles on 1200 tiles 57 -> 64, of 3000 106 -> 78, of 16,000 321 -> 87.
+constexpr uint32_t kSmallBinTiles = 2048;  // LDS counters and cursors: 16 KB
+constexpr uint32_t kSmallBinTris = 2560;   // LDS count bytes: 2.5 KB
 
 // cnt[t]: clipped-triangle count (bits 0-2, at most 4) | kCntClip when the
 // triangle crosses the near or far plane.
@@ -1489,14 +1443,13 @@ __global__ __launch_bounds__(256) void k_bin_count_wide(const SetupRec* __restri
                                                         const DevView* __restrict__ views, const Status* status,
                                                         int TS, const uint32_t* __restrict__ wide_list,
                                                         uint32_t* __restrict__ bincnt, uint32_t* __restrict__ tile_cnt) {
-  __shared__ WaveRows s_rows[4];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63;
   for_each_wide(wide_list, status, [&](uint32_t i) {
     const SetupRec r = setup[i];
     const DevView& vw = views[r.view];
     Spans g;
     spans_init(r, TS, g);
-    const uint32_t c = wave_tiles(r, g, TS, lane, s_rows[wave], [&](uint32_t, int ty, int tx) {
+    const uint32_t c = wave_tiles(g, TS, 0, 1, [&](uint32_t, int tx, int ty) {
       if (!ORDERED) atomicAdd(&tile_cnt[vw.tile_base + (uint32_t)ty * vw.ntx + (uint32_t)tx], 1u);
     });
     if (ORDERED && lane == 0) bincnt[i] = c;
@@ -1562,15 +1515,14 @@ __global__ __launch_bounds__(256) void k_bin_emit_wide(const SetupRec* __restric
                                                        const uint32_t* __restrict__ tile_start,
                                                        uint32_t* __restrict__ tile_cur, uint32_t cap_pairs,
                                                        uint32_t* __restrict__ keys, uint32_t* __restrict__ vals) {
-  __shared__ WaveRows s_rows[4];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63;
   for_each_wide(wide_list, status, [&](uint32_t i) {
     const SetupRec r = setup[i];
     const DevView& vw = views[r.view];
     Spans g;
     spans_init(r, TS, g);
     const uint32_t o = ORDERED ? binoff[i] : 0u;
-    wave_tiles(r, g, TS, lane, s_rows[wave], [&](uint32_t e, int ty, int tx) {
+    wave_tiles(g, TS, 0, 1, [&](uint32_t e, int tx, int ty) {
       const uint32_t key = vw.tile_base + (uint32_t)ty * vw.ntx + (uint32_t)tx;
       const uint32_t pos = ORDERED ? o + e : tile_start[key] + atomicAdd(&tile_cur[key], 1u);
       if (pos < cap_pairs) {
@@ -1582,8 +1534,7 @@ __global__ __launch_bounds__(256) void k_bin_emit_wide(const SetupRec* __restric
 }
 
 // Binning of a small single-view frame in one workgroup of 1024 threads,
-// in place of the general path's dozen launches (which a frame of a few
-// thousand triangles spends mostly starting and draining): per-tile counts
+// in place of the general path's four launches: per-tile counts
 // with LDS atomics from each triangle's bin box (a wave per wide triangle of
 // the emits' list), their scan into the tile ranges, then each
 // triangle's id written into its tiles' lists at LDS-atomic cursors.  The
@@ -1601,9 +1552,10 @@ __global__ __launch_bounds__(1024) void k_bin_small(const SetupRec* __restrict__
   __shared__ uint32_t s_cnt[kSmallBinTiles];
   __shared__ uint32_t s_cur[kSmallBinTiles];
   __shared__ uint32_t s_w[16];
-  __shared__ WaveRows s_rows[16];
+  __shared__ LargeBuf s_large[2];  // the count pass's, the list pass's
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   for (uint32_t k = (uint32_t)tid; k < n_tiles; k += 1024u) s_cnt[k] = 0u;
+  if (tid < 2) s_large[tid].n = 0u;
   __syncthreads();
   const uint32_t n = min(status->n_out, cap_tri);
   const uint2* boxes = bin_boxes(const_cast<uint8_t*>(wflag), cap_tri);
@@ -1614,14 +1566,14 @@ __global__ __launch_bounds__(1024) void k_bin_small(const SetupRec* __restrict__
       box_tiles(boxes[i], [&](uint32_t key) { f(i, key); });
     }
   };
-  auto each_wide_tile = [&](uint32_t nw, auto f) {
-    wave_wide_tiles(wide_list, (uint32_t)wave, 16u, nw, setup, views, TS, s_rows[wave],
-                    [&](uint32_t key, uint32_t i) { f(i, key); });
+  auto each_wide_tile = [&](uint32_t nw, LargeBuf& large, auto f) {
+    wave_wide_tiles<16>(wide_list, (uint32_t)wave, 16u, nw, setup, views, nullptr, TS, large,
+                        [&](uint32_t key, uint32_t i, uint32_t) { f(i, key); });
   };
   // counts
   each_tile([&](uint32_t, uint32_t key) { atomicAdd(&s_cnt[key], 1u); });
   const uint32_t nw = status->n_wide;
-  each_wide_tile(nw, [&](uint32_t, uint32_t key) { atomicAdd(&s_cnt[key], 1u); });
+  each_wide_tile(nw, s_large[0], [&](uint32_t, uint32_t key) { atomicAdd(&s_cnt[key], 1u); });
   __syncthreads();
   // exclusive scan of the counts, 1024 tiles at a time with a carry
   uint32_t carry = 0;
@@ -1660,7 +1612,7 @@ __global__ __launch_bounds__(1024) void k_bin_small(const SetupRec* __restrict__
     if (pos < cap_pairs) vals[pos] = i;
   };
   each_tile(put);
-  each_wide_tile(nw, put);
+  each_wide_tile(nw, s_large[1], put);
 }
 
 __global__ __launch_bounds__(256) void k_ranges_from_counts(const uint32_t* __restrict__ tile_start,
@@ -1801,10 +1753,10 @@ __global__ __launch_bounds__(256) void k_radix_scatter(const uint32_t* __restric
 // or two more sort passes with their scans, 13 to 18 launches of 3 to 15 us
 // each.  1M-triangle 1080p frame: 387 -> 358 us; 150k triangles at 1237x709: 208
 // -> 166 us; 500k triangles at 3840x2160: 300 -> 249 us.)
-constexpr int kPairChunks = 256;         // blocks of 1024 threads: one per CU, twice (triangles, wide triangles)
+constexpr int kPairChunks = 256;         // blocks of 1024 threads: one per CU
 constexpr int kPairT = 1024;
 constexpr int kPairU = 4;                // boxes in flight per thread
-constexpr int kPairCols = 2 * kPairChunks;  // histogram columns: wide chunks first, then the others
+constexpr int kPairCols = kPairChunks;   // histogram columns
 constexpr uint32_t kPairCounters = 8192;    // k_pair_sort's LDS counters: tiles of a segment x depth levels
 // 256 segments, or 2048 where they would leave a segment fewer than 16 depth
 // levels; beyond kPairMaxTiles a segment has more tiles than counters.
@@ -1818,38 +1770,24 @@ static_assert(2048u * (kPairCols + 1u) <= kRadixHistEntries, "histogram and digi
 // most kPairSubmitTris input triangles: a tile's ids that share a key number
 // at most 1/256 of the frame's triangles (with 256 levels), so counting stays
 // far below the tile's blending.  (A transparent pass of 19,600 triangles on
-// 3600 tiles took 13 launches from its emits to the blend by a stable sort of
-// tile keys.)
+// 3600 tiles took 14 launches and some 55 us from its emits to the blend by a
+// stable sort of tile keys, now four and 19.)
 constexpr uint32_t kPairSubmitTris = 65536;
 __device__ inline uint32_t submit_shift(uint32_t n) {  // (n - 1) >> shift <= 255
   return n > 256u ? 24u - (uint32_t)__builtin_clz(n - 1u) : 0u;
 }
 
+__device__ inline uint32_t pair_col() { return xcd_remap(blockIdx.x, (uint32_t)kPairChunks); }
+
 // Visits the pairs of one chunk: f(tile key, triangle, depth key).
 template <class F>
 __device__ inline void pair_chunk(const uint8_t* __restrict__ dkey, const uint32_t* __restrict__ wide_list,
                                   const SetupRec* __restrict__ setup, const DevView* __restrict__ views,
-                                  const Status* __restrict__ status, uint32_t cap_tri, int TS, WaveRows* s_rows, F f) {
-  const int tid = threadIdx.x;
-  if (blockIdx.x < (uint32_t)kPairChunks) {
-    const int lane = tid & 63, wave = tid >> 6;
-    const uint32_t n = min(status->n_wide, cap_tri);
-    for (uint32_t w = blockIdx.x + (uint32_t)(kPairChunks * wave); w < n; w += (uint32_t)(kPairChunks * (kPairT / 64))) {
-      const uint32_t i = (uint32_t)__builtin_amdgcn_readfirstlane((int)wide_list[w]);
-      const SetupRec r = setup[i];
-      const DevView& vw = views[r.view];
-      const uint32_t dk = dkey[i];
-      Spans g;
-      spans_init(r, TS, g);
-      wave_tiles(r, g, TS, lane, s_rows[wave], [&](uint32_t, int ty, int tx) {
-        f(vw.tile_base + (uint32_t)ty * vw.ntx + (uint32_t)tx, i, dk);
-      });
-    }
-    return;
-  }
+                                  const Status* __restrict__ status, uint32_t cap_tri, int TS, LargeBuf& large, F f) {
+  const int tid = threadIdx.x, wave = tid >> 6;
   const uint32_t n = min(status->n_out, cap_tri);
   // consecutive chunks on one XCD: their runs in a segment are neighbours
-  const uint32_t cb = xcd_remap(blockIdx.x - (uint32_t)kPairChunks, (uint32_t)kPairChunks);
+  const uint32_t cb = pair_col();
   const uint32_t C = (n + (uint32_t)kPairChunks - 1u) / (uint32_t)kPairChunks;
   const uint32_t b0 = min(cb * C, n), b1 = min(b0 + C, n);
   const uint2* boxes = bin_boxes(const_cast<uint8_t*>(dkey), cap_tri);
@@ -1866,12 +1804,10 @@ __device__ inline void pair_chunk(const uint8_t* __restrict__ dkey, const uint32
     for (int u = 0; u < kPairU; u++)
       box_tiles(box[u], [&](uint32_t key) { f(key, tb + (uint32_t)(kPairT * u + tid), dk[u]); });
   }
-}
-
-__device__ inline uint32_t pair_col() {
-  return blockIdx.x < (uint32_t)kPairChunks
-             ? blockIdx.x
-             : (uint32_t)kPairChunks + xcd_remap(blockIdx.x - (uint32_t)kPairChunks, (uint32_t)kPairChunks);
+  // its wide triangles
+  wave_wide_tiles<kPairT / 64>(wide_list, blockIdx.x + (uint32_t)kPairChunks * (uint32_t)wave,
+                               (uint32_t)kPairChunks * (kPairT / 64u), min(status->n_wide, cap_tri), setup, views,
+                               dkey, TS, large, f);
 }
 
 template <int DIG>
@@ -1882,10 +1818,11 @@ __global__ __launch_bounds__(kPairT) void k_pair_hist(const uint8_t* __restrict_
                                                       const Status* __restrict__ status, uint32_t cap_tri, int TS,
                                                       uint32_t* __restrict__ hist) {
   __shared__ uint32_t h[DIG];
-  __shared__ WaveRows s_rows[kPairT / 64];
+  __shared__ LargeBuf s_large;
   for (int d = threadIdx.x; d < DIG; d += kPairT) h[d] = 0u;
+  if (threadIdx.x == 0) s_large.n = 0u;
   __syncthreads();
-  pair_chunk(dkey, wide_list, setup, views, status, cap_tri, TS, s_rows,
+  pair_chunk(dkey, wide_list, setup, views, status, cap_tri, TS, s_large,
              [&](uint32_t key, uint32_t, uint32_t) { atomicAdd(&h[key & (DIG - 1u)], 1u); });
   __syncthreads();
   const uint32_t col = pair_col();
@@ -1954,11 +1891,8 @@ __device__ inline uint32_t lds_exclusive_scan(uint32_t* s, uint32_t n, uint32_t*
   return carry;
 }
 
-// Held to 64 VGPRs (a dozen spilled words, in the rows of large triangles), so
-// that a wide block and another share a CU: 20 -> 18 us on the 1M-triangle
-// soup; k_pair_hist, without the scatter's waits, lost more to the spills.
 template <int DIG, bool SUBMIT>
-__global__ __launch_bounds__(kPairT) __attribute__((amdgpu_waves_per_eu(8))) void k_pair_scatter(const uint8_t* __restrict__ dkey,
+__global__ __launch_bounds__(kPairT) void k_pair_scatter(const uint8_t* __restrict__ dkey,
                                                          const uint32_t* __restrict__ wide_list,
                                                          const SetupRec* __restrict__ setup,
                                                          const DevView* __restrict__ views, Status* __restrict__ status,
@@ -1967,9 +1901,10 @@ __global__ __launch_bounds__(kPairT) __attribute__((amdgpu_waves_per_eu(8))) voi
                                                          uint2* __restrict__ pairs) {
   constexpr int kShift = DIG == 256 ? 8 : 11;
   __shared__ uint32_t cur[DIG];
-  __shared__ WaveRows s_rows[kPairT / 64];
+  __shared__ LargeBuf s_large;
   __shared__ uint32_t s_w[kPairT / 64];
   const uint32_t col = pair_col();
+  if (threadIdx.x == 0) s_large.n = 0u;
   for (int d = threadIdx.x; d < DIG; d += kPairT) cur[d] = totals[d];
   __syncthreads();
   const uint32_t all = lds_exclusive_scan<kPairT>(cur, DIG, s_w);
@@ -1980,7 +1915,7 @@ __global__ __launch_bounds__(kPairT) __attribute__((amdgpu_waves_per_eu(8))) voi
   for (int d = threadIdx.x; d < DIG; d += kPairT) cur[d] += hist[(uint32_t)d * kPairCols + col];
   __syncthreads();
   const uint32_t sh = submit_shift(min(status->n_out, cap_tri));
-  pair_chunk(dkey, wide_list, setup, views, status, cap_tri, TS, s_rows,
+  pair_chunk(dkey, wide_list, setup, views, status, cap_tri, TS, s_large,
              [&](uint32_t key, uint32_t i, uint32_t dk) {
                if (SUBMIT) dk = i >> sh;
                const uint32_t pos = atomicAdd(&cur[key & (DIG - 1u)], 1u);
@@ -2158,9 +2093,11 @@ __global__ __launch_bounds__(256) void k_tsort_keys(const uint32_t* __restrict__
 //                  triangles out of the mesh;
 //  k_tsort_merge   sixteen lanes per triangle add up its ranks in the mesh's
 //                  chunks by binary searches and write it to its place.
-// A radix sort took 18 launches a mesh, each about as long as starting it; it
-// stays for larger meshes, whose searches (a sixteenth of n / 1024 chunks a
-// lane) would outgrow it.
+// A radix sort took 18 to 22 launches a mesh, each about as long as starting it
+// (two meshes of 9,800 triangles: some 180 us, now 21; of 33,000: 141, now 58).
+// It stays for larger meshes: the searches, a sixteenth of n / 1024 chunks a
+// lane, grow with the square (two of 65,500: the frame 389 us with these, 358
+// with the radix sort).
 constexpr uint32_t kTsortChunk = 1024, kTsortMax = 32768, kTsortMeshes = 16;
 struct TsortBatch {
   TransMesh m[kTsortMeshes];

