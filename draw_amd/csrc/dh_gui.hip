@@ -158,7 +158,7 @@ __global__ __launch_bounds__(256) void k_gui_raster(const GuiRec* __restrict__ r
                                                     const uint8_t* __restrict__ font, int32_t fw, int32_t fh,
                                                     int32_t fcomp, uint32_t* __restrict__ bgra,
                                                     const float* __restrict__ depth, uint32_t* __restrict__ error) {
-  const uint32_t tile = xcd_remap(blockIdx.x, gridDim.x);
+  const uint32_t tile = xcd_remap_tiles(blockIdx.x, gridDim.x);
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   const int qx0 = (int)(tile % ntx) * 16 + (wave & 1) * 8, qy0 = (int)(tile / ntx) * 16 + (wave >> 1) * 8;
   if (qx0 >= W || qy0 >= H) return;  // the whole wave

@@ -332,7 +332,7 @@ __global__ __launch_bounds__(64 * (TS / 8) * (TS / 8) / QPW) __attribute__((amdg
   constexpr uint32_t kQExact = 1u << 16;
   constexpr int kSmallPx = 8;  // largest side of a small record's rectangle within the tile
 
-  const uint32_t tile = xcd_remap(blockIdx.x, gridDim.x);
+  const uint32_t tile = xcd_remap_tiles(blockIdx.x, gridDim.x);
   const DevView& vw = views[wave_find_view_tile(views, n_views, tile)];
   const uint32_t lt = tile - vw.tile_base;
   const int tx = (int)(lt % vw.ntx), ty = (int)(lt / vw.ntx);
@@ -830,7 +830,7 @@ __global__ __launch_bounds__(64 * NW) void k_raster_tp(
   __shared__ uint32_t s_next;
   __shared__ uint32_t s_nfrag;  // the tile's fragment count (one global atomic per tile)
 
-  const uint32_t tile = xcd_remap(blockIdx.x, gridDim.x);
+  const uint32_t tile = xcd_remap_tiles(blockIdx.x, gridDim.x);
   const DevView& vw = views[wave_find_view_tile(views, n_views, tile)];
   const uint32_t lt = tile - vw.tile_base;
   const int tx0 = (int)(lt % vw.ntx) * TS, ty0 = (int)(lt / vw.ntx) * TS;
@@ -1039,7 +1039,7 @@ __global__ __launch_bounds__(256) void k_blend(const DevView* __restrict__ views
   constexpr int CH = 64;
   __shared__ uint4 s_rec[CH][15];  // the setup record's 6 words, the shading record's 9
   __shared__ float s_unit[256];
-  const uint32_t tile = xcd_remap(blockIdx.x, gridDim.x);
+  const uint32_t tile = xcd_remap_tiles(blockIdx.x, gridDim.x);
   const uint2 rg = ranges[tile];
   if (rg.x >= rg.y) return;  // nothing to blend (the whole block)
   const DevView& vw = views[0];
