@@ -30,6 +30,7 @@ inline Kind handle_kind(dh_handle h) { return (Kind)(h >> 56); }
 struct TexRes {
   uint8_t* d = nullptr;
   int32_t w = 0, h = 0, comp = 0;
+  uint8_t first[3] = {0, 0, 0};  // the first texel
 };
 struct MatRes {
   uint32_t slot = 0;
@@ -213,6 +214,12 @@ int upload_materials(dh_ctx c) {
   return DH_OK;
 }
 
+// An ambient map of one texel: its colour, as the shading computes it.
+void set_ambient(dh::DevMaterial* m, const uint8_t first[3]) {
+  m->ka_one = m->ka_w == 1 && m->ka_h == 1;
+  for (int i = 0; i < 3; i++) m->ka_col[i] = (float)first[i] / 255.0f * m->ka[i];
+}
+
 dh::DevMaterial default_material(const uint8_t* white) {
   dh::DevMaterial m;
   memset(&m, 0, sizeof(m));
@@ -227,6 +234,8 @@ dh::DevMaterial default_material(const uint8_t* white) {
   m.ka_img = white;
   m.kd_w = m.kd_h = m.ka_w = m.ka_h = 1;
   m.kd_comp = m.ka_comp = 3;
+  const uint8_t texel[3] = {255, 255, 255};
+  set_ambient(&m, texel);
   return m;
 }
 
@@ -464,6 +473,7 @@ extern "C" int dh_texture_create(dh_ctx c, const uint8_t* img, int32_t w, int32_
   t.w = w;
   t.h = h;
   t.comp = comp;
+  memcpy(t.first, img, 3);
   const size_t bytes = (size_t)w * (size_t)h * (size_t)comp;
   HIPCHK(c, hipMalloc(reinterpret_cast<void**>(&t.d), bytes + 4));  // +4: 32-bit texel loads
   HIPCHK(c, hipMemcpy(t.d, img, bytes, hipMemcpyHostToDevice));
@@ -484,6 +494,7 @@ extern "C" int dh_material_create(dh_ctx c, const dh_material_desc* d, dh_handle
   }
   m.alpha = d->alpha;
   m.power = d->power;
+  uint8_t ka_first[3] = {255, 255, 255};  // the default map's texel
   const dh_handle maps[2] = {d->map_kd, d->map_ka};
   for (int k = 0; k < 2; k++) {
     if (!maps[k]) continue;
@@ -494,8 +505,10 @@ extern "C" int dh_material_create(dh_ctx c, const dh_material_desc* d, dh_handle
       m.kd_img = it->second.d; m.kd_w = it->second.w; m.kd_h = it->second.h; m.kd_comp = it->second.comp;
     } else {
       m.ka_img = it->second.d; m.ka_w = it->second.w; m.ka_h = it->second.h; m.ka_comp = it->second.comp;
+      memcpy(ka_first, it->second.first, 3);
     }
   }
+  set_ambient(&m, ka_first);
   MatRes r;
   r.slot = (uint32_t)c->res->mat_host.size();
   r.alpha = d->alpha;

@@ -56,6 +56,8 @@ struct DevMaterial {
   const uint8_t* ka_img;
   int32_t kd_w, kd_h, kd_comp;
   int32_t ka_w, ka_h, ka_comp;
+  float ka_col[3];  // ka_one: the texel / 255 * ka
+  int32_t ka_one;   // the ambient map has one texel
 };
 
 // One draw = one IndexedMesh of one Object, in submission order.

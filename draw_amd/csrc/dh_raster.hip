@@ -78,46 +78,68 @@ __device__ inline void fill_unit_table(float* unit, int tid, int nt) {
   for (int k = tid; k < 256; k += nt) unit[k] = div_known((float)k, 255.0f, kInv);
 }
 
+// Device memory behind a pointer read from a table: global accesses, where the
+// compiler would take FLAT ones, which wait for the LDS counter too.
+template <class T>
+using Global = __attribute__((address_space(1))) T;
+template <class T>
+__device__ __forceinline__ Global<T>* as_global(T* p) {
+  return (Global<T>*)p;
+}
+
 // TextureMap::get_rgb_slice's byte offset (rgb_offset) in 32-bit arithmetic:
 // true where the floored coordinates lie in the map, which most do; ok as
-// rgb_offset returns it.  small: the map has fewer than 2^32 bytes.
+// rgb_offset returns it.  small: the map has fewer than 2^32 bytes and 2^24
+// texels a side (full-rate 24-bit products).
 __device__ __forceinline__ bool rgb_offset_in_map(int32_t w, int32_t h, int32_t comp, float u, float v, bool small,
                                          uint32_t* off) {
   const float mu = (float)w - 1.0f, mv = (float)h - 1.0f;
   // f32 as usize: NaN and negatives are 0
   const float fu = fmaxf(floorf(u * mu), 0.0f), fv = fmaxf(floorf(v * mv), 0.0f);
-  *off = (((uint32_t)h - 1u - (uint32_t)fv) * (uint32_t)w + (uint32_t)fu) * (uint32_t)comp;
+  const uint32_t t = __umul24((uint32_t)h - 1u - (uint32_t)fv, (uint32_t)w) + (uint32_t)fu;
+  *off = comp == 4 ? t << 2 : t + (t << 1);
   return small && fu <= mu && fv <= mv;
 }
 __device__ inline bool small_map(int32_t w, int32_t h, int32_t comp) {
-  return (uint64_t)w * (uint64_t)h * (uint64_t)comp < 0xFFFFFFFFull;
+  return (uint64_t)w * (uint64_t)h * (uint64_t)comp < 0xFFFFFFFFull && (w | h) < (1 << 24);
 }
 
-__device__ inline uint32_t fetch_rgb(const uint8_t* img, int32_t comp, uint64_t off) {
-  if (comp == 4) return *reinterpret_cast<const uint32_t*>(img + off);
-  return (uint32_t)img[off] | ((uint32_t)img[off + 1] << 8) | ((uint32_t)img[off + 2] << 16);
+template <class Off>
+__device__ __forceinline__ uint32_t fetch_rgb(const uint8_t* img, int32_t comp, Off off) {
+  Global<const uint8_t>* const t = as_global(img) + off;
+  if (comp == 4) return *(Global<const uint32_t>*)t;
+  return (uint32_t)t[0] | ((uint32_t)t[1] << 8) | ((uint32_t)t[2] << 16);
 }
 
 // Shading of a covered pixel, canvas.rs:685-741; returns B | G<<8 | R<<16 | A<<24.
-// unit: the k / 255 table (fill_unit_table).
+// unit: the k / 255 table (fill_unit_table).  An ambient map of one texel, which
+// materials without one have, is sampled when the material is made: every
+// coordinate falls on it.
 __device__ __forceinline__ uint32_t shade_pixel(const ShadeRec& s, const DevMaterial& m, const FragOut& o, Status* status,
                                        const float* unit) {
   const float u = (s.uv[0] * o.al + s.uv[2] * o.be) + s.uv[4] * o.ga;
   const float v = (s.uv[1] * o.al + s.uv[3] * o.be) + s.uv[5] * o.ga;
-  uint32_t skd, ska;
-  const bool in1 = rgb_offset_in_map(m.kd_w, m.kd_h, m.kd_comp, u, v, small_map(m.kd_w, m.kd_h, m.kd_comp), &skd);
-  const bool in2 = rgb_offset_in_map(m.ka_w, m.ka_h, m.ka_comp, u, v, small_map(m.ka_w, m.ka_h, m.ka_comp), &ska);
-  uint64_t okd = skd, oka = ska;
-  if (!(in1 && in2)) {
+  const bool ka_one = m.ka_one != 0;
+  uint32_t skd, ska = 0;
+  bool in = rgb_offset_in_map(m.kd_w, m.kd_h, m.kd_comp, u, v, small_map(m.kd_w, m.kd_h, m.kd_comp), &skd);
+  if (!ka_one)
+    in &= rgb_offset_in_map(m.ka_w, m.ka_h, m.ka_comp, u, v, small_map(m.ka_w, m.ka_h, m.ka_comp), &ska);
+  uint32_t dk, ak = 0;
+  if (in) {
+    dk = fetch_rgb(m.kd_img, m.kd_comp, skd);
+    if (!ka_one) ak = fetch_rgb(m.ka_img, m.ka_comp, ska);
+  } else {
+    uint64_t okd, oka = 0;
     const bool ok1 = rgb_offset(m.kd_w, m.kd_h, m.kd_comp, u, v, &okd);
-    const bool ok2 = rgb_offset(m.ka_w, m.ka_h, m.ka_comp, u, v, &oka);
+    const bool ok2 = ka_one || rgb_offset(m.ka_w, m.ka_h, m.ka_comp, u, v, &oka);
     if (!(ok1 && ok2)) {
       atomicOr(&status->error, 1u);
       okd = 0;
       oka = 0;
     }
+    dk = fetch_rgb(m.kd_img, m.kd_comp, okd);
+    if (!ka_one) ak = fetch_rgb(m.ka_img, m.ka_comp, oka);
   }
-  const uint32_t dk = fetch_rgb(m.kd_img, m.kd_comp, okd), ak = fetch_rgb(m.ka_img, m.ka_comp, oka);
   const V3 pn = add(add(muls(v3(s.n[0], s.n[1], s.n[2]), o.al), muls(v3(s.n[3], s.n[4], s.n[5]), o.be)),
                     muls(v3(s.n[6], s.n[7], s.n[8]), o.ga));
   const V3 pl = add(add(muls(v3(s.l[0], s.l[1], s.l[2]), o.al), muls(v3(s.l[3], s.l[4], s.l[5]), o.be)),
@@ -129,10 +151,11 @@ __device__ __forceinline__ uint32_t shade_pixel(const ShadeRec& s, const DevMate
                     muls(v3(s.h[6], s.h[7], s.h[8]), o.ga));
   const float h2 = powi_f(dot(ph, pn), m.power);
   const V3 diffuse = v3(unit[dk & 255u], unit[(dk >> 8) & 255u], unit[(dk >> 16) & 255u]);
-  const V3 ambient = v3(unit[ak & 255u], unit[(ak >> 8) & 255u], unit[(ak >> 16) & 255u]);
   const V3 c_l = v3(m.ks[0], m.ks[1], m.ks[2]);
   const V3 c_r = v3(diffuse.x * m.kd[0], diffuse.y * m.kd[1], diffuse.z * m.kd[2]);
-  const V3 c_a = v3(ambient.x * m.ka[0], ambient.y * m.ka[1], ambient.z * m.ka[2]);
+  V3 c_a = v3(m.ka_col[0], m.ka_col[1], m.ka_col[2]);
+  if (!ka_one)
+    c_a = v3(unit[ak & 255u] * m.ka[0], unit[(ak >> 8) & 255u] * m.ka[1], unit[(ak >> 16) & 255u] * m.ka[2]);
   const V3 inner = add(c_a, muls(c_l, sfac));
   const V3 t1 = v3(c_r.x * inner.x, c_r.y * inner.y, c_r.z * inner.z);
   const V3 col = add(t1, muls(c_l, h2));
@@ -147,10 +170,10 @@ __device__ inline uint32_t clear_word(const DevView& vw) {
 }
 __device__ inline void write_pixel(const DevView& vw, uint32_t W, uint32_t H, uint32_t x, uint32_t y, uint32_t bgra,
                                    float depth, uint32_t winner) {
-  const uint32_t p = y * W + x;
-  vw.out_bgra[(H - 1u - y) * W + x] = bgra;  // draw_pixel_coord row flip, canvas.rs:955
-  vw.out_depth[p] = depth;
-  if (vw.out_winner) vw.out_winner[p] = winner;
+  const uint32_t row = __umul24(y, W);
+  as_global(vw.out_bgra)[(H - 1u) * W - row + x] = bgra;  // draw_pixel_coord row flip, canvas.rs:955
+  as_global(vw.out_depth)[row + x] = depth;
+  if (vw.out_winner) as_global(vw.out_winner)[row + x] = winner;
 }
 
 // Shading of up to 64 pixels by one wave; every lane calls it.  A lane's pixel
