@@ -1315,7 +1315,7 @@ uint64_t ctx_scratch_bytes(dh_ctx c) {
 uint64_t scratch_estimate(uint64_t n_in, uint64_t n_tiles, uint64_t n_pixels, uint64_t n_draws,
                           uint64_t n_views) {
   const uint64_t tri = n_in + n_in / 4 + 1024, pairs = 4 * tri + n_tiles;
-  return std::max<uint64_t>(n_in, 1) + 12 * ((n_in + 255) / 256 + 1) + 8 * n_in +
+  return std::max<uint64_t>(n_in, 1) + 12 * geom_blk_stride((n_in + 255) / 256) + 8 * n_in +
          (sizeof(SetupRec) + sizeof(ShadeRec) + 12) * tri + 16 * pairs +
          4ull * kRadixHistEntries + 4096 + 20 * n_tiles + 4 * n_pixels + sizeof(DevDraw) * n_draws +
          sizeof(DevView) * n_views + 2 * sizeof(Status);

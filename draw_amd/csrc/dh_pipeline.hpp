@@ -6,8 +6,8 @@
 namespace dh {
 
 constexpr uint32_t kRadixHistEntries = 2048u * 1024u;  // (up to 11-bit) digits x radix-sort waves
-// words between the three segments of per-block geometry counts
-__host__ __device__ constexpr uint64_t geom_blk_stride(uint64_t n_blk) { return n_blk + 1u; }
+// words between the three segments of per-block geometry counts (16-byte aligned)
+__host__ __device__ constexpr uint64_t geom_blk_stride(uint64_t n_blk) { return (n_blk + 4u) & ~(uint64_t)3; }
 
 struct PipeArgs {
   // inputs
