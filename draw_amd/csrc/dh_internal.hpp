@@ -30,6 +30,13 @@ hipError_t enqueue_gui(const uint4* src, uint4* dst, const GuiLayout& g, uint32_
                        const uint8_t* font, int32_t fw, int32_t fh, int32_t fcomp, uint32_t* bgra, const float* depth,
                        uint32_t* error, hipStream_t s);
 constexpr size_t kGuiRecBytes = 152;  // a 144-byte record and an 8-byte scan rectangle
+// Large reads of canvas buffers into pageable memory (dh_readback.hip): n_seg (at
+// most 3) buffers of n_words words each.  Null from create: not available.
+struct ReadStage;
+ReadStage* read_stage_create(hipStream_t s);
+void read_stage_destroy(ReadStage* st);
+hipError_t read_stage_read(ReadStage* st, const void* const* src, void* const* dst, uint32_t n_seg, uint32_t n_words,
+                           hipStream_t s);
 hipError_t enqueue_bgra_to_rgba(const uint32_t* src, uint32_t* dst, uint32_t n, hipStream_t s);
 // The fixed RGBA staging array of dh_canvas_read_rgba_noalloc: at most
 // kRgbaScratchPixels pixels (one 3840x2160 frame, 31.6 MiB per device).
