@@ -250,6 +250,15 @@ __device__ inline uint32_t wave_find_view_px(const DevView* views, uint32_t n, u
   return v;
 }
 
+// Device memory behind a pointer read from a table: global accesses, where the
+// compiler would take FLAT ones, which wait for the LDS counter too.
+template <class T>
+using Global = __attribute__((address_space(1))) T;
+template <class T>
+__device__ __forceinline__ Global<T>* as_global(T* p) {
+  return (Global<T>*)p;
+}
+
 // XCD-aware block order: workgroups are dispatched round-robin over the 8
 // XCDs, so give each XCD one contiguous run of logical indices (neighbouring
 // tiles share triangles and their records then share one L2).

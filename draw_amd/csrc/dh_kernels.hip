@@ -62,8 +62,25 @@ __device__ inline uint32_t wave_find_draw(const DevDraw* draws, uint32_t n, uint
 }
 
 __device__ inline V3 ld3(const float* a, uint32_t i) {
-  const float* p = a + 3ull * i;
+  Global<const float>* p = as_global(a) + 3ull * i;
   return v3(p[0], p[1], p[2]);
+}
+
+// Runs f(draw index, mine) for each draw among the active lanes' d, mine the
+// lanes that have it, the index wave-uniform: the draw, its view's uniforms and
+// its material come by scalar loads (every lane calls it; one round unless the
+// wave's triangles straddle draws).  Per lane, they were some 60 vector loads of
+// one address each (with global in place of FLAT accesses, 5M micro-triangles:
+// k_geom_emit 172 -> 128 us, k_geom_count 68 -> 53; the 32-view batch 96 -> 87
+// and 37 -> 29).
+template <class F>
+__device__ __forceinline__ void for_each_draw(uint32_t d, bool active, F f) {
+  for (uint64_t todo = __ballot(active); todo;) {
+    const uint32_t d0 = (uint32_t)__builtin_amdgcn_readlane((int)d, __builtin_ctzll(todo));
+    const bool mine = active && d == d0;
+    todo &= ~__ballot(mine);
+    f(d0, mine);
+  }
 }
 
 // Vertex positions of a draw's triangle lt (a, b, c): from the mesh's
@@ -71,12 +88,12 @@ __device__ inline V3 ld3(const float* a, uint32_t i) {
 __device__ inline void tri_positions(const DevDraw& dr, uint32_t lt, V3& a, V3& b, V3& c) {
   if (dr.soa) {
     const uint64_t n = dr.n_tri;
-    const float* s = dr.soa + lt;
+    Global<const float>* s = as_global(dr.soa) + lt;
     a = v3(s[0], s[n], s[2 * n]);
     b = v3(s[3 * n], s[4 * n], s[5 * n]);
     c = v3(s[6 * n], s[7 * n], s[8 * n]);
   } else {
-    const uint32_t* ti = dr.tri + 9ull * lt;
+    Global<const uint32_t>* ti = as_global(dr.tri) + 9ull * lt;
     a = ld3(dr.pos, ti[0]);
     b = ld3(dr.pos, ti[1]);
     c = ld3(dr.pos, ti[2]);
@@ -109,16 +126,15 @@ __device__ inline bool wave_sparse(bool active, uint32_t t, uint32_t span) {
 __device__ inline void tri_vertices(const DevDraw& dr, uint32_t lt, bool sparse, V3 (&P)[3], V3 (&nrm)[3],
                                     float (&u)[3], float (&v)[3]) {
   if (dr.soa && sparse) {
-    const uint4* r = reinterpret_cast<const uint4*>(dr.soa + mesh_records_offset(dr.n_tri)) +
-                     (uint64_t)(kMeshRecFloats / 4u) * lt;
+    typedef float Vec4 __attribute__((ext_vector_type(4)));
+    Global<const Vec4>* r = (Global<const Vec4>*)(dr.soa + mesh_records_offset(dr.n_tri)) +
+                            (uint64_t)(kMeshRecFloats / 4u) * lt;
     float f[24];
 #pragma unroll
     for (int q = 0; q < 6; q++) {
-      const uint4 x = r[q];
-      f[4 * q] = __uint_as_float(x.x);
-      f[4 * q + 1] = __uint_as_float(x.y);
-      f[4 * q + 2] = __uint_as_float(x.z);
-      f[4 * q + 3] = __uint_as_float(x.w);
+      const Vec4 x = r[q];
+#pragma unroll
+      for (int j = 0; j < 4; j++) f[4 * q + j] = x[j];
     }
 #pragma unroll
     for (int k = 0; k < 3; k++) {
@@ -129,7 +145,7 @@ __device__ inline void tri_vertices(const DevDraw& dr, uint32_t lt, bool sparse,
     }
   } else if (dr.soa) {
     const uint64_t n = dr.n_tri;
-    const float* s = dr.soa + lt;
+    Global<const float>* s = as_global(dr.soa) + lt;
 #pragma unroll
     for (int k = 0; k < 3; k++) {
       P[k] = v3(s[(3 * k) * n], s[(3 * k + 1) * n], s[(3 * k + 2) * n]);
@@ -138,12 +154,12 @@ __device__ inline void tri_vertices(const DevDraw& dr, uint32_t lt, bool sparse,
       v[k] = s[(19 + 2 * k) * n];
     }
   } else {
-    const uint32_t* ti = dr.tri + 9ull * lt;
+    Global<const uint32_t>* ti = as_global(dr.tri) + 9ull * lt;
 #pragma unroll
     for (int k = 0; k < 3; k++) {
       P[k] = ld3(dr.pos, ti[k]);
       nrm[k] = ld3(dr.nrm, ti[6 + k]);
-      const float* uv = dr.uv + 2ull * ti[3 + k];
+      Global<const float>* uv = as_global(dr.uv) + 2ull * ti[3 + k];
       u[k] = uv[0];
       v[k] = uv[1];
     }
@@ -928,9 +944,10 @@ __global__ __launch_bounds__(256) void k_geom_count(const DevDraw* __restrict__ 
   uint32_t c = 0;
   bool clip = false;
   const uint32_t d = wave_find_draw(draws, n_draws, t, t < n_in);
-  if (t < n_in) {
-    const DevDraw& dr = draws[d];
+  for_each_draw(d, t < n_in, [&](uint32_t d0, bool mine) {
+    const DevDraw& dr = draws[d0];
     const FrameParamsPod& fr = views[dr.view].fr;
+    if (!mine) return;
     PV a, b, cc;
     tri_positions(dr, t - dr.tri_begin, a.p, b.p, cc.p);
     c = (uint32_t)cull_and_clip(fr, a, b, cc, !(dr.flags & kDrawNoCull), [](int, const PV&, const PV&, const PV&) {});
@@ -938,7 +955,7 @@ __global__ __launch_bounds__(256) void k_geom_count(const DevDraw* __restrict__ 
     // vertices are strictly inside the plane (clip_plane's first branch)
     if (c) clip = !(inside_plane(fr.planes[0], a.p, b.p, cc.p) && inside_plane(fr.planes[1], a.p, b.p, cc.p));
     cnt[t] = (uint8_t)(c | (clip ? kCntClip : 0u));
-  }
+  });
   uint32_t total;
   block_exclusive_scan256(pack_geom(c, clip), s_tmp, &total);
   if (threadIdx.x == 0) {
@@ -995,9 +1012,10 @@ __global__ __launch_bounds__(1024) void k_geom_small(const DevDraw* __restrict__
     uint32_t c = 0;
     bool clip = false;
     const uint32_t d = wave_find_draw(draws, n_draws, t, t < n_in);
-    if (t < n_in) {
-      const DevDraw& dr = draws[d];
+    for_each_draw(d, t < n_in, [&](uint32_t d0, bool mine) {
+      const DevDraw& dr = draws[d0];
       const FrameParamsPod& fr = views[dr.view].fr;
+      if (!mine) return;
       PV a, b, cc;
       tri_positions(dr, t - dr.tri_begin, a.p, b.p, cc.p);
       c = (uint32_t)cull_and_clip(fr, a, b, cc, !(dr.flags & kDrawNoCull),
@@ -1006,7 +1024,7 @@ __global__ __launch_bounds__(1024) void k_geom_small(const DevDraw* __restrict__
       const uint8_t q = (uint8_t)(c | (clip ? kCntClip : 0u));
       cnt[t] = q;
       s_cnt[t] = q;
-    }
+    });
     uint64_t tot;
     const uint64_t ex = block_exclusive_scan1024x3(pack(c, clip), s_w, &tot);
     const uint32_t first = run_o + field(ex, 0);
@@ -1089,54 +1107,63 @@ __device__ __forceinline__ void geom_emit_one(uint2 sv, bool active, bool clip, 
                                               uint32_t cap_tri, Status* __restrict__ status, int TS,
                                               uint32_t* __restrict__ bincnt, uint8_t* __restrict__ wflag,
                                               uint32_t* __restrict__ wide_list, WideBuf* wide, uint32_t span) {
-  uint4 ro[6], so[9];
   const uint32_t t = sv.x, idx = sv.y + k;
-  bool ok = false, skip = false;
   const bool sparse = wave_sparse(active, t, span);
   const uint32_t d = wave_find_draw(draws, n_draws, t, active);
-  if (active) {
-    const DevDraw& dr = draws[d];
+  auto body = [&](uint32_t d0, bool mine) {
+    uint4 ro[6], so[9];
+    bool ok = false, skip = false;
+    const DevDraw& dr = draws[d0];
     const FrameParamsPod& fr = views[dr.view].fr;
-    const uint32_t lt = t - dr.tri_begin;
-    const V3 cam = v3(fr.cam[0], fr.cam[1], fr.cam[2]);
-    const V3 L = v3(fr.light[0], fr.light[1], fr.light[2]);
-    FV v[3];
-    V3 P[3], N[3];
-    float U[3], W[3];
-    tri_vertices(dr, lt, sparse, P, N, U, W);
+    if (mine) {
+      const uint32_t lt = t - dr.tri_begin;
+      const V3 cam = v3(fr.cam[0], fr.cam[1], fr.cam[2]);
+      const V3 L = v3(fr.light[0], fr.light[1], fr.light[2]);
+      FV v[3];
+      V3 P[3], N[3];
+      float U[3], W[3];
+      tri_vertices(dr, lt, sparse, P, N, U, W);
 #pragma unroll
-    for (int q = 0; q < 3; q++) {
-      const V3 p = P[q];
-      v[q].p = p;
-      // per-vertex visual info, scene/mod.rs:920-925
-      const V3 eye_dir = sub(p, cam);
-      const V3 light = normalized(sub(p, L));
-      const V3 eye = normalized(eye_dir);
-      v[q].d = norm(eye_dir);
-      v[q].l = light;
-      v[q].h = normalized(add(light, eye));
-      v[q].n = N[q];
-      v[q].u = U[q];
-      v[q].v = W[q];
-    }
-    // passed the back-face and lateral tests in k_geom_count
-    if (clip) clip_output(fr, v[0], v[1], v[2], k);
-    if (idx >= cap_tri) {
-      atomicOr(&status->overflow, 1u);
-    } else {
-      SetupRec rec;
-      make_setup(fr, v[0], v[1], v[2], dr.material, mats[dr.material], dr.view, dr.group, ro, so, rec);
-      ok = true;
-      // with ordered bins nothing reads a dropped triangle's records
-      skip = BIN != kBinNone && (rec.flags & kDrop);
-      if constexpr (BIN != kBinNone) {
-        const bool is_wide = bin_count_one<BIN>(rec, TS, idx, views[dr.view], bincnt, wflag, bin_boxes(wflag, cap_tri));
-        if (BIN == kBinNear && is_wide) wide_push(*wide, idx, status, wide_list);
+      for (int q = 0; q < 3; q++) {
+        const V3 p = P[q];
+        v[q].p = p;
+        // per-vertex visual info, scene/mod.rs:920-925
+        const V3 eye_dir = sub(p, cam);
+        const V3 light = normalized(sub(p, L));
+        const V3 eye = normalized(eye_dir);
+        v[q].d = norm(eye_dir);
+        v[q].l = light;
+        v[q].h = normalized(add(light, eye));
+        v[q].n = N[q];
+        v[q].u = U[q];
+        v[q].v = W[q];
+      }
+      // passed the back-face and lateral tests in k_geom_count
+      if (clip) clip_output(fr, v[0], v[1], v[2], k);
+      if (idx >= cap_tri) {
+        atomicOr(&status->overflow, 1u);
+      } else {
+        SetupRec rec;
+        make_setup(fr, v[0], v[1], v[2], dr.material, mats[dr.material], dr.view, dr.group, ro, so, rec);
+        ok = true;
+        // with ordered bins nothing reads a dropped triangle's records
+        skip = BIN != kBinNone && (rec.flags & kDrop);
+        if constexpr (BIN != kBinNone) {
+          const bool is_wide = bin_count_one<BIN>(rec, TS, idx, views[dr.view], bincnt, wflag, bin_boxes(wflag, cap_tri));
+          if (BIN == kBinNear && is_wide) wide_push(*wide, idx, status, wide_list);
+        }
       }
     }
-  }
-  wave_store<6>(stage, ro, ok, idx, reinterpret_cast<uint4*>(setup), skip);
-  wave_store<9>(stage, so, ok, idx, reinterpret_cast<uint4*>(shade), skip);
+    wave_store<6>(stage, ro, ok, idx, reinterpret_cast<uint4*>(setup), skip);
+    wave_store<9>(stage, so, ok, idx, reinterpret_cast<uint4*>(shade), skip);
+  };
+  // one draw: scalar loads (for_each_draw); several: per lane, since a second
+  // round would double the launch's longest wave
+  const uint64_t m = __ballot(active);
+  if (!m) return;
+  const uint32_t d0 = (uint32_t)__builtin_amdgcn_readlane((int)d, __builtin_ctzll(m));
+  if (__ballot(active && d != d0) == 0ull) body(d0, active);
+  else body(d, active);
 }
 
 // Both emitter lists (dense: culled triangles take no lane) in one launch, a
@@ -1149,8 +1176,9 @@ __device__ __forceinline__ void geom_emit_one(uint2 sv, bool active, bool clip, 
 // to four inlined copies of the setup (28 KB of code) and 168 VGPRs, its list
 // took 25 us even when short, on a second stream beside the other list's
 // launch: the fork and the join cost some 15 us more.  One copy of the setup
-// serves both lists here (17 KB, 122 VGPRs), at the four waves per SIMD that
-// the LDS of the record stores allows.  Frames, before -> after: 62k triangles
+// serves both lists here (17 KB, twice for waves of one draw and of several;
+// 127 VGPRs), at the four waves per SIMD that the LDS of the record stores
+// allows.  Frames, before -> after: 62k triangles
 // at 800x600 with a GUI 194 -> 179 us, 150k at 1237x709 168 -> 152, the
 // 1M-triangle 1080p soup 357 -> 339, two 125k-triangle shards 403 -> 391.
 template <int BIN>

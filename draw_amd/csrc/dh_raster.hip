@@ -78,15 +78,6 @@ __device__ inline void fill_unit_table(float* unit, int tid, int nt) {
   for (int k = tid; k < 256; k += nt) unit[k] = div_known((float)k, 255.0f, kInv);
 }
 
-// Device memory behind a pointer read from a table: global accesses, where the
-// compiler would take FLAT ones, which wait for the LDS counter too.
-template <class T>
-using Global = __attribute__((address_space(1))) T;
-template <class T>
-__device__ __forceinline__ Global<T>* as_global(T* p) {
-  return (Global<T>*)p;
-}
-
 // TextureMap::get_rgb_slice's byte offset (rgb_offset) in 32-bit arithmetic:
 // true where the floored coordinates lie in the map, which most do; ok as
 // rgb_offset returns it.  small: the map has fewer than 2^32 bytes and 2^24
