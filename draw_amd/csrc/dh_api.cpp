@@ -165,6 +165,7 @@ struct dh_ctx_s {
   DevBuf<uint32_t> grp;       // [groups]: first clipped id
   DevBuf<uint32_t> tperm;     // the triangles being sorted (TransArgs::perm_tmp)
   DevBuf<uint32_t> sort_n;    // [1]
+  std::mutex read_mu;  // threads reading canvases of one context take turns on
   dh::ReadStage* read_stage = nullptr;  // large canvas reads (made for the second one)
   uint64_t large_reads = 0;
   dh_stats stats = {};
@@ -1178,6 +1179,7 @@ extern "C" int dh_canvas_read(dh_ctx c, dh_handle canvas, uint8_t* bgra, float* 
   // the second such read: the first would pay more for it than it saves, and
   // many contexts read once.
   if (pageable && n_seg * n * 4 >= kStagedRead) {
+    std::lock_guard<std::mutex> lk(c->read_mu);
     if (c->large_reads++ == 1) c->read_stage = dh::read_stage_create(c->stream);
     if (c->read_stage) {
       HIPCHK(c, dh::read_stage_read(c->read_stage, src, dst, n_seg, (uint32_t)n, c->stream));

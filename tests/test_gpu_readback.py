@@ -2,6 +2,7 @@
 1 MB where it starts, pixel counts that are no multiple of four, fewer and more chunks than the ring holds,
 one, two and three buffers, changing from read to read.  The arrays equal the device buffers copied directly."""
 import ctypes as C
+import threading
 
 import numpy as np
 import pytest
@@ -31,5 +32,32 @@ def test_staged_reads(W, H):
             assert np.array_equal(f.ravel(), want[0])
             assert d is None or np.array_equal(d.ravel().view(np.uint32), want[1].view(np.uint32))
             assert w is None or np.array_equal(w.ravel(), want[2])
+    finally:
+        r.close()
+
+
+def test_threads_reading_one_context():
+    W, H = 900, 700
+    r = Renderer(0)
+    try:
+        s = workloads.torus_scene(3, W, H)
+        cv = r.render_device(s, frame_uniforms(s), r.mesh_handles(s))
+        want, depth = np.zeros((H, W, 4), np.uint8), np.zeros((H, W), np.float32)
+        r.read_into(cv, want, depth)
+        bad = []
+
+        def reader():
+            for _ in range(20):
+                f, d = np.zeros_like(want), np.zeros_like(depth)
+                r.read_into(cv, f, d)
+                if not (np.array_equal(f, want) and np.array_equal(d, depth)):
+                    bad.append(1)
+
+        ts = [threading.Thread(target=reader) for _ in range(3)]
+        for t in ts:
+            t.start()
+        for t in ts:
+            t.join()
+        assert not bad
     finally:
         r.close()
