@@ -308,10 +308,13 @@ int ensure_scratch(dh_ctx c, uint32_t n_in, uint32_t cap_tri, uint32_t cap_pairs
     c->draws = reinterpret_cast<dh::DevDraw*>(c->tables.p);
     c->views = reinterpret_cast<dh::DevView*>(c->tables.p + c->tables_view_off);
   }
-  c->cap_tri = (uint32_t)std::min<size_t>(c->setup.n, 0xFFFFFFF0u);
-  c->cap_pairs = (uint32_t)std::min<size_t>(c->vals0.n, 0xFFFFFFF0u);
-  // binning keeps the wide-triangle list (up to cap_tri entries) in keys[1] or vals[1]
-  if (c->cap_pairs < c->cap_tri) return fail(c, DH_E_CAPACITY, "bin buffers smaller than the triangle records");
+  // What every buffer of a group holds: one whose growth failed in an earlier
+  // frame has been freed and is now smaller than its fellows.  Binning keeps the
+  // wide-triangle list (up to cap_tri entries) in keys[1] or vals[1].
+  const size_t pairs = std::min({c->keys.n / 2, c->vals0.n, c->vals1.n});
+  const size_t tri = std::min({c->setup.n, c->shade.n, c->bincnt.n, c->binoff.n, (c->big.n - 4) / 3, pairs});
+  c->cap_tri = (uint32_t)std::min<size_t>(tri, 0xFFFFFFF0u);
+  c->cap_pairs = (uint32_t)std::min<size_t>(pairs, 0xFFFFFFF0u);
   return DH_OK;
 }
 

@@ -1,0 +1,110 @@
+"""The library's host code without a device, on a stand-in for the HIP runtime (standin_hip.c): what it hands to
+the kernels after an allocation failed."""
+import os
+import subprocess
+import sys
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+ROOT = os.path.dirname(HERE)
+
+PRELUDE = """
+import ctypes as C, sys
+sys.path.insert(0, {root!r})
+S = C.CDLL({so!r}, mode=C.RTLD_GLOBAL)
+S.standin_room.argtypes, S.standin_room.restype = [C.c_uint64], C.c_int64
+S.standin_fail_alloc.argtypes = [C.c_long]
+S.standin_launches.restype = C.c_long
+S.standin_launch_name.argtypes, S.standin_launch_name.restype = [C.c_long], C.c_char_p
+S.standin_launch_arg.argtypes, S.standin_launch_arg.restype = [C.c_long, C.c_int], C.c_uint64
+S.standin_queries.restype = C.c_uint64
+S.standin_hold_array.argtypes, S.standin_hold_array.restype = [C.c_size_t, C.c_double], C.c_void_p
+import numpy as np
+from draw_amd import workloads
+from draw_amd._lib import DrawHipError
+from draw_amd.render import Renderer, frame_uniforms
+"""
+
+
+@pytest.fixture(scope="module")
+def standin(tmp_path_factory):
+    so = tmp_path_factory.mktemp("standin") / "libstandin.so"
+    subprocess.run(["gcc", "-O1", "-shared", "-fPIC", os.path.join(HERE, "standin_hip.c"), "-o", str(so)], check=True)
+    return str(so)
+
+
+def run(standin, body, timeout=100):
+    r = subprocess.run([sys.executable, "-c", PRELUDE.format(root=ROOT, so=standin) + body], capture_output=True,
+                       text=True, timeout=timeout, cwd=ROOT)
+    assert r.returncode == 0, r.stdout + r.stderr
+    return r.stdout
+
+
+# A frame, a larger one one of whose allocations fails (each in turn), then one of a size between: its kernels must
+# get no capacity beyond the end of any buffer.
+CAPACITIES = """
+def lim32(x):
+    return x & 0xFFFFFFFF
+
+# kernel -> [(pointer argument, bytes it must have, as a function of the arguments)]
+def boxes(cap):
+    return ((cap + 15) & ~15) + 8 * cap
+CHECKS = {
+    "k_geom_emit": [(6, lambda a: 96 * a(8)), (7, lambda a: 144 * a(8)), (11, lambda a: 4 * a(8)),
+                    (12, lambda a: boxes(a(8))), (13, lambda a: 4 * a(8))],
+    "k_pair_hist": [(0, lambda a: boxes(a(5))), (1, lambda a: 4 * a(5)), (2, lambda a: 96 * a(5))],
+    "k_pair_scatter": [(0, lambda a: boxes(a(5))), (10, lambda a: 8 * a(9))],
+    "k_pair_sort": [(0, lambda a: 8 * a(2)), (4, lambda a: 4 * a(2)), (5, lambda a: 8 * a(3)), (6, lambda a: 4 * a(2))],
+    "k_bin_small": [(0, lambda a: 96 * a(3)), (5, lambda a: boxes(a(3))), (6, lambda a: 4 * a(3)), (9, lambda a: 4 * a(8))],
+    "k_bin_emitILb": [(0, lambda a: 96 * a(3)), (6, lambda a: 4 * a(3)), (10, lambda a: 4 * a(9)), (11, lambda a: 4 * a(9))],
+    "k_bin_emit_wide": [(9, lambda a: 4 * a(8)), (10, lambda a: 4 * a(8))],
+    "k_radix_hist": [(0, lambda a: 4 * a(2))],
+    "k_radix_scatter": [(i, lambda a: 4 * a(5)) for i in range(4)],
+}
+seen = set()
+def check(label):
+    for i in range(S.standin_launches(0)):
+        name = S.standin_launch_name(i).decode()
+        for k, rules in CHECKS.items():
+            if k not in name:
+                continue
+            seen.add(k)
+            for arg, need in rules:
+                p, n = S.standin_launch_arg(i, arg), need(lambda j: lim32(S.standin_launch_arg(i, j)))
+                if p:
+                    room = S.standin_room(p)
+                    assert room >= n, f"{label}: {name} argument {arg} needs {n} bytes, its buffer has {room}"
+
+def render(r, n_tri):
+    s = workloads.soup_scene(1, n_tri, 640, 480, 16)
+    return r.render_device(s)
+
+for bins in (1, 2):
+    failed = 0
+    for k in range(64):
+        r = Renderer(0)
+        r.set_bin_order(bins)
+        render(r, 500)
+        s = workloads.soup_scene(1, 60_000, 640, 480, 16)  # its resources first: the frame's own allocations are to fail
+        fr, hs = frame_uniforms(s), r.mesh_handles(s)
+        S.standin_fail_alloc(k)
+        try:
+            r.render_device(s, fr, hs)
+        except DrawHipError:
+            failed += 1
+        S.standin_fail_alloc(-1)
+        S.standin_launches(1)
+        render(r, 9_000)
+        check(f"bins {bins}, allocation {k} failed")
+        n = failed
+        r.close()
+        if n <= k:
+            break
+    assert failed >= 10, failed
+assert seen == set(CHECKS) - {"k_bin_small"}, seen
+"""
+
+
+def test_capacities_after_a_failed_allocation(standin):
+    run(standin, CAPACITIES)
