@@ -111,15 +111,16 @@ struct ReadStage {
       w += e;
     }
   }
-  // Takes chunks until none is left.  While a chunk's flag is down, waiting(spin)
-  // is called; the read ends for all threads when one returns false.
+  // Takes chunks until none is left.  While chunk c's flag is down, waiting(c,
+  // spin) is called; the read ends for all threads when one returns false.
+  bool flag_up(uint32_t c) const {
+    return __atomic_load_n(flags + c % (2u * kHalfChunks), __ATOMIC_ACQUIRE) == ticket + c / kHalfChunks;
+  }
   template <class Waiting>
   void work(Waiting waiting) {
     for (uint32_t c; !stop.load() && (c = next.fetch_add(1)) < chunks;) {
-      const uint32_t* f = flags + c % (2u * kHalfChunks);
-      const uint32_t want = ticket + c / kHalfChunks;
-      for (uint32_t spin = 1; __atomic_load_n(f, __ATOMIC_ACQUIRE) != want; spin++) {
-        if (stop.load() || !waiting(spin)) {
+      for (uint32_t spin = 1; !flag_up(c); spin++) {
+        if (stop.load() || !waiting(c, spin)) {
           stop.store(true);
           return;
         }
@@ -139,7 +140,7 @@ struct ReadStage {
       seen = reads;
       inside++;
       lk.unlock();
-      work([](uint32_t) { return true; });
+      work([](uint32_t, uint32_t) { return true; });
       lk.lock();
       if (--inside == 0) left.notify_all();
     }
@@ -226,21 +227,28 @@ hipError_t read_stage_read(ReadStage* st, const void* const* src, void* const* d
   }
   st->wake.notify_all();
   e = st->launch_next(s);
-  auto waiting = [&](uint32_t spin) {
-    if (e != hipSuccess) return false;
-    const uint32_t before = st->launched;
-    if ((e = st->launch_next(s)) != hipSuccess) return false;
-    if (spin % 4096u || before != st->launched) return true;
-    // all launched parts written, and yet nothing for seconds: they never will be
+  // Launches what can be; now and then asks whether the device has failed, or
+  // has run all it was given and chunk c of it has no flag.
+  bool idle = false;  // every part has been written
+  auto waiting = [&](uint32_t c, uint32_t spin) {
+    if (e == hipSuccess) e = st->launch_next(s);
+    if (e != hipSuccess || spin % 4096u) return e == hipSuccess;
     const hipError_t q = hipStreamQuery(s);
-    if (q != hipSuccess && q != hipErrorNotReady) e = q;
-    if (q == hipErrorNotReady) (void)hipGetLastError();
-    if (q == hipSuccess && spin > (1u << 26)) e = hipErrorUnknown;
+    if (q == hipErrorNotReady) {
+      (void)hipGetLastError();
+      std::this_thread::yield();
+      return true;
+    }
+    idle = st->launched == st->parts;
+    if (q != hipSuccess) e = q;
+    else if (c / kHalfChunks < st->launched && !st->flag_up(c)) e = hipErrorUnknown;
     return e == hipSuccess;
   };
   st->work(waiting);
-  for (uint32_t spin = 1; st->done.load() < st->chunks && !st->stop.load(); spin++) {
-    if (!waiting(spin)) st->stop.store(true);
+  // The other chunks are the helpers', however long they take: once their flags
+  // are all up there is nothing left to do for them here.
+  for (uint32_t spin = 1; st->done.load() < st->chunks && !st->stop.load() && !idle; spin++) {
+    if (!waiting(~0u, spin)) st->stop.store(true);
     _mm_pause();
   }
   {

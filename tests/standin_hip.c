@@ -189,6 +189,9 @@ int __hipPopCallConfiguration(Dim3* grid, Dim3* block, size_t* lds, void** strea
   return 0;
 }
 
+static int g_no_reads; /* k_read_out does nothing, as on a device that stopped */
+void standin_no_reads(int on) { g_no_reads = on; }
+
 /* k_read_out: see its definition for the arguments */
 static void read_out(void** a) {
   const struct {
@@ -211,7 +214,7 @@ int hipLaunchKernel(const void* f, Dim3 grid, Dim3 block, void** args, size_t ld
   const char* name = "?";
   for (int i = 0; i < g_kernels; i++)
     if (g_kernel[i].host == f) name = g_kernel[i].name;
-  if (strstr(name, "k_read_out")) read_out(args);
+  if (strstr(name, "k_read_out") && !g_no_reads) read_out(args);
   if (g_launches < kMaxLaunches) {
     g_launch[g_launches].name = name;
     for (size_t k = 0; k < sizeof kArgs / sizeof *kArgs; k++)

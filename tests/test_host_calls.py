@@ -1,5 +1,5 @@
 """The library's host code without a device, on a stand-in for the HIP runtime (standin_hip.c): what it hands to
-the kernels after an allocation failed."""
+the kernels after an allocation failed, and large canvas reads whose helper threads are late."""
 import os
 import subprocess
 import sys
@@ -108,3 +108,39 @@ assert seen == set(CHECKS) - {"k_bin_small"}, seen
 
 def test_capacities_after_a_failed_allocation(standin):
     run(standin, CAPACITIES)
+
+
+# A helper thread that is not given the processor in the middle of its copy delays the read and does not fail it;
+# a device that stops raising flags does.
+LATE_HELPER = """
+W, H = 1280, 720
+r = Renderer(0)
+cv = r.canvas(W, H)
+p = [C.c_void_p() for _ in range(3)]
+r._check(r.L.dh_canvas_device_ptrs(r.ctx, cv, *(C.byref(q) for q in p)), "dh_canvas_device_ptrs")
+want = np.random.default_rng(1).integers(0, 256, 4 * W * H, np.uint8)
+C.memmove(p[0].value, want.ctypes.data, want.nbytes)
+f, d = np.zeros((H, W, 4), np.uint8), np.zeros((H, W), np.float32)
+for _ in range(3):
+    r.read_into(cv, f, d)
+assert np.array_equal(f.ravel(), want)
+at = S.standin_hold_array(4 * W * H, 3.0)
+r._check(r.L.dh_canvas_read(r.ctx, cv, at, d.ctypes.data, None), "dh_canvas_read")
+assert S.standin_holds() > 0
+assert C.string_at(at, 4 * W * H) == want.tobytes()
+S.standin_no_reads(1)
+try:
+    r.read_into(cv, f, d)
+    raise SystemExit("a read that the device never did")
+except DrawHipError:
+    pass
+S.standin_no_reads(0)
+f[...] = 0
+r.read_into(cv, f, d)
+assert np.array_equal(f.ravel(), want)
+r.close()
+"""
+
+
+def test_a_late_helper_does_not_fail_a_read(standin):
+    run(standin, LATE_HELPER)
