@@ -488,14 +488,28 @@ __device__ inline void make_setup(const FrameParamsPod& fr, const FV& A, const F
   };
   const bool exact = isfinite(R) && exact_edge(ea) && exact_edge(eb) && exact_edge(eg);
   if (exact && __float_as_uint(fa) == 0u && __float_as_uint(fb) == 0u && __float_as_uint(fg) == 0u) flags |= kDrop;
-  // Texture-index safety.  With `exact`, a covered pixel has e_i / f >= 0 and
-  // sum e_i / f = 1, so alpha + beta + gama <= 1 + 2^-24 after rounding; with
-  // all six uv in [0,1] the interpolated u, v lie in [0, 1 + 5*2^-24], and for
-  // maps of at most 16384 texels per side floor(u*(w-1)) <= w-1 and
-  // floor(v*(h-1)) <= h-1: get_rgb_slice (scene/mod.rs:154-168) stays in range.
-  auto unit = [](float t) { return t >= 0.0f && t <= 1.0f; };
-  if ((flags & kFast) && exact && unit(A.u) && unit(A.v) && unit(B.u) && unit(B.v) && unit(C.u) && unit(C.v) &&
-      mat.kd_w <= 16384 && mat.kd_h <= 16384 && mat.ka_w <= 16384 && mat.ka_h <= 16384)
+  // Texture-index safety: no covered pixel reads outside its maps.  With `exact`
+  // its weights are e_i / f >= 0 and sum to 1, so the interpolated u lies within
+  // the vertices' range and the roundings of the weights, products and sums,
+  // ((1 + 2^-24)^4 - 1) sum |u_i| e_i / f <= 2.4e-7 K with K >= every |u_i|.
+  // get_rgb_slice (scene/mod.rs:154-168) takes a negative coordinate for 0.  Its
+  // row floor(v (h - 1)) from the bottom exists while v <= 1 + 1 / (h - 1) -
+  // 1.2e-7, and its texel floor(u (w - 1)) may run on into the r rows below,
+  // r >= floor(v (h - 1)) - 1 (a row for the roundings): u (w - 1) < w (1 + r).
+  // (Records that are not safe are visited one at a time with every lane's
+  // texture index checked.  While only [0, 1] counted as safe, meshes with
+  // coordinates from -0.5 to 0.5 took 206 us for 500k triangles at 1080p and 365
+  // for a 150k soup at 720p; now 123 and 161.)
+  auto in_map = [&](int32_t w, int32_t h) {
+    const float mu = (float)w - 1.0f, mv = (float)h - 1.0f;
+    const float eu = 2.4e-7f * ((fabsf(A.u) + fabsf(B.u)) + fabsf(C.u)) + 1.3e-7f;  // NaN and infinite ones fail below
+    const float ev = 2.4e-7f * ((fabsf(A.v) + fabsf(B.v)) + fabsf(C.v)) + 1.3e-7f;
+    const float u1 = fmaxf(fmaxf(A.u, B.u), C.u), v1 = fmaxf(fmaxf(A.v, B.v), C.v), v0 = fminf(fminf(A.v, B.v), C.v);
+    const float rows = fmaxf(floorf((v0 - ev) * mv) - 1.0f, 0.0f);
+    return ((v1 - 1.0f) + ev) * mv < 0.999f && ((u1 - 1.0f) + eu) * mu < 0.999f * (1.0f + rows * (float)w);
+  };
+  if ((flags & kFast) && exact && max(max(mat.kd_w, mat.kd_h), max(mat.ka_w, mat.ka_h)) <= (1 << 20) &&
+      in_map(mat.kd_w, mat.kd_h) && in_map(mat.ka_w, mat.ka_h))
     flags |= kUvSafe;
   // Depth lower bound for early rejection.  For a UV-safe triangle (exact
   // edge arithmetic) a covered pixel has alpha + beta + gama >= 1 - 2^-24 with
