@@ -66,21 +66,23 @@ __device__ inline V3 ld3(const float* a, uint32_t i) {
   return v3(p[0], p[1], p[2]);
 }
 
-// Runs f(draw index, mine) for each draw among the active lanes' d, mine the
-// lanes that have it, the index wave-uniform: the draw, its view's uniforms and
-// its material come by scalar loads (every lane calls it; one round unless the
-// wave's triangles straddle draws).  Per lane, they were some 60 vector loads of
-// one address each (with global in place of FLAT accesses, 5M micro-triangles:
-// k_geom_emit 172 -> 128 us, k_geom_count 68 -> 53; the 32-view batch 96 -> 87
-// and 37 -> 29).
+// Runs f(draw index) for the active lanes of a wave, d their draws (every lane
+// calls it).  A wave of one draw, as most are, gets the index wave-uniform: the
+// draw, its view's uniforms and its material come by scalar loads.  Per lane,
+// they were some 60 vector loads of one address each (with global in place of
+// FLAT accesses, 5M micro-triangles: k_geom_emit 172 -> 128 us, k_geom_count 68
+// -> 53; the 32-view batch 96 -> 87 and 37 -> 29).  A wave of several draws does
+// load per lane: going round once for each draw cost 1000 meshes of two
+// triangles, 32 rounds a wave, 147 us of geometry kernels (59 per lane).
 template <class F>
-__device__ __forceinline__ void for_each_draw(uint32_t d, bool active, F f) {
-  for (uint64_t todo = __ballot(active); todo;) {
-    const uint32_t d0 = (uint32_t)__builtin_amdgcn_readlane((int)d, __builtin_ctzll(todo));
-    const bool mine = active && d == d0;
-    todo &= ~__ballot(mine);
-    f(d0, mine);
-  }
+__device__ __forceinline__ void by_draw(uint32_t d, bool active, F f) {
+  const uint64_t m = __ballot(active);
+  if (!m) return;
+  const uint32_t d0 = (uint32_t)__builtin_amdgcn_readlane((int)d, __builtin_ctzll(m));
+  const bool one = __ballot(active && d != d0) == 0ull;
+  if (!active) return;
+  if (one) f(d0);
+  else f(d);
 }
 
 // Vertex positions of a draw's triangle lt (a, b, c): from the mesh's
@@ -958,10 +960,9 @@ __global__ __launch_bounds__(256) void k_geom_count(const DevDraw* __restrict__ 
   uint32_t c = 0;
   bool clip = false;
   const uint32_t d = wave_find_draw(draws, n_draws, t, t < n_in);
-  for_each_draw(d, t < n_in, [&](uint32_t d0, bool mine) {
-    const DevDraw& dr = draws[d0];
+  by_draw(d, t < n_in, [&](uint32_t di) {
+    const DevDraw& dr = draws[di];
     const FrameParamsPod& fr = views[dr.view].fr;
-    if (!mine) return;
     PV a, b, cc;
     tri_positions(dr, t - dr.tri_begin, a.p, b.p, cc.p);
     c = (uint32_t)cull_and_clip(fr, a, b, cc, !(dr.flags & kDrawNoCull), [](int, const PV&, const PV&, const PV&) {});
@@ -1026,10 +1027,9 @@ __global__ __launch_bounds__(1024) void k_geom_small(const DevDraw* __restrict__
     uint32_t c = 0;
     bool clip = false;
     const uint32_t d = wave_find_draw(draws, n_draws, t, t < n_in);
-    for_each_draw(d, t < n_in, [&](uint32_t d0, bool mine) {
-      const DevDraw& dr = draws[d0];
+    by_draw(d, t < n_in, [&](uint32_t di) {
+      const DevDraw& dr = draws[di];
       const FrameParamsPod& fr = views[dr.view].fr;
-      if (!mine) return;
       PV a, b, cc;
       tri_positions(dr, t - dr.tri_begin, a.p, b.p, cc.p);
       c = (uint32_t)cull_and_clip(fr, a, b, cc, !(dr.flags & kDrawNoCull),
@@ -1171,8 +1171,7 @@ __device__ __forceinline__ void geom_emit_one(uint2 sv, bool active, bool clip, 
     wave_store<6>(stage, ro, ok, idx, reinterpret_cast<uint4*>(setup), skip);
     wave_store<9>(stage, so, ok, idx, reinterpret_cast<uint4*>(shade), skip);
   };
-  // one draw: scalar loads (for_each_draw); several: per lane, since a second
-  // round would double the launch's longest wave
+  // (as by_draw, but with every lane of the wave in the record stores)
   const uint64_t m = __ballot(active);
   if (!m) return;
   const uint32_t d0 = (uint32_t)__builtin_amdgcn_readlane((int)d, __builtin_ctzll(m));
