@@ -166,8 +166,8 @@ struct dh_ctx_s {
   DevBuf<uint32_t> tperm;     // the triangles being sorted (TransArgs::perm_tmp)
   DevBuf<uint32_t> sort_n;    // [1]
   std::mutex read_mu;  // threads reading canvases of one context take turns on
-  dh::ReadStage* read_stage = nullptr;  // large canvas reads (made for the second one)
-  uint64_t large_reads = 0;
+  dh::ReadStage* read_stage = nullptr;  // large canvas reads
+  uint64_t read_due = 0;                // bytes of them that would have gained from it
   dh_stats stats = {};
   // captured batch launch (DH_BATCH_GRAPH)
   hipGraph_t graph = nullptr;
@@ -1148,9 +1148,13 @@ int find_canvas(dh_ctx c, dh_handle canvas, CanvasRes* out) {
 }  // namespace
 
 namespace {
-// Where the staging ring starts to pay (us, the runtime's copy -> the ring):
-// 0.96 MB 59 (kept), 2.5 MB 160 -> 90, 7.4 MB 445 -> 190.
-constexpr uint64_t kStagedRead = 1u << 20;
+// Where the staging ring starts to pay (us, the runtime's copy -> through the
+// ring): 0.96 MB 59 (kept), 1.4 MB 83 -> 74, 2.5 MB 170 -> 102, 7.4 MB 436 -> 203,
+// 66 MB 3850 -> 1580.  A context's first read through it takes some 80 us more,
+// so it is made once the reads, this one included, have had kStageAfter bytes
+// beyond kStagedRead each that it would have sped up by as much: at the first
+// one of 2.4 MB (175 -> 187 us) or more (7.4 MB 450 -> 330, 66 MB 4.1 -> 2.0 ms).
+constexpr uint64_t kStagedRead = 1u << 20, kStageAfter = 5u << 18;
 }  // namespace
 
 extern "C" int dh_canvas_read(dh_ctx c, dh_handle canvas, uint8_t* bgra, float* depth, uint32_t* winner) {
@@ -1178,12 +1182,10 @@ extern "C" int dh_canvas_read(dh_ctx c, dh_handle canvas, uint8_t* bgra, float* 
   seg(cv.bgra, bgra);
   seg(cv.depth, depth);
   seg(cv.winner, winner);
-  // From kStagedRead bytes on, through the context's staging.  It is made for
-  // the second such read: the first would pay more for it than it saves, and
-  // many contexts read once.
-  if (pageable && n_seg * n * 4 >= kStagedRead) {
+  const uint64_t bytes = n_seg * n * 4;
+  if (pageable && bytes >= kStagedRead) {
     std::lock_guard<std::mutex> lk(c->read_mu);
-    if (c->large_reads++ == 1) c->read_stage = dh::read_stage_create(c->stream);
+    if (!c->read_stage && (c->read_due += bytes - kStagedRead) >= kStageAfter) c->read_stage = dh::read_stage_create();
     if (c->read_stage) {
       HIPCHK(c, dh::read_stage_read(c->read_stage, src, dst, n_seg, (uint32_t)n, c->stream));
       return DH_OK;
@@ -1392,6 +1394,11 @@ void ctx_release_scratch(dh_ctx c) {
   c->status.release(); c->tables.release(); c->draws = nullptr; c->views = nullptr; c->export_buf.release();
   c->grp.release(); c->tperm.release(); c->sort_n.release();
   release_gui(c);
+  {
+    std::lock_guard<std::mutex> lk(c->read_mu);
+    dh::read_stage_destroy(c->read_stage);
+    c->read_stage = nullptr;
+  }
   c->cap_tri = c->cap_pairs = 0;
 }
 }  // namespace dh

@@ -33,7 +33,7 @@ constexpr size_t kGuiRecBytes = 152;  // a 144-byte record and an 8-byte scan re
 // Large reads of canvas buffers into pageable memory (dh_readback.hip): n_seg (at
 // most 3) buffers of n_words words each.  Null from create: not available.
 struct ReadStage;
-ReadStage* read_stage_create(hipStream_t s);
+ReadStage* read_stage_create();
 void read_stage_destroy(ReadStage* st);
 hipError_t read_stage_read(ReadStage* st, const void* const* src, void* const* dst, uint32_t n_seg, uint32_t n_words,
                            hipStream_t s);

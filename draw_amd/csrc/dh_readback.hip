@@ -1,11 +1,11 @@
 // dh_readback.hip -- canvas buffers into a caller's pageable arrays.
 //
-// One kernel writes the buffers into pinned staging in 256 KB chunks and raises
-// a flag in host memory for each; the calling thread and a few helpers copy a
-// chunk out as soon as its flag is up, while the kernel writes the next ones.
+// A kernel writes the buffers into pinned staging in 64 KB chunks and raises a
+// flag in host memory for each; the calling thread and a few helpers copy a
+// chunk out as soon as its flag is up, while the device writes the next ones.
 // A runtime copy to pageable memory stages through pinned memory as well, but
 // one thread copies out, at 18 GB/s: that bounded it (1280x720 frame and depth,
-// 7.4 MB: 445 -> 190 us; 640x480 160 -> 90; 4K 3845 -> 1538; PCIe alone some 140,
+// 7.4 MB: 436 -> 203 us; 640x480 170 -> 102; 4K 3850 -> 1580; PCIe alone some 140,
 // 46 and 1250).
 #if !defined(__HIP_DEVICE_COMPILE__)
 #include <immintrin.h>
@@ -26,10 +26,11 @@
 namespace dh {
 
 namespace {
-constexpr uint32_t kChunkWords = 16384;              // 16-byte words: 256 KB
-constexpr uint32_t kBlockWords = 4096;               // four blocks a chunk
-constexpr uint32_t kHalfChunks = 8;                  // chunks of a staging half (2 MB)
-constexpr uint32_t kHalfWords = kChunkWords * kHalfChunks;
+constexpr uint32_t kChunkWords = 4096;  // 16-byte words: 64 KB, a workgroup's
+constexpr uint32_t kPartChunks = 15;    // chunks of a part, which one piece of staging holds
+constexpr uint32_t kPartWords = kChunkWords * kPartChunks;
+constexpr size_t kPieceBytes = 16ull * kPartWords + 4096;  // and its chunks' flags
+constexpr uint32_t kPieces = 4;
 constexpr int kHelpers = 3;
 constexpr int kMaxSegs = 3;
 
@@ -40,11 +41,19 @@ struct ReadSegs {
 };
 
 // Words [w0, w0 + n) of the segments laid end to end (each padded to 16 bytes)
-// into stage; per finished chunk its flag, by the chunk's last block.  PCIe
-// bounds it.
-__global__ __launch_bounds__(256) void k_read_out(ReadSegs g, uint64_t w0, uint32_t n, uint4* __restrict__ stage,
-                                                  uint32_t* __restrict__ counters, uint32_t* flags, uint32_t ticket) {
-  const uint32_t b0 = blockIdx.x * kBlockWords, b1 = min(b0 + kBlockWords, n);
+// into the staging of one part or two, a chunk per block, and then the chunk's
+// flag, the part's ticket.  PCIe bounds it.
+struct ReadParts {
+  uint4* stage[2];
+  uint32_t* flags[2];
+  uint32_t ticket;  // the first part's; the second's follows
+};
+__global__ __launch_bounds__(256) void k_read_out(ReadSegs g, uint64_t w0, uint32_t n, ReadParts parts) {
+  const uint32_t k = blockIdx.x < kPartChunks ? 0u : 1u, c = blockIdx.x - k * kPartChunks;
+  uint4* const stage = parts.stage[k];
+  w0 += k * kPartWords;
+  n -= k * kPartWords;
+  const uint32_t b0 = c * kChunkWords, b1 = min(b0 + kChunkWords, n);
   for (uint32_t i = b0 + threadIdx.x; i < b1; i += 256u) {
     const uint64_t w = w0 + i;
     const uint64_t w1 = g.n_words16, w2 = 2ull * g.n_words16;
@@ -62,34 +71,35 @@ __global__ __launch_bounds__(256) void k_read_out(ReadSegs g, uint64_t w0, uint3
   }
   __threadfence_system();
   __syncthreads();
-  if (threadIdx.x == 0) {
-    const uint32_t c = b0 / kChunkWords;
-    const uint32_t blocks = (min(kChunkWords, n - c * kChunkWords) + kBlockWords - 1u) / kBlockWords;
-    if (atomicAdd(&counters[c], 1u) + 1u == blocks) {
-      counters[c] = 0u;  // for the next launch
-      __threadfence_system();
-      __hip_atomic_store(&flags[c], ticket, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
-    }
-  }
+  if (threadIdx.x == 0)
+    __hip_atomic_store(&parts.flags[k][c], parts.ticket + k, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 }  // namespace
 
-// A context's staging, a ring of two parts of kHalfChunks chunks, and its helper
-// threads, which sleep between reads.
+// A context's staging and its helper threads, which sleep between reads.  The
+// staging is a ring of pieces, allocated as the reads come (pinned pieces of up
+// to 1 MB take some 40 us each, one of 2 or 4 MB 110 to 740): one before the
+// first read starts, a second behind its first part, two more during the next
+// read.  With all four a launch writes two parts (a launch costs some 5 us of
+// PCIe time, a part takes 19).
 struct ReadStage {
-  uint4* stage = nullptr;        // [2 * kHalfWords], pinned
-  uint4* stage_dev = nullptr;
-  uint32_t* flags = nullptr;     // [2 * kHalfChunks], pinned and coherent: the ticket of the part last written
-  uint32_t* flags_dev = nullptr;
-  uint32_t* counters = nullptr;  // [2 * kHalfChunks], device, zero between launches
+  struct Piece {
+    uint4* stage = nullptr;  // [kPartWords], pinned and coherent, then the chunks' flags: the ticket last written
+    uint4* dev = nullptr;
+    uint32_t* flags() const { return reinterpret_cast<uint32_t*>(stage + kPartWords); }
+    uint32_t* flags_dev() const { return reinterpret_cast<uint32_t*>(dev + kPartWords); }
+  };
+  Piece piece[kPieces];
+  uint32_t n_piece = 0;
   uint32_t ticket = 0, next_ticket = 1;  // part p of a read has ticket + p
 
   // the read under way
   ReadSegs segs{};
   uint8_t* dst[kMaxSegs] = {};
   uint64_t words = 0;
+  uint32_t ring = 0;  // pieces it uses: part p is in piece p % ring
   uint32_t chunks = 0, parts = 0, launched = 0;
-  std::atomic<uint32_t> next{0}, done{0}, done_of[2];  // chunks handed out; copied: in all, of the part in each half
+  std::atomic<uint32_t> next{0}, done{0}, done_of[kPieces];  // chunks handed out; copied: in all, of the part in each piece
   std::atomic<bool> stop{false};
 
   std::mutex mu;
@@ -99,11 +109,24 @@ struct ReadStage {
   bool open = false, quit = false;
   std::vector<std::thread> helpers;
 
-  uint32_t chunks_of(uint32_t p) const { return std::min(kHalfChunks, chunks - p * kHalfChunks); }
-
+  const Piece& piece_of(uint32_t p) const { return piece[p % ring]; }
+  uint32_t chunks_of(uint32_t p) const { return std::min(kPartChunks, chunks - p * kPartChunks); }
+  bool add_piece() {
+    Piece& h = piece[n_piece];
+    hipError_t e = hipSuccess;
+    if (!h.stage) e = hipHostMalloc(reinterpret_cast<void**>(&h.stage), kPieceBytes, hipHostMallocCoherent);
+    if (e == hipSuccess) e = hipHostGetDevicePointer(reinterpret_cast<void**>(&h.dev), h.stage, 0);
+    if (e != hipSuccess) {
+      (void)hipGetLastError();
+      return false;
+    }
+    memset(h.flags(), 0, 4u * kPartChunks);
+    n_piece++;
+    return true;
+  }
   void copy_chunk(uint32_t c) {
     const uint64_t a = (uint64_t)c * kChunkWords, b = std::min<uint64_t>(a + kChunkWords, words);
-    const uint8_t* from = reinterpret_cast<const uint8_t*>(stage + a % (2ull * kHalfWords));
+    const uint8_t* from = reinterpret_cast<const uint8_t*>(piece_of(c / kPartChunks).stage + a % kPartWords);
     for (uint64_t w = a; w < b;) {
       const uint64_t s = w / segs.n_words16, r = w - s * segs.n_words16;
       const uint64_t e = std::min<uint64_t>(b - w, segs.n_words16 - r);
@@ -114,7 +137,8 @@ struct ReadStage {
   // Takes chunks until none is left.  While chunk c's flag is down, waiting(c,
   // spin) is called; the read ends for all threads when one returns false.
   bool flag_up(uint32_t c) const {
-    return __atomic_load_n(flags + c % (2u * kHalfChunks), __ATOMIC_ACQUIRE) == ticket + c / kHalfChunks;
+    const uint32_t p = c / kPartChunks;
+    return __atomic_load_n(piece_of(p).flags() + c % kPartChunks, __ATOMIC_ACQUIRE) == ticket + p;
   }
   template <class Waiting>
   void work(Waiting waiting) {
@@ -127,7 +151,7 @@ struct ReadStage {
         _mm_pause();
       }
       copy_chunk(c);
-      done_of[c / kHalfChunks & 1u].fetch_add(1);
+      done_of[c / kPartChunks % ring].fetch_add(1);
       done.fetch_add(1);
     }
   }
@@ -145,18 +169,27 @@ struct ReadStage {
       if (--inside == 0) left.notify_all();
     }
   }
-  // Launches the next part if its half of the staging is free.
+  // Launches the next part, or two, if their staging is free.
   hipError_t launch_next(hipStream_t s) {
-    if (launched == parts) return hipSuccess;
-    const uint32_t p = launched, h = p & 1u;
-    if (p >= 2u && done_of[h].load() != chunks_of(p - 2u)) return hipSuccess;
-    done_of[h].store(0);
-    const uint64_t w0 = (uint64_t)p * kHalfWords;
-    const uint32_t n = (uint32_t)std::min<uint64_t>(kHalfWords, words - w0);
-    hipLaunchKernelGGL(k_read_out, dim3((n + kBlockWords - 1u) / kBlockWords), dim3(256), 0, s, segs, w0, n,
-                       stage_dev + (size_t)h * kHalfWords, counters + h * kHalfChunks, flags_dev + h * kHalfChunks,
-                       ticket + p);
-    launched++;
+    const uint32_t p = launched, k = std::min(ring == kPieces ? 2u : 1u, parts - p);
+    if (k == 0u) return hipSuccess;
+    for (uint32_t j = p; j < p + k; j++)
+      if (j >= ring && done_of[j % ring].load() != chunks_of(j - ring)) return hipSuccess;
+    ReadParts rp;
+    rp.ticket = ticket + p;
+    uint32_t blocks = 0;
+    for (uint32_t j = 0; j < 2u; j++) {
+      const Piece& h = piece_of(p + (j < k ? j : 0u));
+      rp.stage[j] = h.dev;
+      rp.flags[j] = h.flags_dev();
+      if (j >= k) continue;
+      done_of[(p + j) % ring].store(0);
+      blocks += chunks_of(p + j);
+    }
+    const uint64_t w0 = (uint64_t)p * kPartWords;
+    const uint32_t n = (uint32_t)std::min<uint64_t>((uint64_t)k * kPartWords, words - w0);
+    hipLaunchKernelGGL(k_read_out, dim3(blocks), dim3(256), 0, s, segs, w0, n, rp);
+    launched += k;
     return hipGetLastError();
   }
 };
@@ -169,30 +202,14 @@ void read_stage_destroy(ReadStage* st) {
   }
   st->wake.notify_all();
   for (auto& t : st->helpers) t.join();
-  if (st->stage) (void)hipHostFree(st->stage);
-  if (st->flags) (void)hipHostFree(st->flags);
-  if (st->counters) (void)hipFree(st->counters);
+  for (auto& h : st->piece)
+    if (h.stage) (void)hipHostFree(h.stage);
   delete st;
 }
 
-ReadStage* read_stage_create(hipStream_t s) {
+ReadStage* read_stage_create() {
   ReadStage* st = new (std::nothrow) ReadStage;
-  if (!st) return nullptr;
-  const size_t fb = 2u * kHalfChunks * sizeof(uint32_t);
-  hipError_t e = hipHostMalloc(reinterpret_cast<void**>(&st->stage), 2ull * kHalfWords * 16u, hipHostMallocCoherent);
-  if (e == hipSuccess) e = hipHostGetDevicePointer(reinterpret_cast<void**>(&st->stage_dev), st->stage, 0);
-  if (e == hipSuccess) e = hipHostMalloc(reinterpret_cast<void**>(&st->flags), fb, hipHostMallocCoherent);
-  if (e == hipSuccess) e = hipHostGetDevicePointer(reinterpret_cast<void**>(&st->flags_dev), st->flags, 0);
-  if (e == hipSuccess) e = hipMalloc(reinterpret_cast<void**>(&st->counters), fb);
-  if (e == hipSuccess) e = hipMemsetAsync(st->counters, 0, fb, s);
-  if (e == hipSuccess) memset(st->flags, 0, fb);
-  try {
-    for (int k = 0; e == hipSuccess && k < kHelpers; k++) st->helpers.emplace_back([st] { st->helper(); });
-  } catch (...) {
-    e = hipErrorOutOfMemory;  // no thread: the caller reads the runtime's way
-  }
-  if (e != hipSuccess) {
-    (void)hipGetLastError();
+  if (st && !st->add_piece()) {
     read_stage_destroy(st);
     return nullptr;
   }
@@ -209,24 +226,34 @@ hipError_t read_stage_read(ReadStage* st, const void* const* src, void* const* d
   st->segs.n_words16 = n_words / 4u + (n_words % 4u ? 1u : 0u);
   st->words = (uint64_t)n_seg * st->segs.n_words16;
   st->chunks = (uint32_t)((st->words + kChunkWords - 1u) / kChunkWords);
-  st->parts = (st->chunks + kHalfChunks - 1u) / kHalfChunks;
+  st->parts = (st->chunks + kPartChunks - 1u) / kPartChunks;
   st->ticket = st->next_ticket;
   st->next_ticket += st->parts;
   st->launched = 0;
   st->next.store(0);
   st->done.store(0);
-  st->done_of[0].store(0);
-  st->done_of[1].store(0);
+  for (auto& d : st->done_of) d.store(0);
   st->stop.store(false);
+  st->ring = st->n_piece;
   hipError_t e = st->launch_next(s);
   if (e != hipSuccess) return e;
+  // behind the first part's writing: a second piece, the threads (without either
+  // the read takes longer)
+  if (st->n_piece == 1u && st->parts > 1u && st->add_piece()) st->ring = 2u;
+  e = st->launch_next(s);
+  try {
+    while (st->helpers.size() < (size_t)kHelpers) st->helpers.emplace_back([st] { st->helper(); });
+  } catch (...) {
+  }
   {
     std::lock_guard<std::mutex> lk(st->mu);
     st->reads++;
     st->open = true;
   }
   st->wake.notify_all();
-  e = st->launch_next(s);
+  // more staging for the reads to come
+  for (; st->reads > 1u && st->ring < kPieces && st->n_piece < kPieces && st->parts > st->ring;)
+    if (!st->add_piece()) break;
   // Launches what can be; now and then asks whether the device has failed, or
   // has run all it was given and chunk c of it has no flag.
   bool idle = false;  // every part has been written
@@ -241,7 +268,7 @@ hipError_t read_stage_read(ReadStage* st, const void* const* src, void* const* d
     }
     idle = st->launched == st->parts;
     if (q != hipSuccess) e = q;
-    else if (c / kHalfChunks < st->launched && !st->flag_up(c)) e = hipErrorUnknown;
+    else if (c / kPartChunks < st->launched && !st->flag_up(c)) e = hipErrorUnknown;
     return e == hipSuccess;
   };
   st->work(waiting);

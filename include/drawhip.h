@@ -253,7 +253,12 @@ int dh_device_read(dh_ctx ctx, void* host, const void* dev, uint64_t bytes);
 /* Copy a canvas to host memory: bgra W*H*4 bytes, rows top-down
  * (Canvas::as_bytes_slice, canvas.rs:974-978); depth W*H floats, rows
  * bottom-up (canvas.rs:415); winner W*H ids, rows bottom-up, 0xFFFFFFFF =
- * clear.  Any pointer may be NULL. */
+ * clear.  Any pointer may be NULL.  Reads of 1 MB and more into pageable
+ * memory go through a ring of the context's (up to 4 MB of pinned memory and
+ * three threads, made for its first read of 2.3 MB, or a later one of smaller
+ * ones, and kept until dh_ctx_destroy): the calling thread and those three
+ * spin while the device writes, and sleep between reads.  Reads of one context
+ * from several threads take turns. */
 int dh_canvas_read(dh_ctx ctx, dh_handle canvas, uint8_t* bgra, float* depth, uint32_t* winner);
 /* Frame export (App::export_frame_as, app/mod.rs:316-379): the canvas frame
  * with bytes 0 and 2 of every pixel swapped (BGRA -> RGBA, app/mod.rs:347-351)

@@ -26,7 +26,10 @@ static struct {
 } g_block[kMaxBlocks];
 static long g_fail_in = -1; /* device allocations until the one that fails; -1: none */
 
+static long g_host_left = -1; /* host allocations that succeed; -1: all */
+
 void standin_fail_alloc(long n) { g_fail_in = n; }
+void standin_host_allocs(long n) { g_host_left = n; }
 
 /* bytes from p to the end of its block, -1 if it is in none */
 int64_t standin_room(uint64_t p) {
@@ -52,6 +55,8 @@ int hipMalloc(void** out, size_t n) {
 }
 int hipHostMalloc(void** out, size_t n, unsigned flags) {
   (void)flags;
+  if (g_host_left == 0) return 2;
+  if (g_host_left > 0) g_host_left--;
   return new_block(out, n);
 }
 int hipFree(void* p) {
@@ -198,15 +203,18 @@ static void read_out(void** a) {
     const uint32_t* src[3];
     uint32_t n_seg, n_words4, n_words16;
   }* g = a[0];
+  const struct {
+    uint32_t *stage[2], *flags[2], ticket;
+  }* parts = a[3];
   const uint64_t w0 = *(uint64_t*)a[1];
-  const uint32_t n = *(uint32_t*)a[2], ticket = *(uint32_t*)a[6], chunk = 16384;
-  uint32_t *stage = *(uint32_t**)a[3], *flags = *(uint32_t**)a[5];
+  const uint32_t n = *(uint32_t*)a[2], chunk = 4096, part = 15 * chunk;
   for (uint32_t i = 0; i < n; i++)
     for (uint32_t k = 0; k < 4; k++) {
       const uint64_t e = 4 * ((w0 + i) % g->n_words16) + k;
-      stage[4ull * i + k] = e < g->n_words4 ? g->src[(w0 + i) / g->n_words16][e] : 0;
+      parts->stage[i / part][4 * (i % part) + k] = e < g->n_words4 ? g->src[(w0 + i) / g->n_words16][e] : 0;
     }
-  for (uint32_t c = 0; c * chunk < n; c++) __atomic_store_n(&flags[c], ticket, __ATOMIC_RELEASE);
+  for (uint32_t i = 0; i < n; i += chunk)
+    __atomic_store_n(&parts->flags[i / part][i % part / chunk], parts->ticket + i / part, __ATOMIC_RELEASE);
 }
 
 int hipLaunchKernel(const void* f, Dim3 grid, Dim3 block, void** args, size_t lds, void* stream) {

@@ -1,5 +1,6 @@
 """The library's host code without a device, on a stand-in for the HIP runtime (standin_hip.c): what it hands to
-the kernels after an allocation failed, and large canvas reads whose helper threads are late."""
+the kernels after an allocation failed, and large canvas reads whose helper threads are late or whose staging cannot
+be allocated."""
 import os
 import subprocess
 import sys
@@ -14,7 +15,7 @@ import ctypes as C, sys
 sys.path.insert(0, {root!r})
 S = C.CDLL({so!r}, mode=C.RTLD_GLOBAL)
 S.standin_room.argtypes, S.standin_room.restype = [C.c_uint64], C.c_int64
-S.standin_fail_alloc.argtypes = [C.c_long]
+S.standin_fail_alloc.argtypes = S.standin_host_allocs.argtypes = [C.c_long]
 S.standin_launches.restype = C.c_long
 S.standin_launch_name.argtypes, S.standin_launch_name.restype = [C.c_long], C.c_char_p
 S.standin_launch_arg.argtypes, S.standin_launch_arg.restype = [C.c_long, C.c_int], C.c_uint64
@@ -144,3 +145,46 @@ r.close()
 
 def test_a_late_helper_does_not_fail_a_read(standin):
     run(standin, LATE_HELPER)
+
+
+# Reads of a few megabytes go through the staging from a context's first on, with as much of it as there is; without
+# any, through the runtime's copy.  Smaller ones make it once they would have gained from it.
+STAGING = """
+W, H = 1283, 727
+rng = np.random.default_rng(2)
+for pieces in (0, 1, 2, 3, 4):
+    r = Renderer(0)
+    cv = r.canvas(W, H)
+    p = [C.c_void_p() for _ in range(3)]
+    r._check(r.L.dh_canvas_device_ptrs(r.ctx, cv, *(C.byref(q) for q in p)), "dh_canvas_device_ptrs")
+    S.standin_host_allocs(pieces)
+    for k in range(5):
+        want = [rng.integers(0, 256, 4 * W * H, np.uint8) for _ in p]
+        for q, v in zip(p, want):
+            C.memmove(q.value, v.ctypes.data, v.nbytes)
+        out = [np.zeros(4 * W * H, np.uint8) for _ in p]
+        dst = [None if (k >> i) & 1 else v.ctypes.data for i, v in enumerate(out)]
+        S.standin_launches(1)
+        r._check(r.L.dh_canvas_read(r.ctx, cv, *dst), "dh_canvas_read")
+        n = sum(b"k_read_out" in S.standin_launch_name(i) for i in range(S.standin_launches(0)))
+        assert (n > 0) == (pieces > 0), (pieces, k, n)
+        for d, a, b in zip(dst, out, want):
+            assert d is None or np.array_equal(a, b), (pieces, k)
+    S.standin_host_allocs(-1)
+    r.close()
+for W, H, first in ((480, 360, 3), (361, 363, None)):  # 1.4 MB; just below 1 MB
+    r = Renderer(0)
+    cv = r.canvas(W, H)
+    f, d = np.zeros((H, W, 4), np.uint8), np.zeros((H, W), np.float32)
+    used = []
+    for k in range(6):
+        S.standin_launches(1)
+        r.read_into(cv, f, d)
+        used.append(any(b"k_read_out" in S.standin_launch_name(i) for i in range(S.standin_launches(0))))
+    assert used == [first is not None and k >= first for k in range(6)], used
+    r.close()
+"""
+
+
+def test_reads_with_the_staging_there_is(standin):
+    run(standin, STAGING)
