@@ -934,10 +934,22 @@ __device__ inline void emit_box_pairs(uint2 box, uint32_t i, uint32_t o, uint32_
 // Small single-view frames: at most kSmallBinTris input triangles take one
 // workgroup for the geometry lists (k_geom_small), and with at most
 // kSmallBinTiles tiles one for the binning (k_bin_small): a launch each in
-// place of three and four.  One CU's issue rate sets the limits (frame times,
-// one workgroup -> general kernels): a torus of 2304 triangles on 300 tiles 60
-// -> 67 us, on 1900 74 -> 80, on 2304 90 -> 86, on 3600 117 -> 88; soups of
-// 300 triangles on 1200 tiles 57 -> 64, of 3000 106 -> 78, of 16,000 321 -> 87.
+// place of three and four.
+//
+// The geometry's cost grows with the triangles alone.  Frames, one workgroup ->
+// three launches: soups of 300 triangles 55 -> 58 us, of 900 64 -> 66, of 1200 67 ->
+// 66, of 2500 88 -> 82; tori of 576 48 -> 53, of 2304 61 -> 60, of 3136 64 -> 59, of
+// 6400 74 -> 61; but a frame that no graph replays also saves the host two
+// launches (one of 2312 opaque and 19,600 transparent triangles 174 -> 177).
+//
+// The binning's depends on the wide triangles, which the host does not know.
+// One workgroup -> four launches: compact meshes gain long (tori of 2304
+// triangles on 300, 1200 and 1620 tiles 54 -> 62, 61 -> 67, 67 -> 73; of 6400 58 -> 64,
+// 61 -> 66, 63 -> 68; of 16,384 67 -> 67, 68 -> 67, 68 -> 68), soups, a third of which
+// is wide, lose from 1200 on (of 1800 on 1200 tiles 82 -> 75, of 2500 88 -> 77, of
+// 4000 100 -> 77, of 16,000 209 -> 83).  The limit keeps what a soup below it loses,
+// at most 11 us, near what a mesh above it does, 6.  In tiles, a torus on 1900
+// gains (74 -> 80) and one on 2304 and on 3600 loses (90 -> 86, 117 -> 88).
 constexpr uint32_t kSmallBinTiles = 2048;  // LDS counters and cursors: 16 KB
 constexpr uint32_t kSmallBinTris = 2560;   // LDS count bytes: 2.5 KB
 
@@ -1632,7 +1644,6 @@ __global__ __launch_bounds__(1024) void k_bin_small(const SetupRec* __restrict__
   __syncthreads();
   const uint32_t n = min(status->n_out, cap_tri);
   const uint2* boxes = bin_boxes(const_cast<uint8_t*>(wflag), cap_tri);
-  const DevView& vw = views[0];
   // one pass over the triangles' tiles: f(tile key) for each
   auto each_tile = [&](auto f) {
     for (uint32_t i = (uint32_t)tid; i < n; i += 1024u) {
