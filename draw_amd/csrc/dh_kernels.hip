@@ -1850,13 +1850,24 @@ static_assert(2048u * (kPairCols + 1u) <= kRadixHistEntries, "histogram and digi
 
 // SUBMIT lists hold each tile's triangles in submission order, which the
 // transparent pass blends in: the depth key gives way to the high bits of the
-// id, and k_pair_sort places the few ids that share them by counting.  For at
-// most kPairSubmitTris input triangles: a tile's ids that share a key number
-// at most 1/256 of the frame's triangles (with 256 levels), so counting stays
-// far below the tile's blending.  (A transparent pass of 19,600 triangles on
-// 3600 tiles took 14 launches and some 55 us from its emits to the blend by a
-// stable sort of tile keys, now four and 19.)
-constexpr uint32_t kPairSubmitTris = 65536;
+// id, and k_pair_sort places the ids that share a counter by counting.  (A
+// transparent pass of 19,600 triangles on 3600 tiles took 14 launches and some
+// 55 us from its emits to the blend by a stable sort of tile keys, now four and
+// 19.)  A tile that holds the whole mesh makes that count quadratic, n ids by
+// n / levels each, so at most kPairShare of the input's may share a counter: by
+// 256 segments where these leave levels enough, else by 2048, else by the stable
+// sort.  65,536 triangles in a pane, and all in a few tiles: 1280x720 in 16x16
+// tiles (256 levels) 226 us and 65 ms (256 segments), 238 and 64 (2048), 257 and 60
+// (sorted); 3840x2160 in 16x16 (64 levels, 256 with 2048 segments) 408 us and 73
+// ms, 421 and 67, 442 and 64; in 8x8 (16, 128) 911 us and 100 ms, 927 and 65, 971
+// and 58; 7680x4320 in 8x8 (32 with 2048 segments) 3.18 and 79 ms, 3.27 and 59
+// sorted.
+constexpr uint32_t kPairSubmitTris = 65536, kPairShare = 1024;
+inline bool submit_share(uint32_t n_tri_in, uint32_t n_tiles, uint32_t segments) {
+  const uint32_t nh = (n_tiles + segments - 1u) / segments;  // tiles of a segment
+  const uint32_t levels = std::min(256u, kPairCounters / nh);
+  return levels && n_tri_in <= kPairShare * levels;
+}
 __device__ inline uint32_t submit_shift(uint32_t n) {  // (n - 1) >> shift <= 255
   return n > 256u ? 24u - (uint32_t)__builtin_clz(n - 1u) : 0u;
 }
@@ -2325,7 +2336,9 @@ int enqueue_radix_sort(uint32_t* const keys[2], uint32_t* const vals[2], const u
 PipeArgs enqueue_front(const PipeArgs& a, hipStream_t s) {
   // near-first lists (k_pair_*); a frame of more tiles than their counters
   // take is binned in submission order
-  const bool submit = a.ordered_bins && a.blend_lists && a.n_tri_in <= kPairSubmitTris && a.n_tiles <= kPairMaxTiles;
+  const bool blend_lists = a.ordered_bins && a.blend_lists && a.n_tri_in <= kPairSubmitTris;
+  const bool submit256 = blend_lists && a.n_tiles <= kPairFewTiles && submit_share(a.n_tri_in, a.n_tiles, 256u);
+  const bool submit = submit256 || (blend_lists && submit_share(a.n_tri_in, a.n_tiles, 2048u));
   const bool near = (a.ordered_bins && a.depth_order && a.n_tiles <= kPairMaxTiles) || submit;
   // a small single-view frame is binned by one workgroup (k_bin_small)
   const bool small_bins = near && !submit && a.n_views == 1 && a.n_tiles <= kSmallBinTiles &&
@@ -2388,7 +2401,7 @@ PipeArgs enqueue_front(const PipeArgs& a, hipStream_t s) {
                        wide_list, a.n_tiles, a.cap_pairs, a.vals[0], a.ranges);
   } else if (near) {
     uint2* const pairs = reinterpret_cast<uint2*>(a.keys[0]);  // keys[0] and keys[1] are one buffer
-    const bool few = a.n_tiles <= kPairFewTiles;
+    const bool few = submit ? submit256 : a.n_tiles <= kPairFewTiles;
     const uint32_t dig = few ? 256u : 2048u;
     uint32_t* const totals = a.hist + (size_t)dig * kPairCols;
     const dim3 gp(kPairCols), bp(kPairT);

@@ -1,6 +1,6 @@
 """The library's host code without a device, on a stand-in for the HIP runtime (standin_hip.c): what it hands to
 the kernels after an allocation failed, and large canvas reads whose helper threads are late or whose staging cannot
-be allocated."""
+be allocated, and which lists a transparent pass gets."""
 import os
 import subprocess
 import sys
@@ -188,3 +188,40 @@ for W, H, first in ((480, 360, 3), (361, 363, None)):  # 1.4 MB; just below 1 MB
 
 def test_reads_with_the_staging_there_is(standin):
     run(standin, STAGING)
+
+
+# The submission-ordered lists of a transparent pass rank the ids that share a counter against each other.  However its
+# triangles lie, at most 1024 of the input's may share one; where the counters do not suffice, the radix sort.
+SHARES = """
+from draw_amd.scene import Texture
+def scene(n, W, H):
+    s = workloads.torus_scene(1, W, H)
+    o = workloads.soup_object(n, W, H, 60.0, 0.1, 100.0, 3.0, Texture(alpha=0.5), np.random.default_rng(1))
+    s.objects = [o]
+    return s
+got = {}
+for W, H, tile in ((640, 480, 16), (3840, 2160, 16), (3840, 2160, 8), (7680, 4320, 8), (30000, 30000, 8)):
+    tiles = -(-W // tile) * -(-H // tile)
+    r = Renderer(0, tile, 4 if tile == 16 else 1)
+    for n in (1, 1000, 2000, 16384, 16385, 32768, 32769, 65536, 65537):
+        S.standin_launches(1)
+        r.render_device(scene(n, W, H))
+        names = [S.standin_launch_name(i).decode() for i in range(S.standin_launches(0))]
+        segs = [d for d in (256, 2048) if any(f"k_pair_sortILi{d}ELb1E" in x for x in names)]
+        assert len(segs) <= 1
+        if segs:
+            levels = min(256, 8192 // -(-tiles // segs[0]))
+            assert levels and n <= 1024 * levels, (W, H, tile, n, segs, levels)
+        else:
+            assert any("k_bin_emitILb1E" in x for x in names)
+        got[W, tile, n] = segs[0] if segs else 0
+    r.close()
+assert [got[640, 16, n] for n in (1, 65536, 65537)] == [256, 256, 0]
+assert [got[3840, 16, n] for n in (16385, 65536)] == [256, 256]
+assert [got[3840, 8, n] for n in (16384, 16385, 65536)] == [256, 2048, 2048]
+assert [got[7680, 8, n] for n in (16384, 32768, 32769)] == [2048, 2048, 0]
+"""
+
+
+def test_transparent_lists_by_size(standin):
+    run(standin, SHARES)
