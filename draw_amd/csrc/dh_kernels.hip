@@ -1285,21 +1285,15 @@ __device__ inline uint32_t scan_count(const uint32_t* n_ptr, uint32_t n_const, u
 }
 __device__ inline uint32_t scan_chunk(uint32_t n) { return (((n + kScanG - 1u) / kScanG) + 1023u) & ~1023u; }
 
-// The scans' input: in[i], or in[idx[i]] (a gather fused into the scan).
-__device__ inline uint32_t scan_in(const uint32_t* in, const uint32_t* idx, uint32_t i) {
-  return idx ? in[idx[i]] : in[i];
-}
-
 __global__ __launch_bounds__(256) void k_scan_reduce(const uint32_t* __restrict__ in, const uint32_t* n_ptr,
-                                                     uint32_t n_const, uint32_t cap, uint32_t* __restrict__ partials,
-                                                     const uint32_t* __restrict__ idx) {
+                                                     uint32_t n_const, uint32_t cap, uint32_t* __restrict__ partials) {
   __shared__ uint32_t s_tmp[4];
   const uint32_t n = scan_count(n_ptr, n_const, cap);
   const uint32_t C = scan_chunk(n);
   const uint32_t b0 = blockIdx.x * C;
   const uint32_t b1 = min(b0 + C, n);
   uint32_t s = 0;
-  for (uint32_t i = b0 + threadIdx.x; i < b1; i += 256) s += scan_in(in, idx, i);
+  for (uint32_t i = b0 + threadIdx.x; i < b1; i += 256) s += in[i];
   uint32_t total;
   block_exclusive_scan256(s, s_tmp, &total);
   if (threadIdx.x == 0) partials[blockIdx.x] = total;
@@ -1313,7 +1307,7 @@ __global__ __launch_bounds__(256) void k_scan_apply(const uint32_t* in, uint32_t
                                                     const uint32_t* n_ptr, uint32_t n_const, uint32_t cap,
                                                     const uint32_t* __restrict__ partials, uint32_t* total_out,
                                                     uint32_t cap_check, uint32_t* overflow_word,
-                                                    uint32_t overflow_bit, const uint32_t* __restrict__ idx) {
+                                                    uint32_t overflow_bit) {
   __shared__ uint32_t s_tmp[4];
   const uint32_t n = scan_count(n_ptr, n_const, cap);
   const uint32_t C = scan_chunk(n);
@@ -1337,7 +1331,7 @@ __global__ __launch_bounds__(256) void k_scan_apply(const uint32_t* in, uint32_t
     const uint32_t i0 = tb + threadIdx.x * 4u;
     uint32_t v[4];
 #pragma unroll
-    for (int k = 0; k < 4; k++) v[k] = (i0 + k < b1) ? scan_in(in, idx, i0 + k) : 0u;
+    for (int k = 0; k < 4; k++) v[k] = (i0 + k < b1) ? in[i0 + k] : 0u;
     const uint32_t s4 = v[0] + v[1] + v[2] + v[3];
     uint32_t total;
     uint32_t ex = block_exclusive_scan256(s4, s_tmp, &total) + running;
@@ -1435,19 +1429,19 @@ __global__ __launch_bounds__(1024) void k_scan_segs(ScanSegs segs, uint32_t n) {
   }
 }
 
-// out = exclusive scan of in (or of in[idx[i]] when idx is given).
+// out = exclusive scan of in.
 static void scan_u32(const uint32_t* in, uint32_t* out, const uint32_t* n_ptr, uint32_t n_const, uint32_t cap,
                      uint32_t* partials, uint32_t* total_out, uint32_t cap_check, uint32_t* overflow_word,
-                     uint32_t overflow_bit, hipStream_t s, const uint32_t* idx = nullptr) {
-  if (!n_ptr && n_const <= 4096u && !idx) {
+                     uint32_t overflow_bit, hipStream_t s) {
+  if (!n_ptr && n_const <= 4096u) {
     ScanSegs g{};
     g.s[0] = ScanSeg{in, out, total_out, overflow_word, cap_check, overflow_bit};
     hipLaunchKernelGGL(k_scan_segs, dim3(1), dim3(1024), 0, s, g, n_const);
     return;
   }
-  hipLaunchKernelGGL(k_scan_reduce, dim3(kScanG), dim3(256), 0, s, in, n_ptr, n_const, cap, partials, idx);
+  hipLaunchKernelGGL(k_scan_reduce, dim3(kScanG), dim3(256), 0, s, in, n_ptr, n_const, cap, partials);
   hipLaunchKernelGGL(k_scan_apply, dim3(kScanG), dim3(256), 0, s, in, out, n_ptr, n_const, cap, partials, total_out,
-                     cap_check, overflow_word, overflow_bit, idx);
+                     cap_check, overflow_word, overflow_bit);
 }
 
 // Pass 1 of unordered bins, one thread per clipped triangle: flag wide
@@ -1760,7 +1754,7 @@ __global__ __launch_bounds__(256) void k_radix_hist(const uint32_t* __restrict__
 }
 
 // KEYS_OUT false: only the values are written (a last pass whose sorted keys
-// nobody reads).  vin null: the values are the input positions.  ranges (may be null): [start, end) of each of the first
+// nobody reads).  ranges (may be null): [start, end) of each of the first
 // n_ranges digits in the output, straight from the scanned histogram -- the
 // per-tile lists when this pass sorts by the whole key.
 template <int BITS, bool KEYS_OUT>
@@ -1789,7 +1783,7 @@ __global__ __launch_bounds__(256) void k_radix_scatter(const uint32_t* __restric
     for (int u = 0; u < kRadixU; u++) {
       const uint32_t i = tb + 64u * (uint32_t)u + (uint32_t)lane;
       kk[u] = i < b1 ? kin[i] : 0u;
-      vv[u] = i < b1 ? (vin ? vin[i] : i) : 0u;
+      vv[u] = i < b1 ? vin[i] : 0u;
     }
 #pragma unroll
     for (int u = 0; u < kRadixU; u++) {
@@ -2286,10 +2280,8 @@ void enqueue_mesh_streams(const uint32_t* tri, uint32_t n_tri, const float* pos,
 }
 
 // Stable LSD radix sort of (keys[0], vals[0]) by the low key_bits bits of the
-// keys (vals[0] may be null: the values are then the input positions), *n_ptr
-// items (at most cap): one 8-bit pass when key_bits <= 8, one
-// 11-bit pass when key_bits <= 11, else
-// 8-bit passes.  Returns the index of the buffer pair holding the result.
+// keys, *n_ptr items (at most cap): one 8-bit pass when key_bits <= 8, one
+// 11-bit pass when key_bits <= 11, else 8-bit passes.  Returns the index of the buffer pair holding the result.
 // keys_out false: the sorted keys are not written (the values are).  ranges:
 // when the sort is one pass (key_bits <= 11), [start, end) of each key below
 // n_ranges in the sorted order; not written otherwise.
