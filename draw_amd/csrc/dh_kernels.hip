@@ -685,11 +685,9 @@ __device__ inline uint32_t thread_tiles(const Spans& g, int TS, F f) {
 // are.  A larger one: lanes take its blocks of 8x8 tiles, and the tiles of a
 // block that may hold a covered pixel are tested at once.  f(e, tx, ty) with e
 // numbering the tiles; returns the tile count.  part, parts: a share of the box's
-// blocks (the waves of a workgroup take one each, block by block in turn: 64
-// consecutive blocks a wave left a box of up to 4096 tiles to one wave; two
-// walls of a room over 2040 tiles 42 -> 23 us of binning, the 150k soup at
-// 1237x709 161 -> 148 us a frame, the 1M soup at 1080p 328 -> 318), numbered
-// within the share.
+// blocks, taken in turn by the parts of a workgroup's waves, numbered within the
+// share.  (64 consecutive blocks a wave left a box of up to 4096 tiles to one
+// wave.)
 constexpr int kBoxTiles = 256;
 template <class F>
 __device__ inline uint32_t wave_tiles(const Spans& g, int TS, int part, int parts, F f) {
@@ -750,8 +748,12 @@ __device__ inline WideTri wide_tri(uint32_t id, const SetupRec* __restrict__ set
   return w;
 }
 
-// Triangles of larger boxes that the waves of a block share out.
-constexpr uint32_t kLargeBuf = 64;
+// Triangles of larger boxes that the waves of a block share out: a wave per
+// kShareBlocks of a box's 8x8-tile blocks, the next triangle's on the waves
+// after them.  (2, 4, 8 and 16 blocks a wave, all waves on every box: a room of
+// 20 triangles on 2040 tiles of 32x32 pixels 108, 106, 104, 105, 110 us, of 68 on
+// 2040 of 16x16 77, 74, 73, 75, 81.)
+constexpr uint32_t kLargeBuf = 64, kShareBlocks = 8;
 struct LargeBuf {
   uint32_t n;
   WideTri t[kLargeBuf];
@@ -765,9 +767,8 @@ struct LargeBuf {
 // wave per triangle paid some 2 us of latency for each (k_bin_small of a
 // 2312-triangle frame of 3600 tiles: 105 -> 38 us).  Triangles of larger boxes
 // wait in the block's LDS until every wave is done with the others, and then
-// every wave takes a share of each (150k triangles at 1237x709, 370 of them of
-// such boxes: k_pair_hist 17 -> 15 us, k_pair_scatter 22 -> 21).  Every wave of
-// the block calls it; large.n is 0 before, after a barrier.
+// the waves share them out.  Every wave of the block calls it; large.n is 0
+// before, after a barrier.
 template <int NW, class F>
 __device__ inline void wave_wide_tiles(const uint32_t* __restrict__ list, uint32_t w, uint32_t step, uint32_t n,
                                        const SetupRec* __restrict__ setup, const DevView* __restrict__ views,
@@ -778,6 +779,7 @@ __device__ inline void wave_wide_tiles(const uint32_t* __restrict__ list, uint32
   for (uint64_t w0 = w;; w0 += 64ull * step) {
     WideTri q{};
     bool on;
+    uint32_t part = 0, parts = 0;
     if (w0 < n) {
       const uint64_t at = w0 + (uint64_t)step * (uint32_t)lane;
       on = at < n;
@@ -793,9 +795,22 @@ __device__ inline void wave_wide_tiles(const uint32_t* __restrict__ list, uint32
       }
     } else {
       __syncthreads();
+      const uint32_t n_large = min(large.n, kLargeBuf);
+      if (n_large == 0u) return;
       shared = true;
-      on = (uint32_t)lane < min(large.n, kLargeBuf);
-      if (on) q = large.t[lane];
+      if ((uint32_t)lane < n_large) {
+        q = large.t[lane];
+        const uint32_t nb = (uint32_t)(((q.g.cx1 - q.g.cx0 + 8) >> 3) * ((q.g.cy1 - q.g.cy0 + 8) >> 3));
+        parts = min((nb + kShareBlocks - 1u) / kShareBlocks, (uint32_t)NW);
+      }
+      uint32_t x = parts;  // -> the parts of the triangles up to this one
+#pragma unroll
+      for (int o = 1; o < 64; o <<= 1) {
+        const uint32_t y = __shfl_up(x, o, 64);
+        if (lane >= o) x += y;
+      }
+      part = ((uint32_t)wave + parts - x) % (uint32_t)NW;
+      on = part < parts;
     }
     auto bi = [](auto v, int b) { return (decltype(v))__builtin_amdgcn_readlane((int)v, b); };
     auto bf = [](float v, int b) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), b)); };
@@ -815,7 +830,7 @@ __device__ inline void wave_wide_tiles(const uint32_t* __restrict__ list, uint32
         u.fm[e] = bf(q.g.fm[e], b);
       }
       const uint32_t id = bi(q.id, b), dk = bi(q.dk, b), ntx = bi(q.ntx, b), key0 = bi(q.key0, b);
-      wave_tiles(u, TS, shared ? wave : 0, shared ? NW : 1, [&](uint32_t, int tx, int ty) {
+      wave_tiles(u, TS, (int)bi(part, b), shared ? (int)bi(parts, b) : 1, [&](uint32_t, int tx, int ty) {
         f(key0 + (uint32_t)(ty - u.cy0) * ntx + (uint32_t)(tx - u.cx0), id, dk);
       });
     }
