@@ -511,7 +511,7 @@ __device__ inline void make_setup(const FrameParamsPod& fr, const FV& A, const F
     return ((v1 - 1.0f) + ev) * mv < 0.999f && ((u1 - 1.0f) + eu) * mu < 0.999f * (1.0f + rows * (float)w);
   };
   if ((flags & kFast) && exact && max(max(mat.kd_w, mat.kd_h), max(mat.ka_w, mat.ka_h)) <= (1 << 20) &&
-      in_map(mat.kd_w, mat.kd_h) && in_map(mat.ka_w, mat.ka_h))
+      in_map(mat.kd_w, mat.kd_h) && (mat.ka_one || in_map(mat.ka_w, mat.ka_h)))
     flags |= kUvSafe;
   // Depth lower bound for early rejection.  For a UV-safe triangle (exact
   // edge arithmetic) a covered pixel has alpha + beta + gama >= 1 - 2^-24 with
@@ -947,9 +947,8 @@ __device__ inline void emit_box_pairs(uint2 box, uint32_t i, uint32_t o, uint32_
 
 // ================================================================== geometry
 // Small single-view frames: at most kSmallBinTris input triangles take one
-// workgroup for the geometry lists (k_geom_small), and with at most
-// kSmallBinTiles tiles one for the binning (k_bin_small): a launch each in
-// place of three and four.
+// workgroup for the geometry lists (k_geom_small), and on few tiles one for the
+// binning (k_bin_small, small_bins): a launch each in place of three and four.
 //
 // The geometry's cost grows with the triangles alone.  Frames, one workgroup ->
 // three launches: soups of 300 triangles 55 -> 58 us, of 900 64 -> 66, of 1200 67 ->
@@ -959,14 +958,22 @@ __device__ inline void emit_box_pairs(uint2 box, uint32_t i, uint32_t o, uint32_
 //
 // The binning's depends on the wide triangles, which the host does not know.
 // One workgroup -> four launches: compact meshes gain long (tori of 2304
-// triangles on 300, 1200 and 1620 tiles 54 -> 62, 61 -> 67, 67 -> 73; of 6400 58 -> 64,
-// 61 -> 66, 63 -> 68; of 16,384 67 -> 67, 68 -> 67, 68 -> 68), soups, a third of which
-// is wide, lose from 1200 on (of 1800 on 1200 tiles 82 -> 75, of 2500 88 -> 77, of
-// 4000 100 -> 77, of 16,000 209 -> 83).  The limit keeps what a soup below it loses,
-// at most 11 us, near what a mesh above it does, 6.  In tiles, a torus on 1900
-// gains (74 -> 80) and one on 2304 and on 3600 loses (90 -> 86, 117 -> 88).
-constexpr uint32_t kSmallBinTiles = 2048;  // LDS counters and cursors: 16 KB
-constexpr uint32_t kSmallBinTris = 2560;   // LDS count bytes: 2.5 KB
+// triangles on 300, 1200, 1620 and 2040 tiles 54 -> 62, 60 -> 67, 67 -> 73, 77 -> 78;
+// of 6400 on up to 1620 58 -> 64, 61 -> 66, 63 -> 68; of 16,384 67 -> 67, 68 -> 67, 68
+// -> 68), soups, a third of which is wide, lose from 1200 on (of 1800 on 1200
+// tiles 82 -> 75, of 2500 88 -> 77, of 16,000 209 -> 83), balls of triangles on many
+// tiles (of 2500 on 300, 1200, 1620 and 2040 57 -> 64, 68 -> 72, 82 -> 75, 93 -> 80).
+// kSmallBinTris keeps what a soup below it loses, at most 11 us, near what a
+// mesh above it does, 6.  Beyond kSmallBinTiles what fills the canvas loses (tori
+// of 160, 576 and 2304 on 3600 77 -> 71, 89 -> 75, 112 -> 82) unless it is of a few
+// triangles (none 36 -> 42, one 46 -> 52, a torus of 24 67 -> 68, soups of 10 and 30
+// 55 -> 60, a room of 20 91 -> 90, of 68 90 -> 86).
+constexpr uint32_t kSmallBinTris = 2560;  // LDS count bytes: 2.5 KB
+constexpr uint32_t kSmallBinTiles = 2048;
+constexpr uint32_t kFewBinTris = 32, kFewBinTiles = 4096;  // LDS counters and cursors: 32 KB
+inline bool small_bins(uint32_t n_tri_in, uint32_t n_tiles) {
+  return n_tiles <= kSmallBinTiles ? n_tri_in <= kSmallBinTris : n_tiles <= kFewBinTiles && n_tri_in <= kFewBinTris;
+}
 
 // cnt[t]: clipped-triangle count (bits 0-2, at most 4) | kCntClip when the
 // triangle crosses the near or far plane.
@@ -1643,8 +1650,8 @@ __global__ __launch_bounds__(1024) void k_bin_small(const SetupRec* __restrict__
                                                     const uint32_t* __restrict__ wide_list, uint32_t n_tiles,
                                                     uint32_t cap_pairs, uint32_t* __restrict__ vals,
                                                     uint2* __restrict__ ranges) {
-  __shared__ uint32_t s_cnt[kSmallBinTiles];
-  __shared__ uint32_t s_cur[kSmallBinTiles];
+  __shared__ uint32_t s_cnt[kFewBinTiles];
+  __shared__ uint32_t s_cur[kFewBinTiles];
   __shared__ uint32_t s_w[16];
   __shared__ LargeBuf s_large[2];  // the count pass's, the list pass's
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -2348,8 +2355,7 @@ PipeArgs enqueue_front(const PipeArgs& a, hipStream_t s) {
   const bool submit = submit256 || (blend_lists && submit_share(a.n_tri_in, a.n_tiles, 2048u));
   const bool near = (a.ordered_bins && a.depth_order && a.n_tiles <= kPairMaxTiles) || submit;
   // a small single-view frame is binned by one workgroup (k_bin_small)
-  const bool small_bins = near && !submit && a.n_views == 1 && a.n_tiles <= kSmallBinTiles &&
-                          a.n_tri_in <= kSmallBinTris;
+  const bool one_bin = near && !submit && a.n_views == 1 && small_bins(a.n_tri_in, a.n_tiles);
   if (a.ev[0]) (void)hipEventRecord(a.ev[0], s);
   if (a.tables_src)  // (the transparent pass's were the opaque pass's work)
     hipLaunchKernelGGL(k_frame_begin, dim3(std::min<uint32_t>(cdiv(a.tables_words, 1024), 64u)), dim3(256), 0, s,
@@ -2403,7 +2409,7 @@ PipeArgs enqueue_front(const PipeArgs& a, hipStream_t s) {
   const uint32_t gl = std::min<uint32_t>(cdiv(a.cap_tri, 4096), 1024u);
   const uint32_t gw = std::min<uint32_t>(cdiv(a.cap_tri, 64), 4096u);
   PipeArgs b = a;
-  if (small_bins) {
+  if (one_bin) {
     hipLaunchKernelGGL(k_bin_small, dim3(1), dim3(1024), 0, s, a.setup, a.views, a.status, a.cap_tri, a.TS, wflag,
                        wide_list, a.n_tiles, a.cap_pairs, a.vals[0], a.ranges);
   } else if (near) {

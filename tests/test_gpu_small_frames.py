@@ -32,6 +32,32 @@ def test_limits(renderer, n, slivers):
     assert got[1] == got[2]
 
 
+@pytest.mark.parametrize("n", [0, 1, 31, 32, 33])
+@pytest.mark.parametrize("W,H", [(16384, 8), (16392, 8), (512, 512), (520, 512)])  # 2048, 2049, 4096, 4160 tiles
+def test_few_triangles_on_many_tiles(renderer, n, W, H):
+    s = workloads.soup_scene(17 + n, max(n, 1), W, H, 32, cross_frac=0.3)
+    if n == 0:
+        s.objects = []
+    else:  # half of them across many tiles
+        big = workloads.soup_object((n + 1) // 2, W, H, 60.0, 0.1, 100.0, 3.0, s.objects[0].textures[0],
+                                    np.random.default_rng(n), cross_frac=0.0, median_px=0.2 * W * H, sigma=0.5)
+        s.objects[0].meshes[0].triangles = s.objects[0].meshes[0].triangles[:n // 2]
+        s.objects.append(big)
+    ref = oracle(s)
+    entries = set()
+    renderer.set_tiling(8, 1)
+    try:
+        for mode in (1, 2):
+            renderer.set_bin_order(mode)
+            c, w = renderer.render(s)
+            assert_same(c.frame, c.depth, w, ref, label=f"bin order {mode}")
+            entries.add(renderer.stats()["bin_entries"])
+    finally:
+        renderer.set_bin_order(2)
+        renderer.set_tiling(16, 4)
+    assert len(entries) == 1
+
+
 def _front_slivers(n):
     """sliver_scene's triangles that face the camera, the first n of them."""
     s = workloads.sliver_scene(37, 3 * n, 160, 120)
