@@ -701,8 +701,8 @@ __device__ inline uint32_t thread_tiles(const Spans& g, int TS, F f) {
 // blocks, taken in turn by the parts of a workgroup's waves, numbered within the
 // share.  (64 consecutive blocks a wave left a box of up to 4096 tiles to one
 // wave.)  WHOLE: the tiles of a block that no edge leaves a tile of out are not
-// tested again.  The kernels with a wave per triangle take it (two triangles
-// over 8160 tiles, submission order: 187 -> 174 us a frame); in those that share
+// tested again.  The kernels with a wave per triangle take it (a room of 20
+// triangles on 8160 tiles, submission order: 187 -> 174 us); in those that share
 // the boxes out it cost frames of small boxes 1 us and gave nothing.
 constexpr int kBoxTiles = 256;
 template <bool WHOLE = false, class F>
@@ -1634,7 +1634,6 @@ __global__ __launch_bounds__(256) void k_bin_emit_wide(const SetupRec* __restric
                                                        const uint32_t* __restrict__ tile_start,
                                                        uint32_t* __restrict__ tile_cur, uint32_t cap_pairs,
                                                        uint32_t* __restrict__ keys, uint32_t* __restrict__ vals) {
-  const int lane = threadIdx.x & 63;
   for_each_wide(wide_list, status, [&](uint32_t i) {
     const SetupRec r = setup[i];
     const DevView& vw = views[r.view];
@@ -1870,7 +1869,9 @@ __global__ __launch_bounds__(256) void k_radix_scatter(const uint32_t* __restric
 // (Before: a depth sort of the triangles, a gathered scan, a pair emit and one
 // or two more sort passes with their scans, 13 to 18 launches of 3 to 15 us
 // each.  1M-triangle 1080p frame: 387 -> 358 us; 150k triangles at 1237x709: 208
-// -> 166 us; 500k triangles at 3840x2160: 300 -> 249 us.)
+// -> 166 us; 500k triangles at 3840x2160: 300 -> 249 us.  Hist, scan, scatter and
+// sort take 12, 5, 18 and 13 us of the first, 9, 5, 11 and 7 of the second, 5, 4,
+// 5 and 8 of the third.)
 constexpr int kPairChunks = 256;         // blocks of 1024 threads: one per CU
 constexpr int kPairT = 1024;
 constexpr int kPairU = 4;                // boxes in flight per thread

@@ -306,6 +306,7 @@ __device__ inline uint4 part_word(int sp, const uint4& q0, const uint4& q1, cons
 // -> after): 32-view batch <32, 4> 770 -> 474; 12 mixed requests <16, 1> 432 ->
 // 397; 500k-triangle mesh at 4K 164 -> 146; 5M micro-triangles 155 -> 86; the
 // 1M-triangle 1080p soup, whose lists are long and visits many, 152 -> 151.
+// (340, 297, 151, 64 and 136 with xcd_remap_tiles.)
 template <int TS, int QPW, bool SHADE>
 __global__ __launch_bounds__(64 * (TS / 8) * (TS / 8) / QPW) __attribute__((amdgpu_waves_per_eu(5))) void k_raster(
     const DevView* __restrict__ views, uint32_t n_views, const uint2* __restrict__ ranges,
