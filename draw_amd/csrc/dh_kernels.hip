@@ -2322,10 +2322,11 @@ void enqueue_mesh_streams(const uint32_t* tri, uint32_t n_tri, const float* pos,
 
 // Stable LSD radix sort of (keys[0], vals[0]) by the low key_bits bits of the
 // keys, *n_ptr items (at most cap): one 8-bit pass when key_bits <= 8, one
-// 11-bit pass when key_bits <= 11, else 8-bit passes.  Returns the index of the buffer pair holding the result.
-// keys_out false: the sorted keys are not written (the values are).  ranges:
-// when the sort is one pass (key_bits <= 11), [start, end) of each key below
-// n_ranges in the sorted order; not written otherwise.
+// 11-bit pass when key_bits <= 11, else 8-bit passes.  Returns the index of the
+// buffer pair holding the result.  keys_out false: the sorted keys are not
+// written (the values are).  ranges: when the sort is one pass (key_bits <= 11),
+// [start, end) of each key below n_ranges in the sorted order; not written
+// otherwise.
 int enqueue_radix_sort(uint32_t* const keys[2], uint32_t* const vals[2], const uint32_t* n_ptr, uint32_t cap,
                        int key_bits, uint32_t* hist, uint32_t* partials, hipStream_t s, bool keys_out,
                        uint2* ranges, uint32_t n_ranges) {
